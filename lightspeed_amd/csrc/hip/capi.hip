@@ -409,27 +409,6 @@ void build_pairlist(lsjk_pairlist* pl)
         for (int Lp = 0; Lp <= maxLp; Lp++)
             if (pl->h_row_start[(size_t)r * (maxLp + 1) + Lp + 1] > pl->h_row_start[(size_t)r * (maxLp + 1) + Lp])
                 pl->h_rows[b1->h_L[r]][Lp].push_back(r);
-    // triangle enumerations (a <= b) for the symmetric-mode launches with equal row momenta; the
-    // symmetric mode depends on the list being used on both sides with a symmetric D24, not on the
-    // list itself being symmetric, so every list gets them (for every Lp <= kMaxL)
-    std::vector<int> tri_start[kMaxL + 1][kMaxL + 1][kMaxL + 1];
-    {
-        for (int L = 0; L <= kMaxL; L++)
-            for (int La = 0; La <= kMaxL; La++)
-                for (int Lb = 0; Lb <= kMaxL; Lb++) {
-                    const auto& A = pl->h_rows[L][La];
-                    const auto& B = pl->h_rows[L][Lb];
-                    auto& pre = pl->h_tri_pre[L][La][Lb];
-                    auto& st = tri_start[L][La][Lb];
-                    pre.assign(A.size() + 1, 0);
-                    st.assign(A.size(), 0);
-                    for (size_t i = 0; i < A.size(); i++) {
-                        st[i] = (int)(std::lower_bound(B.begin(), B.end(), A[i]) - B.begin());
-                        pre[i + 1] = pre[i] + (long long)(B.size() - st[i]);
-                    }
-                }
-    }
-
     // uploads
     pl->d_p1 = dev_upload(pl->h_p1);
     pl->d_p2 = dev_upload(pl->h_p2);
@@ -442,7 +421,6 @@ void build_pairlist(lsjk_pairlist* pl)
     pl->d_ebound = dev_upload(eb);
     pl->h_eb = eb;
     pl->h_eprim = eprim;
-    pl->d_eprim = dev_upload(eprim);
     pl->d_ecart = dev_upload(ecart);
     pl->d_eblk = dev_upload(eblk);
     pl->d_keblk = dev_upload(keblk);
@@ -451,10 +429,6 @@ void build_pairlist(lsjk_pairlist* pl)
     for (int L = 0; L <= kMaxL; L++)
         for (int Lp = 0; Lp <= kMaxL; Lp++) {
             pl->d_rows[L][Lp] = dev_upload(pl->h_rows[L][Lp]);
-            for (int Lb = 0; Lb <= kMaxL; Lb++) {
-                    pl->d_tri_pre[L][Lp][Lb] = dev_upload(pl->h_tri_pre[L][Lp][Lb]);
-                    pl->d_tri_start[L][Lp][Lb] = dev_upload(tri_start[L][Lp][Lb]);
-                }
         }
     pl->d_cls_start = dev_upload(pl->cls_start);
     pl->d_cls_L1 = dev_upload(pl->cls_L1);
@@ -493,7 +467,6 @@ void free_pairlist(lsjk_pairlist* pl)
     dev_free(pl->d_hgeom);
     dev_free(pl->d_row_start);
     dev_free(pl->d_ebound);
-    dev_free(pl->d_eprim);
     dev_free(pl->d_ecart);
     dev_free(pl->d_eblk);
     dev_free(pl->d_keblk);
@@ -502,10 +475,6 @@ void free_pairlist(lsjk_pairlist* pl)
     for (int L = 0; L <= lsjk::kMaxL; L++)
         for (int Lp = 0; Lp <= lsjk::kMaxL; Lp++) {
             dev_free(pl->d_rows[L][Lp]);
-            for (int Lb = 0; Lb <= lsjk::kMaxL; Lb++) {
-                dev_free(pl->d_tri_pre[L][Lp][Lb]);
-                dev_free(pl->d_tri_start[L][Lp][Lb]);
-            }
         }
     dev_free(pl->d_piv_row_start);
     dev_free(pl->d_piv_b);
@@ -516,9 +485,10 @@ void free_pairlist(lsjk_pairlist* pl)
     pl->jtasks.clear();
     dev_free(pl->jtasks_sym.d_tasks);
     pl->jtasks_sym = lsjk::JTaskList();
-    for (auto& kv : pl->kunits) dev_free(kv.second.first);
-    pl->kunits.clear();
-    pl->kcost.clear();
+    dev_free(pl->grad.d_g);
+    dev_free(pl->grad.d_b);
+    dev_free(pl->grad.d_prim);
+    pl->grad = lsjk_pairlist::GradPairs();
     for (auto& kv : pl->kunits_g) dev_free(kv.second.first);
     pl->kunits_g.clear();
     pl->kcost_g.clear();
@@ -559,8 +529,6 @@ void drop_caches_for(lsjk_pairlist* pl, unsigned long long uid)
         pl->jtasks.erase(it);
     }
     auto by_uid = [uid](const auto& k) { return k.first == uid; };
-    erase_if_key(pl->kunits, by_uid, true);
-    erase_if_key(pl->kcost, by_uid, false);
     erase_if_key(pl->kunits_g, by_uid, true);
     pl->kunits_gen++;
     erase_if_key(pl->kcost_g, by_uid, false);
@@ -595,78 +563,83 @@ long long j_chunk(long long nket, long long ntile, int L)
     return std::min(c, few);
 }
 
-// K work units of one class.  A unit is (row1, block of kKTile row3s, chunk of at most kKChunk2 of
-// row1's partners); its cost estimate is (chunk partners) x (partners of the block's row3s) from
-// the bound-screened lists alone (D only removes quartets, it never adds).  In the triangle mode
-// row3s below row1 are not counted and units without work are dropped.  Heavy units are
-// dispatched first (so that long units do not finish after the rest of the launch), in an order
-// that keeps each XCD on neighbouring rows (see below).
-std::pair<const lsjk::KUnit*, int> get_kunits(const lsjk_pairlist* pl12c, const lsjk_pairlist* pl34, int L1, int L2,
-                                              int L3, int L4, bool tri, double* cost_out)
+// The exchange gradient's pairs of a symmetric list: each unordered pair once, by class, the shell of
+// higher angular momentum first, sorted by bound (descending) inside a class (see GPair).
+const lsjk_pairlist::GradPairs& get_grad_pairs(lsjk_pairlist* pl)
 {
-    using lsjk::KUnit;
-    lsjk_pairlist* pl12 = const_cast<lsjk_pairlist*>(pl12c);
-    const int cls = ((((L1 * 3 + L2) * 3 + L3) * 3 + L4) << 1) | (tri ? 1 : 0);
-    const auto key = std::make_pair(pl34->uid, cls);
-    auto it = pl12->kunits.find(key);
-    if (it == pl12->kunits.end()) {
-        const auto& rows1 = pl12->h_rows[L1][L2];
-        const auto& rows3 = pl34->h_rows[L3][L4];
-        const int m12 = pl12->kmaxL2 + 1, m34 = pl34->kmaxL2 + 1;
-        std::vector<long long> n4(rows3.size());
-        for (size_t j = 0; j < rows3.size(); j++) {
-            const size_t r3 = (size_t)rows3[j];
-            n4[j] = pl34->h_row_start[r3 * m34 + L4 + 1] - pl34->h_row_start[r3 * m34 + L4];
-        }
-        const int nb3 = (int)((rows3.size() + lsjk::kKTile - 1) / lsjk::kKTile);
-        std::vector<std::pair<long long, KUnit>> v;
-        double total = 0.0;
-        for (size_t i1 = 0; i1 < rows1.size(); i1++) {
-            const size_t r1 = (size_t)rows1[i1];
-            const int n2 = pl12->h_row_start[r1 * m12 + L2 + 1] - pl12->h_row_start[r1 * m12 + L2];
-            for (int ib = 0; ib < nb3; ib++) {
-                long long sum4 = 0;
-                const size_t j0 = (size_t)ib * lsjk::kKTile, j1 = std::min(rows3.size(), j0 + lsjk::kKTile);
-                for (size_t j = j0; j < j1; j++)
-                    if (!tri || rows3[j] >= (int)r1) sum4 += n4[j];
-                if (sum4 == 0) continue;
-                for (int e = 0; e < n2; e += lsjk::kKChunk2) {
-                    const int cnt = std::min(lsjk::kKChunk2, n2 - e);
-                    v.push_back({(long long)cnt * sum4, KUnit{(int)i1, ib, e, cnt}});
-                    total += (double)cnt * (double)sum4;
-                }
-            }
-        }
-        // Dispatch order: coarse cost buckets (powers of two), heaviest bucket first; inside a bucket
-        // the units stay in row order (v is built row-major) and are split into 8 contiguous ranges
-        // that are interleaved, so that with the round-robin workgroup-to-XCD dispatch each XCD (one
-        // L2) works through neighbouring rows of D and K.
-        auto bucket = [](long long c) { return c > 0 ? 63 - __builtin_clzll((unsigned long long)c) : 0; };
-        std::stable_sort(v.begin(), v.end(), [&](const std::pair<long long, KUnit>& a,
-                                                 const std::pair<long long, KUnit>& b) {
-            return bucket(a.first) > bucket(b.first);
-        });
-        std::vector<KUnit> u;
-        u.reserve(v.size());
-        for (size_t s0 = 0; s0 < v.size();) {
-            size_t s1 = s0;
-            while (s1 < v.size() && bucket(v[s1].first) == bucket(v[s0].first)) s1++;
-            const size_t n = s1 - s0, chunk = (n + 7) / 8;
-            for (size_t k = 0; k < chunk; k++)
-                for (size_t x = 0; x < 8; x++) {
-                    const size_t src = s0 + x * chunk + k;
-                    if (x * chunk + k < n) u.push_back(v[src].second);
-                }
-            s0 = s1;
-        }
-        if (u.size() > (size_t)std::numeric_limits<int>::max())
-            throw LsjkError(LSJK_E_UNSUPPORTED, "lsjk: too many exchange work units");
-        KUnit* d = u.empty() ? nullptr : dev_upload(u);
-        it = pl12->kunits.insert({key, {(void*)d, (int)u.size()}}).first;
-        pl12->kcost[key] = total;
+    using namespace lsjk;
+    auto& gd = pl->grad;
+    if (gd.built) return gd;
+    const Basis* b = pl->b1;
+    std::vector<int> order(pl->npair);
+    std::vector<int> cls(pl->npair);
+    for (int k = 0; k < pl->npair; k++) {
+        const int Li = b->h_L[pl->h_p1[k]], Lj = b->h_L[pl->h_p2[k]];
+        order[k] = k;
+        cls[k] = std::max(Li, Lj) * (kMaxL + 1) + std::min(Li, Lj);
+        gd.n[std::max(Li, Lj)][std::min(Li, Lj)]++;
     }
-    if (cost_out) *cost_out = pl12->kcost[key];
-    return {static_cast<const KUnit*>(it->second.first), it->second.second};
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+        return cls[x] != cls[y] ? cls[x] < cls[y] : pl->h_bound[x] > pl->h_bound[y];
+    });
+    int at = 0;
+    for (int L1 = 0; L1 <= kMaxL; L1++)
+        for (int L2 = 0; L2 <= L1; L2++) {
+            gd.start[L1][L2] = at;
+            at += gd.n[L1][L2];
+        }
+    std::vector<double> g((size_t)kGPairDoubles * pl->npair);
+    std::vector<float> bound(pl->npair);
+    std::vector<int2> prim(pl->npair);
+    for (int q = 0; q < pl->npair; q++) {
+        const int k = order[q];
+        int i = pl->h_p1[k], j = pl->h_p2[k];
+        if (b->h_L[i] < b->h_L[j]) std::swap(i, j);
+        const double ei = b->h_e[i], ej = b->h_e[j], p = ei + ej, ip = 1.0 / p;
+        double R2 = 0.0;
+        for (int d = 0; d < 3; d++) {
+            const double dd = b->h_xyz[3 * i + d] - b->h_xyz[3 * j + d];
+            R2 += dd * dd;
+        }
+        double* r = g.data() + (size_t)kGPairDoubles * q;
+        r[0] = p;
+        r[1] = b->h_c[i] * b->h_c[j] * std::exp(-ei * ej * ip * R2) * kKPrefRoot * ip * (i == j ? 0.5 : 1.0);
+        for (int d = 0; d < 3; d++) {
+            const double A = b->h_xyz[3 * i + d], B = b->h_xyz[3 * j + d], P = (ei * A + ej * B) * ip;
+            r[2 + d] = P;
+            r[5 + d] = P - A;
+            r[8 + d] = A - B;
+        }
+        r[11] = 0.5 * ip;
+        r[12] = 2.0 * ei;
+        r[13] = 2.0 * ej;
+        const int ids[4] = {b->h_cart[i], b->h_cart[j], b->h_blk[i], b->h_blk[j]};
+        std::memcpy(&r[14], ids, sizeof(ids));
+        bound[q] = pl->h_bound[k];
+        prim[q] = make_int2(i, j);
+    }
+    gd.d_g = dev_upload(g);
+    gd.d_b = dev_upload(bound);
+    gd.d_prim = dev_upload(prim);
+    gd.built = true;
+    return gd;
+}
+
+// How one class pair of the exchange gradient is cut into waves.  chunk: pairs of class 2 one wave
+// walks for its tile of 64 class-1 pairs, for about 8 waves per SIMD.  Classes with all components
+// expanded take at least 8 (staging the Rys table and the six additions per lane stay a small
+// share).  The others cost 0.02-0.2 ms per quartet and wave (36 to 1296 components on up to 5
+// roots): they go down to one pair and, below 2048 waves, cut its (c, d) components into nslice
+// slices as well, each forming the 2-D integrals again (a tenth of the work).
+void grad_split(int L1, int L2, int L3, int L4, int n1, int n2, int* chunk, int* nslice)
+{
+    const long long tiles = (n1 + 63) / 64, steps = tiles * n2;
+    const bool expanded = lsjk::grad_expanded(L1, L2, L3, L4);
+    *chunk = (int)std::max<long long>(expanded ? 8 : 1, (steps + 8191) / 8192);
+    *nslice = 1;
+    const long long waves = tiles * ((n2 + *chunk - 1) / *chunk);
+    if (!expanded && waves < 2048)
+        *nslice = (int)std::min<long long>(lsjk::ncart(L3) * lsjk::ncart(L4), (2047 + waves) / waves);
 }
 
 // Spatial rank of every basis-1 primitive of a list: primitives sorted by the Morton code of
@@ -1847,7 +1820,6 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
                 ka.thredp = thredp;
                 ka.count = S.counting ? 1 : 0;
                 ka.symmetric = symmode ? 1 : 0;
-                ka.tri = tri ? 1 : 0;
                 const lsjk_pairlist* sides[2] = {pl12, pl34};
                 KSide* ks[2] = {&ka.s12, &ka.s34};
                 const int Ls[2] = {L1, L3}, Lps[2] = {L2, L4};
@@ -3148,57 +3120,69 @@ int lsjk_exchange_grad(const lsjk_pairlist* pl, const double* D13_dev, const dou
         Ewald ew;
         check_ewald(nterm, scales, omegas, ew);
         hipStream_t st = S.stream;
-        double* Dsh = nullptr;
+        const auto& gd = get_grad_pairs(const_cast<lsjk_pairlist*>(pl));
+        const size_t nn = (size_t)b->ncart * b->ncart;
+        KGradPrepArgs pa{};
+        double* gp = nullptr;
         Workspace wsp;
-        wsp.add(&Dsh, (size_t)b->nblk * b->nblk);
+        wsp.add(&pa.Dsh, (size_t)b->nblk * b->nblk);
+        wsp.add(&pa.S13, nn);
+        wsp.add(&pa.S24, nn);
+        wsp.add(&pa.A13, nn);
+        wsp.add(&pa.A24, nn);
+        wsp.add(&gp, (size_t)6 * pl->npair);
         wsp.commit();
         launch_fill(S.d_sc, sizeof(CallScalars), st);
-        launch_k_blockmax(D24_dev, b->ncart, b->d_blk_cart, b->d_blk_L, b->nblk, b->d_blk_cart, b->d_blk_L, b->nblk, Dsh,
-                          b->nblk, nullptr, nullptr, 0, S.d_sc, st);
-        if (ew.n > 0) {
-            for (int L1 = 0; L1 <= b->maxL; L1++)
-                for (int L2 = 0; L2 <= b->maxL; L2++)
-                    for (int L3 = 0; L3 <= b->maxL; L3++)
-                        for (int L4 = 0; L4 <= b->maxL; L4++) {
-                            if (pl->h_rows[L1][L2].empty() || pl->h_rows[L3][L4].empty()) continue;
-                            const auto units = get_kunits(pl, pl, L1, L2, L3, L4, false, nullptr);
-                            if (units.second == 0) continue;
-                            KArgs ka{};
-                            ka.rys = S.rys;
-                            ka.ew = ew;
-                            ka.thresp = thresp;
-                            ka.thredp = thresp;
-                            KSide* ks[2] = {&ka.s12, &ka.s34};
-                            const int Ls[2] = {L1, L3}, Lps[2] = {L2, L4};
-                            for (int q = 0; q < 2; q++) {
-                                KSide& s = *ks[q];
-                                s.row_start = pl->d_row_start;
-                                s.maxLp = pl->kmaxL2;
-                                s.eb = pl->d_ebound;
-                                s.ecart = pl->d_ecart;
-                                s.eblk = pl->d_eblk;
-                                s.eg = pl->d_egeom;
-                                s.eg32 = pl->d_egeom32;
-                                s.nent = pl->nent;
-                                s.rows = pl->d_rows[Ls[q]][Lps[q]];
-                                s.nrows = (int)pl->h_rows[Ls[q]][Lps[q]].size();
-                                s.cart = b->d_cart;
+        launch_fill(gp, std::max<size_t>(1, (size_t)6 * pl->npair) * sizeof(double), st);
+        pa.D13 = D13_dev;
+        pa.D24 = D24_dev;
+        pa.n = b->ncart;
+        pa.nblk = b->nblk;
+        pa.blk_cart = b->d_blk_cart;
+        pa.blk_L = b->d_blk_L;
+        pa.flags = S.d_sc->queue;
+        pa.sc = S.d_sc;
+        launch_k_grad_prep(pa, st);
+        // all class pairs (the lane's class x the walked one), heaviest first over the side streams
+        auto pass = [&](const double* X13, const double* X24) {
+            Fanout fo;
+            fo.begin();
+            for (int Lt = 4 * kMaxL; Lt >= 0; Lt--)
+                for (int L1 = 0; L1 <= kMaxL; L1++)
+                    for (int L2 = 0; L2 <= L1; L2++)
+                        for (int L3 = 0; L3 <= kMaxL; L3++)
+                            for (int L4 = 0; L4 <= L3; L4++) {
+                                if (L1 + L2 + L3 + L4 != Lt || gd.n[L1][L2] == 0 || gd.n[L3][L4] == 0) continue;
+                                KGradArgs ka{};
+                                ka.rys = S.rys;
+                                ka.ew = ew;
+                                ka.thresp = thresp;
+                                ka.g1 = gd.d_g + (size_t)kGPairDoubles * gd.start[L1][L2];
+                                ka.g2 = gd.d_g + (size_t)kGPairDoubles * gd.start[L3][L4];
+                                ka.b1 = gd.d_b + gd.start[L1][L2];
+                                ka.b2 = gd.d_b + gd.start[L3][L4];
+                                ka.n1 = gd.n[L1][L2];
+                                ka.n2 = gd.n[L3][L4];
+                                grad_split(L1, L2, L3, L4, ka.n1, ka.n2, &ka.chunk, &ka.nslice);
+                                ka.X13 = X13;
+                                ka.X24 = X24;
+                                ka.ldx = b->ncart;
+                                ka.Dsh = pa.Dsh;
+                                ka.nblk = b->nblk;
+                                ka.gp = gp + (size_t)6 * gd.start[L1][L2];
+                                ka.sc = S.d_sc;
+                                launch_k_grad(L1, L2, L3, L4, ka, fo.pick());
                             }
-                            ka.D = D24_dev;
-                            ka.ldD = b->ncart;
-                            ka.Dsh = Dsh;
-                            ka.ldDsh = b->nblk;
-                            ka.maxb12 = pl->maxbound;
-                            ka.maxb34 = pl->maxbound;
-                            ka.sc = S.d_sc;
-                            ka.D13 = D13_dev;
-                            ka.ldD13 = b->ncart;
-                            ka.G = G_dev;
-                            ka.exp1 = ka.exp2 = ka.exp3 = ka.exp4 = b->d_e;
-                            ka.atom1 = ka.atom2 = ka.atom3 = ka.atom4 = b->d_atom;
-                            ka.eprim12 = ka.eprim34 = pl->d_eprim;
-                            launch_k_quartets(L1, L2, L3, L4, kRouteGrad, ka, units.first, units.second, st);
-                        }
+            fo.end();
+        };
+        if (ew.n > 0) {
+            pass(pa.S13, pa.S24);
+            // the antisymmetric parts contribute only where both densities have one
+            unsigned int anti[2] = {0, 0};
+            HIPCHK(hipMemcpyAsync(anti, pa.flags, sizeof(anti), hipMemcpyDeviceToHost, st));
+            HIPCHK(hipStreamSynchronize(st));
+            if (anti[0] && anti[1]) pass(pa.A13, pa.A24);
+            launch_k_grad_atoms(gp, gd.d_prim, b->d_atom, pl->npair, b->natom, G_dev, st);
         }
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(st));

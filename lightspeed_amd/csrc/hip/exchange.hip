@@ -15,11 +15,9 @@ LSJK_KET_EXTERN(0) LSJK_KET_EXTERN(1) LSJK_KET_EXTERN(2)
 #undef LSJK_KET_EXTERN
 
 template <int L1, int L2>
-void launch_k_grad_l12(int L3, int L4, const KArgs& a, const KUnit* units, int nunits, hipStream_t s);
-#define LSJK_GRAD_EXTERN(X, Y) \
-    extern template void launch_k_grad_l12<X, Y>(int, int, const KArgs&, const KUnit*, int, hipStream_t);
-LSJK_GRAD_EXTERN(0, 0) LSJK_GRAD_EXTERN(0, 1) LSJK_GRAD_EXTERN(0, 2)
-LSJK_GRAD_EXTERN(1, 0) LSJK_GRAD_EXTERN(1, 1) LSJK_GRAD_EXTERN(1, 2)
+void launch_k_grad_l12(int L3, int L4, const KGradArgs& a, hipStream_t s);
+#define LSJK_GRAD_EXTERN(X, Y) extern template void launch_k_grad_l12<X, Y>(int, int, const KGradArgs&, hipStream_t);
+LSJK_GRAD_EXTERN(0, 0) LSJK_GRAD_EXTERN(1, 0) LSJK_GRAD_EXTERN(1, 1)
 LSJK_GRAD_EXTERN(2, 0) LSJK_GRAD_EXTERN(2, 1) LSJK_GRAD_EXTERN(2, 2)
 #undef LSJK_GRAD_EXTERN
 
@@ -113,15 +111,89 @@ void launch_permute(const double* in, int ldi, int nr, int nc, const int* pr, co
                        ldo);
 }
 
-void launch_k_quartets(int L1, int L2, int L3, int L4, int route, const KArgs& a, const KUnit* units, int nunits,
-                       hipStream_t s)
+__global__ __launch_bounds__(256) void k_grad_prep(KGradPrepArgs a)
 {
-    if (nunits <= 0) return;
-    if (route != kRouteGrad) throw std::runtime_error("lsjk: tile kernels serve the gradient route only");
-#define G(X, Y) \
-    if (L1 == X && L2 == Y) return launch_k_grad_l12<X, Y>(L3, L4, a, units, nunits, s);
-    G(0, 0) G(0, 1) G(0, 2) G(1, 0) G(1, 1) G(1, 2) G(2, 0) G(2, 1) G(2, 2)
-#undef G
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (long long)a.nblk * a.nblk) return;
+    const int bi = (int)(t / a.nblk), bj = (int)(t - (long long)bi * a.nblk);
+    const int oi = a.blk_cart[bi], oj = a.blk_cart[bj], ni = ncart(a.blk_L[bi]), nj = ncart(a.blk_L[bj]);
+    double m = 0.0;
+    bool anti13 = false, anti24 = false;
+    for (int i = oi; i < oi + ni; i++)
+        for (int j = oj; j < oj + nj; j++) {
+            const size_t ij = (size_t)i * a.n + j, ji = (size_t)j * a.n + i;
+            const double u = a.D13[ij], v = a.D13[ji], x = a.D24[ij], y = a.D24[ji];
+            a.S13[ij] = 0.5 * (u + v);
+            a.A13[ij] = 0.5 * (u - v);
+            a.S24[ij] = 0.5 * (x + y);
+            a.A24[ij] = 0.5 * (x - y);
+            anti13 = anti13 || u != v;
+            anti24 = anti24 || x != y;
+            m = fmax(m, fmax(fabs(x), fabs(y)));
+        }
+    a.Dsh[t] = m;
+    if (anti13) atomicOr(a.flags, 1u);
+    if (anti24) atomicOr(a.flags + 1, 1u);
+    atomicMax(&a.sc->dmax_bits, (unsigned long long)__double_as_longlong(m));
+}
+
+void launch_k_grad_prep(const KGradPrepArgs& a, hipStream_t s)
+{
+    const long long n = (long long)a.nblk * a.nblk;
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_grad_prep, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
+}
+
+// Atoms are few and pairs many, so each workgroup sums in LDS first (one global atomic per atom and
+// axis) while the atoms fit kGradAtomsLds; above that the additions spread over enough addresses.
+constexpr int kGradAtomsLds = 1024;
+__global__ __launch_bounds__(256) void k_grad_atoms(const double* __restrict__ gp, const int2* __restrict__ prim,
+                                                    const int* __restrict__ atom, int npair, int natom,
+                                                    double* __restrict__ G)
+{
+    extern __shared__ double s_g[];
+    const bool lds = natom <= kGradAtomsLds;
+    if (lds) {
+        for (int i = threadIdx.x; i < 3 * natom; i += blockDim.x) s_g[i] = 0.0;
+        __syncthreads();
+    }
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < npair; i += gridDim.x * blockDim.x) {
+        const int2 pr = prim[i];
+        const int2 at = make_int2(atom[pr.x], atom[pr.y]);
+        for (int d = 0; d < 3; d++) {
+            const double a = gp[(size_t)6 * i + d], b = gp[(size_t)6 * i + 3 + d];
+            if (lds) {
+                atomicAdd(&s_g[3 * at.x + d], a);
+                atomicAdd(&s_g[3 * at.y + d], b);
+            } else {
+                atomic_add(G + 3 * (size_t)at.x + d, a);
+                atomic_add(G + 3 * (size_t)at.y + d, b);
+            }
+        }
+    }
+    if (lds) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < 3 * natom; i += blockDim.x)
+            if (s_g[i] != 0.0) atomic_add(G + i, s_g[i]);
+    }
+}
+
+void launch_k_grad_atoms(const double* gp, const int2* prim, const int* atom, int npair, int natom, double* G,
+                         hipStream_t s)
+{
+    if (npair <= 0) return;
+    const int grid = std::min((npair + 255) / 256, 256);
+    const size_t lds = natom <= kGradAtomsLds ? (size_t)3 * natom * sizeof(double) : 0;
+    hipLaunchKernelGGL(k_grad_atoms, dim3(grid), dim3(256), lds, s, gp, prim, atom, npair, natom, G);
+}
+
+void launch_k_grad(int L1, int L2, int L3, int L4, const KGradArgs& a, hipStream_t s)
+{
+    if (a.n1 <= 0 || a.n2 <= 0) return;
+#define CASE(X, Y) \
+    if (L1 == X && L2 == Y) return launch_k_grad_l12<X, Y>(L3, L4, a, s);
+    CASE(0, 0) CASE(1, 0) CASE(1, 1) CASE(2, 0) CASE(2, 1) CASE(2, 2)
+#undef CASE
 }
 
 void launch_k_ket(int L1, int L2, int L3, int L4, int route, const KArgs& a, const KGroups& kg, const KUnitG* units,

@@ -8,13 +8,10 @@
 //   * pairs (1,2) and (3,4) taken from the K-invert partner lists with b >= thresp/(maxb*D24max)
 //     (KBlock::build21 / build_symmetric, src/cpp/core/kvec.cpp:128-232; exchange.cpp:54-71),
 //   * quartet sieve float(b12*b34) * max|D24 block| >= thresp (exchange.cpp:145-152, 186).
-// The reference loops pivot pairs (2,4) and scatters each quartet's (1,3) block with atomics.  Here
-// one wave owns a tile of outputs (one row-1 primitive x 16 row-3 primitives): its lanes test the
-// (2,4) partner combinations of each output pair, compact the survivors into an LDS queue, evaluate
-// them 64 at a time, and add each quartet's N1 x N3 block to the tile's LDS accumulator, which is
-// flushed to K with one atomic add per element.  With a symmetric D24 and one list on both sides
-// only row1 <= row3 is computed and the transposed block is added as well (K = K^T), the same 2x
-// the reference's D24symm half-sieve (exchange.cpp:138-139, 326-336) obtains.
+// The reference loops pivot pairs (2,4) and scatters each quartet's (1,3) block with atomics; here a
+// wave holds 64 ket pairs and walks one bra row's partners (see k_ket).  With a symmetric D24 and one
+// list on both sides K = K^T halves the work, the same 2x the reference's D24symm half-sieve
+// (exchange.cpp:138-139, 326-336) obtains.
 //
 // Integrals: Rys quadrature with the 2-D integrals built by the vertical recurrence on centres
 // A and C and the horizontal transfer to B and D (Rys, Dupuis & King, J. Comput. Chem. 4, 154
@@ -303,242 +300,6 @@ __device__ __forceinline__ void k_quartet(const RysTable& tab, const void* s_tab
 #pragma unroll
             for (int c = 0; c < N3; c++) acc[a][c] += (double)qacc[a][c];
     }
-}
-
-// Derivatives of one primitive quartet with respect to the centres A, B, C (D by translational
-// invariance, dE/dD = -(dE/dA + dE/dB + dE/dC)), contracted with D13[a][c] D24[b][d]:
-//   d/dA_x (ab|cd) = 2 alpha (a+1x b|cd) - a_x (a-1x b|cd), likewise B (beta), C (gamma),
-// from 2-D Rys integrals with L1, L2, L3 raised by one (reference exchange_grad.cpp).
-template <int L1, int L2, int L3, int L4>
-__device__ __forceinline__ void k_quartet_grad(const RysTable& tab, const Ewald& ew, const KEnt<double>& e12,
-                                               const KEnt<double>& e34, double alpha, double beta, double gamma,
-                                               const double (&D13)[ncart(L1)][ncart(L3)],
-                                               const double (&D24)[ncart(L2)][ncart(L4)], double (&gA)[3],
-                                               double (&gB)[3], double (&gC)[3])
-{
-    constexpr int N1 = ncart(L1), N2 = ncart(L2), N3 = ncart(L3), N4 = ncart(L4);
-    constexpr int NR = (L1 + L2 + L3 + L4 + 1) / 2 + 1;
-    const double p = e12.p, q = e34.p;
-    const double pq = p + q;
-    const double rpq = rsqrt_pos(pq);
-    const double ipq = rpq * rpq;
-    const double rho = p * q * ipq;
-    const double PQx = e12.Px - e34.Px, PQy = e12.Py - e34.Py, PQz = e12.Pz - e34.Pz;
-    const double r2 = PQx * PQx + PQy * PQy + PQz * PQz;
-    const double base = e12.K * e34.K * rpq;  // 2 pi^(5/2) K_AB K_CD / (p q sqrt(p + q))
-    const double qf = q * ipq, pf = p * ipq;
-    const double i2p = e12.i2p, i2q = e34.i2p;
-    for (int it = 0; it < ew.n; it++) {
-        const double om = ew.omega[it];
-        double d2 = 1.0;
-        double pref = ew.alpha[it] * base;
-        if (__double_as_longlong(om) != __double_as_longlong(-1.0)) {  // erf-attenuated term (bit test: scalar)
-            d2 = om * om / (rho + om * om);
-            pref *= sqrt(d2);
-        }
-        double x[NR], w[NR];
-        rys_roots<NR>(tab, rho * d2 * r2, x, w);
-        // roots one after another (not unrolled): keeps the derivative kernels' code size and
-        // compile time bounded
-#pragma unroll 1
-        for (int i = 0; i < NR; i++) {
-            const double u = x[i] * d2;
-            const double B00 = 0.5 * u * ipq;
-            const double B10 = i2p * (1.0 - u * qf);
-            const double B01 = i2q * (1.0 - u * pf);
-            const double cq = u * qf, cp = u * pf;
-            Axis4<double, L1 + 1, L2 + 1, L3 + 1, L4> I[3];
-            rys_axis<double, L1 + 1, L2 + 1, L3 + 1, L4>(pref * w[i], e12.PAx - cq * PQx, e34.PAx + cp * PQx, B10, B01,
-                                                         B00, e12.ABx, e34.ABx, I[0]);
-            rys_axis<double, L1 + 1, L2 + 1, L3 + 1, L4>(1.0, e12.PAy - cq * PQy, e34.PAy + cp * PQy, B10, B01, B00,
-                                                         e12.ABy, e34.ABy, I[1]);
-            rys_axis<double, L1 + 1, L2 + 1, L3 + 1, L4>(1.0, e12.PAz - cq * PQz, e34.PAz + cp * PQz, B10, B01, B00,
-                                                         e12.ABz, e34.ABz, I[2]);
-            // (a, c) run as ordinary loops (the 2-D integrals are then indexed at run time), the
-            // partner components (b, d) and the three axes are expanded at compile time
-#pragma unroll 1
-            for (int a = 0; a < N1; a++) {
-                int an[3];
-                for (int k = 0; k < 3; k++) an[k] = cart_lk(L1, a, k);
-#pragma unroll 1
-                for (int c = 0; c < N3; c++) {
-                    int cn[3];
-                    for (int k = 0; k < 3; k++) cn[k] = cart_lk(L3, c, k);
-                    const double d13 = D13[a][c];
-                    if (d13 == 0.0) continue;
-                    static_for<N2>([&](auto B_) {
-                        constexpr int b = decltype(B_)::value;
-                        static_for<N4>([&](auto D_) {
-                            constexpr int d = decltype(D_)::value;
-                            const double wgt = d13 * D24[b][d];
-                            double base3[3], dA[3], dB[3], dC[3];
-                            static_for<3>([&](auto K_) {
-                                constexpr int k = decltype(K_)::value;
-                                constexpr int ib = cart_lk(L2, b, k), id = cart_lk(L4, d, k);
-                                const int ia = an[k], ic = cn[k];
-                                const auto& V = I[k].v;
-                                base3[k] = V[ia][ib][ic][id];
-                                double va = 2.0 * alpha * V[ia + 1][ib][ic][id];
-                                if (ia > 0) va -= ia * V[ia - 1][ib][ic][id];
-                                double vb = 2.0 * beta * V[ia][ib + 1][ic][id];
-                                if constexpr (ib > 0) vb -= ib * V[ia][ib - 1][ic][id];
-                                double vc = 2.0 * gamma * V[ia][ib][ic + 1][id];
-                                if (ic > 0) vc -= ic * V[ia][ib][ic - 1][id];
-                                dA[k] = va;
-                                dB[k] = vb;
-                                dC[k] = vc;
-                            });
-                            gA[0] += wgt * dA[0] * base3[1] * base3[2];
-                            gA[1] += wgt * base3[0] * dA[1] * base3[2];
-                            gA[2] += wgt * base3[0] * base3[1] * dA[2];
-                            gB[0] += wgt * dB[0] * base3[1] * base3[2];
-                            gB[1] += wgt * base3[0] * dB[1] * base3[2];
-                            gB[2] += wgt * base3[0] * base3[1] * dB[2];
-                            gC[0] += wgt * dC[0] * base3[1] * base3[2];
-                            gC[1] += wgt * base3[0] * dC[1] * base3[2];
-                            gC[2] += wgt * base3[0] * base3[1] * dC[2];
-                        });
-                    });
-                }
-            }
-        }
-    }
-}
-
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
-constexpr int kKQueue = 128;
-
-// Exchange gradient.  One wave per tile = (row1, block of kKTile row3s) of a class (L1 L2 | L3 L4).
-// For each (row1, row3) of the tile the lanes test the sieve over the candidate rectangle
-// (partners that can pass with the global D maximum), compact the passing (2,4) combinations into
-// an LDS queue shared by all pairs of the tile, and evaluate the quartets 64 at a time; each
-// quartet's derivative contributions go to the four atoms' gradients with atomics.
-template <int L1, int L2, int L3, int L4>
-__global__ __launch_bounds__(64) void k_tiles_grad(KArgs a, const KUnit* __restrict__ units)
-{
-    __shared__ int s_e2[kKQueue], s_e4[kKQueue], s_t[kKQueue];
-    const int lane = threadIdx.x;
-    const KUnit unit = units[blockIdx.x];
-    const int r1 = a.s12.rows[unit.i1];
-    const int j3a = unit.ib * kKTile;
-    const int j3b = min(j3a + kKTile, a.s34.nrows);
-
-    const float thresp = a.thresp;
-    const double dmax = __longlong_as_double((long long)a.sc->dmax_bits);
-    const float thre12 = (float)((double)thresp / ((double)a.maxb34 * dmax));
-    const float thre34 = (float)((double)thresp / ((double)a.maxb12 * dmax));
-    // this unit's chunk of row1's partners (bound order, so the surviving ones are a prefix)
-    const int a0 = a.s12.row_start[r1 * (a.s12.maxLp + 1) + L2] + unit.e2off;
-    const int a1 = a0 + unit.e2cnt;
-    const float b12top = a.s12.eb[a0];
-    // partners of row1 that can pass with the largest possible ket bound are a prefix
-    int n2max = 0;
-    for (int k = lane; k < a1 - a0; k += 64) n2max += (a.s12.eb[a0 + k] >= thre12) ? 1 : 0;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) n2max += __shfl_xor(n2max, o);
-
-    int qn = 0;  // queue length (wave-uniform)
-    // inlined at both call sites: an outlined copy would take the address of the kernel arguments
-    auto evaluate = [&](int slot) __attribute__((always_inline)) {
-        constexpr int N1 = ncart(L1), N2 = ncart(L2), N3 = ncart(L3), N4 = ncart(L4);
-        const int e2 = s_e2[slot], e4 = s_e4[slot], tt = s_t[slot];
-        const KEnt<double> E12 = load_ent(a.s12.eg, e2), E34 = load_ent(a.s34.eg, e4);
-        double Db[N2][N4];
-#pragma unroll
-        for (int b = 0; b < N2; b++)
-#pragma unroll
-            for (int d = 0; d < N4; d++) Db[b][d] = a.D[(size_t)(E12.cart + b) * a.ldD + (E34.cart + d)];
-        const int r3 = a.s34.rows[j3a + tt];
-        const int p2 = a.eprim12[e2], p4 = a.eprim34[e4];
-        const int o1 = a.s12.cart[r1], o3 = a.s34.cart[r3];
-        double D13[N1][N3];
-#pragma unroll
-        for (int i = 0; i < N1; i++)
-#pragma unroll
-            for (int j = 0; j < N3; j++) D13[i][j] = a.D13[(size_t)(o1 + i) * a.ldD13 + (o3 + j)];
-        double gA[3] = {0.0, 0.0, 0.0}, gB[3] = {0.0, 0.0, 0.0}, gC[3] = {0.0, 0.0, 0.0};
-        k_quartet_grad<L1, L2, L3, L4>(a.rys, a.ew, E12, E34, a.exp1[r1], a.exp2[p2], a.exp3[r3], D13, Db, gA, gB, gC);
-        const int at1 = a.atom1[r1], at2 = a.atom2[p2], at3 = a.atom3[r3], at4 = a.atom4[p4];
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            atomic_add(a.G + 3 * at1 + k, gA[k]);
-            atomic_add(a.G + 3 * at2 + k, gB[k]);
-            atomic_add(a.G + 3 * at3 + k, gC[k]);
-            atomic_add(a.G + 3 * at4 + k, -(gA[k] + gB[k] + gC[k]));
-        }
-    };
-
-    for (int t = j3a; t < j3b && n2max > 0; t++) {
-        const int r3 = a.s34.rows[t];
-        const int c0 = a.s34.row_start[r3 * (a.s34.maxLp + 1) + L4];
-        const int c1 = a.s34.row_start[r3 * (a.s34.maxLp + 1) + L4 + 1];
-        const float b34top = a.s34.eb[c0];
-        if (!(b34top >= thre34)) continue;
-        int n2 = 0, n4 = 0;
-        for (int k = lane; k < n2max; k += 64)
-            n2 += ((double)(a.s12.eb[a0 + k] * b34top) * dmax >= (double)thresp) ? 1 : 0;
-        for (int k = lane; k < c1 - c0; k += 64) {
-            const float b = a.s34.eb[c0 + k];
-            n4 += (b >= thre34 && (double)(b12top * b) * dmax >= (double)thresp) ? 1 : 0;
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            n2 += __shfl_xor(n2, o);
-            n4 += __shfl_xor(n4, o);
-        }
-        const int ntot = n2 * n4;
-        for (int base = 0; base < ntot; base += 64) {
-            const int f = base + lane;
-            bool pass = false;
-            int e2 = 0, e4 = 0;
-            if (f < ntot) {
-                const int j2 = f / n4;
-                e2 = a0 + j2;
-                e4 = c0 + (f - j2 * n4);
-                const float b12 = a.s12.eb[e2], b34 = a.s34.eb[e4];
-                if (b12 >= thre12 && b34 >= thre34) {
-                    const double dblk = a.Dsh[(size_t)a.s12.eblk[e2] * a.ldDsh + a.s34.eblk[e4]];
-                    const double est = (double)(b12 * b34) * dblk;
-                    pass = est >= (double)thresp;
-                }
-            }
-            const unsigned long long m = __ballot(pass);
-            if (pass) {
-                const int pos = qn + __popcll(m & ((1ull << lane) - 1ull));
-                s_e2[pos] = e2;
-                s_e4[pos] = e4;
-                s_t[pos] = t - j3a;
-            }
-            qn += __popcll(m);
-            if (qn >= 64) {
-                __syncthreads();
-                evaluate(lane);
-                __syncthreads();
-                const int rest = qn - 64;
-                int m2 = 0, m4 = 0, mt = 0;
-                if (lane < rest) {
-                    m2 = s_e2[64 + lane];
-                    m4 = s_e4[64 + lane];
-                    mt = s_t[64 + lane];
-                }
-                __syncthreads();
-                if (lane < rest) {
-                    s_e2[lane] = m2;
-                    s_e4[lane] = m4;
-                    s_t[lane] = mt;
-                }
-                qn = rest;
-            }
-        }
-    }
-    __syncthreads();
-    if (lane < qn) evaluate(lane);
 }
 
 // One packed FP64 entry at a wave-uniform index, through scalar loads (K view ids).
@@ -969,20 +730,6 @@ void launch_k_ket_l1(int L2, int L3, int L4, int route, const KArgs& a, const KG
 #undef C4
 #undef CASE
 #undef ONE
-}
-
-// Launch of one exchange-gradient class (instantiated per (L1, L2) in exchange_grad_<L1><L2>.hip).
-template <int L1, int L2>
-void launch_k_grad_l12(int L3, int L4, const KArgs& a, const KUnit* units, int nunits, hipStream_t s)
-{
-    dim3 grid((unsigned)nunits), block(64);
-#define CASE(C, D)                                                                                  \
-    if (L3 == C && L4 == D) {                                                                       \
-        hipLaunchKernelGGL((k_tiles_grad<L1, L2, C, D>), grid, block, 0, s, a, units);             \
-        return;                                                                                     \
-    }
-    CASE(0, 0) CASE(0, 1) CASE(0, 2) CASE(1, 0) CASE(1, 1) CASE(1, 2) CASE(2, 0) CASE(2, 1) CASE(2, 2)
-#undef CASE
 }
 
 }  // namespace lsjk

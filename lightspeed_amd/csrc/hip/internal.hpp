@@ -88,7 +88,6 @@ struct PairList {
     int* d_row_start = nullptr;
     int nent = 0;
     float* d_ebound = nullptr;
-    int* d_eprim = nullptr;   // partner primitive
     int* d_ecart = nullptr;   // partner Cartesian offset
     int* d_eblk = nullptr;    // partner block id
     int* d_keblk = nullptr;   // partner block id in the K view order (Basis::h_kblk)
@@ -105,11 +104,6 @@ struct PairList {
     // rows with at least one partner of angular momentum Lp, per (row L, Lp), in primitive order
     std::vector<int> h_rows[kMaxL + 1][kMaxL + 1];
     int* d_rows[kMaxL + 1][kMaxL + 1] = {};
-    // triangle enumeration for a symmetric list: units (a in rows[L][La], b in rows[L][Lb], a <= b);
-    // tri_start[i] = first index into rows[L][Lb] with b >= a_i, tri_pre[i] = units before row i
-    std::vector<long long> h_tri_pre[kMaxL + 1][kMaxL + 1][kMaxL + 1];
-    long long* d_tri_pre[kMaxL + 1][kMaxL + 1][kMaxL + 1] = {};
-    int* d_tri_start[kMaxL + 1][kMaxL + 1][kMaxL + 1] = {};
     // batch list (lsjk_batch_create): pairs of one molecule only; nmol molecules, h_mol[p] the
     // molecule of basis-1 primitive p; in each Hermite group the molecules' pairs are contiguous,
     // molecule m at [h_hmol[L][m], h_hmol[L][m + 1]), each sorted by bound.  Quartets are formed
@@ -143,10 +137,16 @@ struct PairList {
     std::map<unsigned long long, JTaskList> jtasks;
     // the symmetric J kernel's task list (this list on both sides), built with the list
     JTaskList jtasks_sym;
-    // cached K gradient unit lists (device pointer, count) keyed by (ket list uid, class, triangle flag)
-    std::map<std::pair<unsigned long long, int>, std::pair<void*, int>> kunits;
-    // cost of the class's units (sum over units of partner-count products), same key
-    std::map<std::pair<unsigned long long, int>, double> kcost;
+    // exchange gradient: the list's pairs by class (L1 >= L2, the shell of higher angular momentum
+    // first), bound order; built on first use (get_grad_pairs)
+    struct GradPairs {
+        bool built = false;
+        int start[kMaxL + 1][kMaxL + 2] = {{0}};  // class (L1, L2): pairs [start, start + n)
+        int n[kMaxL + 1][kMaxL + 1] = {{0}};
+        double* d_g = nullptr;   // kGPairDoubles doubles each
+        float* d_b = nullptr;    // bounds
+        int2* d_prim = nullptr;  // {primitive A, primitive B}
+    } grad;
     // host copies of the entry bounds and partner primitives (K view order)
     std::vector<float> h_eb;
     std::vector<int> h_eprim;

@@ -16,7 +16,6 @@ __host__ __device__ constexpr int kcount_index(int L1, int L2, int L3, int L4)
 constexpr int kRoutePlain = 0;  // est >= thresp, FP64 (thredp <= thresp)
 constexpr int kRouteHi = 1;     // est >= thredp, FP64
 constexpr int kRouteLo = 2;     // thresp <= est < thredp, FP32 arithmetic, FP64 accumulation
-constexpr int kRouteGrad = 3;   // exchange gradient: est >= thresp, FP64 derivative integrals
 constexpr int kRouteMixed = 4;  // K build: est >= thredp in FP64 and thresp <= est < thredp in FP32, one launch
 
 struct JPrepArgs {
@@ -134,16 +133,46 @@ struct OneEArgs {
 void launch_one_e_st(int LA, int LB, const OneEArgs& a, int k0, int nk, hipStream_t s);
 void launch_one_e_v(int LA, int LB, const OneEArgs& a, int k0, int nk, int hstart, size_t hoff, hipStream_t s);
 
-// K gradient: one wave per tile = (row1, kKTile consecutive row3s) of fixed angular momenta.
-constexpr int kKTile = 16;
-// Row-1 partners per gradient work unit: a tile's partner range is split into chunks of this size
-// so that no unit is much heavier than the rest.
-constexpr int kKChunk2 = 64;
-// A K gradient work unit: row1 = rows1[i1], row3 block ib (rows3[ib*kKTile ...]), row1's partners
-// [e2off, e2off + e2cnt) of the class's partner angular momentum.
-struct KUnit {
-    int i1, ib, e2off, e2cnt;
+// Exchange gradient (exchange_grad_impl.hpp): the lanes' pairs (class 1, n1 of them) against chunks
+// of `chunk` pairs of class 2; records of kGPairDoubles doubles and bounds, both in bound order.
+constexpr int kGPairDoubles = 16;
+struct KGradArgs {
+    RysTable rys;
+    Ewald ew;
+    float thresp;
+    const double *g1, *g2;
+    const float *b1, *b2;
+    int n1, n2, chunk, nslice;
+    const double *X13, *X24;  // both symmetric or both antisymmetric, ncart x ncart
+    int ldx;
+    const double* Dsh;  // block maxima of |D24|, the larger of the two triangles', nblk x nblk
+    int nblk;
+    double* gp;  // the class-1 pairs' sums, 6 doubles each (dE/dA, dE/dB)
+    CallScalars* sc;
 };
+void launch_k_grad(int L1, int L2, int L3, int L4, const KGradArgs& a, hipStream_t s);
+// Classes whose components are all expanded at compile time: up to (pp|pp).  Above that the (c, d)
+// components run as a loop (the 2-D integrals are indexed at run time there, the a and b components
+// stay expanded), which bounds the code: (dd|dd) has 1296 components.
+constexpr bool grad_expanded(int L1, int L2, int L3, int L4)
+{
+    return ncart(L1) * ncart(L2) * ncart(L3) * ncart(L4) <= 81;
+}
+// Per block pair: the symmetric and antisymmetric parts of D13 and D24, the block maxima of D24
+// (the larger of the two triangles'), max|D24|, and flags[0], flags[1] = whether D13, D24 have an
+// antisymmetric part.
+struct KGradPrepArgs {
+    const double *D13, *D24;
+    int n, nblk;
+    const int *blk_cart, *blk_L;
+    double *S13, *S24, *A13, *A24, *Dsh;
+    unsigned int* flags;
+    CallScalars* sc;
+};
+void launch_k_grad_prep(const KGradPrepArgs& a, hipStream_t s);
+// G[atom] += the pairs' sums (gp: 6 doubles each; prim: {primitive A, primitive B}; atom: of a primitive).
+void launch_k_grad_atoms(const double* gp, const int2* prim, const int* atom, int npair, int natom, double* G,
+                         hipStream_t s);
 
 // K build: ket groups.  The rows of one (row L, partner L) class of the ket list are put in
 // spatial (Morton) order and cut into groups of kgroup_size(L, Lp) consecutive rows; the partner
@@ -208,9 +237,6 @@ struct KArgs {
     int symmetric;  // compute only row1 <= row3 and add the transposed block
     int mirror_diag;  // symmetric mode, a class evaluated for its mirror class as well: the
                       // transposed block is added on the diagonal (row1 == row3) too
-    int tri;        // units are the (row1 <= row3) pairs given by tri_pre / tri_start
-    const long long* tri_pre;
-    const int* tri_start;
     KSide s12, s34;
     const double* D;     // D24, ncart2 x ncart4
     int ldD;
@@ -224,13 +250,6 @@ struct KArgs {
     const float* tau;
     float tau_smin;
     CallScalars* sc;
-    // exchange gradient (kRouteGrad): G (natom x 3) += d/dR sum D13_ac D24_bd (ab|cd)
-    const double* D13;
-    int ldD13;
-    double* G;
-    const double *exp1, *exp2, *exp3, *exp4;  // primitive exponents of the four bases
-    const int *atom1, *atom2, *atom3, *atom4; // primitive atoms
-    const int *eprim12, *eprim34;             // partner primitive of each entry
 };
 
 struct CountJArgs {
@@ -313,9 +332,6 @@ void launch_permute(const double* in, int ldi, int nr, int nc, const int* pr, co
 void launch_k_blockmax(const double* D, int ldD, const int* blk_cart2, const int* blk_L2, int nblk2,
                        const int* blk_cart4, const int* blk_L4, int nblk4, double* Dsh, int ldDsh, const int* blk_lo,
                        const int* blk_hi, int band, CallScalars* sc, hipStream_t s);
-// Exchange gradient classes (route kRouteGrad) over KUnit tiles.
-void launch_k_quartets(int L1, int L2, int L3, int L4, int route, const KArgs& a, const KUnit* units, int nunits,
-                       hipStream_t s);
 // Learned-screen training data: per K unit, the largest M_q / (b12 b34) over its quartets with
 // b12 b34 >= smin (classes with s and p functions only).
 void launch_k_unit_mag_sp(int L1, int L2, int L3, int L4, const KArgs& a, const KGroups& kg, const KUnitG* units,
