@@ -242,6 +242,32 @@ void check_ewald(int nterm, const double* scales, const double* omegas, lsjk::Ew
 
 // ------------------------------------------------------------------ pair-list layouts
 
+// The packed K entry of row primitive r of b1 and partner primitive s of b2 (kKEntDoubles, see KEnt).
+void kent_record(const lsjk::Basis* b1, int r, const lsjk::Basis* b2, int s, double* g)
+{
+    const double er = b1->h_e[r], es = b2->h_e[s], p = er + es, ip = 1.0 / p;
+    double R2 = 0.0;
+    for (int d = 0; d < 3; d++) {
+        const double dd = b1->h_xyz[3 * r + d] - b2->h_xyz[3 * s + d];
+        R2 += dd * dd;
+    }
+    g[0] = p;
+    // K_AB sqrt(2 pi^(5/2)) / p: the product of the two sides' values times (p + q)^(-1/2) is the
+    // quartet prefactor 2 pi^(5/2) K_AB K_CD / (p q sqrt(p + q))
+    g[1] = b1->h_c[r] * b2->h_c[s] * std::exp(-er * es * ip * R2) * lsjk::kKPrefRoot * ip;
+    for (int d = 0; d < 3; d++) {
+        const double A = b1->h_xyz[3 * r + d], B = b2->h_xyz[3 * s + d];
+        const double P = (er * A + es * B) * ip;
+        g[2 + d] = P;
+        g[5 + d] = P - A;
+        g[8 + d] = A - B;
+    }
+    const int ids[2] = {b2->h_cart[s], b2->h_blk[s]}, kids[2] = {b2->h_kcart[ids[0]], b2->h_kblk[ids[1]]};
+    std::memcpy(&g[11], ids, sizeof(ids));
+    g[12] = 0.5 * ip;
+    std::memcpy(&g[13], kids, sizeof(kids));
+}
+
 void build_pairlist(lsjk_pairlist* pl)
 {
     using namespace lsjk;
@@ -363,35 +389,15 @@ void build_pairlist(lsjk_pairlist* pl)
     std::vector<double> eg32((size_t)kKEnt32Doubles * (size_t)std::max(ne, 1), 0.0);
     for (int q = 0; q < ne; q++) {
         const Ent& e = ents[q];
-        int r = e.row, s = e.part;
-        double er = b1->h_e[r], es = b2->h_e[s], p = er + es, ip = 1.0 / p;
-        double R2 = 0.0;
-        for (int d = 0; d < 3; d++) {
-            double dd = b1->h_xyz[3 * r + d] - b2->h_xyz[3 * s + d];
-            R2 += dd * dd;
-        }
+        const int r = e.row, s = e.part;
         eb[q] = e.b;
         eprim[q] = s;
         ecart[q] = b2->h_cart[s];
         eblk[q] = b2->h_blk[s];
-        double* g = eg.data() + (size_t)kKEntDoubles * q;
-        g[0] = p;
-        // K_AB sqrt(2 pi^(5/2)) / p: the product of the two sides' values times (p + q)^(-1/2) is the
-        // quartet prefactor 2 pi^(5/2) K_AB K_CD / (p q sqrt(p + q))
-        g[1] = b1->h_c[r] * b2->h_c[s] * std::exp(-er * es * ip * R2) * kKPrefRoot * ip;
-        for (int d = 0; d < 3; d++) {
-            const double A = b1->h_xyz[3 * r + d], B = b2->h_xyz[3 * s + d];
-            const double P = (er * A + es * B) * ip;
-            g[2 + d] = P;
-            g[5 + d] = P - A;
-            g[8 + d] = A - B;
-        }
-        const int ids[2] = {ecart[q], eblk[q]};
-        std::memcpy(&g[11], ids, sizeof(ids));
-        g[12] = 0.5 * ip;
         keblk[q] = b2->h_kblk[eblk[q]];
-        const int kids[2] = {b2->h_kcart[ecart[q]], keblk[q]};
-        std::memcpy(&g[13], kids, sizeof(kids));
+        const int ids[2] = {ecart[q], eblk[q]}, kids[2] = {b2->h_kcart[ecart[q]], keblk[q]};
+        double* g = eg.data() + (size_t)kKEntDoubles * q;
+        kent_record(b1, r, b2, s, g);
         // FP32-route copy: P in FP64, the rest rounded to FP32
         double* h = eg32.data() + (size_t)kKEnt32Doubles * q;
         h[0] = g[2];
@@ -421,9 +427,15 @@ void build_pairlist(lsjk_pairlist* pl)
     pl->d_ebound = dev_upload(eb);
     pl->h_eb = eb;
     pl->h_eprim = eprim;
-    pl->d_ecart = dev_upload(ecart);
-    pl->d_eblk = dev_upload(eblk);
-    pl->d_keblk = dev_upload(keblk);
+    {
+        std::vector<int4> ebk(ne + 2, make_int4(0, 0, 0, 0));  // k_ket reads up to two entries past a row's end
+        for (int q = 0; q < ne; q++) {
+            std::memcpy(&ebk[q].x, &eb[q], sizeof(float));
+            ebk[q].y = keblk[q];
+            ebk[q].z = b2->h_kcart[ecart[q]];
+        }
+        pl->d_ebk = dev_upload(ebk);
+    }
     pl->d_egeom = dev_upload(eg);
     pl->d_egeom32 = dev_upload(eg32);
     for (int L = 0; L <= kMaxL; L++)
@@ -467,9 +479,7 @@ void free_pairlist(lsjk_pairlist* pl)
     dev_free(pl->d_hgeom);
     dev_free(pl->d_row_start);
     dev_free(pl->d_ebound);
-    dev_free(pl->d_ecart);
-    dev_free(pl->d_eblk);
-    dev_free(pl->d_keblk);
+    dev_free(pl->d_ebk);
     dev_free(pl->d_egeom);
     dev_free(pl->d_egeom32);
     for (int L = 0; L <= lsjk::kMaxL; L++)
@@ -494,6 +504,7 @@ void free_pairlist(lsjk_pairlist* pl)
     pl->kcost_g.clear();
     for (auto& kv : pl->kgroups) {
         dev_free(kv.second.d_slot);
+        dev_free(kv.second.d_ent);
         dev_free(kv.second.d_grp_slot);
         dev_free(kv.second.d_grp_rows);
         dev_free(kv.second.d_grp_rank);
@@ -739,11 +750,42 @@ const lsjk_pairlist::KGroupData& get_kgroups(lsjk_pairlist* pl, int L, int Lp, i
         }
         std::stable_sort(v.begin(), v.end(), [&](const int2& a, const int2& b) { return pl->h_eb[a.x] > pl->h_eb[b.x]; });
         while (v.size() % 64) v.push_back(make_int2(-1, 0));
-        for (size_t c = 0; c < v.size(); c += 64) G.chunk_b.push_back(pl->h_eb[v[c].x]);
+        for (size_t c = 0; c < v.size(); c += 64) {
+            G.chunk_b.push_back(pl->h_eb[v[c].x]);
+            // inside a chunk by the partner's K view column: neighbouring lanes then gather D from the
+            // same cache lines
+            auto col = [&](const int2& s) {
+                return s.x < 0 ? std::numeric_limits<int>::max()
+                               : pl->b2->h_kcart[pl->b2->h_cart[pl->h_eprim[s.x]]];
+            };
+            std::stable_sort(v.begin() + c, v.begin() + c + 64,
+                             [&](const int2& a, const int2& b) { return col(a) < col(b); });
+        }
         slot.insert(slot.end(), v.begin(), v.end());
         G.grp_slot[g + 1] = (int)slot.size();
     }
-    G.d_slot = dev_upload(slot);
+    {
+        const lsjk::Basis *b1 = pl->b1, *b2 = pl->b2;
+        std::vector<int4> packed(slot.size());
+        std::vector<double> ent(13 * slot.size(), 0.0);
+        for (size_t q = 0; q < slot.size(); q++) {
+            const int e = slot[q].x;
+            packed[q] = make_int4(e, slot[q].y, 0, 0);
+            if (e < 0) continue;
+            const int g = (int)(std::upper_bound(G.grp_slot.begin(), G.grp_slot.end(), (int)q) - G.grp_slot.begin()) - 1;
+            const int s = pl->h_eprim[e];
+            std::memcpy(&packed[q].z, &pl->h_eb[e], sizeof(float));
+            packed[q].w = b2->h_kblk[b2->h_blk[s]];
+            double rec[lsjk::kKEntDoubles];
+            kent_record(b1, grp_rows[(size_t)g * gsize + slot[q].y], b2, s, rec);
+            for (int f = 0; f < 11; f++) ent[f * slot.size() + q] = rec[f];
+            ent[11 * slot.size() + q] = rec[12];
+            const long long cart = b2->h_kcart[b2->h_cart[s]];
+            std::memcpy(&ent[12 * slot.size() + q], &cart, sizeof(cart));
+        }
+        G.d_ent = dev_upload(ent);
+        G.d_slot = dev_upload(packed);
+    }
     G.d_grp_slot = dev_upload(G.grp_slot);
     G.d_grp_rows = dev_upload(grp_rows);
     G.slot = slot;
@@ -977,6 +1019,8 @@ lsjk::KGroups kgroups_args(const lsjk_pairlist::KGroupData& G)
     lsjk::KGroups k;
     k.gsize = G.gsize;
     k.slot = G.d_slot;
+    k.ent = G.d_ent;
+    k.nslot = (int)G.slot.size();
     k.grp_slot = G.d_grp_slot;
     k.grp_rows = G.d_grp_rows;
     k.grp_rank = G.d_grp_rank;
@@ -1398,6 +1442,14 @@ struct CallOpts {
     const std::map<int, int>* orient_set = nullptr; // exchange: store and use these orientations
 };
 
+// Elements of KArgs::rw for a bra list and the ket partners' basis.  It is formed up to 4 GiB (about
+// 20,000 primitives with 18,000 shells); 0 above that: the kernel then sieves with the largest |D|.
+size_t rowmax_elems(const lsjk_pairlist* pl12, const lsjk::Basis* b4)
+{
+    const size_t n = (size_t)pl12->nrow * (pl12->kmaxL2 + 1) * (size_t)lsjk::blk_ld(b4);
+    return n * sizeof(unsigned int) <= (size_t)4 << 30 ? n : 0;
+}
+
 void commit_ws(Workspace& wsp, const CallOpts& o, const char* who)
 {
     if (o.ws) {
@@ -1596,6 +1648,8 @@ void basis_free(lsjk_basis* b)
     dev_free(b->d_blk_L);
     dev_free(b->d_blk_lo);
     dev_free(b->d_blk_hi);
+    dev_free(b->d_prim_lo);
+    dev_free(b->d_prim_hi);
     dev_free(b->d_kcart);
     dev_free(b->d_kblk);
     delete b;
@@ -1759,33 +1813,53 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
         }
         double* Dsh = nullptr;
         double* Ks = nullptr;
+        unsigned int* rw = nullptr;  // the bra rows' maxima over their partners (KArgs::rw)
         // K view copies of D24 and of its block maxima (Basis::kperm): the kernel gathers from them
         double* Dk = nullptr;
         double* Dshk = nullptr;
         const bool kview = b2->kperm || b4->kperm;
         Workspace wsp;
-        wsp.add(&Dsh, blk_elems(b2, b4));
         if (kview) {
             wsp.add(&Dk, mat_elems(b2, b4));
             wsp.add(&Dshk, blk_elems(b2, b4));
+        } else {
+            wsp.add(&Dsh, blk_elems(b2, b4));
         }
+        const size_t nrw = rowmax_elems(pl12, b4);
+        if (nrw) wsp.add(&rw, nrw);
         if (tune) wsp.add(&Ks, mat_elems(b1, b3));
         commit_ws(wsp, o, who);
         const bool timed = !o.graph;
 
         if (timed) HIPCHK(hipEventRecord(S.ev[0], st));
         launch_fill(S.d_sc, sizeof(CallScalars), st);
-        launch_k_blockmax(D24_dev, mat_ld(b4), b2->d_blk_cart, b2->d_blk_L, b2->nblk, b4->d_blk_cart, b4->d_blk_L,
-                          b4->nblk, Dsh, blk_ld(b4), b2->d_blk_lo, b2->d_blk_hi, b2->ldblk, S.d_sc, st);
         if (kview) {
-            launch_permute(D24_dev, mat_ld(b4), b2->ncart, b4->ncart, b2->kperm ? b2->d_kcart : nullptr,
-                           b4->kperm ? b4->d_kcart : nullptr, Dk, mat_ld(b4), st);
-            launch_permute(Dsh, blk_ld(b4), b2->nblk, b4->nblk, b2->kperm ? b2->d_kblk : nullptr,
-                           b4->kperm ? b4->d_kblk : nullptr, Dshk, blk_ld(b4), st);
+            KViewArgs va{};
+            va.D = D24_dev;
+            va.ld = mat_ld(b4);
+            va.bc2 = b2->d_blk_cart;
+            va.bL2 = b2->d_blk_L;
+            va.bc4 = b4->d_blk_cart;
+            va.bL4 = b4->d_blk_L;
+            va.nb2 = b2->nblk;
+            va.nb4 = b4->nblk;
+            va.kc2 = b2->kperm ? b2->d_kcart : nullptr;
+            va.kc4 = b4->kperm ? b4->d_kcart : nullptr;
+            va.kb2 = b2->kperm ? b2->d_kblk : nullptr;
+            va.kb4 = b4->kperm ? b4->d_kblk : nullptr;
+            va.Dk = Dk;
+            va.Dshk = Dshk;
+            va.sc = S.d_sc;
+            launch_k_kview(va, st);
         } else {
+            launch_k_blockmax(D24_dev, mat_ld(b4), b2->d_blk_cart, b2->d_blk_L, b2->nblk, b4->d_blk_cart, b4->d_blk_L,
+                              b4->nblk, Dsh, blk_ld(b4), b2->d_blk_lo, b2->d_blk_hi, b2->ldblk, S.d_sc, st);
             Dk = const_cast<double*>(D24_dev);
             Dshk = Dsh;
         }
+        if (rw)
+            launch_k_rowmax(pl12->d_row_start, pl12->nrow, pl12->kmaxL2, pl12->d_ebk, Dshk, blk_ld(b4),
+                            b4->nblk, b1->d_prim_lo, b1->d_prim_hi, thresp, pl34->maxbound, S.d_sc, rw, blk_ld(b4), st);
         HIPCHK(hipGetLastError());
         if (timed) HIPCHK(hipEventRecord(S.ev[1], st));
         S.kid.clear();
@@ -1828,9 +1902,7 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
                     KSide& sd = *ks[q];
                     sd.row_start = pl->d_row_start;
                     sd.maxLp = pl->kmaxL2;
-                    sd.eb = pl->d_ebound;
-                    sd.ecart = pl->d_ecart;
-                    sd.eblk = pl->d_keblk;  // the K view order of Dshk
+                    sd.ebk = pl->d_ebk;
                     sd.eg = pl->d_egeom;
                     sd.eg32 = pl->d_egeom32;
                     sd.nent = pl->nent;
@@ -1846,6 +1918,9 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
                 ka.ldD = mat_ld(b4);
                 ka.Dsh = Dshk;
                 ka.ldDsh = blk_ld(b4);
+                ka.rw = rw;
+                ka.ldrw = blk_ld(b4);
+                ka.rwlo = b1->d_prim_lo;
                 ka.K = K;
                 ka.ldK = mat_ld(b3);
                 ka.maxb12 = pl12->maxbound;
@@ -2414,6 +2489,13 @@ lsjk_batch* batch_new(int nmol, const lsjk_pairlist* const* lists)
         bb->ldblk = std::max(bb->ldblk, 1);
         bb->d_blk_lo = dev_upload(bb->h_blk_lo);
         bb->d_blk_hi = dev_upload(bb->h_blk_hi);
+        std::vector<int> plo(mol.size()), phi(mol.size());
+        for (size_t i = 0; i < mol.size(); i++) {
+            plo[i] = mb0[mol[i]];
+            phi[i] = mb0[mol[i] + 1];
+        }
+        bb->d_prim_lo = dev_upload(plo);
+        bb->d_prim_hi = dev_upload(phi);
         b->nelem = mat_elems(bb, bb);
         // pairs: class by class ((L1, L2) in L1-major order), molecule by molecule, each molecule's
         // pairs of the class in its own (bound-sorted) order
@@ -2440,7 +2522,7 @@ lsjk_batch* batch_new(int nmol, const lsjk_pairlist* const* lists)
 }
 
 // Bytes of the per-call buffers of one J + K build of a batch (as coulomb_call / exchange_call
-// carve them from a workspace): kb, kd, jp (and kd32 on the mixed route); Dsh.
+// carve them from a workspace): kb, kd, jp (and kd32 on the mixed route); Dsh, the rows' maxima.
 size_t batch_ws_bytes(const lsjk_batch* b, bool mixed, size_t* jbytes)
 {
     auto r = [](size_t n) { return (std::max<size_t>(1, n) + 255) & ~size_t(255); };
@@ -2449,7 +2531,7 @@ size_t batch_ws_bytes(const lsjk_batch* b, bool mixed, size_t* jbytes)
     size_t j = r((size_t)pl->npair * sizeof(float)) + r(h * sizeof(double)) + r(h * sizeof(double));
     if (mixed) j += r(h * sizeof(float));
     *jbytes = j;
-    return j + r(blk_elems(b->basis, b->basis) * sizeof(double));
+    return j + r(blk_elems(b->basis, b->basis) * sizeof(double)) + r(rowmax_elems(pl, b->basis) * sizeof(unsigned int));
 }
 
 void batch_jk(lsjk_batch* b, const double* D_dev, int nterm, const double* scales, const double* omegas, float thresp,
@@ -2794,9 +2876,7 @@ int lsjk_unit_magnitudes(const lsjk_pairlist* pl, int L1, int L2, int L3, int L4
             KSide& sd = *ks[q];
             sd.row_start = pl->d_row_start;
             sd.maxLp = pl->kmaxL2;
-            sd.eb = pl->d_ebound;
-            sd.ecart = pl->d_ecart;
-            sd.eblk = pl->d_eblk;
+            sd.ebk = pl->d_ebk;
             sd.eg = pl->d_egeom;
             sd.eg32 = pl->d_egeom32;
             sd.nent = pl->nent;

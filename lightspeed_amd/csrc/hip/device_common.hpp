@@ -355,6 +355,24 @@ __device__ __forceinline__ double wave_sum_last(double v)
     return v;
 }
 
+// Largest of the 64 lanes' values (every lane active), as a wave-uniform value: the moves of
+// wave_sum_last with max in place of the sum.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ unsigned int dpp_umax(unsigned int v)
+{
+    return max(v, (unsigned int)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROW_MASK, 0xf, false));
+}
+__device__ __forceinline__ unsigned int wave_umax(unsigned int v)
+{
+    v = dpp_umax<0xB1, 0xf>(v);
+    v = dpp_umax<0x4E, 0xf>(v);
+    v = dpp_umax<0x141, 0xf>(v);
+    v = dpp_umax<0x140, 0xf>(v);
+    v = dpp_umax<0x142, 0xa>(v);
+    v = dpp_umax<0x143, 0xc>(v);
+    return (unsigned int)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 // McMurchie-Davidson Hermite expansion coefficients for one axis:
 // E[t][i][j] for i <= LA, j <= LB, t <= i + j (Helgaker, Jorgensen & Olsen eqs. 9.5.6-9.5.7):
 //   E^{i+1,j}_t = E^{ij}_{t-1}/(2p) + X_PA E^{ij}_t + (t+1) E^{ij}_{t+1}

@@ -1,17 +1,19 @@
 // Exchange (K) build: small helper kernels (D block maxima, fills, copies) and the class
-// dispatcher; the quartet kernels are in exchange_impl.hpp (instantiated by exchange_l<L1>.hip).
+// dispatcher; the quartet kernels are in exchange_impl.hpp (instantiated by exchange_k<L1><L2>.hip).
 #include "internal.hpp"
 #include "kernels.hpp"
 
 namespace lsjk {
 
-template <int L1>
-void launch_k_ket_l1(int L2, int L3, int L4, int route, const KArgs& a, const KGroups& kg, const KUnitG* units,
-                     int nunits, hipStream_t s);
-#define LSJK_KET_EXTERN(X)                                                                                   \
-    extern template void launch_k_ket_l1<X>(int, int, int, int, const KArgs&, const KGroups&, const KUnitG*, int, \
-                                            hipStream_t);
-LSJK_KET_EXTERN(0) LSJK_KET_EXTERN(1) LSJK_KET_EXTERN(2)
+template <int L1, int L2>
+void launch_k_ket_l12(int L3, int L4, int route, const KArgs& a, const KGroups& kg, const KUnitG* units, int nunits,
+                      hipStream_t s);
+#define LSJK_KET_EXTERN(X, Y)                                                                                \
+    extern template void launch_k_ket_l12<X, Y>(int, int, int, const KArgs&, const KGroups&, const KUnitG*, int, \
+                                                hipStream_t);
+LSJK_KET_EXTERN(0, 0) LSJK_KET_EXTERN(0, 1) LSJK_KET_EXTERN(0, 2)
+LSJK_KET_EXTERN(1, 0) LSJK_KET_EXTERN(1, 1) LSJK_KET_EXTERN(1, 2)
+LSJK_KET_EXTERN(2, 0) LSJK_KET_EXTERN(2, 1) LSJK_KET_EXTERN(2, 2)
 #undef LSJK_KET_EXTERN
 
 template <int L1, int L2>
@@ -47,16 +49,96 @@ __global__ void k_blockmax(const double* D, int ldD, const int* bc2, const int* 
     atomicMax(&sc->dmax_bits, (unsigned long long)__double_as_longlong(m));
 }
 
-// out[pr[i] * ldo + pc[j]] = in[i * ldi + j] for i < nr, j < nc (pr, pc permutations; null: the
-// identity on that side).  One thread per element, rows of `in` read coalesced.
-__global__ void k_permute(const double* __restrict__ in, int ldi, int nr, int nc, const int* __restrict__ pr,
-                          const int* __restrict__ pc, double* __restrict__ out, int ldo)
+// One workgroup per (row, partner L) key, threads over the ket blocks (coalesced rows of the block
+// maxima).  Bound by L2 reads of the maxima, 8 bytes per (partner, block).
+__global__ __launch_bounds__(256) void k_rowmax(const int* __restrict__ row_start, int maxLp,
+                                                const int4* __restrict__ ebk,
+                                                const double* __restrict__ Dsh, int ldDsh, int ncol,
+                                                const int* __restrict__ rwlo, const int* __restrict__ rwhi,
+                                                float thresp, float maxb34, const CallScalars* __restrict__ sc,
+                                                unsigned int* __restrict__ rw, int ldrw)
+{
+    const int key = blockIdx.x;
+    const int a0 = ld_const(row_start + key);
+    const int a1 = ld_const(row_start + key + 1);
+    if (a0 == a1) return;
+    const int row = key / (maxLp + 1);
+    const int lo = rwlo ? ld_const(rwlo + row) : 0, hi = rwhi ? ld_const(rwhi + row) : ncol;
+    const double dmax = __longlong_as_double((long long)sc->dmax_bits);
+    const float thre12 = (float)((double)thresp / ((double)maxb34 * dmax));
+    // the partners that count: sorted, so a prefix
+    int n = a1 - a0;
+    if (__int_as_float(ld_const(&ebk[a1 - 1].x)) < thre12) {
+        int l = 0;
+        while (l < n) {
+            const int mid = (l + n) / 2;
+            if (__int_as_float(ld_const(&ebk[a0 + mid].x)) < thre12)
+                n = mid;
+            else
+                l = mid + 1;
+        }
+        n = l;
+    }
+    for (int c = lo + (int)threadIdx.x; c < hi; c += 256) {
+        double w = 0.0, d = 0.0;
+        // eight partners' loads in flight (the last one again past the end)
+        for (int k = 0; k < n; k += 8) {
+            double v[8];
+            float b[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const int e = a0 + min(k + q, n - 1);
+                b[q] = __int_as_float(ld_const(&ebk[e].x));
+                v[q] = Dsh[(size_t)ld_const(&ebk[e].y) * ldDsh + c];
+            }
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                w = fmax(w, (double)b[q] * v[q]);
+                d = fmax(d, v[q]);
+            }
+        }
+        // upper halves, rounded up (values are finite or infinite and non-negative)
+        auto up16 = [](double v) { return (unsigned int)min((__float_as_uint(__double2float_ru(v)) + 0xffffu) >> 16, 0x7f80u); };
+        rw[(size_t)key * ldrw + (c - lo)] = up16(w) << 16 | up16(d);
+    }
+}
+
+void launch_k_rowmax(const int* row_start, int nrow, int maxLp, const int4* ebk, const double* Dsh, int ldDsh, int ncol,
+                     const int* rwlo, const int* rwhi, float thresp, float maxb34,
+                     const CallScalars* sc, unsigned int* rw, int ldrw, hipStream_t s)
+{
+    const long long keys = (long long)nrow * (maxLp + 1);
+    if (keys == 0 || ncol == 0) return;
+    hipLaunchKernelGGL(k_rowmax, dim3((unsigned)keys), dim3(256), 0, s, row_start, maxLp, ebk, Dsh, ldDsh, ncol,
+                       rwlo, rwhi, thresp, maxb34, sc, rw, ldrw);
+}
+
+// The K view of D24 in one pass: per (block2, block4) the block's values and its maximum, at the two
+// blocks' places in the K view order (kc, kb: null for a basis that keeps its order), and the global
+// maximum.  One thread per block pair: D is read once, coalesced along the ket blocks.
+__global__ __launch_bounds__(256) void k_kview(KViewArgs a)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)nr * nc) return;
-    const int i = (int)(t / nc), j = (int)(t - (long long)i * nc);
-    const int oi = pr ? pr[i] : i, oj = pc ? pc[j] : j;
-    out[(size_t)oi * ldo + oj] = in[(size_t)i * ldi + j];
+    if (t >= (long long)a.nb2 * a.nb4) return;
+    const int i2 = (int)(t / a.nb4), i4 = (int)(t - (long long)i2 * a.nb4);
+    const int o2 = a.bc2[i2], o4 = a.bc4[i4], n2 = ncart(a.bL2[i2]), n4 = ncart(a.bL4[i4]);
+    const int k2 = a.kc2 ? a.kc2[o2] : o2, k4 = a.kc4 ? a.kc4[o4] : o4;  // a block's functions stay together
+    double m = 0.0;
+    for (int b = 0; b < n2; b++)
+        for (int d = 0; d < n4; d++) {
+            const double v = a.D[(size_t)(o2 + b) * a.ld + (o4 + d)];
+            a.Dk[(size_t)(k2 + b) * a.ld + (k4 + d)] = v;
+            m = fmax(m, fabs(v));
+        }
+    a.Dshk[(size_t)(a.kb2 ? a.kb2[i2] : i2) * a.nb4 + (a.kb4 ? a.kb4[i4] : i4)] = m;
+    atomicMax(&a.sc->dmax_bits, (unsigned long long)__double_as_longlong(m));
+}
+
+void launch_k_kview(const KViewArgs& a, hipStream_t s)
+{
+    const long long n = (long long)a.nb2 * a.nb4;
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_kview, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
 }
 
 __global__ void fill_zero(unsigned int* p, size_t n)
@@ -100,15 +182,6 @@ void launch_k_blockmax(const double* D, int ldD, const int* bc2, const int* bL2,
     if (n == 0) return;
     hipLaunchKernelGGL(k_blockmax, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, D, ldD, bc2, bL2, nb2, bc4,
                        bL4, nb4, Dsh, ldDsh, blo, bhi, band, sc);
-}
-
-void launch_permute(const double* in, int ldi, int nr, int nc, const int* pr, const int* pc, double* out, int ldo,
-                    hipStream_t s)
-{
-    const long long n = (long long)nr * nc;
-    if (n == 0) return;
-    hipLaunchKernelGGL(k_permute, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, ldi, nr, nc, pr, pc, out,
-                       ldo);
 }
 
 __global__ __launch_bounds__(256) void k_grad_prep(KGradPrepArgs a)
@@ -200,12 +273,10 @@ void launch_k_ket(int L1, int L2, int L3, int L4, int route, const KArgs& a, con
                   int nunits, hipStream_t s)
 {
     if (nunits <= 0) return;
-    if (L1 == 0)
-        launch_k_ket_l1<0>(L2, L3, L4, route, a, kg, units, nunits, s);
-    else if (L1 == 1)
-        launch_k_ket_l1<1>(L2, L3, L4, route, a, kg, units, nunits, s);
-    else
-        launch_k_ket_l1<2>(L2, L3, L4, route, a, kg, units, nunits, s);
+#define CASE(X, Y) \
+    if (L1 == X && L2 == Y) return launch_k_ket_l12<X, Y>(L3, L4, route, a, kg, units, nunits, s);
+    CASE(0, 0) CASE(0, 1) CASE(0, 2) CASE(1, 0) CASE(1, 1) CASE(1, 2) CASE(2, 0) CASE(2, 1) CASE(2, 2)
+#undef CASE
 }
 
 }  // namespace lsjk

@@ -1,6 +1,6 @@
 // Exchange (K) quartet kernel templates, shared by the translation units that instantiate them
-// (exchange_l0.hip, exchange_l1.hip, exchange_l2.hip: one per bra row angular momentum L1, so the
-// 243 instantiations compile in parallel).
+// (exchange_k<L1><L2>.hip: one per bra row and partner angular momentum, so the 324 instantiations
+// compile in parallel).
 // Direct exchange (K) build on gfx950.
 //
 // K13 += sum_{2,4} (12|34) D24 over the quartets the reference evaluates
@@ -133,32 +133,6 @@ __device__ __forceinline__ KEnt<double> load_ent(const double* __restrict__ eg, 
     return e;
 }
 
-// One packed FP32-route entry: an 80-byte record (P as 3 doubles; p, Kp, P - A, A - B, 1/(2p) as
-// floats; {cart, blk}; K view {cart, blk}); KV: take the K view ids.
-template <bool KV = false>
-__device__ __forceinline__ KEnt<float> load_ent32(const double* __restrict__ eg32, int i)
-{
-    const double* g = static_cast<const double*>(__builtin_assume_aligned(eg32 + (size_t)i * kKEnt32Doubles, 16));
-    KEnt<float> e;
-    e.Px = g[0];
-    e.Py = g[1];
-    e.Pz = g[2];
-    const float* f = reinterpret_cast<const float*>(g + 3);
-    e.p = f[0];
-    e.K = f[1];
-    e.PAx = f[2];
-    e.PAy = f[3];
-    e.PAz = f[4];
-    e.ABx = f[5];
-    e.ABy = f[6];
-    e.ABz = f[7];
-    e.i2p = f[8];
-    const int* ids = reinterpret_cast<const int*>(g + (KV ? 9 : 8));
-    e.cart = ids[0];
-    e.blk = ids[1];
-    return e;
-}
-
 template <typename Real>
 __device__ __forceinline__ Real kdiv(Real a, Real b)
 {
@@ -182,8 +156,9 @@ __device__ __forceinline__ Real krsqrt(Real x)
 // copied to LDS at s_tab (FP64 block for Real = double, FP32 block for Real = float); otherwise
 // the global table is read.  KETD (L3 = 0 only): e34's P - A holds Q - D, and the ket's 2-D
 // integrals (ab|0d) are recurred at D directly, as (ab|d0) with D in the place of C (the same
-// integrals; no transfer from C, so C - D is not needed).
-template <typename Real, int L1, int L2, int L3, int L4, bool STAGED, bool KETD = false>
+// integrals; no transfer from C, so C - D is not needed).  BARE: the operator is one bare 1/r term
+// whose scale the caller has put into e34's Kp; otherwise the terms of ew are summed.
+template <typename Real, int L1, int L2, int L3, int L4, bool STAGED, bool KETD = false, bool BARE = false>
 __device__ __forceinline__ void k_quartet(const RysTable& tab, const void* s_tab, const Ewald& ew,
                                           const KEnt<Real>& e12, const KEnt<Real>& e34,
                                           const Real (&Db)[ncart(L2)][ncart(L4)], double (&acc)[ncart(L1)][ncart(L3)])
@@ -215,8 +190,10 @@ __device__ __forceinline__ void k_quartet(const RysTable& tab, const void* s_tab
 #pragma unroll
             for (int c = 0; c < N3; c++) qacc[a][c] = Real(0);
     }
-    // one operator term: Rys roots at T = rho d2 |PQ|^2, assembly with prefactor pref
-    auto term = [&](Real pref, Real d2) __attribute__((always_inline)) {
+    // one operator term: Rys roots at T = rho d2 |PQ|^2, assembly with prefactor pref (d2: the number,
+    // or the constant one for a bare term)
+    auto term = [&](Real pref, auto d2_) __attribute__((always_inline)) {
+        const Real d2 = (Real)d2_;
         Real x[NR], w[NR];
         if constexpr (std::is_same<Real, float>::value)
             rys_roots_f32<NR, STAGED>(tab, STAGED ? static_cast<const float*>(s_tab) : tab.coef32 + tab.offset32[NR],
@@ -275,12 +252,8 @@ __device__ __forceinline__ void k_quartet(const RysTable& tab, const void* s_tab
             });
         }
     };
-    // one bare 1/r term (the common case): d2 = 1 and no term loop.  Taken for the light classes
-    // only, where the loop's overhead is a visible share of a quartet; for the others the second
-    // copy of the quartet code measured slower.
-    constexpr bool kPlainBranch = L1 + L2 + L3 + L4 <= 2;
-    if (kPlainBranch && ew.plain) {
-        term((Real)ew.alpha[0] * base, Real(1));
+    if constexpr (BARE) {
+        term(base, std::integral_constant<int, 1>{});
     } else {
         for (int it = 0; it < ew.n; it++) {
             const double om = ew.omega[it];
@@ -300,6 +273,30 @@ __device__ __forceinline__ void k_quartet(const RysTable& tab, const void* s_tab
 #pragma unroll
             for (int c = 0; c < N3; c++) acc[a][c] += (double)qacc[a][c];
     }
+}
+
+// The entry of one ket slot from the group's fields in slot order (KGroups::ent; K view ids): a wave's
+// slots are mostly consecutive, so each field is a few cache lines, where a 128-byte record per lane
+// is one line per lane and load.
+__device__ __forceinline__ KEnt<double> load_slot(const double* __restrict__ ent, int nslot, int s)
+{
+    auto f = [&](int i) __attribute__((always_inline)) { return (ent + (size_t)i * nslot)[s]; };
+    KEnt<double> e;
+    e.p = f(0);
+    e.K = f(1);
+    e.Px = f(2);
+    e.Py = f(3);
+    e.Pz = f(4);
+    e.PAx = f(5);
+    e.PAy = f(6);
+    e.PAz = f(7);
+    e.ABx = f(8);
+    e.ABy = f(9);
+    e.ABz = f(10);
+    e.i2p = f(11);
+    e.cart = (int)__double_as_longlong(f(12));
+    e.blk = 0;
+    return e;
 }
 
 // One packed FP64 entry at a wave-uniform index, through scalar loads (K view ids).
@@ -351,16 +348,14 @@ __device__ __forceinline__ KEnt<float> load_ent32_uniform(const double* __restri
 
 // LDS of one k_ket workgroup: the staged table blocks first, FP64 (routes with FP64 quartets,
 // nrys <= 3) then FP32 (routes with FP32 quartets, nrys <= 5), then kKWaves group accumulators
-// (gsize x N1 x N3 doubles each, gsize = rows per ket group).  The FP64 table at address 0 keeps a bin's coefficient offsets
+// (gsize x N1 x N3 doubles each, gsize = rows per ket group) and kKWaves slot queues.  The FP64 table at address 0 keeps a bin's coefficient offsets
 // (0..8 nrys * 24 bytes) inside the immediate offset field of the paired LDS reads, so the table
 // lookup needs one address per bin.
 template <int L1, int L2, int L3, int L4, int ROUTE>
 struct KKetLds {
     static constexpr int NR = (L1 + L2 + L3 + L4) / 2 + 1;
-    static constexpr bool HAS32 = ROUTE == kRouteLo || ROUTE == kRouteMixed;
-    static constexpr bool HAS64 = ROUTE != kRouteLo;
-    static constexpr bool STAGED64 = HAS64 && rys_staged(NR);
-    static constexpr bool STAGED32 = HAS32 && rys32_staged(NR);
+    static constexpr bool STAGED64 = rys_staged(NR);
+    static constexpr bool STAGED32 = ROUTE == kRouteMixed && rys32_staged(NR);
     static constexpr int N13 = ncart(L1) * ncart(L3);  // accumulator doubles per group row
     static __host__ __device__ size_t bytes64(const RysTable& tab)
     {
@@ -374,7 +369,7 @@ struct KKetLds {
     }
     static size_t bytes(const RysTable& tab, int gsize)
     {
-        return acc_offset(tab) + (size_t)kKWaves * gsize * N13 * sizeof(double);
+        return acc_offset(tab) + (size_t)kKWaves * (gsize * N13 * sizeof(double) + kKQueueBytes);
     }
 };
 
@@ -399,44 +394,78 @@ __device__ __forceinline__ KEnt<float> ent_to_f32(const KEnt<double>& e)
     return f;
 }
 
-// Waves per SIMD the compiler is asked to keep room for (register budget 512 / waves), per plain
-// route class: classes whose register count sits just above an occupancy step are held below it
-// where that costs at most a few spilled dwords and measured faster (classes that already spill,
-// or spill more, ran 15-55 % slower when held).  1 = no constraint.
+// Waves per SIMD the compiler is asked to keep room for (register budget 512 / waves): FP64 classes
+// with an operator-term loop whose register count sits just above an occupancy step are held below it
+// where that costs at most a few spilled dwords and measured faster (classes that already spill, or
+// spill more, ran 15-55 % slower when held).  The bare 1/r kernels need no hold ((ss|ss) 44 registers,
+// (ss|sp) 77).  1 = no constraint.
 constexpr int kket_class(int L1, int L2, int L3, int L4) { return ((L1 * 3 + L2) * 3 + L3) * 3 + L4; }
-constexpr int kket_waves(int L1, int L2, int L3, int L4, int route)
+constexpr int kket_waves(int L1, int L2, int L3, int L4, int route, bool bare)
 {
-    if (route != kRoutePlain) return 1;
+    if (route != kRoutePlain || bare) return 1;
     switch (kket_class(L1, L2, L3, L4)) {
     case kket_class(0, 0, 0, 0):
-        return 8;  // 62 -> 57 VGPRs, no spill
+        return 8;
     case kket_class(0, 0, 0, 1):
     case kket_class(0, 0, 2, 0):
     case kket_class(0, 0, 1, 1):
-        return 5;  // 98-108 -> 96 VGPRs, 12-32 bytes spilled
+        return 5;
     default:
         return 1;
     }
 }
 
+// The lane's number, formed anew at each use: the address arithmetic that depends on it stays inside
+// the loop that uses it instead of holding registers through the bra walk.
+__device__ __forceinline__ int lane_id()
+{
+    int z = 0;
+    asm volatile("" : "+s"(z));
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, (unsigned int)z));
+}
+
+// The kernel's arguments (KArgs, then KGroups) in constant memory, through a pointer formed anew at
+// each call: what only the sieve and the ends of a walk read is then loaded there, instead of
+// holding scalar registers (and, once those run out, vector registers) through the bra walk.
+struct KKernArgs {
+    KArgs a;
+    KGroups kg;
+};
+__device__ __forceinline__ const __attribute__((address_space(4))) KKernArgs* kernel_args()
+{
+    auto p = (const __attribute__((address_space(4))) KKernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 // K build over ket groups.  Each wave of the workgroup takes one unit (bra row r1, chunks of ket
-// group g); for each 64-slot chunk, lane l holds ket pair (r3, 4) of slot l in registers and the
-// wave walks r1's partners 2 in bound order (wave-uniform, scalar loads), stopping where even the
-// chunk's largest ket bound cannot pass with the largest D block.  Each lane tests the reference's
-// sieve float(b12 b34) max|D24 block| >= thresp for its (2, 4) and, where it passes, evaluates the
-// quartet into FP64 register accumulators for (r1, r3) (reference exchange.cpp:145-152, 186).  On
-// the mixed route (one launch) quartets with est >= thredp are evaluated in FP64 and the others in
+// group g).  It first sieves the unit's ket slots: a slot (r3, 4) can pass with some partner 2 of r1
+// only if b34 max_2(b12 max|D24 block|) >= thresp, and the maximum over r1's partners per ket block is
+// formed once per call (KArgs::rw).  Slots that can are packed into a queue in LDS; 64 at a time, lane
+// l holds one ket pair in registers and the wave walks r1's partners 2 in bound order (wave-uniform,
+// scalar loads) down to the smallest bound with which any of the 64 can pass.  Each lane tests the
+// reference's sieve float(b12 b34) max|D24 block| >= thresp for its (2, 4) and, where it passes,
+// evaluates the quartet into FP64 register accumulators for (r1, r3) (reference
+// exchange.cpp:145-152, 186).  Without the packing a chunk of 64 slots was walked whenever its largest
+// bound passed with the largest |D| anywhere: with a density that decays over distance most chunks
+// then held no quartet ((H2O)128 / 6-31G*, (ss|ss): 451 k walk steps for 39 k with a quartet in a
+// sample of rows, 35 k steps packed), and in the triangle mode chunks of earlier rows were walked too.
+// On the mixed route (one launch) quartets with est >= thredp are evaluated in FP64 and the others in
 // FP32, except that a wave step holding any FP64 quartet evaluates all of its quartets in FP64
-// (never less precision than the route asks for, and one evaluation per step).  At the end of a chunk the lanes add their
-// accumulators into the wave's LDS block of the group (row position t); at the end of the unit
-// the block is added to K with one atomic per element, plus the transposed block in the symmetric
-// mode (K = K^T) for r3 != r1.
-template <int L1, int L2, int L3, int L4, int ROUTE>
-__global__ __launch_bounds__(64 * kKWaves) __attribute__((amdgpu_waves_per_eu(kket_waves(L1, L2, L3, L4, ROUTE)))) void k_ket(KArgs a, KGroups kg, const KUnitG* __restrict__ units, int nunits)
+// (never less precision than the route asks for, and one evaluation per step).  After a walk the
+// lanes add their accumulators into the wave's LDS block of the group (row position t); at the end of
+// the unit the block is added to K with one atomic per element, plus the transposed block in the
+// symmetric mode (K = K^T) for r3 != r1.
+template <int L1, int L2, int L3, int L4, int ROUTE, bool BARE>
+__global__ __launch_bounds__(64 * kKWaves) __attribute__((amdgpu_waves_per_eu(kket_waves(L1, L2, L3, L4, ROUTE, BARE)))) void k_ket(KArgs a, KGroups kg, const KUnitG* __restrict__ units, int nunits)
 {
     using Lds = KKetLds<L1, L2, L3, L4, ROUTE>;
-    constexpr bool LO = ROUTE == kRouteLo;        // FP32 only
     constexpr bool SPLIT = ROUTE == kRouteMixed;  // FP64 and FP32 in one launch
+    // D24 blocks of up to three values are loaded ahead and sieved themselves; larger ones are sieved
+    // by their block maxima first and loaded where they pass.  The walk's gathers are what bounds the
+    // light classes (the vector cache looks up one line per clock: 90-98 % of its cycles on (ss|ss) and
+    // (ss|sp) with a gather of the maximum and one of the value per step).
+    constexpr bool DIRECT = ncart(L2) * ncart(L4) <= 3;
     constexpr int NR = Lds::NR;
     constexpr int N1 = ncart(L1), N2 = ncart(L2), N3 = ncart(L3), N4 = ncart(L4), N13 = N1 * N3;
     extern __shared__ double s_dyn[];
@@ -446,7 +475,10 @@ __global__ __launch_bounds__(64 * kKWaves) __attribute__((amdgpu_waves_per_eu(kk
     float* s_tab32 = reinterpret_cast<float*>(reinterpret_cast<char*>(s_dyn) + Lds::bytes64(a.rys));
     const int G = kg.gsize;  // rows per ket group
     const int ACC = G * N13;  // accumulator doubles per wave
-    double* s_acc = reinterpret_cast<double*>(reinterpret_cast<char*>(s_dyn) + Lds::acc_offset(a.rys)) + w * ACC;
+    double* s_acc0 = reinterpret_cast<double*>(reinterpret_cast<char*>(s_dyn) + Lds::acc_offset(a.rys));
+    double* s_acc = s_acc0 + w * ACC;
+    // the wave's queue: slots and their largest b34 max|D24 block| (bits), kKQueue of each
+    int* q_wave = reinterpret_cast<int*>(s_acc0 + kKWaves * ACC) + w * (2 * kKQueue);
     if constexpr (Lds::STAGED64) rys_stage_lds<NR>(a.rys, s_tab64);
     if constexpr (Lds::STAGED32) rys32_stage_lds<NR>(a.rys, s_tab32);
     for (int q = lane; q < ACC; q += 64) s_acc[q] = 0.0;
@@ -464,11 +496,11 @@ __global__ __launch_bounds__(64 * kKWaves) __attribute__((amdgpu_waves_per_eu(kk
         a0 = min(a1, a0 + (prange & 0xffff));
         if (prange >> 16) a1 = min(a1, a0 + (prange >> 16));
     }
+    if (a0 >= a1) return;
     const int s0 = ld_const(kg.grp_slot + g) + 64 * (crange & 0xffff);
     const int s1 = min(ld_const(kg.grp_slot + g + 1), s0 + 64 * (crange >> 16));
 
-    // quartets with est at or above `thresp` here (and, on the FP32 route, below thredp) are evaluated
-    const float thresp = (ROUTE == kRouteHi) ? a.thredp : a.thresp;
+    const float thresp = a.thresp;
     const double dmax = __longlong_as_double((long long)a.sc->dmax_bits);
     // learned route: the unit's certified factor tau <= 1 (est tau bounds every quartet's
     // contribution), so the thresholds scale by 1 / tau.  It holds for quartets whose Schwarz
@@ -479,126 +511,204 @@ __global__ __launch_bounds__(64 * kKWaves) __attribute__((amdgpu_waves_per_eu(kk
     const double thredp = (double)a.thredp / tau;
     const float thre12 = (float)(thr / ((double)a.maxb34 * dmax));
     const float thre34 = (float)(thr / ((double)a.maxb12 * dmax));
-    const float b12top = ld_const(a.s12.eb + a0);
+    const float b12top = __int_as_float(ld_const(&a.s12.ebk[a0].x));
 
+    // evaluated quartets of the wave and the FP32 part of them, wave steps with one (scalar registers)
     unsigned long long nq = 0, nq32 = 0;
-    unsigned int nsteps = 0;  // wave steps with an evaluated quartet (counting mode)
+    unsigned int nsteps = 0;
     bool any = false;
-    for (int c0 = s0; c0 < s1; c0 += 64) {
-        const float b34max = ld_const(kg.chunk_b + (c0 >> 6));
-        // no quartet of this chunk can pass, and the later chunks of the group hold smaller bounds
-        if (!(b34max >= thre34) || (double)(b12top * b34max) * dmax < thr) break;
-        const int2 sl = kg.slot[c0 + lane];
-        const int e4 = max(sl.x, 0);
-        const float b34 = a.s34.eb[e4];
-        const bool valid = sl.x >= 0 && kg.grp_rank[g * G + sl.y] >= rank1 && b34 >= thre34;
-        const int blk4 = a.s34.eblk[e4];
-        KEnt<double> E34;
-        KEnt<float> E34f;
+    int c0 = s0, qn = 0;  // next slot to sieve; queue length (wave-uniform)
+    for (;;) {
+        int s4 = 0;             // the lane's slot
+        unsigned int x4 = 0u;   // its largest b34 max|D24 block| (bits; 0: none)
+        bool valid = false, direct = false;
+        while (qn < 64 && c0 < s1) {
+            const auto* A = kernel_args();
+            const float b34max = ld_const(A->kg.chunk_b + (c0 >> 6));
+            // no quartet of this chunk can pass, and the later chunks of the group hold smaller bounds
+            if (!(b34max >= thre34) || (double)(b12top * b34max) * dmax < thr) {
+                c0 = s1;
+                break;
+            }
+            const int4* slots = A->kg.slot;
+            const int4 sl = slots[c0 + lane_id()];
+            const float b34 = __int_as_float(sl.z);
+            bool can = sl.x >= 0 && b34 >= thre34;
+            if (rank1 >= 0) {
+                const int* ranks = A->kg.grp_rank;
+                can = can && ranks[g * G + sl.y] >= rank1;
+            }
+            // x: the largest b34 max|D24 block| of the slot
+            float x;
+            if (const unsigned int* rw = A->a.rw) {
+                // the row's maxima over its partners
+                rw += (size_t)(r1 * (A->a.s12.maxLp + 1) + L2) * A->a.ldrw;
+                if (const int* lo = A->a.rwlo) rw -= ld_const(lo + r1);
+                const unsigned int wd = can ? rw[sl.w] : 0u;
+                // margin for the rounding of float(b12 b34) and of the products here
+                can = can && (double)b34 * (double)__uint_as_float(wd & 0xffff0000u) * (1.0 + 1.0e-6) >= thr;
+                x = b34 * __uint_as_float(wd << 16);
+            } else {
+                x = (float)((double)b34 * dmax);
+            }
+            const unsigned long long m = __ballot(can);
+            // a full chunk, or the unit's last one with nothing queued, goes as it is
+            if (qn == 0 && m != 0ull && (m == ~0ull || c0 + 64 >= s1)) {
+                direct = true;
+                valid = can;
+                s4 = c0 + lane_id();
+                x4 = can ? __float_as_uint(x) : 0u;
+                c0 += 64;
+                break;
+            }
+            if (can) {
+                int* q = q_wave + qn + __builtin_amdgcn_mbcnt_hi((unsigned int)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)m, 0));
+                q[0] = c0 + lane_id();
+                q[kKQueue] = __float_as_int(x);
+            }
+            qn += __popcll(m);
+            c0 += 64;
+        }
+        if (!direct) {
+            if (qn == 0) break;
+            // LDS of one wave: its reads below follow its writes above in order
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const int ln = lane_id();
+            valid = ln < qn;
+            int* q = q_wave + ln;
+            // an empty lane takes the first queued slot, so that its loads stay in range
+            s4 = valid ? q[0] : q_wave[0];
+            x4 = valid ? (unsigned int)q[kKQueue] : 0u;
+            // the slots left over move to the front
+            const int me = q[64], mx = q[kKQueue + 64];
+            __builtin_amdgcn_wave_barrier();
+            qn = max(qn - 64, 0);
+            if (ln < qn) {
+                q[0] = me;
+                q[kKQueue] = mx;
+            }
+        }
+        const auto* A = kernel_args();
+        const int4* slots = A->kg.slot;
+        const int4 sl = slots[s4];
+        const int t4 = sl.y;
+        // an empty lane's bound is not a number: no estimate of it passes
+        const float b34 = valid ? __int_as_float(sl.z) : __builtin_nanf("");
+        // the slot's entry, from the fields in slot order (neighbouring lanes, neighbouring addresses)
+        KEnt<double> E34 = load_slot(A->kg.ent, A->kg.nslot, s4);
         // s-type C with a higher D: the quartets recur at D (k_quartet KETD), from Q - D = (Q - C) + (C - D)
         constexpr bool KETD = L3 == 0 && L4 > 0;
-        if constexpr (LO) {
-            E34f = load_ent32<true>(a.s34.eg32, e4);
-            if constexpr (KETD) {
-                E34f.PAx += E34f.ABx;
-                E34f.PAy += E34f.ABy;
-                E34f.PAz += E34f.ABz;
-            }
-        } else {
-            E34 = load_ent<true>(a.s34.eg, e4);
-            if constexpr (KETD) {
-                E34.PAx += E34.ABx;
-                E34.PAy += E34.ABy;
-                E34.PAz += E34.ABz;
-            }
-            if constexpr (SPLIT) E34f = ent_to_f32(E34);
+        if constexpr (KETD) {
+            E34.PAx += E34.ABx;
+            E34.PAy += E34.ABy;
+            E34.PAz += E34.ABz;
         }
-        const int cart4 = LO ? E34f.cart : E34.cart;
-        const double* __restrict__ dsh = a.Dsh + blk4;
-        const double* __restrict__ dcol = a.D + cart4;
+        if constexpr (BARE) E34.K *= A->a.ew.alpha[0];
+        KEnt<float> E34f;
+        if constexpr (SPLIT) E34f = ent_to_f32(E34);
+        const double* __restrict__ dsh = A->a.Dsh + sl.w;
+        const double* __restrict__ dcol = A->a.D + E34.cart;
         double acc[N1][N3];
 #pragma unroll
         for (int i = 0; i < N1; i++)
 #pragma unroll
             for (int j = 0; j < N3; j++) acc[i][j] = 0.0;
         bool hit = false;
-        // Bra partners below bstop cannot pass with any slot of the chunk: float(b12 b34max) dmax
-        // < thr for b12 < thr / (b34max dmax) (1 - 2^-22), and below thre12 the partner fails the
-        // truncation.  The partners are sorted, so the walk stops at the first one below bstop
-        // (compared as bit patterns: the bounds are non-negative floats).
-        const float bstop = fmaxf(thre12, (float)(thr / ((double)b34max * dmax)) * (1.0f - 4.0f * 1.1920929e-7f));
+        // Bra partners below bstop cannot pass with any of the 64 slots: float(b12 b34) max|D24 block| <
+        // thr for b12 < thr / x (1 - 2^-20) with the largest x of the slots (rounding of the bound
+        // product and of x), and below thre12 the partner fails the truncation.  The partners are
+        // sorted, so the walk stops at the first one below bstop (compared as bit patterns: the bounds
+        // are non-negative floats).
+        const float xmax = __uint_as_float(wave_umax(x4));
+        const float bstop = fmaxf(thre12, (float)(thr / (double)xmax) * (1.0f - 8.0f * 1.1920929e-7f));
         const unsigned int bstop_bits = __builtin_amdgcn_readfirstlane(__float_as_uint(bstop));
-        // the next partner's bound, block and D block maximum are loaded one step ahead
-        float b12n = ld_const(a.s12.eb + a0);
-        double dnext = valid ? dsh[(size_t)ld_const(a.s12.eblk + a0) * a.ldDsh] : 0.0;
+        // Loads run ahead of their use: a partner's bound and ids two steps (the list is padded), its D
+        // block maximum (or D block) one step.
+        const int4* __restrict__ ebk12 = a.s12.ebk;
+        auto load_block = [&](int cart, auto& Db) __attribute__((always_inline)) {
+            using Real = typename std::remove_reference<decltype(Db[0][0])>::type;
+#pragma unroll
+            for (int b = 0; b < N2; b++)
+#pragma unroll
+                for (int d = 0; d < N4; d++) Db[b][d] = (Real)dcol[(size_t)(cart + b) * a.ldD + d];
+        };
+        int bn = ld_const(&ebk12[a0].x), bn2 = ld_const(&ebk12[a0 + 1].x);
+        int id1 = ld_const(DIRECT ? &ebk12[a0].z : &ebk12[a0].y);
+        int id2 = ld_const(DIRECT ? &ebk12[a0 + 1].z : &ebk12[a0 + 1].y);
+        double dnext = 0.0, Dnext[DIRECT ? N2 : 1][DIRECT ? N4 : 1];
+        if constexpr (DIRECT)
+            load_block(id1, Dnext);
+        else
+            dnext = dsh[(size_t)id1 * a.ldDsh];
         for (int k = a0; k < a1; k++) {
-            const float b12 = b12n;
-            if (__float_as_uint(b12) < bstop_bits) break;
-            const double dblk = dnext;
-            if (k + 1 < a1) {
-                b12n = ld_const(a.s12.eb + k + 1);
-                const int blk2n = ld_const(a.s12.eblk + k + 1);
-                if (valid) dnext = dsh[(size_t)blk2n * a.ldDsh];
+            const float b12 = __int_as_float(bn);
+            if ((unsigned int)bn < bstop_bits) break;
+            double dblk = dnext, Db[DIRECT ? N2 : 1][DIRECT ? N4 : 1];
+            if constexpr (DIRECT) {
+                // the block's own maximum; the block past the row's last partner may be of another
+                // size: the last one is loaded again in its place
+                if (k + 1 < a1) id1 = id2;
+                dblk = 0.0;
+#pragma unroll
+                for (int b = 0; b < N2; b++)
+#pragma unroll
+                    for (int d = 0; d < N4; d++) {
+                        Db[b][d] = Dnext[b][d];
+                        dblk = (N2 * N4 == 1) ? fabs(Db[b][d]) : fmax(dblk, fabs(Db[b][d]));
+                    }
+                load_block(id1, Dnext);
+                id2 = ld_const(&ebk12[k + 2].z);
+            } else {
+                dnext = dsh[(size_t)id2 * a.ldDsh];
+                id2 = ld_const(&ebk12[k + 2].y);
             }
-            bool pass = false, low = LO;
-            if (valid) {
-                const double est = (double)(b12 * b34) * dblk;
-                pass = est >= thr;
-                if constexpr (LO) pass = pass && !(est >= thredp);
-                if constexpr (SPLIT) low = !(est >= thredp);
-            }
+            bn = bn2;
+            bn2 = ld_const(&ebk12[k + 2].x);
+            const double est = (double)(b12 * b34) * dblk;
+            const bool pass = est >= thr;
             const unsigned long long m = __ballot(pass);
             if (m == 0ull) continue;
-            if (a.count) nsteps++;
-            if constexpr (ROUTE == kRoutePlain || ROUTE == kRouteHi) {
-                const KEnt<double> E12 = load_ent_uniform(a.s12.eg, k);
-                if (pass) {
-                    double Db[N2][N4];
-#pragma unroll
-                    for (int b = 0; b < N2; b++)
-#pragma unroll
-                        for (int d = 0; d < N4; d++) Db[b][d] = dcol[(size_t)(E12.cart + b) * a.ldD + d];
-                    k_quartet<double, L1, L2, L3, L4, Lds::STAGED64, KETD>(a.rys, s_tab64, a.ew, E12, E34, Db, acc);
-                    nq++;
-                    hit = true;
-                }
-                continue;
-            }
+            nsteps++;
+            nq += __popcll(m);
             // mixed route: a wave step with any quartet at or above thredp evaluates all its
             // quartets in FP64 (at least the precision the route asks for); the other steps in FP32
-            const bool step32 = LO || (SPLIT && __ballot(pass && !low) == 0ull);
-            if (!step32) {
+            const bool step32 = SPLIT && __ballot(pass && est >= thredp) == 0ull;
+            if (!SPLIT || !step32) {
                 const KEnt<double> E12 = load_ent_uniform(a.s12.eg, k);
                 if (pass) {
-                    double Db[N2][N4];
-#pragma unroll
-                    for (int b = 0; b < N2; b++)
-#pragma unroll
-                        for (int d = 0; d < N4; d++) Db[b][d] = dcol[(size_t)(E12.cart + b) * a.ldD + d];
-                    k_quartet<double, L1, L2, L3, L4, Lds::STAGED64, KETD>(a.rys, s_tab64, a.ew, E12, E34, Db, acc);
+                    if constexpr (DIRECT) {
+                        k_quartet<double, L1, L2, L3, L4, Lds::STAGED64, KETD, BARE>(a.rys, s_tab64, a.ew, E12, E34, Db, acc);
+                    } else {
+                        double Dq[N2][N4];
+                        load_block(E12.cart, Dq);
+                        k_quartet<double, L1, L2, L3, L4, Lds::STAGED64, KETD, BARE>(a.rys, s_tab64, a.ew, E12, E34, Dq, acc);
+                    }
                 }
-            } else {
+            } else if constexpr (SPLIT) {
+                nq32 += __popcll(m);
                 const KEnt<float> E12f = load_ent32_uniform(a.s12.eg32, k);
                 if (pass) {
-                    float Dbf[N2][N4];
+                    float Dq[N2][N4];
+                    if constexpr (DIRECT) {
 #pragma unroll
-                    for (int b = 0; b < N2; b++)
+                        for (int b = 0; b < N2; b++)
 #pragma unroll
-                        for (int d = 0; d < N4; d++) Dbf[b][d] = (float)dcol[(size_t)(E12f.cart + b) * a.ldD + d];
-                    k_quartet<float, L1, L2, L3, L4, Lds::STAGED32, KETD>(a.rys, s_tab32, a.ew, E12f, E34f, Dbf, acc);
+                            for (int d = 0; d < N4; d++) Dq[b][d] = (float)Db[b][d];
+                    } else {
+                        load_block(E12f.cart, Dq);
+                    }
+                    k_quartet<float, L1, L2, L3, L4, Lds::STAGED32, KETD, BARE>(a.rys, s_tab32, a.ew, E12f, E34f, Dq, acc);
                 }
             }
-            if (pass) {
-                nq++;
-                if (step32) nq32++;
-                hit = true;
-            }
+            hit = hit || pass;
         }
         if (hit) {
 #pragma unroll
             for (int i = 0; i < N1; i++)
 #pragma unroll
-                for (int j = 0; j < N3; j++) atomicAdd(&s_acc[sl.y * N13 + i * N3 + j], acc[i][j]);
+                for (int j = 0; j < N3; j++) atomicAdd(&s_acc[t4 * N13 + i * N3 + j], acc[i][j]);
         }
         any = any || (__ballot(hit) != 0ull);
     }
@@ -607,24 +717,24 @@ __global__ __launch_bounds__(64 * kKWaves) __attribute__((amdgpu_waves_per_eu(kk
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int o1 = ld_const(a.s12.cart + r1);
-        for (int q = lane; q < ACC; q += 64) {
+        const auto* A = kernel_args();
+        const int *rows3 = A->kg.grp_rows, *cart3 = A->a.s34.cart;
+        double* K = A->a.K;
+        const int ldK = A->a.ldK;
+        const bool sym = A->a.symmetric, diag = A->a.mirror_diag;
+        const int o1 = ld_const(A->a.s12.cart + r1);
+        for (int q = lane_id(); q < ACC; q += 64) {
             const double v = s_acc[q];
             if (v == 0.0) continue;
             const int t = q / N13, ij = q - t * N13, i = ij / N3, j = ij - i * N3;
-            const int r3 = kg.grp_rows[g * G + t];
-            const int o3 = a.s34.cart[r3];
-            atomic_add(a.K + (size_t)(o1 + i) * a.ldK + (o3 + j), v);
-            if (a.symmetric && (r1 != r3 || a.mirror_diag)) atomic_add(a.K + (size_t)(o3 + j) * a.ldK + (o1 + i), v);
+            const int r3 = rows3[g * G + t];
+            const int o3 = cart3[r3];
+            atomic_add(K + (size_t)(o1 + i) * ldK + (o3 + j), v);
+            if (sym && (r1 != r3 || diag)) atomic_add(K + (size_t)(o3 + j) * ldK + (o1 + i), v);
         }
     }
     if (a.count) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            nq += __shfl_xor(nq, o);
-            nq32 += __shfl_xor(nq32, o);
-        }
-        if (lane == 0 && nq) {
+        if (lane_id() == 0 && nq) {
             atomicAdd(&a.sc->counts[kcount_index(L1, L2, L3, L4)], nq);
             if (nq32) atomicAdd(&a.sc->counts32[kcount_index(L1, L2, L3, L4)], nq32);
             atomicAdd(&a.sc->wsteps[kcount_index(L1, L2, L3, L4)], (unsigned long long)nsteps);
@@ -663,13 +773,13 @@ __global__ __launch_bounds__(64 * kKWaves) void k_unit_mag(KArgs a, KGroups kg, 
     const int s1 = min(ld_const(kg.grp_slot + g + 1), s0 + 64 * (crange >> 16));
     float best = 0.0f;
     for (int c0 = s0; c0 < s1; c0 += 64) {
-        const int2 sl = kg.slot[c0 + lane];
+        const int4 sl = kg.slot[c0 + lane];
         const int e4 = max(sl.x, 0);
         const bool valid = sl.x >= 0 && kg.grp_rank[g * G + sl.y] >= rank1;
-        const double b34 = (double)a.s34.eb[e4];
+        const double b34 = (double)__int_as_float(sl.z);
         const KEnt<double> E34 = load_ent(a.s34.eg, e4);
         for (int k = a0; k < a1; k++) {
-            const double b12 = (double)ld_const(a.s12.eb + k);
+            const double b12 = (double)__int_as_float(ld_const(&a.s12.ebk[k].x));
             const KEnt<double> E12 = load_ent_uniform(a.s12.eg, k);
             if (valid && b12 * b34 >= (double)smin) {
                 double m = 0.0;
@@ -700,34 +810,32 @@ __global__ __launch_bounds__(64 * kKWaves) void k_unit_mag(KArgs a, KGroups kg, 
     if (lane == 0) out[u] = best;
 }
 
-// Launch of one K build class at row angular momentum L1 (instantiated in exchange_l<L1>.hip).
-template <int L1>
-void launch_k_ket_l1(int L2, int L3, int L4, int route, const KArgs& a, const KGroups& kg, const KUnitG* units,
-                     int nunits, hipStream_t s)
+// Launch of one K build class with bra row and partner angular momenta L1, L2 (instantiated in
+// exchange_k<L1><L2>.hip).
+template <int L1, int L2>
+void launch_k_ket_l12(int L3, int L4, int route, const KArgs& a, const KGroups& kg, const KUnitG* units, int nunits,
+                      hipStream_t s)
 {
     dim3 grid((unsigned)((nunits + kKWaves - 1) / kKWaves)), block(64 * kKWaves);
-#define ONE(B, C, D, R)                                                                             \
+#define ONE(C, D, R)                                                                                \
     {                                                                                               \
-        const size_t lds = KKetLds<L1, B, C, D, R>::bytes(a.rys, kg.gsize);                         \
-        if (lds > kMaxLdsPerGroup || lds != kket_lds_bytes(a.rys, L1, B, C, D, R, kg.gsize))       \
+        auto* kernel = a.ew.plain ? k_ket<L1, L2, C, D, R, true> : k_ket<L1, L2, C, D, R, false>;   \
+        const size_t lds = KKetLds<L1, L2, C, D, R>::bytes(a.rys, kg.gsize);                        \
+        if (lds > kMaxLdsPerGroup || lds != kket_lds_bytes(a.rys, L1, L2, C, D, R, kg.gsize))      \
             throw std::runtime_error("lsjk: k_ket LDS request too large or inconsistent");         \
-        hipLaunchKernelGGL((k_ket<L1, B, C, D, R>), grid, block, lds, s, a, kg, units, nunits);     \
+        hipLaunchKernelGGL(kernel, grid, block, lds, s, a, kg, units, nunits);                      \
     }
-#define CASE(B, C, D)                                                                               \
-    if (L2 == B && L3 == C && L4 == D) {                                                            \
+#define CASE(C, D)                                                                                  \
+    if (L3 == C && L4 == D) {                                                                       \
         if (route == kRouteMixed)                                                                   \
-            ONE(B, C, D, kRouteMixed)                                                               \
+            ONE(C, D, kRouteMixed)                                                                  \
         else if (route == kRoutePlain)                                                              \
-            ONE(B, C, D, kRoutePlain)                                                               \
+            ONE(C, D, kRoutePlain)                                                                  \
         else                                                                                        \
             throw std::runtime_error("lsjk: k_ket route not instantiated");                         \
         return;                                                                                     \
     }
-#define C4(B, C) CASE(B, C, 0) CASE(B, C, 1) CASE(B, C, 2)
-#define C3(B) C4(B, 0) C4(B, 1) C4(B, 2)
-    C3(0) C3(1) C3(2)
-#undef C3
-#undef C4
+    CASE(0, 0) CASE(0, 1) CASE(0, 2) CASE(1, 0) CASE(1, 1) CASE(1, 2) CASE(2, 0) CASE(2, 1) CASE(2, 2)
 #undef CASE
 #undef ONE
 }

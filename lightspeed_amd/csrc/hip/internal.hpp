@@ -33,6 +33,7 @@ struct Basis {
     std::vector<int> h_mol;           // molecule of each primitive (batch basis)
     std::vector<int> h_blk_lo, h_blk_hi;  // per block: its molecule's block range (batch basis)
     int *d_blk_lo = nullptr, *d_blk_hi = nullptr;
+    int *d_prim_lo = nullptr, *d_prim_hi = nullptr;  // the same range per primitive
     // K view order: the exchange kernel reads D and its block maxima from copies whose blocks are
     // ordered by angular momentum, then spatially (Morton order of the shell centres), so that the
     // partners of a group of nearby rows are neighbouring columns.  h_kcart[i] = position of
@@ -88,9 +89,7 @@ struct PairList {
     int* d_row_start = nullptr;
     int nent = 0;
     float* d_ebound = nullptr;
-    int* d_ecart = nullptr;   // partner Cartesian offset
-    int* d_eblk = nullptr;    // partner block id
-    int* d_keblk = nullptr;   // partner block id in the K view order (Basis::h_kblk)
+    int4* d_ebk = nullptr;    // KSide::ebk, 2 pads at the end
     double* d_egeom = nullptr; // packed entries (12 doubles each: p, K, P, P-A, A-B, {cart, blk})
     double* d_egeom32 = nullptr; // FP32-route entries (64 bytes each: P in FP64, 8 floats, {cart, blk})
     // pivot view for counting (rows = basis-2 primitives, partners = basis-1 primitives, bounds
@@ -156,7 +155,8 @@ struct PairList {
     // K ket groups per (row L, partner L) (kernels.hpp KGroups), built on first use
     struct KGroupData {
         int gsize = 16;  // rows per group
-        int2* d_slot = nullptr;
+        int4* d_slot = nullptr;
+        double* d_ent = nullptr;  // KGroups::ent
         int* d_grp_slot = nullptr;
         int* d_grp_rows = nullptr;
         int* d_grp_rank = nullptr;

@@ -187,9 +187,19 @@ constexpr int kgroup_size(int L, int Lp) { return (L == 0 && Lp > 0) ? 64 : ((L 
 // These are the defaults: lsjk_autotune picks 16, 32 or 64 rows per (row L, partner L) of a list
 // (KGroups::gsize), where every class over that ket pair fits the LDS limit (kket_lds_bytes).
 constexpr int kKWaves = 4;  // waves (independent work units) per workgroup
+// k_ket's queue of ket slots that can pass the sieve: slot and largest b34 max|D24 block|; at most 63
+// left over + 64 new.
+constexpr int kKQueue = 128;
+constexpr size_t kKQueueBytes = kKQueue * 2 * sizeof(int);
 struct KGroups {
     int gsize;             // rows per group
-    const int2* slot;      // [nslot] {entry index or -1 (padding), position of the row in the group}
+    // [nslot] {entry index or -1 (padding), position of the row in the group, bits of the entry's
+    // bound, the partner's block id in the K view order}
+    const int4* slot;
+    // [13][nslot] the slots' entries by field: p, Kp, P (3), P - A (3), A - B (3), 1/(2p), the partner's
+    // Cartesian offset in the K view order (zeros for padding)
+    const double* ent;
+    int nslot;
     const int* grp_slot;   // [ngroup + 1] first slot of each group
     const int* grp_rows;   // [ngroup * group size] row primitive at each position (-1: none)
     const int* grp_rank;   // [ngroup * group size] spatial rank of that row (INT_MAX: none)
@@ -216,9 +226,8 @@ constexpr int kKEnt32Doubles = 10;
 struct KSide {
     const int* row_start;  // [nrow * (maxLp+1) + 1]
     int maxLp;
-    const float* eb;       // entry bound
-    const int* ecart;      // partner Cartesian offset
-    const int* eblk;       // partner block id
+    // per entry {bits of the bound, the partner's block id and Cartesian offset in the K view order, 0}
+    const int4* ebk;
     const double* eg;      // packed entries, kKEntDoubles doubles each (see KEnt)
     const double* eg32;    // FP32-route entries, kKEnt32Doubles doubles each
     int nent;
@@ -245,6 +254,13 @@ struct KArgs {
     double* K;           // K13, ncart1 x ncart3
     int ldK;
     float maxb12, maxb34;  // max_bound of the two lists
+    // Per bra row key r1 * (s12.maxLp + 1) + L2 and ket block: the largest b12 max|D24 block| over the
+    // row's partners (upper 16 bits) and the largest max|D24 block| (lower 16), each the upper half
+    // of a float, rounded up (launch_k_rowmax), at rw[key * ldrw + blk4 - (rwlo ? rwlo[r1] : 0)];
+    // nullptr: not formed.  They only bound what a slot can reach, so 8 bits of mantissa do.
+    const unsigned int* rw;
+    int ldrw;
+    const int* rwlo;
     // learned route (nullptr: none): per unit the certified factor tau in (0, 1] of the Schwarz
     // estimate, applied while thresp >= tau_smin max|D24|
     const float* tau;
@@ -318,17 +334,31 @@ int persistent_grid(const void* kernel, int block, size_t lds, long long nwork_g
 inline size_t kket_lds_bytes(const RysTable& tab, int L1, int L2, int L3, int L4, int route, int gsize)
 {
     const int NR = (L1 + L2 + L3 + L4) / 2 + 1;
-    const bool has32 = route == kRouteLo || route == kRouteMixed, has64 = route != kRouteLo;
     size_t b = 0;
-    if (has64 && rys_staged(NR)) b += rys_lds_doubles(tab.nbin[NR], NR) * sizeof(double);
-    if (has32 && rys32_staged(NR)) b += rys32_lds_floats(tab.nbin[NR], NR) * sizeof(float);
+    if (rys_staged(NR)) b += rys_lds_doubles(tab.nbin[NR], NR) * sizeof(double);
+    if (route == kRouteMixed && rys32_staged(NR)) b += rys32_lds_floats(tab.nbin[NR], NR) * sizeof(float);
     b = (b + 7) & ~(size_t)7;
-    return b + (size_t)kKWaves * gsize * ncart(L1) * ncart(L3) * sizeof(double);
+    return b + (size_t)kKWaves * (gsize * ncart(L1) * ncart(L3) * sizeof(double) + kKQueueBytes);
 }
 
-// out[pr[i] * ldo + pc[j]] = in[i * ldi + j] (the K view copies of D and of its block maxima).
-void launch_permute(const double* in, int ldi, int nr, int nc, const int* pr, const int* pc, double* out, int ldo,
-                    hipStream_t s);
+// KArgs::rw of one exchange call: rows x (maxLp + 1) keys by ldrw ket blocks, from the block maxima
+// (K view order) and the bra list's partner lists.  Partners below thresp / (maxb34 max|D24|) fail the
+// sieve with every ket and are left out.
+void launch_k_rowmax(const int* row_start, int nrow, int maxLp, const int4* ebk, const double* Dsh, int ldDsh, int ncol,
+                     const int* rwlo, const int* rwhi, float thresp, float maxb34,
+                     const CallScalars* sc, unsigned int* rw, int ldrw, hipStream_t s);
+
+// The K view copies of D24 (ncart2 x ncart4, stride ld) and of its block maxima (nb2 x nb4), and max|D24|.
+struct KViewArgs {
+    const double* D;
+    int ld;
+    const int *bc2, *bL2, *bc4, *bL4;  // blocks' Cartesian offsets and angular momenta
+    int nb2, nb4;
+    const int *kc2, *kc4, *kb2, *kb4;  // K view places of Cartesian functions and blocks (null: unchanged)
+    double *Dk, *Dshk;
+    CallScalars* sc;
+};
+void launch_k_kview(const KViewArgs& a, hipStream_t s);
 void launch_k_blockmax(const double* D, int ldD, const int* blk_cart2, const int* blk_L2, int nblk2,
                        const int* blk_cart4, const int* blk_L4, int nblk4, double* Dsh, int ldDsh, const int* blk_lo,
                        const int* blk_hi, int band, CallScalars* sc, hipStream_t s);
