@@ -56,8 +56,6 @@ struct Session {
     int device = 0;
     hipStream_t stream = nullptr;
     double* d_rys_coef = nullptr;
-    double* d_rys_r2 = nullptr;
-    double* d_rys_w = nullptr;
     float* d_rys_coef32 = nullptr;
     lsjk::RysTable rys{};
     lsjk::CallScalars* d_sc = nullptr;
@@ -106,9 +104,8 @@ void dev_free(T*& p)
 
 // FP32 Rys rule derived from the FP64 table: on each bin, the degree-(kRysNcoef32-1) Chebyshev
 // interpolant (at the Chebyshev points of the first kind) of each FP64 polynomial, converted to
-// monomial coefficients in the bin variable u and rounded to FP32.  Blocks are padded to a
-// multiple of 4 floats so every block starts 16-byte aligned.
-void build_rys_f32(std::vector<float>& out, int* offset32)
+// monomial coefficients in v = u / 2 and rounded to FP32 (rys_offset(n, kRysNcoef32)).
+void build_rys_f32(std::vector<float>& out)
 {
     constexpr int NC = LSJK_RYS_NCOEF, M = lsjk::kRysNcoef32;
     // monomial coefficients of the Chebyshev polynomials T_0..T_{M-1}
@@ -120,10 +117,7 @@ void build_rys_f32(std::vector<float>& out, int* offset32)
     double node[M];
     for (int j = 0; j < M; j++) node[j] = std::cos(M_PI * (j + 0.5) / M);
     out.clear();
-    offset32[0] = 0;
-    for (int n = 1; n <= 9; n++) {
-        while (out.size() % 4) out.push_back(0.0f);
-        offset32[n] = (int)out.size();
+    for (int n = 1; n <= 9; n++)
         for (int b = 0; b < lsjk_rys_nbin[n]; b++)
             for (int i = 0; i < n; i++)
                 for (int xw = 0; xw < 2; xw++) {
@@ -141,10 +135,8 @@ void build_rys_f32(std::vector<float>& out, int* offset32)
                         ck *= (k == 0 ? 1.0 : 2.0) / M;
                         for (int q = 0; q < M; q++) mono[q] += ck * Tm[k][q];
                     }
-                    for (int q = 0; q < M; q++) out.push_back((float)mono[q]);
+                    for (int q = 0; q < M; q++) out.push_back((float)std::ldexp(mono[q], q));
                 }
-    }
-    while (out.size() % 4) out.push_back(0.0f);
 }
 
 void require_init()
@@ -2671,27 +2663,19 @@ int lsjk_init(int device)
         int lds = 0;
         HIPCHK(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
         S.max_lds = (size_t)lds;
+        // coefficient k times 2^k: the device's bin variable is v = u / 2 (exact)
         std::vector<double> coef(lsjk_rys_coef, lsjk_rys_coef + sizeof(lsjk_rys_coef) / sizeof(double));
-        std::vector<double> r2(lsjk_rys_asym_r2, lsjk_rys_asym_r2 + sizeof(lsjk_rys_asym_r2) / sizeof(double));
-        std::vector<double> w(lsjk_rys_asym_w, lsjk_rys_asym_w + sizeof(lsjk_rys_asym_w) / sizeof(double));
+        for (size_t i = 0; i < coef.size(); i++) coef[i] = std::ldexp(coef[i], (int)(i % LSJK_RYS_NCOEF));
         S.d_rys_coef = dev_upload(coef);
-        S.d_rys_r2 = dev_upload(r2);
-        S.d_rys_w = dev_upload(w);
         S.rys.coef = S.d_rys_coef;
-        S.rys.asym_r2 = S.d_rys_r2;
-        S.rys.asym_w = S.d_rys_w;
-        for (int n = 0; n < 10; n++) {
-            S.rys.offset[n] = lsjk_rys_offset[n];
-            S.rys.nbin[n] = lsjk_rys_nbin[n];
-            S.rys.h_inv[n] = (n > 0) ? 1.0 / lsjk_rys_h[n] : 0.0;
-            S.rys.Tc[n] = lsjk_rys_Tc[n];
-        }
-        {
-            std::vector<float> c32;
-            build_rys_f32(c32, S.rys.offset32);
-            S.d_rys_coef32 = dev_upload(c32);
-            S.rys.coef32 = S.d_rys_coef32;
-        }
+        std::vector<float> c32;
+        build_rys_f32(c32);
+        S.d_rys_coef32 = dev_upload(c32);
+        S.rys.coef32 = S.d_rys_coef32;
+        for (int n = 1; n < 10; n++)
+            if (lsjk_rys_nbin[n] != lsjk::kRysNbin[n] || lsjk_rys_offset[n] != lsjk::rys_offset(n) || lsjk_rys_h[n] != 1.0 ||
+                lsjk_rys_Tc[n] != lsjk_rys_nbin[n])
+                throw LsjkError(LSJK_E_INVALID, "lsjk_init: rys_asym.inc and rys_table.inc do not belong together");
         HIPCHK(hipMalloc((void**)&S.d_sc, sizeof(lsjk::CallScalars)));
         for (auto& e : S.ev) HIPCHK(hipEventCreate(&e));
         // device address of the no-alloc scratch array on this device (the device is current)
@@ -2710,8 +2694,6 @@ int lsjk_finalize(void)
         if (!S.init) return;
         (void)hipStreamSynchronize(S.stream);
         dev_free(S.d_rys_coef);
-        dev_free(S.d_rys_r2);
-        dev_free(S.d_rys_w);
         dev_free(S.d_rys_coef32);
         dev_free(S.d_sc);
         if (S.ws) (void)hipFree(S.ws);
@@ -3156,7 +3138,7 @@ int lsjk_coulomb_grad(const lsjk_pairlist* pl, const double* Dbra_dev, const dou
                     qa.ket_hstart = pl->hstart[L34];
                     qa.ket_d = kd + pl->hoff[L34];
                     qa.sc = S.d_sc;
-                    launch_j_quartets_grad(L12 + 1, L34, qa, (const JTask*)seg.d_tasks + seg.off[L12][L34],
+                    launch_j_quartets(L12 + 1, L34, kRoutePlain, qa, (const JTask*)seg.d_tasks + seg.off[L12][L34],
                                            seg.cnt[L12][L34], &S.d_sc->queue[jcount_index(L12, L34)], st);
                 }
             JGradArgs ga{};

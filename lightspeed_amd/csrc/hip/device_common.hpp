@@ -102,68 +102,89 @@ __device__ __forceinline__ void static_for(F&& f)
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// Rys table in device memory: pointers set up by the library at init.
-struct RysTable {
-    const double* coef;      // [offset[n] + bin*n*2*NCOEF + root*2*NCOEF + {x|w}*NCOEF + k]
-    const double* asym_r2;   // [n(n-1)/2 + i]
-    const double* asym_w;
-    int offset[10];
-    int nbin[10];
-    double h_inv[10];
-    double Tc[10];
-    // FP32 rule for the single-precision route: same bins, kRysNcoef32 coefficients per
-    // polynomial, layout [offset32[n] + bin*n*2*kRysNcoef32 + root*2*kRysNcoef32 + {x|w}*kRysNcoef32 + k]
-    const float* coef32;
-    int offset32[10];
-};
+#include "../common/rys_asym.inc"
 
+// Rys table in device memory, set up by the library at init: per nrys n, root and bin the
+// coefficients of x = t^2 and of the weight in v = T - b - 1/2 on [b, b + 1), FP64 at
+// rys_offset(n) + bin n 2 kRysNcoef + root 2 kRysNcoef + {x|w} kRysNcoef + k, and the FP32 rule for
+// the single-precision route (same bins, kRysNcoef32 coefficients per polynomial).
+struct RysTable {
+    const double* coef;
+    const float* coef32;
+};
+constexpr int kRysNcoef = 12;
 // Coefficients per polynomial of the FP32 rule: a degree-5 Chebyshev interpolant of the FP64
 // polynomial on each bin reaches the FP32 rounding floor (1.2e-7 relative to F0).
 constexpr int kRysNcoef32 = 6;
-
-// Evaluate the nrys-root rule: x_i = t_i^2, w_i.  The oracle's rys_eval evaluates the same rule
-// (same table, same asymptotic formula; here 1/T and T^(-1/2) come from one rsqrt).
-// A non-finite T takes the asymptotic branch (no table access), and the bin is clamped, so the
-// table is never read out of bounds.
-template <int NRYS>
-__device__ __forceinline__ void rys_roots(const RysTable& tab, double T, double* x, double* w)
+__host__ __device__ constexpr int rys_offset(int n, int ncoef = kRysNcoef)
 {
-    constexpr int NC = 12;  // LSJK_RYS_NCOEF
-    if (!(T < tab.Tc[NRYS])) {
-        const double s = rsqrt(T);
-        const double iT = s * s;
-#pragma unroll
-        for (int i = 0; i < NRYS; i++) {
-            x[i] = tab.asym_r2[NRYS * (NRYS - 1) / 2 + i] * iT;
-            w[i] = tab.asym_w[NRYS * (NRYS - 1) / 2 + i] * s;
-        }
-        return;
-    }
-    const double sT = T * tab.h_inv[NRYS];  // 0 <= T < Tc here
-    const int b = min((int)sT, tab.nbin[NRYS] - 1);
-    const double u = 2.0 * (sT - b) - 1.0;
-    const double* c = tab.coef + tab.offset[NRYS] + (size_t)b * NRYS * 2 * NC;
+    int o = 0;
+    for (int k = 1; k < n; k++) o += kRysNbin[k] * k * 2 * ncoef;
+    return o;
+}
+
+// Bin b of T in [0, Tc) and v = T - b - 1/2: adding 1.5 2^52 rounds T - 1/2 to an integer in the low
+// word of the sum, which is the bin (at a bin's edge either neighbour, whose polynomials both hold
+// there).  Four FP64 additions, where a conversion to an integer and back takes two quarter-rate
+// instructions.  The bin is clamped, so the table is never read out of bounds.
+template <int NRYS>
+__device__ __forceinline__ int rys_bin(double T, double& v)
+{
+    constexpr double kRound = 6755399441055744.0;
+    const double a = T - 0.5, t = a + kRound;
+    v = a - (t - kRound);
+    return (int)min((unsigned int)__double2loint(t), (unsigned int)(kRysNbin[NRYS] - 1));
+}
+
+// Large-T rule: x_i = r2_i / T, w_i = W_i / sqrt(T), 1/T and T^(-1/2) from one rsqrt; the constants
+// are compile-time.
+template <int NRYS, typename Real>
+__device__ __forceinline__ void rys_asym(double T, Real* x, Real* w)
+{
+    const double s = rsqrt(T);
+    const double iT = s * s;
 #pragma unroll
     for (int i = 0; i < NRYS; i++) {
-        const double* cx = c + i * 2 * NC;
-        const double* cw = cx + NC;
-        double px = cx[NC - 1];
-        double pw = cw[NC - 1];
+        x[i] = (Real)(kRysAsymR2[NRYS * (NRYS - 1) / 2 + i] * iT);
+        w[i] = (Real)(kRysAsymW[NRYS * (NRYS - 1) / 2 + i] * s);
+    }
+}
+
+// The bin polynomials of all roots at v; c: the bin's NRYS x {x|w} x NC coefficients.
+template <int NRYS, int NC, typename Real>
+__device__ __forceinline__ void rys_poly(const Real* c, Real v, Real* x, Real* w)
+{
+#pragma unroll
+    for (int i = 0; i < NRYS; i++) {
+        const Real* cx = c + i * 2 * NC;
+        const Real* cw = cx + NC;
+        Real px = cx[NC - 1], pw = cw[NC - 1];
 #pragma unroll
         for (int k = NC - 2; k >= 0; k--) {
-            px = fma(px, u, cx[k]);
-            pw = fma(pw, u, cw[k]);
+            px = fma(px, v, cx[k]);
+            pw = fma(pw, v, cw[k]);
         }
         x[i] = px;
         w[i] = pw;
     }
 }
 
+// Evaluate the nrys-root rule from the global table: x_i = t_i^2, w_i (the oracle's rys_eval evaluates
+// the same rule).  A non-finite T takes the asymptotic branch (no table access).
+template <int NRYS>
+__device__ __forceinline__ void rys_roots(const RysTable& tab, double T, double* x, double* w)
+{
+    if (!(T < (double)kRysNbin[NRYS])) return rys_asym<NRYS>(T, x, w);
+    double v;
+    const int b = rys_bin<NRYS>(T, v);
+    rys_poly<NRYS, kRysNcoef>(tab.coef + rys_offset(NRYS) + (size_t)b * NRYS * 2 * kRysNcoef, v, x, w);
+}
+
 // LDS copy of the table block of one nrys: [bin][root][x|w][12] doubles with one pad double per
 // bin, so that lanes reading the same coefficient of different bins hit different LDS banks (an
 // unpadded bin of 24 nrys doubles puts every bin on the same few banks).
 __host__ __device__ constexpr int rys_lds_stride(int nrys) { return nrys * 2 * 12 + 1; }
-__host__ __device__ constexpr size_t rys_lds_doubles(int nbin, int nrys) { return (size_t)nbin * rys_lds_stride(nrys); }
+__host__ __device__ constexpr size_t rys_lds_doubles(int nrys) { return (size_t)kRysNbin[nrys] * rys_lds_stride(nrys); }
 
 // Kernels stage the table block in LDS for nrys <= 3 (at most 27.6 KB, so several workgroups
 // share a CU); for more roots they read it from global memory (rys_roots).
@@ -182,9 +203,9 @@ __device__ __forceinline__ void rys_roots_any(const RysTable& tab, const double*
 template <int NRYS>
 __device__ __forceinline__ void rys_stage_lds(const RysTable& tab, double* s_coef)
 {
-    constexpr int B = NRYS * 2 * 12, S = rys_lds_stride(NRYS);
-    const int n = tab.nbin[NRYS] * B;
-    const double* src = tab.coef + tab.offset[NRYS];
+    constexpr int B = NRYS * 2 * kRysNcoef, S = rys_lds_stride(NRYS);
+    constexpr int n = kRysNbin[NRYS] * B;
+    const double* src = tab.coef + rys_offset(NRYS);
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         const int b = i / B;
         s_coef[b * S + (i - b * B)] = src[i];
@@ -193,38 +214,12 @@ __device__ __forceinline__ void rys_stage_lds(const RysTable& tab, double* s_coe
 
 // rys_roots with the coefficients of this nrys read from LDS (staged by rys_stage_lds).
 template <int NRYS>
-__device__ __forceinline__ void rys_roots_lds(const RysTable& tab, const double* s_coef, double T, double* x,
-                                              double* w)
+__device__ __forceinline__ void rys_roots_lds(const double* s_coef, double T, double* x, double* w)
 {
-    constexpr int NC = 12;
-    if (!(T < tab.Tc[NRYS])) {
-        const double s = rsqrt(T);
-        const double iT = s * s;
-#pragma unroll
-        for (int i = 0; i < NRYS; i++) {
-            x[i] = tab.asym_r2[NRYS * (NRYS - 1) / 2 + i] * iT;
-            w[i] = tab.asym_w[NRYS * (NRYS - 1) / 2 + i] * s;
-        }
-        return;
-    }
-    const double sT = T * tab.h_inv[NRYS];  // 0 <= T < Tc here
-    const int b = min((int)sT, tab.nbin[NRYS] - 1);
-    const double u = 2.0 * (sT - b) - 1.0;
-    const double* c = s_coef + (size_t)b * rys_lds_stride(NRYS);
-#pragma unroll
-    for (int i = 0; i < NRYS; i++) {
-        const double* cx = c + i * 2 * NC;
-        const double* cw = cx + NC;
-        double px = cx[NC - 1];
-        double pw = cw[NC - 1];
-#pragma unroll
-        for (int k = NC - 2; k >= 0; k--) {
-            px = fma(px, u, cx[k]);
-            pw = fma(pw, u, cw[k]);
-        }
-        x[i] = px;
-        w[i] = pw;
-    }
+    if (!(T < (double)kRysNbin[NRYS])) return rys_asym<NRYS>(T, x, w);
+    double v;
+    const int b = rys_bin<NRYS>(T, v);
+    rys_poly<NRYS, kRysNcoef>(s_coef + __umul24(b, rys_lds_stride(NRYS)), v, x, w);
 }
 
 template <int NRYS>
@@ -232,7 +227,7 @@ __device__ __forceinline__ void rys_roots_any(const RysTable& tab, const double*
                                               double* w)
 {
     if constexpr (rys_staged(NRYS))
-        rys_roots_lds<NRYS>(tab, s_coef, T, x, w);
+        rys_roots_lds<NRYS>(s_coef, T, x, w);
     else
         rys_roots<NRYS>(tab, T, x, w);
 }
@@ -245,40 +240,15 @@ __host__ __device__ constexpr int rys32_lds_stride(int nrys) { return nrys * 2 *
 // from `c32`: the global table (LDS = false) or an LDS copy of this nrys block with padded bins
 // (LDS = true).
 template <int NRYS, bool LDS>
-__device__ __forceinline__ void rys_roots_f32(const RysTable& tab, const float* c32, double T, float* x, float* w)
+__device__ __forceinline__ void rys_roots_f32(const float* c32, double T, float* x, float* w)
 {
-    constexpr int NC = kRysNcoef32;
-    if (!(T < tab.Tc[NRYS])) {
-        const double s = rsqrt(T);
-        const double iT = s * s;
-#pragma unroll
-        for (int i = 0; i < NRYS; i++) {
-            x[i] = (float)(tab.asym_r2[NRYS * (NRYS - 1) / 2 + i] * iT);
-            w[i] = (float)(tab.asym_w[NRYS * (NRYS - 1) / 2 + i] * s);
-        }
-        return;
-    }
-    const double sT = T * tab.h_inv[NRYS];  // 0 <= T < Tc here
-    const int b = min((int)sT, tab.nbin[NRYS] - 1);
-    const float u = (float)(2.0 * (sT - b) - 1.0);
-    const float* c = c32 + (size_t)b * (LDS ? rys32_lds_stride(NRYS) : NRYS * 2 * NC);
-#pragma unroll
-    for (int i = 0; i < NRYS; i++) {
-        const float* cx = c + i * 2 * NC;
-        const float* cw = cx + NC;
-        float px = cx[NC - 1];
-        float pw = cw[NC - 1];
-#pragma unroll
-        for (int k = NC - 2; k >= 0; k--) {
-            px = fmaf(px, u, cx[k]);
-            pw = fmaf(pw, u, cw[k]);
-        }
-        x[i] = px;
-        w[i] = pw;
-    }
+    if (!(T < (double)kRysNbin[NRYS])) return rys_asym<NRYS>(T, x, w);
+    double v;
+    const int b = rys_bin<NRYS>(T, v);
+    rys_poly<NRYS, kRysNcoef32>(c32 + __umul24(b, LDS ? rys32_lds_stride(NRYS) : NRYS * 2 * kRysNcoef32), (float)v, x, w);
 }
 
-__host__ __device__ constexpr size_t rys32_lds_floats(int nbin, int nrys) { return (size_t)nbin * rys32_lds_stride(nrys); }
+__host__ __device__ constexpr size_t rys32_lds_floats(int nrys) { return (size_t)kRysNbin[nrys] * rys32_lds_stride(nrys); }
 
 // Kernels of the FP32 route stage the FP32 block in LDS for nrys <= 5 (at most 14.2 KB).
 __host__ __device__ constexpr bool rys32_staged(int nrys) { return nrys <= 5; }
@@ -288,8 +258,8 @@ template <int NRYS>
 __device__ __forceinline__ void rys32_stage_lds(const RysTable& tab, float* s_coef)
 {
     constexpr int B = NRYS * 2 * kRysNcoef32, S = rys32_lds_stride(NRYS);
-    const int n = tab.nbin[NRYS] * B;
-    const float* src = tab.coef32 + tab.offset32[NRYS];
+    constexpr int n = kRysNbin[NRYS] * B;
+    const float* src = tab.coef32 + rys_offset(NRYS, kRysNcoef32);
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         const int b = i / B;
         s_coef[b * S + (i - b * B)] = src[i];

@@ -300,7 +300,7 @@ void launch_k_grad_l12(int L3, int L4, const KGradArgs& a, hipStream_t s)
 #define CASE(C, D)                                                                               \
     if (L3 == C && L4 == D) {                                                                    \
         constexpr int NR = (L1 + L2 + C + D + 1) / 2 + 1;                                        \
-        const size_t lds = rys_staged(NR) ? rys_lds_doubles(a.rys.nbin[NR], NR) * sizeof(double) : 0; \
+        const size_t lds = rys_staged(NR) ? rys_lds_doubles(NR) * sizeof(double) : 0; \
         hipLaunchKernelGGL((k_grad<L1, L2, C, D>), grid, block, lds, s, a);                      \
         return;                                                                                  \
     }

@@ -196,10 +196,10 @@ __device__ __forceinline__ void k_quartet(const RysTable& tab, const void* s_tab
         const Real d2 = (Real)d2_;
         Real x[NR], w[NR];
         if constexpr (std::is_same<Real, float>::value)
-            rys_roots_f32<NR, STAGED>(tab, STAGED ? static_cast<const float*>(s_tab) : tab.coef32 + tab.offset32[NR],
+            rys_roots_f32<NR, STAGED>(STAGED ? static_cast<const float*>(s_tab) : tab.coef32 + rys_offset(NR, kRysNcoef32),
                                       (double)(rho * d2) * r2, x, w);
         else if constexpr (STAGED)
-            rys_roots_lds<NR>(tab, static_cast<const double*>(s_tab), rho * d2 * r2, x, w);
+            rys_roots_lds<NR>(static_cast<const double*>(s_tab), rho * d2 * r2, x, w);
         else
             rys_roots<NR>(tab, rho * d2 * r2, x, w);
 #pragma unroll
@@ -359,12 +359,12 @@ struct KKetLds {
     static constexpr int N13 = ncart(L1) * ncart(L3);  // accumulator doubles per group row
     static __host__ __device__ size_t bytes64(const RysTable& tab)
     {
-        return STAGED64 ? rys_lds_doubles(tab.nbin[NR], NR) * sizeof(double) : 0;
+        return STAGED64 ? rys_lds_doubles(NR) * sizeof(double) : 0;
     }
     // byte offset of the accumulators: after both tables, 8-byte aligned
     static __host__ __device__ size_t acc_offset(const RysTable& tab)
     {
-        const size_t b = bytes64(tab) + (STAGED32 ? rys32_lds_floats(tab.nbin[NR], NR) * sizeof(float) : 0);
+        const size_t b = bytes64(tab) + (STAGED32 ? rys32_lds_floats(NR) * sizeof(float) : 0);
         return (b + 7) & ~(size_t)7;
     }
     static size_t bytes(const RysTable& tab, int gsize)

@@ -313,10 +313,10 @@ void launch_j_bra_scatter(int LA, int LB, const JScatterArgs& a, int k0, int nk,
 __host__ __device__ constexpr bool js_enabled(int L12, int L34) { return L12 >= L34 && L34 == 0; }
 void launch_j_quartets_sym(int L12, int L34, int route, const JQuartetArgs& a, const JTask* tasks, int ntask,
                            unsigned int* qctr, hipStream_t s);
+// Bra order 5 (gradients: bra order L12 + 1) runs the FP64 route only.
 void launch_j_quartets(int L12, int L34, int route, const JQuartetArgs& a, const JTask* tasks, int ntask,
                        unsigned int* qctr, hipStream_t s);
-void launch_j_quartets_grad(int L12p1, int L34, const JQuartetArgs& a, const JTask* tasks, int ntask,
-                            unsigned int* qctr, hipStream_t s);
+
 
 // Work-queue counters of one call (CallScalars::queue, zeroed with the call's scalars): J classes
 // at jcount_index.
@@ -335,8 +335,8 @@ inline size_t kket_lds_bytes(const RysTable& tab, int L1, int L2, int L3, int L4
 {
     const int NR = (L1 + L2 + L3 + L4) / 2 + 1;
     size_t b = 0;
-    if (rys_staged(NR)) b += rys_lds_doubles(tab.nbin[NR], NR) * sizeof(double);
-    if (route == kRouteMixed && rys32_staged(NR)) b += rys32_lds_floats(tab.nbin[NR], NR) * sizeof(float);
+    if (rys_staged(NR)) b += rys_lds_doubles(NR) * sizeof(double);
+    if (route == kRouteMixed && rys32_staged(NR)) b += rys32_lds_floats(NR) * sizeof(float);
     b = (b + 7) & ~(size_t)7;
     return b + (size_t)kKWaves * (gsize * ncart(L1) * ncart(L3) * sizeof(double) + kKQueueBytes);
 }

@@ -236,6 +236,15 @@ def main():
     with open(OUT, "w") as fh:
         fh.write("\n".join(lines) + "\n")
     print("wrote", os.path.normpath(OUT), "doubles:", off)
+    # the compile-time part for the device, whose bin arithmetic needs bins of width 1
+    assert all(table[n][1] == 1.0 and table[n][3] == table[n][0] for n in range(1, NMAX + 1))
+    with open(os.path.join(os.path.dirname(OUT), "rys_asym.inc"), "w") as fh:
+        fh.write("/* Generated by lightspeed_amd/tables/gen_rys.py with rys_table.inc -- do not edit.\n"
+                 " * Compile-time part of the Rys table for the device: bins of width 1 per nrys (Tc = the number of\n"
+                 " * bins), and the large-T rule, packed [n][i] with offset n (n - 1) / 2.\n */\n")
+        fh.write("constexpr int kRysNbin[%d] = {0, %s};\n" % (NMAX + 1, ", ".join(str(table[n][0]) for n in range(1, NMAX + 1))))
+        fh.write("constexpr double kRysAsymR2[%d] = {%s};\n" % (len(r2s), ", ".join("%.17e" % v for v in r2s)))
+        fh.write("constexpr double kRysAsymW[%d] = {%s};\n" % (len(Ws), ", ".join("%.17e" % v for v in Ws)))
 
 
 if __name__ == "__main__":
