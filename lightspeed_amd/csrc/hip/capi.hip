@@ -57,6 +57,7 @@ struct Session {
     hipStream_t stream = nullptr;
     double* d_rys_coef = nullptr;
     float* d_rys_coef32 = nullptr;
+    double* d_boys = nullptr;
     lsjk::RysTable rys{};
     lsjk::CallScalars* d_sc = nullptr;
     void* ws = nullptr;
@@ -137,6 +138,45 @@ void build_rys_f32(std::vector<float>& out)
                     }
                     for (int q = 0; q < M; q++) out.push_back((float)std::ldexp(mono[q], q));
                 }
+}
+
+// The Boys tables (boys_offset): per bin the degree-11 Chebyshev interpolant of F_L, as monomial
+// coefficients in v, from its power series F_L(T) = exp(-T) sum_k (2T)^k / ((2L+1)(2L+3)..(2L+2k+1)) in
+// extended precision, and exp(-(b + 1/2)).
+std::vector<double> build_boys()
+{
+    constexpr int M = lsjk::kRysNcoef;
+    typedef long double ld;
+    const ld pi = std::acos((ld)-1);
+    ld Tm[M][M] = {};
+    Tm[0][0] = 1;
+    Tm[1][1] = 1;
+    for (int k = 2; k < M; k++)
+        for (int j = 0; j < M; j++) Tm[k][j] = (j > 0 ? 2 * Tm[k - 1][j - 1] : 0) - Tm[k - 2][j];
+    std::vector<double> out;
+    for (int L = 2; L <= 4; L++)
+        for (int b = 0; b < lsjk::kRysNbin[L / 2 + 1]; b++) {
+            ld f[M];
+            for (int j = 0; j < M; j++) {
+                const ld T = b + (ld)0.5 + (ld)0.5 * std::cos(pi * (j + (ld)0.5) / M);
+                ld term = (ld)1 / (2 * L + 1), sum = term;
+                for (int k = 1; k < 400 && term > sum * (ld)1e-22; k++) {
+                    term *= 2 * T / (2 * L + 2 * k + 1);
+                    sum += term;
+                }
+                f[j] = std::exp(-T) * sum;
+            }
+            ld mono[M] = {};
+            for (int k = 0; k < M; k++) {
+                ld ck = 0;
+                for (int j = 0; j < M; j++) ck += f[j] * std::cos(pi * k * (j + (ld)0.5) / M);
+                ck *= (k == 0 ? (ld)1 : (ld)2) / M;
+                for (int q = 0; q < M; q++) mono[q] += ck * Tm[k][q];
+            }
+            for (int q = 0; q < M; q++) out.push_back((double)std::ldexp(mono[q], q));
+            out.push_back((double)std::exp(-(b + (ld)0.5)));
+        }
+    return out;
 }
 
 void require_init()
@@ -413,7 +453,20 @@ void build_pairlist(lsjk_pairlist* pl)
     pl->d_bound = dev_upload(pl->h_bound);
     pl->d_hpos = dev_upload(hpos);
     pl->d_K = dev_upload(K);
-    pl->d_hb = dev_upload(pl->h_hb);
+    {
+        // the ket side reads one pair past a range's end
+        std::vector<float> hb(pl->h_hb);
+        hb.push_back(0.0f);
+        pl->d_hb = dev_upload(hb);
+        std::vector<double> rec((size_t)kJKetDoubles * (n + 1), 0.0);
+        for (int h = 0; h < n; h++) {
+            double* r = rec.data() + (size_t)kJKetDoubles * h;
+            r[0] = hgeom[h];
+            r[1] = hgeom[(size_t)4 * n + h];
+            for (int d = 0; d < 3; d++) r[2 + d] = hgeom[(size_t)(d + 1) * n + h];
+        }
+        pl->d_hrec = dev_upload(rec);
+    }
     pl->d_hgeom = dev_upload(hgeom);
     pl->d_row_start = dev_upload(pl->h_row_start);
     pl->d_ebound = dev_upload(eb);
@@ -469,6 +522,7 @@ void free_pairlist(lsjk_pairlist* pl)
     dev_free(pl->d_K);
     dev_free(pl->d_hb);
     dev_free(pl->d_hgeom);
+    dev_free(pl->d_hrec);
     dev_free(pl->d_row_start);
     dev_free(pl->d_ebound);
     dev_free(pl->d_ebk);
@@ -1474,8 +1528,9 @@ static void coulomb_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, c
         double* kd = nullptr;
         double* jp = nullptr;
         Workspace wsp;
-        wsp.add(&kb, (size_t)pl34->npair);
-        wsp.add(&kd, pl34->hoff[2 * kMaxL + 1]);
+        // one ket more than the list's: the kernels read one past a range's end
+        wsp.add(&kb, (size_t)pl34->npair + 1);
+        wsp.add(&kd, pl34->hoff[2 * kMaxL + 1] + kMaxHerm);
         wsp.add(&jp, pl12->hoff[2 * kMaxL + 1]);
         float* kd32 = nullptr;
         if (mixed) wsp.add(&kd32, pl34->hoff[2 * kMaxL + 1]);
@@ -1554,8 +1609,7 @@ static void coulomb_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, c
                     qa.jp = jp + pl12->hoff[L12];
                     qa.ket_b = kb;
                     qa.ket_static_b = pl34->d_hb;
-                    qa.ket_geom = pl34->d_hgeom;
-                    qa.ket_n = pl34->npair;
+                    qa.ket_rec = pl34->d_hrec;
                     qa.ket_hstart = pl34->hstart[L34];
                     qa.ket_d = kd + pl34->hoff[L34];
                     qa.ket_d32 = kd32 ? kd32 + pl34->hoff[L34] : nullptr;
@@ -2520,7 +2574,7 @@ size_t batch_ws_bytes(const lsjk_batch* b, bool mixed, size_t* jbytes)
     auto r = [](size_t n) { return (std::max<size_t>(1, n) + 255) & ~size_t(255); };
     const lsjk_pairlist* pl = b->list;
     const size_t h = pl->hoff[2 * lsjk::kMaxL + 1];
-    size_t j = r((size_t)pl->npair * sizeof(float)) + r(h * sizeof(double)) + r(h * sizeof(double));
+    size_t j = r(((size_t)pl->npair + 1) * sizeof(float)) + r((h + lsjk::kMaxHerm) * sizeof(double)) + r(h * sizeof(double));
     if (mixed) j += r(h * sizeof(float));
     *jbytes = j;
     return j + r(blk_elems(b->basis, b->basis) * sizeof(double)) + r(rowmax_elems(pl, b->basis) * sizeof(unsigned int));
@@ -2672,6 +2726,8 @@ int lsjk_init(int device)
         build_rys_f32(c32);
         S.d_rys_coef32 = dev_upload(c32);
         S.rys.coef32 = S.d_rys_coef32;
+        S.d_boys = dev_upload(build_boys());
+        S.rys.boys = S.d_boys;
         for (int n = 1; n < 10; n++)
             if (lsjk_rys_nbin[n] != lsjk::kRysNbin[n] || lsjk_rys_offset[n] != lsjk::rys_offset(n) || lsjk_rys_h[n] != 1.0 ||
                 lsjk_rys_Tc[n] != lsjk_rys_nbin[n])
@@ -2695,6 +2751,7 @@ int lsjk_finalize(void)
         (void)hipStreamSynchronize(S.stream);
         dev_free(S.d_rys_coef);
         dev_free(S.d_rys_coef32);
+        dev_free(S.d_boys);
         dev_free(S.d_sc);
         if (S.ws) (void)hipFree(S.ws);
         S.ws = nullptr;
@@ -3090,8 +3147,8 @@ int lsjk_coulomb_grad(const lsjk_pairlist* pl, const double* Dbra_dev, const dou
         double* kd = nullptr;
         double* vp = nullptr;
         Workspace wsp;
-        wsp.add(&kb, (size_t)pl->npair);
-        wsp.add(&kd, pl->hoff[2 * kMaxL + 1]);
+        wsp.add(&kb, (size_t)pl->npair + 1);
+        wsp.add(&kd, pl->hoff[2 * kMaxL + 1] + kMaxHerm);
         wsp.add(&vp, hoff2[2 * kMaxL + 1]);
         wsp.commit();
         const JTaskList& seg = *get_jtasks(pl, pl);
@@ -3133,8 +3190,7 @@ int lsjk_coulomb_grad(const lsjk_pairlist* pl, const double* Dbra_dev, const dou
                     qa.jp = vp + hoff2[L12];
                     qa.ket_b = kb;
                     qa.ket_static_b = pl->d_hb;
-                    qa.ket_geom = pl->d_hgeom;
-                    qa.ket_n = pl->npair;
+                    qa.ket_rec = pl->d_hrec;
                     qa.ket_hstart = pl->hstart[L34];
                     qa.ket_d = kd + pl->hoff[L34];
                     qa.sc = S.d_sc;
@@ -3369,8 +3425,9 @@ int lsjk_count_quartets(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, co
         double* Dsh = nullptr;
         unsigned long long* out = nullptr;
         Workspace wsp;
-        wsp.add(&kb, (size_t)pl34->npair);
-        wsp.add(&kd, pl34->hoff[2 * kMaxL + 1]);
+        // one ket more than the list's: the kernels read one past a range's end
+        wsp.add(&kb, (size_t)pl34->npair + 1);
+        wsp.add(&kd, pl34->hoff[2 * kMaxL + 1] + kMaxHerm);
         wsp.add(&Dsh, (size_t)b2->nblk * b4->nblk);
         wsp.add(&out, 2 * 625);
         wsp.commit();

@@ -12,8 +12,9 @@
 // Kernels (one launch each per call, per class):
 //   j_ket_prep<LA,LB>    one thread per ket pair: truncated bound, Hermite density d_u.
 //   j_quartets<L12,L34>  one wave per (64 bra pairs x ket chunk) task: each lane owns one bra
-//                        pair and sweeps the chunk's kets, staged through LDS; Hermite integrals
-//                        R_{t+u} by Rys quadrature; jp_t += sum_u R_{t+u} d_u in registers.
+//                        pair and sweeps the chunk's kets (scalar loads); Hermite integrals R_{t+u}
+//                        from Boys functions or by Rys quadrature; jp_t += sum_u R_{t+u} d_u in
+//                        registers (coulomb_impl.hpp).
 //   j_bra_scatter<LA,LB> one thread per bra pair: J_ab += K sum_t E E E jp_t (symmetrised).
 #include "internal.hpp"
 #include "kernels.hpp"

@@ -109,14 +109,91 @@ __device__ __forceinline__ void for_each_root(const RysTable& tab, const void* s
     }
 }
 
-// Hermite Coulomb integrals R_{tuv} (t+u+v <= L) of one bra-ket pair by Rys quadrature:
-// R_{tuv} = pref * sum_i w_i Hx_t Hy_u Hz_v.
+// FP64 Hermite integrals of total order 2 .. 4 come from Boys functions by the McMurchie-Davidson
+// recursion (J. Comput. Phys. 26, 218 (1978)): one polynomial (F_L) and an exponential instead of one
+// polynomial per root and weight, and no sum over roots (order 4: about 130 FP64 operations against
+// 340, order 2: 50 against 108), with 13 table doubles per bin against 24 nrys.  Order 0 and 1 cost the
+// same either way; orders above 4 keep the factorised root sum (their recursion does not fit the
+// registers).
+constexpr bool j_md(int L) { return L >= 2 && L <= 4; }
+
+template <int L, int N>
+__device__ __forceinline__ void md_level(const double (&b)[L + 1], double X, double Y, double Z,
+                                         double (&out)[nherm(L - N)])
+{
+    // R^(N)_t, |t| <= L - N, from R^(N+1): R^(n)_{t + 1_i} = X_i R^(n+1)_t + t_i R^(n+1)_{t - 1_i}
+    out[0] = b[N];
+    if constexpr (N < L) {
+        double prev[nherm(L - N - 1)];
+        md_level<L, N + 1>(b, X, Y, Z, prev);
+        static_for<nherm(L - N) - 1>([&](auto I_) {
+            constexpr int t = decltype(I_)::value + 1;
+            constexpr int tx = herm_tx(t), ty = herm_ty(t), tz = herm_tz(t);
+            // an axis of power one where there is one: its step has no second term
+            constexpr int ax = tx == 1 ? 0 : ty == 1 ? 1 : tz == 1 ? 2 : tx > 0 ? 0 : ty > 0 ? 1 : 2;
+            constexpr int n = ax == 0 ? tx : ax == 1 ? ty : tz;
+            constexpr int lx = tx - (ax == 0), ly = ty - (ax == 1), lz = tz - (ax == 2);
+            const double D = ax == 0 ? X : ax == 1 ? Y : Z;
+            if constexpr (n > 1)
+                out[t] = fma(D, prev[herm_index(lx, ly, lz)],
+                             double(n - 1) * prev[herm_index(lx - (ax == 0), ly - (ax == 1), lz - (ax == 2))]);
+            else
+                out[t] = D * prev[herm_index(lx, ly, lz)];
+        });
+    }
+}
+
+template <int L>
+__device__ __forceinline__ void hermite_R_md(const double* s_boys, const Ewald& ew, double p, double c12, double q,
+                                             double c34, double X, double Y, double Z, double (&R)[nherm(L)])
+{
+    const double psum = p + q;
+    const double rs = rsqrt_pos(psum);
+    const double rho = p * q * (rs * rs);
+    const double base = c12 * c34 * rs;  // 2 pi^{5/2} / (p q sqrt(p+q))
+    const double r2 = X * X + Y * Y + Z * Z;
+    double b[L + 1], F[L + 1];
+    if (ew.plain) {
+        boys_lds<L>(s_boys, rho * r2, F);
+        double f = ew.alpha[0] * base;
+#pragma unroll
+        for (int n = 0; n <= L; n++) {
+            b[n] = f * F[n];
+            f *= -2.0 * rho;
+        }
+    } else {
+        // the operator's terms differ in the Boys argument and the powers of d^2 only: one recursion
+#pragma unroll
+        for (int n = 0; n <= L; n++) b[n] = 0.0;
+        for (int it = 0; it < ew.n; it++) {
+            const double om = ew.omega[it];
+            double d2 = 1.0, f = ew.alpha[it] * base;
+            if (__double_as_longlong(om) != __double_as_longlong(-1.0)) {  // erf-attenuated term (bit test: scalar)
+                d2 = om * om / (rho + om * om);
+                f *= sqrt(d2);
+            }
+            const double rd = rho * d2;
+            boys_lds<L>(s_boys, rd * r2, F);
+#pragma unroll
+            for (int n = 0; n <= L; n++) {
+                b[n] = fma(f, F[n], b[n]);
+                f *= -2.0 * rd;
+            }
+        }
+    }
+    md_level<L, 0>(b, X, Y, Z, R);
+}
+
+// Hermite Coulomb integrals R_{tuv} (t+u+v <= L) of one bra-ket pair, by Rys quadrature
+// (R_{tuv} = pref * sum_i w_i Hx_t Hy_u Hz_v) or from Boys functions (j_md).
 template <typename Real, int L>
 __device__ __forceinline__ void hermite_R(const RysTable& tab, const void* s_tab, const Ewald& ew, double p12,
                                           double c12, double p34, double c34, double X, double Y, double Z,
                                           Real (&R)[nherm(L)])
 {
     constexpr int HL = nherm(L);
+    if constexpr (std::is_same<Real, double>::value && j_md(L))
+        return hermite_R_md<L>(static_cast<const double*>(s_tab), ew, p12, c12, p34, c34, X, Y, Z, R);
 #pragma unroll
     for (int t = 0; t < HL; t++) R[t] = Real(0);
     for_each_root<Real, L>(tab, s_tab, ew, p12, c12, p34, c34, X, Y, Z, [&](const HermRoot<Real, L>& H) __attribute__((always_inline)) {
@@ -175,54 +252,64 @@ __device__ __forceinline__ void hermite_contract_factorized(const RysTable& tab,
     });
 }
 
-// LDS of one j_quartets workgroup: the FP64 table block (routes with FP64 quartets, nrys <= 3),
-// then the FP32 block (routes with FP32 quartets).
+// LDS of one j_quartets workgroup: the FP64 table (the Boys table of the class's order for j_md, the
+// Rys block for nrys <= 3), then the FP32 Rys block on the mixed route.
 template <int L12, int L34, int ROUTE>
 struct JLds {
-    static constexpr int NR = (L12 + L34) / 2 + 1;
-    static constexpr bool HAS32 = ROUTE == kRouteLo || ROUTE == kRouteMixed;
-    static constexpr bool STAGED64 = ROUTE != kRouteLo && rys_staged(NR);
-    static __host__ __device__ size_t bytes64(const RysTable& tab)
+    static constexpr int L = L12 + L34, NR = L / 2 + 1;
+    static constexpr bool HAS32 = ROUTE == kRouteMixed;
+    static constexpr bool STAGED64 = j_md(L) || rys_staged(NR);
+    static constexpr size_t kBytes64 =
+        j_md(L) ? boys_lds_doubles(L) * sizeof(double) : rys_staged(NR) ? rys_lds_doubles(NR) * sizeof(double) : 0;
+    static constexpr size_t kBytes = kBytes64 + (HAS32 ? rys32_lds_floats(NR) * sizeof(float) : 0);
+    static __device__ __forceinline__ void stage(const RysTable& tab, double* s64, float* s32)
     {
-        return STAGED64 ? rys_lds_doubles(NR) * sizeof(double) : 0;
-    }
-    static size_t bytes(const RysTable& tab)
-    {
-        return bytes64(tab) + (HAS32 ? rys32_lds_floats(NR) * sizeof(float) : 0);
+        if constexpr (j_md(L))
+            boys_stage_lds<L>(tab, s64);
+        else if constexpr (rys_staged(NR))
+            rys_stage_lds<NR>(tab, s64);
+        if constexpr (HAS32) rys32_stage_lds<NR>(tab, s32);
+        if constexpr (STAGED64 || HAS32) __syncthreads();
     }
 };
 
+// One ket pair's geometry at a wave-uniform index (scalar loads).
+struct JKet {
+    double q, c, x, y, z;
+};
+__device__ __forceinline__ JKet load_ket(const double* __restrict__ rec, int k)
+{
+    const double* g = rec + (size_t)k * kJKetDoubles;
+    return {ld_const(g), ld_const(g + 1), ld_const(g + 2), ld_const(g + 3), ld_const(g + 4)};
+}
+
 // Persistent kernel: each wave takes (64 bra pairs x ket range) tasks from a queue until it is
-// empty.  The workgroup's waves share an LDS copy of the Rys table (FP64 rule for nrys <= 3 on the
-// routes with FP64 quartets, the FP32 rule on the routes with FP32 quartets).  Lanes own bra
-// pairs; the kets are read at wave-uniform addresses (scalar loads), in bound order.  ROUTE
-// selects the quartets by est = B12 * B34' (kRoutePlain / kRouteHi / kRouteLo), or evaluates
-// the mixed route in one launch (kRouteMixed): a ket step with any quartet at or above thredp is
-// evaluated in FP64, the others in FP32.
+// empty.  The workgroup's waves share an LDS copy of the tables (JLds).  Lanes own bra pairs; the
+// kets are read at wave-uniform addresses (scalar loads) one ket ahead of their use, in bound order
+// (the lists and per-call buffers are padded by one ket).  Quartets with est = B12 * B34' at or above
+// thresp are evaluated in FP64 (kRoutePlain), or on the mixed route (kRouteMixed) a ket step with any
+// quartet at or above thredp in FP64 and the others in FP32.
 template <int L12, int L34, int ROUTE>
 __global__ __launch_bounds__(256) void j_quartets(JQuartetArgs a, const JTask* __restrict__ tasks, int ntask,
                                                   unsigned int* qctr)
 {
     using Lds = JLds<L12, L34, ROUTE>;
-    constexpr int H12 = nherm(L12), H34 = nherm(L34), L = L12 + L34, HL = nherm(L), NR = L / 2 + 1;
-    constexpr bool LO = ROUTE == kRouteLo;
+    constexpr int H12 = nherm(L12), H34 = nherm(L34), L = L12 + L34, HL = nherm(L);
     constexpr bool MIXED = ROUTE == kRouteMixed;
+    constexpr int DN = H34 <= 4 ? H34 : 1;  // ket densities loaded ahead
     extern __shared__ double s_dyn[];
     double* s_tab64 = s_dyn;
-    float* s_tab32 = reinterpret_cast<float*>(reinterpret_cast<char*>(s_dyn) + Lds::bytes64(a.rys));
-    if constexpr (Lds::STAGED64) rys_stage_lds<NR>(a.rys, s_tab64);
-    if constexpr (Lds::HAS32) rys32_stage_lds<NR>(a.rys, s_tab32);
-    if constexpr (Lds::STAGED64 || Lds::HAS32) __syncthreads();
+    float* s_tab32 = reinterpret_cast<float*>(reinterpret_cast<char*>(s_dyn) + Lds::kBytes64);
+    Lds::stage(a.rys, s_tab64, s_tab32);
 
     const int lane = threadIdx.x & 63;
     const float thresp = a.thresp;
-    // quartets at or above `thre_lo` (and, on the FP32 route, below thredp) are evaluated
-    const float thre_lo = (ROUTE == kRouteHi) ? a.thredp : thresp;
     const float max34 = __uint_as_float(a.sc->max34_bits);
     const float thre_bra = thresp / max34;
     const double dmax = __longlong_as_double((long long)a.sc->dmax_bits);
+    // evaluated quartets and wave steps with one (scalar registers)
     unsigned long long nq = 0, nq32 = 0;
-    unsigned int nsteps = 0;  // wave steps with an evaluated quartet (counting mode)
+    unsigned int nsteps = 0;
 
     for (;;) {
         const int t = (int)wave_take(qctr);
@@ -248,51 +335,58 @@ __global__ __launch_bounds__(256) void j_quartets(JQuartetArgs a, const JTask* _
             c12 = a.bra_geom[4 * a.bra_n + bra];
         }
         const bool bra_ok = active && (B12 >= thre_bra);
+        if (!bra_ok) B12 = __builtin_nanf("");  // no estimate of the lane passes
         double jp[H12];
 #pragma unroll
         for (int u = 0; u < H12; u++) jp[u] = 0.0;
 
         // Early exit: B34' <= float(dmax * B34) and the static ket bounds are sorted, so no ket with
-        // static bound below kstop = thre_lo / (B12max dmax) (1 - 2^-21) can pass with a bra of the
+        // static bound below kstop = thresp / (B12max dmax) (1 - 2^-21) can pass with a bra of the
         // tile; the test compares bit patterns (non-negative floats) on the scalar unit.
-        const float kstop = (float)((double)thre_lo / ((double)B12max * dmax)) * (1.0f - 4.0f * 1.1920929e-7f);
+        const float kstop = (float)((double)thresp / ((double)B12max * dmax)) * (1.0f - 4.0f * 1.1920929e-7f);
         const unsigned int kstop_bits = __builtin_amdgcn_readfirstlane(__float_as_uint(kstop));
-        // the next ket's bounds are loaded one step ahead
         float bsn = ld_const(a.ket_static_b + task.ket0), kbn = ld_const(a.ket_b + task.ket0);
+        JKet kn = load_ket(a.ket_rec, task.ket0);
+        double dn[DN];
+        const double* __restrict__ kd = a.ket_d + (size_t)(task.ket0 - a.ket_hstart) * H34;
+#pragma unroll
+        for (int u = 0; u < DN; u++) dn[u] = ld_const(kd + u);
         for (int k = task.ket0; k < task.ket1; k++) {
             const float bs = bsn, kb = kbn;
             if (__float_as_uint(bs) < kstop_bits) break;
-            if (k + 1 < task.ket1) {
-                bsn = ld_const(a.ket_static_b + k + 1);
-                kbn = ld_const(a.ket_b + k + 1);
-            }
-            const float est = B12 * kb;
-            bool take = bra_ok && est >= thre_lo;
-            if constexpr (LO) take = take && !(est >= a.thredp);
-            bool step32 = LO;
-            if constexpr (MIXED) step32 = __ballot(take && est >= a.thredp) == 0ull;
-            if (a.count && __ballot(take) != 0ull) nsteps++;
-            if (!take) continue;
-            nq++;
-            if (step32) nq32++;
-            const double q = ld_const(a.ket_geom + k);
-            const double c34 = ld_const(a.ket_geom + 4 * a.ket_n + k);
-            const double X = Px - ld_const(a.ket_geom + a.ket_n + k);
-            const double Y = Py - ld_const(a.ket_geom + 2 * a.ket_n + k);
-            const double Z = Pz - ld_const(a.ket_geom + 3 * a.ket_n + k);
+            const JKet ket = kn;
+            double d0[DN];
+#pragma unroll
+            for (int u = 0; u < DN; u++) d0[u] = dn[u];
+            bsn = ld_const(a.ket_static_b + k + 1);
+            kbn = ld_const(a.ket_b + k + 1);
+            kn = load_ket(a.ket_rec, k + 1);
             const size_t dofs = (size_t)(k - a.ket_hstart) * H34;
-            // one quartet in the arithmetic of `acc`'s element type, reading the ket density of
-            // that precision and the matching table block
+#pragma unroll
+            for (int u = 0; u < DN; u++) dn[u] = ld_const(a.ket_d + dofs + H34 + u);
+            const float est = B12 * kb;
+            const bool take = est >= thresp;
+            const unsigned long long m = __ballot(take);
+            if (m == 0ull) continue;
+            nsteps++;
+            nq += __popcll(m);
+            const bool step32 = MIXED && __ballot(take && est >= a.thredp) == 0ull;
+            if (MIXED && step32) nq32 += __popcll(m);
+            if (!take) continue;
+            const double X = Px - ket.x, Y = Py - ket.y, Z = Pz - ket.z;
+            // one quartet in the arithmetic of `acc`'s element type, with the ket density of that
+            // precision and the matching table
             auto contract = [&](auto& acc, const auto* dsrc, const void* tab) __attribute__((always_inline)) {
                 using Real = typename std::remove_reference<decltype(acc[0])>::type;
                 Real dreg[H34];
 #pragma unroll
-                for (int u = 0; u < H34; u++) dreg[u] = ld_const(dsrc + dofs + u);
+                for (int u = 0; u < H34; u++)
+                    dreg[u] = (std::is_same<Real, double>::value && DN == H34) ? (Real)d0[u] : (Real)ld_const(dsrc + dofs + u);
                 if constexpr (L >= 5) {
-                    hermite_contract_factorized<Real, L12, L34>(a.rys, tab, a.ew, p12, c12, q, c34, X, Y, Z, dreg, acc);
+                    hermite_contract_factorized<Real, L12, L34>(a.rys, tab, a.ew, p12, c12, ket.q, ket.c, X, Y, Z, dreg, acc);
                 } else {
                     Real R[HL];
-                    hermite_R<Real, L>(a.rys, tab, a.ew, p12, c12, q, c34, X, Y, Z, R);
+                    hermite_R<Real, L>(a.rys, tab, a.ew, p12, c12, ket.q, ket.c, X, Y, Z, R);
                     static_for<H34>([&](auto U_) {
                         constexpr int u = decltype(U_)::value;
                         constexpr int ux = herm_tx(u), uy = herm_ty(u), uz = herm_tz(u);
@@ -304,7 +398,7 @@ __global__ __launch_bounds__(256) void j_quartets(JQuartetArgs a, const JTask* _
                     });
                 }
             };
-            auto fp32 = [&]() __attribute__((always_inline)) {
+            if (MIXED && step32) {
                 // FP32 quartet, FP64 accumulation
                 float jq[H12];
 #pragma unroll
@@ -312,14 +406,6 @@ __global__ __launch_bounds__(256) void j_quartets(JQuartetArgs a, const JTask* _
                 contract(jq, a.ket_d32, s_tab32);
 #pragma unroll
                 for (int u = 0; u < H12; u++) jp[u] += (double)jq[u];
-            };
-            if constexpr (LO) {
-                fp32();
-            } else if constexpr (MIXED) {
-                if (step32)
-                    fp32();
-                else
-                    contract(jp, a.ket_d, s_tab64);
             } else {
                 contract(jp, a.ket_d, s_tab64);
             }
@@ -331,18 +417,11 @@ __global__ __launch_bounds__(256) void j_quartets(JQuartetArgs a, const JTask* _
                 if (jp[u] != 0.0) atomic_add(dst + u, jp[u]);
         }
     }
-    if (a.count) {
-        // per-wave reduction of the evaluated-quartet counts
-        for (int o = 32; o > 0; o >>= 1) {
-            nq += __shfl_xor(nq, o);
-            nq32 += __shfl_xor(nq32, o);
-        }
-        if (lane == 0 && nq) {
-            atomicAdd(&a.sc->counts[a.count_cls], nq);
-            if (nq32) atomicAdd(&a.sc->counts32[a.count_cls], nq32);
-            atomicAdd(&a.sc->wsteps[a.count_cls], (unsigned long long)nsteps);
-            atomicAdd(&a.sc->wlanes[a.count_cls], nq);
-        }
+    if (a.count && lane == 0 && nq) {
+        atomicAdd(&a.sc->counts[a.count_cls], nq);
+        if (nq32) atomicAdd(&a.sc->counts32[a.count_cls], nq32);
+        atomicAdd(&a.sc->wsteps[a.count_cls], (unsigned long long)nsteps);
+        atomicAdd(&a.sc->wlanes[a.count_cls], nq);
     }
 }
 
@@ -362,21 +441,19 @@ __global__ __launch_bounds__(256) void j_quartets_sym(JQuartetArgs a, const JTas
 {
     using Lds = JLds<L12, L34, ROUTE>;
     constexpr bool MIXED = ROUTE == kRouteMixed;
-    constexpr int H12 = nherm(L12), H34 = nherm(L34), L = L12 + L34, HL = nherm(L), NR = L / 2 + 1;
+    constexpr int H12 = nherm(L12), H34 = nherm(L34), L = L12 + L34, HL = nherm(L);
     constexpr bool SAME = L12 == L34;
     extern __shared__ double s_dyn[];
     double* s_tab64 = s_dyn;
-    float* s_tab32 = reinterpret_cast<float*>(reinterpret_cast<char*>(s_dyn) + Lds::bytes64(a.rys));
-    if constexpr (Lds::STAGED64) rys_stage_lds<NR>(a.rys, s_tab64);
-    if constexpr (Lds::HAS32) rys32_stage_lds<NR>(a.rys, s_tab32);
-    if constexpr (Lds::STAGED64 || Lds::HAS32) __syncthreads();
+    float* s_tab32 = reinterpret_cast<float*>(reinterpret_cast<char*>(s_dyn) + Lds::kBytes64);
+    Lds::stage(a.rys, s_tab64, s_tab32);
     const int lane = threadIdx.x & 63;
     const float thre_lo = a.thresp;
     const float max34 = __uint_as_float(a.sc->max34_bits);
     const float thre_bra = a.thresp / max34;
     const double dmax = __longlong_as_double((long long)a.sc->dmax_bits);
-    unsigned long long nqa = 0, nqb = 0, nq32a = 0, nq32b = 0;
-    unsigned long long nlanes = 0;  // integrals evaluated (one serves both uses; counting mode)
+    // evaluated quartets of each use, integrals (one serves both uses), wave steps (scalar registers)
+    unsigned long long nqa = 0, nqb = 0, nq32a = 0, nq32b = 0, nlanes = 0;
     unsigned int nsteps = 0;
 
     for (;;) {
@@ -407,6 +484,8 @@ __global__ __launch_bounds__(256) void j_quartets_sym(JQuartetArgs a, const JTas
             for (int u = 0; u < H12; u++) dx[u] = a.bra_d[(size_t)(x - a.bra_hstart) * H12 + u];
         }
         const bool bra_ok = active && (Bx >= thre_bra);
+        if (!bra_ok) Bx = __builtin_nanf("");    // no estimate of the lane passes in the first use,
+        if (!active) kbx = __builtin_nanf("");  // or in the second
         double jp[H12];
 #pragma unroll
         for (int u = 0; u < H12; u++) jp[u] = 0.0;
@@ -416,41 +495,44 @@ __global__ __launch_bounds__(256) void j_quartets_sym(JQuartetArgs a, const JTas
         const float kstop = (float)((double)thre_lo / ((double)B12max * dmax)) * (1.0f - 8.0f * 1.1920929e-7f);
         const unsigned int kstop_bits = __builtin_amdgcn_readfirstlane(__float_as_uint(kstop));
         float bsn = ld_const(a.ket_static_b + task.ket0), kbn = ld_const(a.ket_b + task.ket0);
+        JKet kn = load_ket(a.ket_rec, task.ket0);
         for (int k = task.ket0; k < task.ket1; k++) {
             const float By = bsn, kby = kbn;
             if (__float_as_uint(By) < kstop_bits) break;
-            if (k + 1 < task.ket1) {
-                bsn = ld_const(a.ket_static_b + k + 1);
-                kbn = ld_const(a.ket_b + k + 1);
-            }
-            const bool takeA = bra_ok && (!SAME || k <= x) && Bx * kby >= thre_lo;
-            const bool takeB = active && (By >= thre_bra) && (!SAME || k < x) && By * kbx >= thre_lo;
-            const unsigned long long mB = __ballot(takeB);
-            if ((__ballot(takeA) | mB) == 0ull) continue;
-            if (a.count) nsteps++;
-            bool step32 = false;
-            if constexpr (MIXED)
-                step32 = __ballot((takeA && Bx * kby >= a.thredp) || (takeB && By * kbx >= a.thredp)) == 0ull;
-            const double q = ld_const(a.ket_geom + k);
-            const double c34 = ld_const(a.ket_geom + 4 * a.ket_n + k);
-            const double X = Px - ld_const(a.ket_geom + a.ket_n + k);
-            const double Y = Py - ld_const(a.ket_geom + 2 * a.ket_n + k);
-            const double Z = Pz - ld_const(a.ket_geom + 3 * a.ket_n + k);
+            const JKet ket = kn;
             const size_t dofs = (size_t)(k - a.ket_hstart) * H34;
             double dy[H34];
 #pragma unroll
             for (int u = 0; u < H34; u++) dy[u] = ld_const(a.ket_d + dofs + u);
+            bsn = ld_const(a.ket_static_b + k + 1);
+            kbn = ld_const(a.ket_b + k + 1);
+            kn = load_ket(a.ket_rec, k + 1);
+            const float ea = Bx * kby, eb = By * kbx;
+            const bool takeA = (!SAME || k <= x) && ea >= thre_lo;
+            const bool takeB = (By >= thre_bra) && (!SAME || k < x) && eb >= thre_lo;
+            const unsigned long long mA = __ballot(takeA), mB = __ballot(takeB);
+            if ((mA | mB) == 0ull) continue;
+            nsteps++;
+            nqa += __popcll(mA);
+            nqb += __popcll(mB);
+            nlanes += __popcll(mA | mB);
+            bool step32 = false;
+            if constexpr (MIXED) {
+                step32 = __ballot((takeA && ea >= a.thredp) || (takeB && eb >= a.thredp)) == 0ull;
+                if (step32) {
+                    nq32a += __popcll(mA);
+                    nq32b += __popcll(mB);
+                }
+            }
+            const double X = Px - ket.x, Y = Py - ket.y, Z = Pz - ket.z;
             double jy[H34];
 #pragma unroll
             for (int u = 0; u < H34; u++) jy[u] = 0.0;
             if (takeA || takeB) {
-                nqa += takeA ? 1 : 0;
-                nqb += takeB ? 1 : 0;
-                nlanes++;
                 // one integral in the arithmetic Real, both uses; the A part lands in accA
                 auto both = [&](auto* R, auto* accA, const void* tab) __attribute__((always_inline)) {
                     using Real = typename std::remove_reference<decltype(R[0])>::type;
-                    hermite_R<Real, L>(a.rys, tab, a.ew, p12, c12, q, c34, X, Y, Z,
+                    hermite_R<Real, L>(a.rys, tab, a.ew, p12, c12, ket.q, ket.c, X, Y, Z,
                                        *reinterpret_cast<Real(*)[HL]>(R));
                     const Real wa = takeA ? Real(1) : Real(0), wb = takeB ? Real(1) : Real(0);
                     static_for<H34>([&](auto U_) {
@@ -478,8 +560,6 @@ __global__ __launch_bounds__(256) void j_quartets_sym(JQuartetArgs a, const JTas
                     both(R, ja, s_tab32);
 #pragma unroll
                     for (int u = 0; u < H12; u++) jp[u] += (double)ja[u];
-                    nq32a += takeA ? 1 : 0;
-                    nq32b += takeB ? 1 : 0;
                 } else {
                     double R[HL];
                     both(R, jp, s_tab64);
@@ -505,37 +585,22 @@ __global__ __launch_bounds__(256) void j_quartets_sym(JQuartetArgs a, const JTas
                 if (jp[u] != 0.0) atomic_add(dst + u, jp[u]);
         }
     }
-    if (a.count) {
-        for (int o = 32; o > 0; o >>= 1) {
-            nqa += __shfl_xor(nqa, o);
-            nqb += __shfl_xor(nqb, o);
-            nlanes += __shfl_xor(nlanes, o);
+    if (a.count && lane == 0) {
+        if (nqa) atomicAdd(&a.sc->counts[a.count_cls], nqa);
+        if (nqb) atomicAdd(&a.sc->counts[a.count_cls2], nqb);
+        if (nlanes) {
+            atomicAdd(&a.sc->wsteps[a.count_cls], (unsigned long long)nsteps);
+            atomicAdd(&a.sc->wlanes[a.count_cls], nlanes);
         }
-        if (lane == 0) {
-            if (nqa) atomicAdd(&a.sc->counts[a.count_cls], nqa);
-            if (nqb) atomicAdd(&a.sc->counts[a.count_cls2], nqb);
-            if (nlanes) {
-                atomicAdd(&a.sc->wsteps[a.count_cls], (unsigned long long)nsteps);
-                atomicAdd(&a.sc->wlanes[a.count_cls], nlanes);
-            }
-        }
-        if constexpr (MIXED) {
-            for (int o = 32; o > 0; o >>= 1) {
-                nq32a += __shfl_xor(nq32a, o);
-                nq32b += __shfl_xor(nq32b, o);
-            }
-            if (lane == 0) {
-                if (nq32a) atomicAdd(&a.sc->counts32[a.count_cls], nq32a);
-                if (nq32b) atomicAdd(&a.sc->counts32[a.count_cls2], nq32b);
-            }
-        }
+        if (nq32a) atomicAdd(&a.sc->counts32[a.count_cls], nq32a);
+        if (nq32b) atomicAdd(&a.sc->counts32[a.count_cls2], nq32b);
     }
 }
 
 template <int L12, int L34, int ROUTE>
 void launch_jq(const JQuartetArgs& a, const JTask* tasks, int ntask, unsigned int* qctr, hipStream_t s)
 {
-    const size_t lds = JLds<L12, L34, ROUTE>::bytes(a.rys);
+    const size_t lds = JLds<L12, L34, ROUTE>::kBytes;
     const int grid = persistent_grid((const void*)j_quartets<L12, L34, ROUTE>, 256, lds, ((long long)ntask + 3) / 4);
     hipLaunchKernelGGL((j_quartets<L12, L34, ROUTE>), dim3(grid), dim3(256), lds, s, a, tasks, ntask, qctr);
 }

@@ -111,6 +111,7 @@ __device__ __forceinline__ void static_for(F&& f)
 struct RysTable {
     const double* coef;
     const float* coef32;
+    const double* boys;  // Boys tables of orders 2 .. 4 (boys_offset)
 };
 constexpr int kRysNcoef = 12;
 // Coefficients per polynomial of the FP32 rule: a degree-5 Chebyshev interpolant of the FP64
@@ -230,6 +231,65 @@ __device__ __forceinline__ void rys_roots_any(const RysTable& tab, const double*
         rys_roots_lds<NRYS>(s_coef, T, x, w);
     else
         rys_roots<NRYS>(tab, T, x, w);
+}
+
+// Boys table of order L (2 .. 4): on the Rys bins of L / 2 + 1 roots the coefficients of F_L in
+// v = T - b - 1/2 (degree 11) and exp(-(b + 1/2)), 13 doubles per bin (odd: lanes in different bins
+// fall on different LDS banks).
+constexpr int kBoysDoubles = kRysNcoef + 1;
+__host__ __device__ constexpr size_t boys_lds_doubles(int L) { return (size_t)kRysNbin[L / 2 + 1] * kBoysDoubles; }
+__host__ __device__ constexpr size_t boys_offset(int L)
+{
+    size_t o = 0;
+    for (int k = 2; k < L; k++) o += boys_lds_doubles(k);
+    return o;
+}
+template <int L>
+__device__ __forceinline__ void boys_stage_lds(const RysTable& tab, double* s)
+{
+    for (int i = threadIdx.x; i < (int)boys_lds_doubles(L); i += blockDim.x) s[i] = tab.boys[boys_offset(L) + i];
+}
+
+// F_0 .. F_L at T from the staged table: F_L by its polynomial, exp(-T) = exp(-(b + 1/2)) exp(-v) with
+// the degree-12 Chebyshev interpolant of exp(-v) on |v| <= 1/2 (5e-18), then downward,
+// F_{n-1} = (2 T F_n + exp(-T)) / (2 n - 1), which is stable.  From T = Tc on (where exp(-T) is below
+// rounding) F_n = F_{n-1} (n - 1/2) / T.
+template <int L>
+__device__ __forceinline__ void boys_lds(const double* s, double T, double (&F)[L + 1])
+{
+    constexpr int NR = L / 2 + 1;
+    if (!(T < (double)kRysNbin[NR])) {
+        const double r = rsqrt(T), iT = r * r;
+        F[0] = kRysAsymW[0] * r;
+#pragma unroll
+        for (int n = 1; n <= L; n++) F[n] = F[n - 1] * ((n - 0.5) * iT);
+        return;
+    }
+    double v;
+    const double* c = s + __umul24(rys_bin<NR>(T, v), kBoysDoubles);
+    constexpr double kExp[13] = {1.0,
+                                 -9.99999999999999889e-01,
+                                 5.00000000000000000e-01,
+                                 -1.66666666666680646e-01,
+                                 4.16666666666676636e-02,
+                                 -8.33333333288569476e-03,
+                                 1.38888888885692970e-03,
+                                 -1.98412704550513576e-04,
+                                 2.48015877398097512e-05,
+                                 -2.75569101863640885e-06,
+                                 2.75570271694439541e-07,
+                                 -2.51828992381847868e-08,
+                                 2.09701512151694754e-09};
+    double f = c[kRysNcoef - 1], e = kExp[12];
+#pragma unroll
+    for (int k = kRysNcoef - 2; k >= 0; k--) f = fma(f, v, c[k]);
+#pragma unroll
+    for (int k = 11; k >= 0; k--) e = fma(e, v, kExp[k]);
+    e *= c[kRysNcoef];
+    F[L] = f;
+    const double T2 = T + T;
+#pragma unroll
+    for (int n = L; n >= 1; n--) F[n - 1] = fma(T2, F[n], e) * (1.0 / (2 * n - 1));
 }
 
 // LDS copy of the FP32 table block of one nrys: bins of nrys 2 kRysNcoef32 floats plus one pad.

@@ -81,6 +81,7 @@ struct PairList {
     size_t hoff[2 * kMaxL + 2] = {0}; // offset (in doubles) of group in the H-strided buffers
     float* d_hb = nullptr;             // static bound, Hermite order
     double* d_hgeom = nullptr;         // p, Px, Py, Pz, sqrt(2 pi^(5/2))/p (SoA, 5 * npair), Hermite order
+    double* d_hrec = nullptr;          // kJKetDoubles per pair (JQuartetArgs::ket_rec), Hermite order, one pad
     std::vector<float> h_hb;
     // K view
     int nrow = 0;                      // = b1->nprim

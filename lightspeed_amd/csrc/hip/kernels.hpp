@@ -14,9 +14,7 @@ __host__ __device__ constexpr int kcount_index(int L1, int L2, int L3, int L4)
 // Precision routes of a quartet kernel launch (the reference's documented mixed precision,
 // intbox.hpp:736-742: FP64 when est >= thredp, FP32 when thresp <= est < thredp, else skipped).
 constexpr int kRoutePlain = 0;  // est >= thresp, FP64 (thredp <= thresp)
-constexpr int kRouteHi = 1;     // est >= thredp, FP64
-constexpr int kRouteLo = 2;     // thresp <= est < thredp, FP32 arithmetic, FP64 accumulation
-constexpr int kRouteMixed = 4;  // K build: est >= thredp in FP64 and thresp <= est < thredp in FP32, one launch
+constexpr int kRouteMixed = 4;  // est >= thredp in FP64 and thresp <= est < thredp in FP32, one launch
 
 struct JPrepArgs {
     const int* p1;
@@ -38,6 +36,7 @@ struct JPrepArgs {
     CallScalars* sc;
 };
 
+constexpr int kJKetDoubles = 6;
 struct JQuartetArgs {
     RysTable rys;
     Ewald ew;
@@ -53,8 +52,7 @@ struct JQuartetArgs {
     // ket (Hermite order of the ket list)
     const float* ket_b;         // truncated bounds (per call)
     const float* ket_static_b;  // Schwarz bounds
-    const double* ket_geom;
-    int ket_n;
+    const double* ket_rec;      // kJKetDoubles per pair: p, sqrt(2 pi^(5/2))/p, P (3), 0
     int ket_hstart;
     const double* ket_d;  // Hermite densities of the ket group
     const float* ket_d32; // their FP32 copy (FP32 route)
