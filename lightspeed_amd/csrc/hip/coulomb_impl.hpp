@@ -65,9 +65,10 @@ __device__ __forceinline__ void herm_factors(Real pref_w, Real U, Real X, Real Y
     }
 }
 
-// Calls f(HermRoot) for every Rys root of every operator term of one bra-ket pair.
+// Calls f(HermRoot) for every Rys root of every operator term of one bra-ket pair (BARE: of one bare 1/r
+// term, its scale in c12).
 // c12, c34: sqrt(2 pi^(5/2)) / p of each pair, so that c12 c34 (p + q)^(-1/2) = 2 pi^(5/2) / (p q sqrt(p + q)).
-template <typename Real, int L, typename F>
+template <typename Real, int L, bool BARE, typename F>
 __device__ __forceinline__ void for_each_root(const RysTable& tab, const void* s_tab, const Ewald& ew, double p12,
                                               double c12, double p34, double c34, double X, double Y, double Z, F&& f)
 {
@@ -80,7 +81,8 @@ __device__ __forceinline__ void for_each_root(const RysTable& tab, const void* s
     const double r2 = X * X + Y * Y + Z * Z;
     const Real Xr = (Real)X, Yr = (Real)Y, Zr = (Real)Z;
     // one operator term: Rys roots at T = rho d2 r2, Hermite factors with prefactor pref
-    auto term = [&](Real pref, Real d2) __attribute__((always_inline)) {
+    auto term = [&](Real pref, auto d2_) __attribute__((always_inline)) {
+        const Real d2 = (Real)d2_;
         const double T = (double)(rho * d2) * r2;
         Real x[NR], w[NR];
         roots_real<Real, NR>(tab, s_tab, T, x, w);
@@ -91,9 +93,9 @@ __device__ __forceinline__ void for_each_root(const RysTable& tab, const void* s
             f(H);
         }
     };
-    if (ew.plain) {
-        // one bare 1/r term: d2 = 1, no term loop (the common case)
-        term((Real)ew.alpha[0] * base, Real(1));
+    if constexpr (BARE) {
+        // one bare 1/r term, its scale in c12: no term loop
+        term(base, std::integral_constant<int, 1>{});
         return;
     }
     for (int it = 0; it < ew.n; it++) {
@@ -143,7 +145,7 @@ __device__ __forceinline__ void md_level(const double (&b)[L + 1], double X, dou
     }
 }
 
-template <int L>
+template <int L, bool BARE>
 __device__ __forceinline__ void hermite_R_md(const double* s_boys, const Ewald& ew, double p, double c12, double q,
                                              double c34, double X, double Y, double Z, double (&R)[nherm(L)])
 {
@@ -153,9 +155,9 @@ __device__ __forceinline__ void hermite_R_md(const double* s_boys, const Ewald& 
     const double base = c12 * c34 * rs;  // 2 pi^{5/2} / (p q sqrt(p+q))
     const double r2 = X * X + Y * Y + Z * Z;
     double b[L + 1], F[L + 1];
-    if (ew.plain) {
+    if constexpr (BARE) {
         boys_lds<L>(s_boys, rho * r2, F);
-        double f = ew.alpha[0] * base;
+        double f = base;
 #pragma unroll
         for (int n = 0; n <= L; n++) {
             b[n] = f * F[n];
@@ -186,17 +188,17 @@ __device__ __forceinline__ void hermite_R_md(const double* s_boys, const Ewald& 
 
 // Hermite Coulomb integrals R_{tuv} (t+u+v <= L) of one bra-ket pair, by Rys quadrature
 // (R_{tuv} = pref * sum_i w_i Hx_t Hy_u Hz_v) or from Boys functions (j_md).
-template <typename Real, int L>
+template <typename Real, int L, bool BARE>
 __device__ __forceinline__ void hermite_R(const RysTable& tab, const void* s_tab, const Ewald& ew, double p12,
                                           double c12, double p34, double c34, double X, double Y, double Z,
                                           Real (&R)[nherm(L)])
 {
     constexpr int HL = nherm(L);
     if constexpr (std::is_same<Real, double>::value && j_md(L))
-        return hermite_R_md<L>(static_cast<const double*>(s_tab), ew, p12, c12, p34, c34, X, Y, Z, R);
+        return hermite_R_md<L, BARE>(static_cast<const double*>(s_tab), ew, p12, c12, p34, c34, X, Y, Z, R);
 #pragma unroll
     for (int t = 0; t < HL; t++) R[t] = Real(0);
-    for_each_root<Real, L>(tab, s_tab, ew, p12, c12, p34, c34, X, Y, Z, [&](const HermRoot<Real, L>& H) __attribute__((always_inline)) {
+    for_each_root<Real, L, BARE>(tab, s_tab, ew, p12, c12, p34, c34, X, Y, Z, [&](const HermRoot<Real, L>& H) __attribute__((always_inline)) {
         static_for<HL>([&](auto T_) {
             constexpr int t = decltype(T_)::value;
             constexpr int tx = herm_tx(t), ty = herm_ty(t), tz = herm_tz(t);
@@ -209,13 +211,13 @@ __device__ __forceinline__ void hermite_R(const RysTable& tab, const void* s_tab
 // Hermite integrals are never held at once:
 //   A[uy][tz] = sum_uz Hz[tz+uz] d[ux,uy,uz];  B[ty][tz] = sum_uy Hy[ty+uy] A[uy][tz];
 //   jp[tx,ty,tz] += Hx[tx+ux] B[ty][tz]   (for each ux).
-template <typename Real, int L12, int L34, typename Acc>
+template <typename Real, int L12, int L34, bool BARE, typename Acc>
 __device__ __forceinline__ void hermite_contract_factorized(const RysTable& tab, const void* s_tab, const Ewald& ew,
                                                             double p12, double c12, double p34, double c34, double X,
                                                             double Y, double Z, const Real (&d)[nherm(L34)], Acc& jp)
 {
     constexpr int L = L12 + L34;
-    for_each_root<Real, L>(tab, s_tab, ew, p12, c12, p34, c34, X, Y, Z, [&](const HermRoot<Real, L>& H) __attribute__((always_inline)) {
+    for_each_root<Real, L, BARE>(tab, s_tab, ew, p12, c12, p34, c34, X, Y, Z, [&](const HermRoot<Real, L>& H) __attribute__((always_inline)) {
         static_for<L34 + 1>([&](auto UX_) {
             constexpr int ux = decltype(UX_)::value;
             Real A[L34 + 1 - ux][L12 + 1];
@@ -283,14 +285,25 @@ __device__ __forceinline__ JKet load_ket(const double* __restrict__ rec, int k)
     return {ld_const(g), ld_const(g + 1), ld_const(g + 2), ld_const(g + 3), ld_const(g + 4)};
 }
 
+// Waves per SIMD asked of the compiler (register budget 512 / waves) for the bare 1/r FP64 kernels that
+// sit one to three registers above an occupancy step and reach it without spilling ((1|3) and the
+// symmetric (3|0) spill when held, and measured 0.21 against 0.18 ms and no faster); 1 = no constraint.
+constexpr int j_waves(int L12, int L34, int route, bool bare)
+{
+    if (route != kRoutePlain || !bare) return 1;
+    if (L12 == 1 && (L34 == 1 || L34 == 2)) return 5;  // 97, 99 registers; step at 96
+    if (L12 == 2 && L34 == 3) return 4;                // 129; step at 128
+    return 1;
+}
+
 // Persistent kernel: each wave takes (64 bra pairs x ket range) tasks from a queue until it is
 // empty.  The workgroup's waves share an LDS copy of the tables (JLds).  Lanes own bra pairs; the
 // kets are read at wave-uniform addresses (scalar loads) one ket ahead of their use, in bound order
 // (the lists and per-call buffers are padded by one ket).  Quartets with est = B12 * B34' at or above
 // thresp are evaluated in FP64 (kRoutePlain), or on the mixed route (kRouteMixed) a ket step with any
 // quartet at or above thredp in FP64 and the others in FP32.
-template <int L12, int L34, int ROUTE>
-__global__ __launch_bounds__(256) void j_quartets(JQuartetArgs a, const JTask* __restrict__ tasks, int ntask,
+template <int L12, int L34, int ROUTE, bool BARE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(j_waves(L12, L34, ROUTE, BARE)))) void j_quartets(JQuartetArgs a, const JTask* __restrict__ tasks, int ntask,
                                                   unsigned int* qctr)
 {
     using Lds = JLds<L12, L34, ROUTE>;
@@ -333,6 +346,7 @@ __global__ __launch_bounds__(256) void j_quartets(JQuartetArgs a, const JTask* _
             Py = a.bra_geom[2 * a.bra_n + bra];
             Pz = a.bra_geom[3 * a.bra_n + bra];
             c12 = a.bra_geom[4 * a.bra_n + bra];
+            if constexpr (BARE) c12 *= a.ew.alpha[0];
         }
         const bool bra_ok = active && (B12 >= thre_bra);
         if (!bra_ok) B12 = __builtin_nanf("");  // no estimate of the lane passes
@@ -383,10 +397,10 @@ __global__ __launch_bounds__(256) void j_quartets(JQuartetArgs a, const JTask* _
                 for (int u = 0; u < H34; u++)
                     dreg[u] = (std::is_same<Real, double>::value && DN == H34) ? (Real)d0[u] : (Real)ld_const(dsrc + dofs + u);
                 if constexpr (L >= 5) {
-                    hermite_contract_factorized<Real, L12, L34>(a.rys, tab, a.ew, p12, c12, ket.q, ket.c, X, Y, Z, dreg, acc);
+                    hermite_contract_factorized<Real, L12, L34, BARE>(a.rys, tab, a.ew, p12, c12, ket.q, ket.c, X, Y, Z, dreg, acc);
                 } else {
                     Real R[HL];
-                    hermite_R<Real, L>(a.rys, tab, a.ew, p12, c12, ket.q, ket.c, X, Y, Z, R);
+                    hermite_R<Real, L, BARE>(a.rys, tab, a.ew, p12, c12, ket.q, ket.c, X, Y, Z, R);
                     static_for<H34>([&](auto U_) {
                         constexpr int u = decltype(U_)::value;
                         constexpr int ux = herm_tx(u), uy = herm_ty(u), uz = herm_tz(u);
@@ -435,7 +449,7 @@ __global__ __launch_bounds__(256) void j_quartets(JQuartetArgs a, const JTask* _
 // contributions of a ket step are summed over the wave and added to J_y by one lane.  ROUTE
 // kRoutePlain: FP64; kRouteMixed: a ket step in which no lane's estimate reaches thredp, in either
 // use, is evaluated in FP32 (table, R, contraction; FP64 accumulation), the others in FP64.
-template <int L12, int L34, int ROUTE>
+template <int L12, int L34, int ROUTE, bool BARE>
 __global__ __launch_bounds__(256) void j_quartets_sym(JQuartetArgs a, const JTask* __restrict__ tasks, int ntask,
                                                       unsigned int* qctr)
 {
@@ -480,6 +494,7 @@ __global__ __launch_bounds__(256) void j_quartets_sym(JQuartetArgs a, const JTas
             Py = a.bra_geom[2 * a.bra_n + x];
             Pz = a.bra_geom[3 * a.bra_n + x];
             c12 = a.bra_geom[4 * a.bra_n + x];
+            if constexpr (BARE) c12 *= a.ew.alpha[0];
 #pragma unroll
             for (int u = 0; u < H12; u++) dx[u] = a.bra_d[(size_t)(x - a.bra_hstart) * H12 + u];
         }
@@ -532,7 +547,7 @@ __global__ __launch_bounds__(256) void j_quartets_sym(JQuartetArgs a, const JTas
                 // one integral in the arithmetic Real, both uses; the A part lands in accA
                 auto both = [&](auto* R, auto* accA, const void* tab) __attribute__((always_inline)) {
                     using Real = typename std::remove_reference<decltype(R[0])>::type;
-                    hermite_R<Real, L>(a.rys, tab, a.ew, p12, c12, ket.q, ket.c, X, Y, Z,
+                    hermite_R<Real, L, BARE>(a.rys, tab, a.ew, p12, c12, ket.q, ket.c, X, Y, Z,
                                        *reinterpret_cast<Real(*)[HL]>(R));
                     const Real wa = takeA ? Real(1) : Real(0), wb = takeB ? Real(1) : Real(0);
                     static_for<H34>([&](auto U_) {
@@ -600,9 +615,11 @@ __global__ __launch_bounds__(256) void j_quartets_sym(JQuartetArgs a, const JTas
 template <int L12, int L34, int ROUTE>
 void launch_jq(const JQuartetArgs& a, const JTask* tasks, int ntask, unsigned int* qctr, hipStream_t s)
 {
+    // one bare 1/r term (the common case) has kernels without the operator-term loop
+    auto* kernel = a.ew.plain ? j_quartets<L12, L34, ROUTE, true> : j_quartets<L12, L34, ROUTE, false>;
     const size_t lds = JLds<L12, L34, ROUTE>::kBytes;
-    const int grid = persistent_grid((const void*)j_quartets<L12, L34, ROUTE>, 256, lds, ((long long)ntask + 3) / 4);
-    hipLaunchKernelGGL((j_quartets<L12, L34, ROUTE>), dim3(grid), dim3(256), lds, s, a, tasks, ntask, qctr);
+    const int grid = persistent_grid((const void*)kernel, 256, lds, ((long long)ntask + 3) / 4);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, s, a, tasks, ntask, qctr);
 }
 
 // All ket orders of one bra order: both routes, or the FP64 route only (order 5: gradients).

@@ -9,9 +9,10 @@ void launch_j_quartets_sym(int L12, int L34, int route, const JQuartetArgs& a, c
     if (ntask <= 0) return;
 #define ONE(X, Y, R)                                                                                     \
     {                                                                                                    \
+        auto* kernel = a.ew.plain ? j_quartets_sym<X, Y, R, true> : j_quartets_sym<X, Y, R, false>;      \
         const size_t lds = JLds<X, Y, R>::kBytes;                                                        \
-        const int grid = persistent_grid((const void*)j_quartets_sym<X, Y, R>, 256, lds, ((long long)ntask + 3) / 4); \
-        hipLaunchKernelGGL((j_quartets_sym<X, Y, R>), dim3(grid), dim3(256), lds, s, a, tasks, ntask, qctr); \
+        const int grid = persistent_grid((const void*)kernel, 256, lds, ((long long)ntask + 3) / 4);     \
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, s, a, tasks, ntask, qctr);                \
         return;                                                                                          \
     }
 #define CASE(X, Y)                                                                                       \
