@@ -3175,28 +3175,33 @@ int lsjk_coulomb_grad(const lsjk_pairlist* pl, const double* Dbra_dev, const dou
                               pl->hstart[L], pl->hoff[L], st);
         }
         if (ew.n > 0) {
-            for (int L12 = 0; L12 <= 2 * kMaxL; L12++)
-                for (int L34 = 0; L34 <= 2 * kMaxL; L34++) {
-                    if (seg.cnt[L12][L34] == 0) continue;
-                    JQuartetArgs qa{};
-                    qa.rys = S.rys;
-                    qa.ew = ew;
-                    qa.thresp = thresp;
-                    qa.thredp = thresp;
-                    qa.bra_b = pl->d_hb;
-                    qa.bra_geom = pl->d_hgeom;
-                    qa.bra_n = pl->npair;
-                    qa.bra_hstart = pl->hstart[L12];
-                    qa.jp = vp + hoff2[L12];
-                    qa.ket_b = kb;
-                    qa.ket_static_b = pl->d_hb;
-                    qa.ket_rec = pl->d_hrec;
-                    qa.ket_hstart = pl->hstart[L34];
-                    qa.ket_d = kd + pl->hoff[L34];
-                    qa.sc = S.d_sc;
-                    launch_j_quartets(L12 + 1, L34, kRoutePlain, qa, (const JTask*)seg.d_tasks + seg.off[L12][L34],
-                                           seg.cnt[L12][L34], &S.d_sc->queue[jcount_index(L12, L34)], st);
-                }
+            // the group pairs over the side streams, heaviest first
+            Fanout fo;
+            fo.begin();
+            for (int Lt = 4 * kMaxL; Lt >= 0; Lt--)
+                for (int L12 = 0; L12 <= 2 * kMaxL; L12++)
+                    for (int L34 = 0; L34 <= 2 * kMaxL; L34++) {
+                        if (L12 + L34 != Lt || seg.cnt[L12][L34] == 0) continue;
+                        JQuartetArgs qa{};
+                        qa.rys = S.rys;
+                        qa.ew = ew;
+                        qa.thresp = thresp;
+                        qa.thredp = thresp;
+                        qa.bra_b = pl->d_hb;
+                        qa.bra_geom = pl->d_hgeom;
+                        qa.bra_n = pl->npair;
+                        qa.bra_hstart = pl->hstart[L12];
+                        qa.jp = vp + hoff2[L12];
+                        qa.ket_b = kb;
+                        qa.ket_static_b = pl->d_hb;
+                        qa.ket_rec = pl->d_hrec;
+                        qa.ket_hstart = pl->hstart[L34];
+                        qa.ket_d = kd + pl->hoff[L34];
+                        qa.sc = S.d_sc;
+                        launch_j_quartets(L12 + 1, L34, kRoutePlain, qa, (const JTask*)seg.d_tasks + seg.off[L12][L34],
+                                               seg.cnt[L12][L34], &S.d_sc->queue[jcount_index(L12, L34)], fo.pick());
+                    }
+            fo.end();
             JGradArgs ga{};
             ga.p1 = pl->d_p1;
             ga.p2 = pl->d_p2;

@@ -193,18 +193,8 @@ __device__ __forceinline__ void k_quartet_grad(const RysTable& tab, const double
                     });
                 });
             } else {
-#pragma unroll 1
-                for (int cd = slice; cd < N3 * N4; cd += nslice) {
-                    const int c = cd / N4, d = cd - c * N4;
-                    double S[3][L1 + 2][L2 + 2];
-#pragma unroll
-                    for (int k = 0; k < 3; k++) {
-                        const int ic = cart_lk(L3, c, k), id = cart_lk(L4, d, k);
-#pragma unroll
-                        for (int ia = 0; ia < L1 + 2; ia++)
-#pragma unroll
-                            for (int ib = 0; ib < L2 + 2; ib++) S[k][ia][ib] = I[k].v[ia][ib][ic][id];
-                    }
+                // one (c, d): its 2-D integrals S(k, i, j) and the weights of the four blocks
+                auto component = [&](int c, int d, auto&& S) __attribute__((always_inline)) {
                     double a3c[N1], a3d[N1], a4c[N1], a4d[N1];
 #pragma unroll
                     for (int a = 0; a < N1; a++) {
@@ -221,13 +211,37 @@ __device__ __forceinline__ void k_quartet_grad(const RysTable& tab, const double
                         b4c[b] = gbc ? x24b[(size_t)b * ldx + oc + c] : 0.0;
                         b4d[b] = gbd ? x24b[(size_t)b * ldx + od + d] : 0.0;
                     }
-                    bra(
-                        [&](auto K_, auto I_, auto J_) __attribute__((always_inline)) {
-                            return S[decltype(K_)::value][decltype(I_)::value][decltype(J_)::value];
-                        },
-                        [&](int a, int b) __attribute__((always_inline)) {
-                            return a3c[a] * b4d[b] + b3c[b] * a4d[a] + a3d[a] * b4c[b] + b3d[b] * a4c[a];
+                    bra(S, [&](int a, int b) __attribute__((always_inline)) {
+                        return a3c[a] * b4d[b] + b3c[b] * a4d[a] + a3d[a] * b4c[b] + b3d[b] * a4c[a];
+                    });
+                };
+                if constexpr (grad_unrolled(L1, L2, L3, L4)) {
+                    static_for<N3 * N4>([&](auto CD_) {
+                        constexpr int cd = decltype(CD_)::value, c = cd / N4, d = cd - c * N4;
+                        if (nslice > 1 && cd % nslice != slice) return;
+                        component(c, d, [&](auto K_, auto I_, auto J_) __attribute__((always_inline)) {
+                            constexpr int k = decltype(K_)::value;
+                            constexpr int ic = cart_lk(L3, c, k), id = cart_lk(L4, d, k);
+                            return I[k].v[decltype(I_)::value][decltype(J_)::value][ic][id];
                         });
+                    });
+                } else {
+#pragma unroll 1
+                    for (int cd = slice; cd < N3 * N4; cd += nslice) {
+                        const int c = cd / N4, d = cd - c * N4;
+                        double S[3][L1 + 2][L2 + 2];
+#pragma unroll
+                        for (int k = 0; k < 3; k++) {
+                            const int ic = cart_lk(L3, c, k), id = cart_lk(L4, d, k);
+#pragma unroll
+                            for (int ia = 0; ia < L1 + 2; ia++)
+#pragma unroll
+                                for (int ib = 0; ib < L2 + 2; ib++) S[k][ia][ib] = I[k].v[ia][ib][ic][id];
+                        }
+                        component(c, d, [&](auto K_, auto I_, auto J_) __attribute__((always_inline)) {
+                            return S[decltype(K_)::value][decltype(I_)::value][decltype(J_)::value];
+                        });
+                    }
                 }
             }
         }

@@ -149,13 +149,14 @@ struct KGradArgs {
     CallScalars* sc;
 };
 void launch_k_grad(int L1, int L2, int L3, int L4, const KGradArgs& a, hipStream_t s);
-// Classes whose components are all expanded at compile time: up to (pp|pp).  Above that the (c, d)
-// components run as a loop (the 2-D integrals are indexed at run time there, the a and b components
-// stay expanded), which bounds the code: (dd|dd) has 1296 components.
-constexpr bool grad_expanded(int L1, int L2, int L3, int L4)
-{
-    return ncart(L1) * ncart(L2) * ncart(L3) * ncart(L4) <= 81;
-}
+// How a class's components are formed.  Expanded: every component at compile time with the weight
+// blocks in registers, up to (pp|pp).  Unrolled: the (c, d) components at compile time, each loading
+// its weights, up to (dd|pp); they can be cut over waves.  Above that (648 and 1296
+// components) the (c, d) components run as a loop, the 2-D integrals indexed at run time in scratch,
+// which bounds the code.
+constexpr int grad_ncomp(int L1, int L2, int L3, int L4) { return ncart(L1) * ncart(L2) * ncart(L3) * ncart(L4); }
+constexpr bool grad_expanded(int L1, int L2, int L3, int L4) { return grad_ncomp(L1, L2, L3, L4) <= 81; }
+constexpr bool grad_unrolled(int L1, int L2, int L3, int L4) { return grad_ncomp(L1, L2, L3, L4) <= 324; }
 // Per block pair: the symmetric and antisymmetric parts of D13 and D24, the block maxima of D24
 // (the larger of the two triangles'), max|D24|, and flags[0], flags[1] = whether D13, D24 have an
 // antisymmetric part.

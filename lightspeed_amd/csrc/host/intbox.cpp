@@ -196,9 +196,13 @@ std::shared_ptr<Tensor> IntBox::coulombGrad(const std::shared_ptr<ResourceList>&
     // bra-centre derivatives with each density in the bra role (d/dR of (12|34) = bra part + ket
     // part, and the ket part of (12|34) is the bra part of (34|12))
     check(lsjk_coulomb_grad(d, d12.d(), d34.d(), (int)s.size(), s.data(), o.data(), thresp, thredp, dG.d()));
-    check(lsjk_coulomb_grad(d, d34.d(), d12.d(), (int)s.size(), s.data(), o.data(), thresp, thredp, dG.d()));
+    // one density in both roles: the two parts are equal
+    const bool same = D12 == D34;
+    if (!same)
+        check(lsjk_coulomb_grad(d, d34.d(), d12.d(), (int)s.size(), s.data(), o.data(), thresp, thredp, dG.d()));
     auto Gn = std::make_shared<Tensor>(std::vector<size_t>{natom, 3}, "G");
     check(lsjk_memcpy_dtoh(Gn->data().data(), dG.p, 3 * natom * sizeof(double)));
+    if (same) Gn->scale(2.0);
     if (!G) return Gn;
     G->axpby(Gn, 1.0, 1.0);
     return G;
