@@ -1178,12 +1178,12 @@ struct Fanout {
     void begin()
     {
         HIPCHK(hipEventRecord(S.fork, S.stream));
-        for (int i = 0; i < kSide; i++) HIPCHK(hipStreamWaitEvent(S.side[i], S.fork, 0));
+        for (int i = 0; i < S.nside; i++) HIPCHK(hipStreamWaitEvent(S.side[i], S.fork, 0));
     }
     hipStream_t pick() { return S.side[(next++) % S.nside]; }
     void end()
     {
-        for (int i = 0; i < kSide; i++) {
+        for (int i = 0; i < S.nside; i++) {
             HIPCHK(hipEventRecord(S.join[i], S.side[i]));
             HIPCHK(hipStreamWaitEvent(S.stream, S.join[i], 0));
         }
@@ -1506,6 +1506,27 @@ void commit_ws(Workspace& wsp, const CallOpts& o, const char* who)
     }
 }
 
+// The classes of a list as one launch's segments.
+lsjk::JSegments jsegments(const lsjk_pairlist* pl)
+{
+    lsjk::JSegments g{};
+    for (size_t c = 0; c + 1 < pl->cls_start.size(); c++) {
+        const int nk = pl->cls_start[c + 1] - pl->cls_start[c], L = pl->cls_L1[c] + pl->cls_L2[c];
+        if (nk <= 0) continue;
+        g.L1[g.n] = pl->cls_L1[c];
+        g.L2[g.n] = pl->cls_L2[c];
+        g.k0[g.n] = pl->cls_start[c];
+        g.nk[g.n] = nk;
+        g.hstart[g.n] = pl->hstart[L];
+        g.hoff[g.n] = pl->hoff[L];
+        g.block0[g.n] = g.nblock;
+        g.nblock += (nk + 255) / 256;
+        g.maxL = std::max({g.maxL, pl->cls_L1[c], pl->cls_L2[c]});
+        g.n++;
+    }
+    return g;
+}
+
 // lsjk_coulomb: workspace, task lists, the launches on the library stream.
 static void coulomb_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, const double* D34_dev, int nterm,
                          const double* scales, const double* omegas, float thresp, float thredp, double* J12_dev,
@@ -1570,11 +1591,7 @@ static void coulomb_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, c
         pa.kd = kd;
         pa.kd32 = kd32;
         pa.sc = sc;
-        for (size_t c = 0; c + 1 < pl34->cls_start.size(); c++) {
-            int L = pl34->cls_L1[c] + pl34->cls_L2[c];
-            launch_j_ket_prep(pl34->cls_L1[c], pl34->cls_L2[c], pa, pl34->cls_start[c],
-                              pl34->cls_start[c + 1] - pl34->cls_start[c], pl34->hstart[L], pl34->hoff[L], st);
-        }
+        launch_j_ket_prep(pa, jsegments(pl34), st);
         HIPCHK(hipGetLastError());
 
         if (timed) HIPCHK(hipEventRecord(S.ev[1], st));
@@ -1663,11 +1680,7 @@ static void coulomb_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, c
         sa.thresp = thresp;
         sa.sc = sc;
         if (ew.n > 0) {
-            for (size_t c = 0; c + 1 < pl12->cls_start.size(); c++) {
-                int L = pl12->cls_L1[c] + pl12->cls_L2[c];
-                launch_j_bra_scatter(pl12->cls_L1[c], pl12->cls_L2[c], sa, pl12->cls_start[c],
-                                     pl12->cls_start[c + 1] - pl12->cls_start[c], pl12->hstart[L], pl12->hoff[L], st);
-            }
+            launch_j_bra_scatter(sa, jsegments(pl12), st);
             HIPCHK(hipGetLastError());
         }
         if (timed) {
@@ -3169,11 +3182,7 @@ int lsjk_coulomb_grad(const lsjk_pairlist* pl, const double* Dbra_dev, const dou
         pa.kb = kb;
         pa.kd = kd;
         pa.sc = S.d_sc;
-        for (size_t c = 0; c + 1 < pl->cls_start.size(); c++) {
-            int L = pl->cls_L1[c] + pl->cls_L2[c];
-            launch_j_ket_prep(pl->cls_L1[c], pl->cls_L2[c], pa, pl->cls_start[c], pl->cls_start[c + 1] - pl->cls_start[c],
-                              pl->hstart[L], pl->hoff[L], st);
-        }
+        launch_j_ket_prep(pa, jsegments(pl), st);
         if (ew.n > 0) {
             // the group pairs over the side streams, heaviest first
             Fanout fo;
@@ -3330,9 +3339,12 @@ static void one_e_st(const lsjk_pairlist* pl, double* Sout, double* Tout)
     a.S = Sout;
     a.T = Tout;
     a.ld = b2->ncart;
+    Fanout fo;
+    fo.begin();
     for (size_t c = 0; c + 1 < pl->cls_start.size(); c++)
         launch_one_e_st(pl->cls_L1[c], pl->cls_L2[c], a, pl->cls_start[c], pl->cls_start[c + 1] - pl->cls_start[c],
-                        S.stream);
+                        fo.pick());
+    fo.end();
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(S.stream));
 }
@@ -3386,11 +3398,19 @@ int lsjk_potential(const lsjk_pairlist* pl, int nterm, const double* scales, con
         a.xyzc = dxyzc;
         a.nA = ncharge;
         a.vp = vp;
+        // the charges are cut so that the classes together give about 32 waves per compute unit, with at
+        // least 4 charges a wave; the classes run side by side
+        const long long waves = ((long long)pl->npair + 63) / 64 + (long long)pl->cls_L1.size();
+        const int nsplit = (int)std::max<long long>(1, std::min<long long>((ncharge + 3) / 4, 32ll * S.num_cu / waves));
+        if (nsplit > 1) launch_fill(vp, pl->hoff[2 * kMaxL + 1] * sizeof(double), st);
+        Fanout fo;
+        fo.begin();
         for (size_t c = 0; c + 1 < pl->cls_start.size(); c++) {
             const int L = pl->cls_L1[c] + pl->cls_L2[c];
             launch_one_e_v(pl->cls_L1[c], pl->cls_L2[c], a, pl->cls_start[c], pl->cls_start[c + 1] - pl->cls_start[c],
-                           pl->hstart[L], pl->hoff[L], st);
+                           nsplit, pl->hstart[L], pl->hoff[L], fo.pick());
         }
+        fo.end();
         JScatterArgs sa{};
         sa.p1 = pl->d_p1;
         sa.p2 = pl->d_p2;
@@ -3405,11 +3425,7 @@ int lsjk_potential(const lsjk_pairlist* pl, int nterm, const double* scales, con
         sa.symmetric = pl->symmetric;
         sa.screen = 0;
         sa.sc = S.d_sc;
-        for (size_t c = 0; c + 1 < pl->cls_start.size(); c++) {
-            const int L = pl->cls_L1[c] + pl->cls_L2[c];
-            launch_j_bra_scatter(pl->cls_L1[c], pl->cls_L2[c], sa, pl->cls_start[c],
-                                 pl->cls_start[c + 1] - pl->cls_start[c], pl->hstart[L], pl->hoff[L], st);
-        }
+        launch_j_bra_scatter(sa, jsegments(pl), st);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(st));
     });
@@ -3448,11 +3464,7 @@ int lsjk_count_quartets(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, co
             pa.D = D34_dev; pa.ldD = b4->ncart; pa.symmetric = pl34->symmetric;
             pa.thre_ket = thresp / pl12->maxbound;
             pa.kb = kb; pa.kd = kd; pa.sc = S.d_sc;
-            for (size_t c = 0; c + 1 < pl34->cls_start.size(); c++) {
-                int L = pl34->cls_L1[c] + pl34->cls_L2[c];
-                launch_j_ket_prep(pl34->cls_L1[c], pl34->cls_L2[c], pa, pl34->cls_start[c],
-                                  pl34->cls_start[c + 1] - pl34->cls_start[c], pl34->hstart[L], pl34->hoff[L], st);
-            }
+            launch_j_ket_prep(pa, jsegments(pl34), st);
             CountJArgs ca{};
             ca.thresp = thresp;
             ca.bra_bound = pl12->d_bound;

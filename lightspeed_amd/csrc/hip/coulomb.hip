@@ -9,26 +9,25 @@
 //     the transposed bra transform (herm_to_cart, hermite.cpp:207-411).
 // The same set of primitive quartets is evaluated; only the order of evaluation differs.
 //
-// Kernels (one launch each per call, per class):
-//   j_ket_prep<LA,LB>    one thread per ket pair: truncated bound, Hermite density d_u.
+// Kernels:
+//   j_ket_prep           one thread per ket pair, all classes: truncated bound, Hermite density d_u.
 //   j_quartets<L12,L34>  one wave per (64 bra pairs x ket chunk) task: each lane owns one bra
 //                        pair and sweeps the chunk's kets (scalar loads); Hermite integrals R_{t+u}
 //                        from Boys functions or by Rys quadrature; jp_t += sum_u R_{t+u} d_u in
 //                        registers (coulomb_impl.hpp).
-//   j_bra_scatter<LA,LB> one thread per bra pair: J_ab += K sum_t E E E jp_t (symmetrised).
+//   j_bra_scatter        one thread per bra pair, all classes: J_ab += K sum_t E E E jp_t
+//                        (symmetrised).
 #include "internal.hpp"
 #include "kernels.hpp"
 
 namespace lsjk {
 
 // ------------------------------------------------------------------ ket preparation
+// One pair k of class (LA, LB), whose Hermite group starts at pair hstart and buffer offset hoff.
 template <int LA, int LB>
-__global__ __launch_bounds__(256) void j_ket_prep(JPrepArgs a, int k0, int nk, int hstart, size_t hoff)
+__device__ __forceinline__ void ket_prep(const JPrepArgs& a, int k, int hstart, size_t hoff)
 {
     constexpr int NA = ncart(LA), NB = ncart(LB), L = LA + LB, H = nherm(L);
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nk) return;
-    const int k = k0 + i;
     const int ia = a.p1[k], ib = a.p2[k];
     const int ca = a.cartA[ia], cb = a.cartB[ib];
     const int pos = a.hpos[k];
@@ -186,12 +185,9 @@ __global__ __launch_bounds__(256) void j_grad_scatter(JGradArgs a, int k0, int n
 
 // ------------------------------------------------------------------ bra scatter
 template <int LA, int LB>
-__global__ __launch_bounds__(256) void j_bra_scatter(JScatterArgs a, int k0, int nk, int hstart, size_t hoff)
+__device__ __forceinline__ void bra_scatter(const JScatterArgs& a, int k, int hstart, size_t hoff)
 {
     constexpr int NA = ncart(LA), NB = ncart(LB), L = LA + LB, H = nherm(L);
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nk) return;
-    const int k = k0 + i;
     if (a.screen) {
         const float max34 = __uint_as_float(a.sc->max34_bits);
         const float thre_bra = a.thresp / max34;
@@ -243,24 +239,54 @@ __global__ __launch_bounds__(256) void j_bra_scatter(JScatterArgs a, int k0, int
 // ------------------------------------------------------------------ launchers
 #define LSJK_L2_CASES(F) F(0, 0) F(0, 1) F(0, 2) F(1, 0) F(1, 1) F(1, 2) F(2, 0) F(2, 1) F(2, 2)
 
-void launch_j_ket_prep(int LA, int LB, const JPrepArgs& a, int k0, int nk, int hstart, size_t hoff, hipStream_t s)
+// All classes of a list in one launch: a workgroup finds its class among the (at most 9) segments.  One
+// launch per class cost more than the classes' own time on small lists (5 us each against 2-9 us).
+// The registers are those of the heaviest class in the list's maximum angular momentum (MAXL), which
+// leaves fewer waves per SIMD for the light ones; a list of 100,000 pairs still fits the device at once.
+template <int MAXL, typename F>
+__device__ __forceinline__ void for_segment(const JSegments& seg, F&& f)
 {
-    if (nk <= 0) return;
-    dim3 grid((nk + 255) / 256), block(256);
-#define CASE(X, Y) \
-    if (LA == X && LB == Y) { hipLaunchKernelGGL((j_ket_prep<X, Y>), grid, block, 0, s, a, k0, nk, hstart, hoff); return; }
+    int c = 0;
+    while (c + 1 < seg.n && (int)blockIdx.x >= seg.block0[c + 1]) c++;
+    const int i = ((int)blockIdx.x - seg.block0[c]) * 256 + (int)threadIdx.x;
+    if (i >= seg.nk[c]) return;
+    const int k = seg.k0[c] + i, L1 = seg.L1[c], L2 = seg.L2[c];
+#define CASE(X, Y)                                                                  \
+    if constexpr (X <= MAXL && Y <= MAXL)                                           \
+        if (L1 == X && L2 == Y)                                                     \
+            return f(std::integral_constant<int, X>{}, std::integral_constant<int, Y>{}, k, seg.hstart[c], seg.hoff[c]);
     LSJK_L2_CASES(CASE)
 #undef CASE
 }
 
-void launch_j_bra_scatter(int LA, int LB, const JScatterArgs& a, int k0, int nk, int hstart, size_t hoff, hipStream_t s)
+template <int MAXL>
+__global__ __launch_bounds__(256) void j_ket_prep(JPrepArgs a, JSegments seg)
 {
-    if (nk <= 0) return;
-    dim3 grid((nk + 255) / 256), block(256);
-#define CASE(X, Y) \
-    if (LA == X && LB == Y) { hipLaunchKernelGGL((j_bra_scatter<X, Y>), grid, block, 0, s, a, k0, nk, hstart, hoff); return; }
-    LSJK_L2_CASES(CASE)
-#undef CASE
+    for_segment<MAXL>(seg, [&](auto A_, auto B_, int k, int hstart, size_t hoff) __attribute__((always_inline)) {
+        ket_prep<decltype(A_)::value, decltype(B_)::value>(a, k, hstart, hoff);
+    });
+}
+
+template <int MAXL>
+__global__ __launch_bounds__(256) void j_bra_scatter(JScatterArgs a, JSegments seg)
+{
+    for_segment<MAXL>(seg, [&](auto A_, auto B_, int k, int hstart, size_t hoff) __attribute__((always_inline)) {
+        bra_scatter<decltype(A_)::value, decltype(B_)::value>(a, k, hstart, hoff);
+    });
+}
+
+void launch_j_ket_prep(const JPrepArgs& a, const JSegments& seg, hipStream_t s)
+{
+    if (seg.nblock <= 0) return;
+    auto* kernel = seg.maxL == 0 ? j_ket_prep<0> : seg.maxL == 1 ? j_ket_prep<1> : j_ket_prep<2>;
+    hipLaunchKernelGGL(kernel, dim3(seg.nblock), dim3(256), 0, s, a, seg);
+}
+
+void launch_j_bra_scatter(const JScatterArgs& a, const JSegments& seg, hipStream_t s)
+{
+    if (seg.nblock <= 0) return;
+    auto* kernel = seg.maxL == 0 ? j_bra_scatter<0> : seg.maxL == 1 ? j_bra_scatter<1> : j_bra_scatter<2>;
+    hipLaunchKernelGGL(kernel, dim3(seg.nblock), dim3(256), 0, s, a, seg);
 }
 
 void launch_j_grad_scatter(int LA, int LB, const JGradArgs& a, int k0, int nk, int hstart, size_t hoff,

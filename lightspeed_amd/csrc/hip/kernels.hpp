@@ -129,7 +129,9 @@ struct OneEArgs {
     double* vp;  // Hermite accumulators (Hermite order, same layout as the J bra buffer)
 };
 void launch_one_e_st(int LA, int LB, const OneEArgs& a, int k0, int nk, hipStream_t s);
-void launch_one_e_v(int LA, int LB, const OneEArgs& a, int k0, int nk, int hstart, size_t hoff, hipStream_t s);
+// nsplit: parts the charges are cut into (more than one: the accumulators are added to).
+void launch_one_e_v(int LA, int LB, const OneEArgs& a, int k0, int nk, int nsplit, int hstart, size_t hoff,
+                    hipStream_t s);
 
 // Exchange gradient (exchange_grad_impl.hpp): the lanes' pairs (class 1, n1 of them) against chunks
 // of `chunk` pairs of class 2; records of kGPairDoubles doubles and bounds, both in bound order.
@@ -301,9 +303,15 @@ struct CountKArgs {
 void launch_count_j(const CountJArgs& a, int k0, int nk, int L1, int L2, hipStream_t s);
 void launch_count_k(const CountKArgs& a, hipStream_t s);
 
-void launch_j_ket_prep(int LA, int LB, const JPrepArgs& a, int k0, int nk, int hstart, size_t hoff, hipStream_t s);
-void launch_j_bra_scatter(int LA, int LB, const JScatterArgs& a, int k0, int nk, int hstart, size_t hoff,
-                          hipStream_t s);
+// The classes of a pair list as segments of one launch: workgroups [block0[c], block0[c + 1]) take the
+// pairs [k0[c], k0[c] + nk[c]) of class (L1[c], L2[c]).
+struct JSegments {
+    int n, nblock, maxL;
+    int L1[9], L2[9], k0[9], nk[9], hstart[9], block0[9];
+    size_t hoff[9];
+};
+void launch_j_ket_prep(const JPrepArgs& a, const JSegments& seg, hipStream_t s);
+void launch_j_bra_scatter(const JScatterArgs& a, const JSegments& seg, hipStream_t s);
 // Group pairs (L12 >= L34) of the symmetric J kernel: with one list on both sides it evaluates each
 // bra-ket pair of the two groups once for both J blocks (the triangle within one group).  Used
 // where measured faster than the two one-way launches: s-type kets (one Hermite component to

@@ -12,8 +12,7 @@
 //
 // Kernels: one_e_st<LA,LB> (thread per pair, list order), one_e_v<LA,LB> (thread per pair,
 // writes the pair's Hermite accumulators); j_bra_scatter then transforms V.
-#include "internal.hpp"
-#include "kernels.hpp"
+#include "coulomb_impl.hpp"
 
 namespace lsjk {
 
@@ -72,10 +71,20 @@ __global__ __launch_bounds__(256) void one_e_st(OneEArgs a, int k0, int nk)
     });
 }
 
+// Potential of the point charges [nA blockIdx.y / gridDim.y, ...) at each pair's Hermite functions, added
+// to the pair's accumulators (zero before) when the charges are cut, stored otherwise.  Hermite
+// integrals from Boys functions (orders 2-4; md_level) or the one-root Rys rule (F_0, F_1), with the
+// table in LDS.
 template <int LA, int LB>
 __global__ __launch_bounds__(256) void one_e_v(OneEArgs a, int k0, int nk, int hstart, size_t hoff)
 {
-    constexpr int L = LA + LB, H = nherm(L), NR = L / 2 + 1;
+    constexpr int L = LA + LB, H = nherm(L);
+    extern __shared__ double s_tab[];
+    if constexpr (j_md(L))
+        boys_stage_lds<L>(a.rys, s_tab);
+    else
+        rys_stage_lds<1>(a.rys, s_tab);
+    __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nk) return;
     const int k = k0 + i;
@@ -85,50 +94,55 @@ __global__ __launch_bounds__(256) void one_e_v(OneEArgs a, int k0, int nk, int h
     const double Px = (eA * a.xA[ia] + eB * a.xB[ib]) * ip;
     const double Py = (eA * a.yA[ia] + eB * a.yB[ib]) * ip;
     const double Pz = (eA * a.zA[ia] + eB * a.zB[ib]) * ip;
+    const int A0 = (int)((long long)a.nA * blockIdx.y / gridDim.y);
+    const int A1 = (int)((long long)a.nA * (blockIdx.y + 1) / gridDim.y);
     double acc[H];
 #pragma unroll
     for (int t = 0; t < H; t++) acc[t] = 0.0;
-    for (int it = 0; it < a.ew.n; it++) {
-        const double om = a.ew.omega[it];
-        double pref = a.ew.alpha[it] * 2.0 * kPi * ip, d2 = 1.0;
-        if (om != -1.0) {
-            d2 = om * om / (p + om * om);
-            pref *= sqrt(d2);
-        }
-        for (int A = 0; A < a.nA; A++) {
-            const double X = Px - ld_const(a.xyzc + 4 * A), Y = Py - ld_const(a.xyzc + 4 * A + 1);
-            const double Z = Pz - ld_const(a.xyzc + 4 * A + 2), cA = ld_const(a.xyzc + 4 * A + 3);
-            double x[NR], w[NR];
-            rys_roots<NR>(a.rys, p * d2 * (X * X + Y * Y + Z * Z), x, w);
+    for (int A = A0; A < A1; A++) {
+        const double X = Px - ld_const(a.xyzc + 4 * A), Y = Py - ld_const(a.xyzc + 4 * A + 1);
+        const double Z = Pz - ld_const(a.xyzc + 4 * A + 2), cA = ld_const(a.xyzc + 4 * A + 3);
+        const double r2 = X * X + Y * Y + Z * Z;
+        // the operator's terms differ in the Boys argument and the powers of d^2 only
+        double b[L + 1];
 #pragma unroll
-            for (int r = 0; r < NR; r++) {
-                const double U = -2.0 * p * d2 * x[r];
-                double Hx[L + 1], Hy[L + 1], Hz[L + 1];
-                Hx[0] = -pref * w[r] * cA;
-                Hy[0] = 1.0;
-                Hz[0] = 1.0;
-                if constexpr (L > 0) {
-                    Hx[1] = U * X * Hx[0];
-                    Hy[1] = U * Y;
-                    Hz[1] = U * Z;
-                }
+        for (int n = 0; n <= L; n++) b[n] = 0.0;
+        for (int it = 0; it < a.ew.n; it++) {
+            const double om = a.ew.omega[it];
+            double f = -cA * a.ew.alpha[it] * 2.0 * kPi * ip, d2 = 1.0;
+            if (om != -1.0) {
+                d2 = om * om / (p + om * om);
+                f *= sqrt(d2);
+            }
+            const double pd = p * d2;
+            double F[L + 1];
+            if constexpr (j_md(L)) {
+                boys_lds<L>(s_tab, pd * r2, F);
+            } else {
+                double x, w;
+                rys_roots_lds<1>(s_tab, pd * r2, &x, &w);
+                F[0] = w;
+                if constexpr (L == 1) F[1] = w * x;
+            }
 #pragma unroll
-                for (int u = 1; u < L; u++) {
-                    Hx[u + 1] = U * (X * Hx[u] + u * Hx[u - 1]);
-                    Hy[u + 1] = U * (Y * Hy[u] + u * Hy[u - 1]);
-                    Hz[u + 1] = U * (Z * Hz[u] + u * Hz[u - 1]);
-                }
-                static_for<H>([&](auto T_) {
-                    constexpr int t = decltype(T_)::value;
-                    constexpr int tx = herm_tx(t), ty = herm_ty(t), tz = herm_tz(t);
-                    acc[t] += Hx[tx] * Hy[ty] * Hz[tz];
-                });
+            for (int n = 0; n <= L; n++) {
+                b[n] = fma(f, F[n], b[n]);
+                f *= -2.0 * pd;
             }
         }
+        double R[H];
+        md_level<L, 0>(b, X, Y, Z, R);
+#pragma unroll
+        for (int t = 0; t < H; t++) acc[t] += R[t];
     }
     double* dst = a.vp + hoff + (size_t)(a.hpos[k] - hstart) * H;
+    if (gridDim.y == 1) {
 #pragma unroll
-    for (int t = 0; t < H; t++) dst[t] = acc[t];
+        for (int t = 0; t < H; t++) dst[t] = acc[t];
+    } else {
+#pragma unroll
+        for (int t = 0; t < H; t++) atomic_add(dst + t, acc[t]);
+    }
 }
 
 #define LSJK_ONE_E_CASES(LAUNCH) \
@@ -144,13 +158,16 @@ void launch_one_e_st(int LA, int LB, const OneEArgs& a, int k0, int nk, hipStrea
 #undef L_ST
 }
 
-void launch_one_e_v(int LA, int LB, const OneEArgs& a, int k0, int nk, int hstart, size_t hoff, hipStream_t s)
+void launch_one_e_v(int LA, int LB, const OneEArgs& a, int k0, int nk, int nsplit, int hstart, size_t hoff,
+                    hipStream_t s)
 {
     if (nk <= 0) return;
-    dim3 grid((nk + 255) / 256), block(256);
+    dim3 grid((nk + 255) / 256, nsplit), block(256);
+    const int L = LA + LB;
+    const size_t lds = (j_md(L) ? boys_lds_doubles(L) : rys_lds_doubles(1)) * sizeof(double);
 #define L_V(X, Y)                                                                                   \
     if (LA == X && LB == Y) {                                                                       \
-        hipLaunchKernelGGL((one_e_v<X, Y>), grid, block, 0, s, a, k0, nk, hstart, hoff);            \
+        hipLaunchKernelGGL((one_e_v<X, Y>), grid, block, lds, s, a, k0, nk, hstart, hoff);            \
         return;                                                                                     \
     }
     LSJK_ONE_E_CASES(L_V)
