@@ -279,6 +279,16 @@ int lsjk_free(void* ptr);
 int lsjk_memcpy_htod(void* dst, const void* src, size_t bytes);
 int lsjk_memcpy_dtoh(void* dst, const void* src, size_t bytes);
 int lsjk_memset_zero(void* dst, size_t bytes);
+/* A device buffer for one call's operands or results, from the blocks that the session keeps (at most
+ * 128 MiB of idle ones, freed by lsjk_finalize).  Release it with busy = 0 when nothing queued uses it
+ * any more (after a call that waits: a copy to the host), else with busy = 1: it is then freed, which
+ * waits.  Not for lsjk_free. */
+int lsjk_buffer_acquire(void** ptr, size_t bytes);
+int lsjk_buffer_release(void* ptr, int busy);
+/* lsjk_memcpy_htod and lsjk_memset_zero without waiting: in order before the builds that follow.  src
+ * stays as it is until a call that waits has returned. */
+int lsjk_enqueue_htod(void* dst, const void* src, size_t bytes);
+int lsjk_enqueue_zero(void* dst, size_t bytes);
 /* Device-to-device copy by a plain copy kernel (16-byte loads and stores); also the reference
  * kernel for calibrating HBM byte counters. */
 int lsjk_memcpy_dtod(void* dst, const void* src, size_t bytes);

@@ -80,8 +80,74 @@ struct Session {
     std::vector<hipEvent_t> kev;      // event pool for per-launch timing
     std::vector<int> kid;             // launch ids of the last call (count index)
     std::vector<double> kms;          // their durations (ms)
+    // lsjk_buffer_acquire's blocks: on loan (with their sizes), and given back, the oldest first
+    std::map<void*, size_t> lent;
+    std::vector<std::pair<void*, size_t>> idle;
+    size_t idle_bytes = 0;
 };
 Session S;
+
+// hipMalloc; out of memory, the idle blocks go first.
+hipError_t device_malloc(void** p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && !S.idle.empty()) {
+        (void)hipGetLastError();
+        for (auto& b : S.idle) (void)hipFree(b.first);
+        S.idle.clear();
+        S.idle_bytes = 0;
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
+// Blocks for one call's operands and results, kept when they come back: hipMalloc and hipFree (which
+// waits for the device) cost as much as the kernels of a small call.  A block serves requests of at
+// least half its size, and the idle ones are bounded (kIdleBytes, kIdleBlocks; the oldest is freed),
+// so at most this much stays with the session; lsjk_finalize frees it.  Under g_mu, like every call.
+constexpr size_t kIdleBytes = size_t(128) << 20, kIdleBlocks = 16, kBlockUnit = size_t(64) << 10;
+
+void* block_get(size_t bytes)
+{
+    bytes = (std::max<size_t>(bytes, 1) + kBlockUnit - 1) / kBlockUnit * kBlockUnit;
+    size_t best = S.idle.size();
+    for (size_t i = 0; i < S.idle.size(); i++)
+        if (S.idle[i].second >= bytes && S.idle[i].second <= 2 * bytes &&
+            (best == S.idle.size() || S.idle[i].second < S.idle[best].second))
+            best = i;
+    if (best < S.idle.size()) {
+        const auto b = S.idle[best];
+        S.idle.erase(S.idle.begin() + best);
+        S.idle_bytes -= b.second;
+        S.lent[b.first] = b.second;
+        return b.first;
+    }
+    void* p = nullptr;
+    HIPCHK(device_malloc(&p, bytes));
+    S.lent[p] = bytes;
+    return p;
+}
+
+// `busy`: work that uses the block may still be queued (hipFree waits for it; such a block is not kept).
+void block_put(void* p, bool busy)
+{
+    if (!p) return;
+    const auto it = S.lent.find(p);
+    const size_t bytes = it == S.lent.end() ? 0 : it->second;  // 0: of a session that has ended
+    if (it != S.lent.end()) S.lent.erase(it);
+    if (busy || !bytes || bytes > kIdleBytes) {
+        HIPCHK(hipFree(p));
+        return;
+    }
+    while (!S.idle.empty() && (S.idle_bytes + bytes > kIdleBytes || S.idle.size() >= kIdleBlocks)) {
+        const auto old = S.idle.front();
+        S.idle.erase(S.idle.begin());
+        S.idle_bytes -= old.second;
+        (void)hipFree(old.first);
+    }
+    S.idle.push_back({p, bytes});
+    S.idle_bytes += bytes;
+}
 
 constexpr int kSide = 4;
 
@@ -90,7 +156,7 @@ T* dev_upload(const std::vector<T>& v)
 {
     T* p = nullptr;
     size_t bytes = std::max<size_t>(1, v.size()) * sizeof(T);
-    HIPCHK(hipMalloc((void**)&p, bytes));
+    HIPCHK(device_malloc((void**)&p, bytes));
     if (!v.empty()) HIPCHK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
     return p;
 }
@@ -224,7 +290,7 @@ struct Workspace {
             if (S.ws) HIPCHK(hipFree(S.ws));
             S.ws = nullptr;
             S.ws_bytes = 0;
-            HIPCHK(hipMalloc(&S.ws, total));
+            HIPCHK(device_malloc(&S.ws, total));
             S.ws_bytes = total;
         }
         size_t off = 0;
@@ -1439,7 +1505,7 @@ const float* screen_tau(lsjk_screen* sc, const lsjk_pairlist* pl12, const lsjk_p
     float* df = nullptr;
     std::vector<float> f(nunits);
     try {
-        HIPCHK(hipMalloc((void**)&df, std::max(nunits, 1) * sizeof(float)));
+        HIPCHK(device_malloc((void**)&df, std::max(nunits, 1) * sizeof(float)));
         lsjk::launch_mlp_forward(sc->d_params, sc->ni, nunits, dx, df, S.stream);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(S.stream));
@@ -2186,8 +2252,8 @@ void autotune(lsjk_pairlist* pl, const double* D_dev, int nterm, const double* s
             dev_free(*b);
         }
     } restore{S.nside, S.profiling, S.counting, &dJ, &dK};
-    HIPCHK(hipMalloc((void**)&dJ, n * sizeof(double)));
-    HIPCHK(hipMalloc((void**)&dK, n * sizeof(double)));
+    HIPCHK(device_malloc((void**)&dJ, n * sizeof(double)));
+    HIPCHK(device_malloc((void**)&dK, n * sizeof(double)));
     S.counting = false;
     struct ForcePlain {
         lsjk_pairlist* pl;
@@ -2643,7 +2709,7 @@ void batch_jk(lsjk_batch* b, const double* D_dev, int nterm, const double* scale
         if (b->ws) HIPCHK(hipFree(b->ws));
         b->ws = nullptr;
         b->ws_bytes = 0;
-        HIPCHK(hipMalloc(&b->ws, need));
+        HIPCHK(device_malloc(&b->ws, need));
         b->ws_bytes = need;
     }
     if (b->graphs.size() >= kBatchGraphsKept) {
@@ -2745,7 +2811,7 @@ int lsjk_init(int device)
             if (lsjk_rys_nbin[n] != lsjk::kRysNbin[n] || lsjk_rys_offset[n] != lsjk::rys_offset(n) || lsjk_rys_h[n] != 1.0 ||
                 lsjk_rys_Tc[n] != lsjk_rys_nbin[n])
                 throw LsjkError(LSJK_E_INVALID, "lsjk_init: rys_asym.inc and rys_table.inc do not belong together");
-        HIPCHK(hipMalloc((void**)&S.d_sc, sizeof(lsjk::CallScalars)));
+        HIPCHK(device_malloc((void**)&S.d_sc, sizeof(lsjk::CallScalars)));
         for (auto& e : S.ev) HIPCHK(hipEventCreate(&e));
         // device address of the no-alloc scratch array on this device (the device is current)
         S.scratch = nullptr;
@@ -2762,6 +2828,7 @@ int lsjk_finalize(void)
     return guarded([&] {
         if (!S.init) return;
         (void)hipStreamSynchronize(S.stream);
+        for (auto& b : S.idle) (void)hipFree(b.first);
         dev_free(S.d_rys_coef);
         dev_free(S.d_rys_coef32);
         dev_free(S.d_boys);
@@ -2940,7 +3007,7 @@ int lsjk_unit_magnitudes(const lsjk_pairlist* pl, int L1, int L2, int L3, int L4
             sd.cart = pl->b1->d_cart;
         }
         float* d = nullptr;
-        HIPCHK(hipMalloc((void**)&d, (size_t)units.second * sizeof(float)));
+        HIPCHK(device_malloc((void**)&d, (size_t)units.second * sizeof(float)));
         try {
             launch_k_unit_mag_sp(L1, L2, L3, L4, ka, kg, units.first, units.second, smin, d, S.stream);
             HIPCHK(hipGetLastError());
@@ -3541,13 +3608,40 @@ int lsjk_malloc(void** ptr, size_t bytes)
     return guarded([&] {
         require_init();
         if (!ptr) throw LsjkError(LSJK_E_INVALID, "lsjk_malloc: null pointer");
-        HIPCHK(hipMalloc(ptr, std::max<size_t>(bytes, 1)));
+        HIPCHK(device_malloc(ptr, std::max<size_t>(bytes, 1)));
     });
 }
 int lsjk_free(void* ptr)
 {
     return guarded([&] {
         if (ptr) HIPCHK(hipFree(ptr));
+    });
+}
+int lsjk_buffer_acquire(void** ptr, size_t bytes)
+{
+    return guarded([&] {
+        require_init();
+        if (!ptr) throw LsjkError(LSJK_E_INVALID, "lsjk_buffer_acquire: null pointer");
+        *ptr = block_get(bytes);
+    });
+}
+int lsjk_buffer_release(void* ptr, int busy)
+{
+    return guarded([&] { block_put(ptr, busy != 0); });
+}
+int lsjk_enqueue_htod(void* dst, const void* src, size_t bytes)
+{
+    return guarded([&] {
+        require_init();
+        if (bytes) HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, S.stream));
+    });
+}
+int lsjk_enqueue_zero(void* dst, size_t bytes)
+{
+    return guarded([&] {
+        require_init();
+        lsjk::launch_fill(dst, bytes, S.stream);
+        HIPCHK(hipGetLastError());
     });
 }
 int lsjk_memcpy_htod(void* dst, const void* src, size_t bytes)

@@ -4,6 +4,7 @@
 // around its kernels (src/cpp/intbox/cpu/coulomb.cpp:26-35, 186-193).
 #include <algorithm>
 #include <cstring>
+#include <exception>
 
 #include "../../../include/lsjk.h"
 #include "lightspeed.hpp"
@@ -17,13 +18,15 @@ void check(int rc)
     if (rc != LSJK_OK) throw std::runtime_error(std::string("lightspeed_amd HIP backend: ") + lsjk_last_error());
 }
 
-// RAII device buffer
+// RAII device buffer of one call, which reads its result back (and so waits) before it ends; left by
+// an exception, copies and kernels that use it may still be queued.
 struct DevBuf {
     void* p = nullptr;
-    explicit DevBuf(size_t bytes) { check(lsjk_malloc(&p, bytes)); }
+    int unwinding = std::uncaught_exceptions();
+    explicit DevBuf(size_t bytes) { check(lsjk_buffer_acquire(&p, bytes)); }
     ~DevBuf()
     {
-        if (p) lsjk_free(p);
+        if (p) lsjk_buffer_release(p, std::uncaught_exceptions() > unwinding);
     }
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
@@ -86,8 +89,8 @@ std::shared_ptr<Tensor> IntBox::coulomb(const std::shared_ptr<ResourceList>& res
     auto Dc = PureTransform::pureToCart2(b3, b4, D34);
     const size_t nD = b3->ncart() * b4->ncart(), nJ = b1->ncart() * b2->ncart();
     DevBuf dD(nD * sizeof(double)), dJ(nJ * sizeof(double));
-    check(lsjk_memcpy_htod(dD.p, Dc->data().data(), nD * sizeof(double)));
-    check(lsjk_memset_zero(dJ.p, nJ * sizeof(double)));
+    check(lsjk_enqueue_htod(dD.p, Dc->data().data(), nD * sizeof(double)));
+    check(lsjk_enqueue_zero(dJ.p, nJ * sizeof(double)));
     coulomb_device(ewald, pl12, pl34, dD.d(), thresp, thredp, dJ.d());
     auto Jc = std::make_shared<Tensor>(std::vector<size_t>{b1->ncart(), b2->ncart()}, "J");
     check(lsjk_memcpy_dtoh(Jc->data().data(), dJ.p, nJ * sizeof(double)));
@@ -110,8 +113,8 @@ std::shared_ptr<Tensor> IntBox::exchange(const std::shared_ptr<ResourceList>& re
     auto Dc = PureTransform::pureToCart2(b2, b4, D24);
     const size_t nD = b2->ncart() * b4->ncart(), nK = b1->ncart() * b3->ncart();
     DevBuf dD(nD * sizeof(double)), dK(nK * sizeof(double));
-    check(lsjk_memcpy_htod(dD.p, Dc->data().data(), nD * sizeof(double)));
-    check(lsjk_memset_zero(dK.p, nK * sizeof(double)));
+    check(lsjk_enqueue_htod(dD.p, Dc->data().data(), nD * sizeof(double)));
+    check(lsjk_enqueue_zero(dK.p, nK * sizeof(double)));
     exchange_device(ewald, pl12, pl34, dD.d(), D24symm, thresp, thredp, dK.d());
     auto Kc = std::make_shared<Tensor>(std::vector<size_t>{b1->ncart(), b3->ncart()}, "K");
     check(lsjk_memcpy_dtoh(Kc->data().data(), dK.p, nK * sizeof(double)));
@@ -132,7 +135,7 @@ std::shared_ptr<Tensor> one_electron(OneE kind, const char* who, const std::shar
     require_ready(who, resources, pl, pl);
     const size_t n = b1->ncart() * b2->ncart();
     DevBuf dM(std::max<size_t>(n, 1) * sizeof(double));
-    check(lsjk_memset_zero(dM.p, std::max<size_t>(n, 1) * sizeof(double)));
+    check(lsjk_enqueue_zero(dM.p, std::max<size_t>(n, 1) * sizeof(double)));
     lsjk_pairlist* d = pl->device_handle();
     if (kind == OneE::S) {
         check(lsjk_overlap(d, dM.d()));
@@ -187,9 +190,9 @@ std::shared_ptr<Tensor> IntBox::coulombGrad(const std::shared_ptr<ResourceList>&
     auto Dc34 = PureTransform::pureToCart2(b, b, D34);
     const size_t nD = b->ncart() * b->ncart();
     DevBuf d12(nD * sizeof(double)), d34(nD * sizeof(double)), dG(std::max<size_t>(1, 3 * natom) * sizeof(double));
-    check(lsjk_memcpy_htod(d12.p, Dc12->data().data(), nD * sizeof(double)));
-    check(lsjk_memcpy_htod(d34.p, Dc34->data().data(), nD * sizeof(double)));
-    check(lsjk_memset_zero(dG.p, std::max<size_t>(1, 3 * natom) * sizeof(double)));
+    check(lsjk_enqueue_htod(d12.p, Dc12->data().data(), nD * sizeof(double)));
+    check(lsjk_enqueue_htod(d34.p, Dc34->data().data(), nD * sizeof(double)));
+    check(lsjk_enqueue_zero(dG.p, std::max<size_t>(1, 3 * natom) * sizeof(double)));
     std::vector<double> s, o;
     ewald_arrays(ewald, s, o);
     lsjk_pairlist* d = pl->device_handle();
@@ -228,9 +231,9 @@ std::shared_ptr<Tensor> IntBox::exchangeGrad(const std::shared_ptr<ResourceList>
     auto Dc24 = PureTransform::pureToCart2(b, b, D24);
     const size_t nD = b->ncart() * b->ncart();
     DevBuf d13(nD * sizeof(double)), d24(nD * sizeof(double)), dG(std::max<size_t>(1, 3 * natom) * sizeof(double));
-    check(lsjk_memcpy_htod(d13.p, Dc13->data().data(), nD * sizeof(double)));
-    check(lsjk_memcpy_htod(d24.p, Dc24->data().data(), nD * sizeof(double)));
-    check(lsjk_memset_zero(dG.p, std::max<size_t>(1, 3 * natom) * sizeof(double)));
+    check(lsjk_enqueue_htod(d13.p, Dc13->data().data(), nD * sizeof(double)));
+    check(lsjk_enqueue_htod(d24.p, Dc24->data().data(), nD * sizeof(double)));
+    check(lsjk_enqueue_zero(dG.p, std::max<size_t>(1, 3 * natom) * sizeof(double)));
     std::vector<double> s, o;
     ewald_arrays(ewald, s, o);
     check(lsjk_exchange_grad(pl->device_handle(), d13.d(), d24.d(), (int)s.size(), s.data(), o.data(), thresp, thredp,
