@@ -521,14 +521,15 @@ def main():
 
         def launch_name(kind, lid):
             # template arguments as the profiler prints them: route 0 plain FP64, 4 mixed (FP64 and FP32
-            # parts in one launch)
+            # parts in one launch); true: the kernels for one bare 1/r term, the operator here
             if kind == "J":
                 if (lid >> 24) & 1:
-                    return "j_quartets_sym<%d, %d>" % ((lid & 0xfff) // 5, (lid & 0xfff) % 5)
-                return "j_quartets<%d, %d, %d>" % (lid // 5, lid % 5, 4 if j_mixed else 0)
+                    return "j_quartets_sym<%d, %d, %d, true>" % ((lid & 0xfff) // 5, (lid & 0xfff) % 5,
+                                                                 4 if j_mixed else 0)
+                return "j_quartets<%d, %d, %d, true>" % (lid // 5, lid % 5, 4 if j_mixed else 0)
             m = mirror(lid)
             k_route = 4 if (routes[rname][0] > thresp and ck32[lid] + (ck32[m] if m != lid else 0) > 0) else 0
-            return "k_ket<%d, %d, %d, %d, %d>" % (cls_of(lid - 256) + (k_route,))
+            return "k_ket<%d, %d, %d, %d, %d, true>" % (cls_of(lid - 256) + (k_route,))
 
         def lane_use(kind, lid):
             """Share of the wave's lanes evaluating an integral in the launch's busy wave steps."""

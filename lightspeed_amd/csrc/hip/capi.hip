@@ -1900,6 +1900,27 @@ lsjk_basis* basis_new(int nprim, const double* c, const double* e, const double*
 
 }  // namespace
 
+// Which of two mirror classes runs, the first (L1 L2 | L3 L4) with L1 < L3, or L1 = L3 and L2 < L4
+// (steps_c wave steps over nunits units), or its mirror (steps_m)?  By the wave steps, weighed by what a
+// step costs in either orientation; all pairs timed in both at (H2O)64/6-31G**, (H2O)128/6-31G* and
+// (H2O)30/cc-pVDZ (decaying densities) and C19H40/cc-pVDZ:
+//  * L1 < L3: the mirror's ket has the lower row, whose transfer from C is shorter or absent (L3 = 0)
+//    and whose lists fill the lanes better.  At equal steps (ss|ds) 1.27, 1.64, 0.58, 0.68 ms against
+//    (ds|ss) 0.55, 0.81, 0.21, 0.64; (ss|ps) 1.69, 1.62, 1.39, 1.94 against 1.64, 1.43, 0.80, 1.58;
+//    (sd|pp) with 1.02-1.14 of its steps 0.54, 0.50, 0.16, 0.33 against 0.48, 0.38, 0.15, 0.32.  The
+//    mirror is kept up to 1.25 times the steps; beyond, (ps|ds) and (pd|ds) kinds are faster as they are.
+//  * L1 = L3 = 0: the first class's ket (s L4) recurs at D and comes in groups of 64 rows, worth about a
+//    quarter of the steps ((ss|sd) 0.61 and 0.97 ms with 1.22 of the steps of (sd|ss), 1.01 and 1.64) if
+//    its fewer, longer units still fill the device's 24 waves per CU three times; with fewer, the last
+//    ones run alone ((ss|sp) 1.47 against 0.82 ms at 16500 units of equal steps, 1.98 against 1.71 at
+//    13000, but 1.98 against 2.25 at 20700 and 1.84 against 2.27 at 83000).
+bool first_orientation(int L1, int L3, double steps_c, double steps_m, int nunits)
+{
+    if (L1 < L3) return 1.25 * steps_c < steps_m;
+    if (L1 == 0) return nunits >= 3 * 24 * S.num_cu ? steps_c <= 1.25 * steps_m : 1.05 * steps_c < steps_m;
+    return steps_c <= steps_m;
+}
+
 // lsjk_exchange: workspace, unit lists, mirror-class choices, the launches on the library stream.
 static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, const double* D24_dev, int D24symm,
                           int nterm, const double* scales, const double* omegas, float thresp, float thredp,
@@ -2084,9 +2105,9 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
             // Symmetric mode (K = K^T): a class and its mirror (L3 L4 | L1 L2) hold the same quartets
             // with bra and ket swapped, so one of them, over all row pairs and with the transposed
             // block, gives both.  Which one runs faster depends on the class shapes and the lists.
-            // By default the orientation with fewer estimated wave steps is kept (the unit lists'
-            // cost: (bra partner, ket chunk) steps that pass the bound test with |D| <= 1), a
-            // deterministic choice; the autotuner times both (twice each, on the library stream,
+            // By default first_orientation picks by estimated wave steps (the unit lists' cost: (bra
+            // partner, ket chunk) steps that pass the bound test with |D| <= 1), a deterministic
+            // choice; the autotuner times both (twice each, on the library stream,
             // into a scratch K) and keeps the faster.  A class that is its own mirror takes the row
             // triangle instead.
             if (symmode && !tune && !orient && ew.n > 0 && !o.graph) {
@@ -2097,14 +2118,16 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
                             for (int L4 = 0; L4 <= b4->maxL; L4++) {
                                 const int c = kcount_index(L1, L2, L3, L4), m = kcount_index(L3, L4, L1, L2);
                                 if (c >= m) continue;
+                                int nunits = 0;  // of the class asked for last
                                 auto steps = [&](int A, int B, int C, int D_) {
+                                    nunits = 0;
                                     if (pl12->h_rows[A][B].empty() || pl34->h_rows[C][D_].empty()) return 0.0;
                                     double cost = 0.0;
-                                    get_kunits_g(pl12, pl34, A, B, C, D_, false, thresp, &cost);
+                                    nunits = (int)get_kunits_g(pl12, pl34, A, B, C, D_, false, thresp, &cost).second;
                                     return cost;
                                 };
-                                const double sc = steps(L1, L2, L3, L4), sm = steps(L3, L4, L1, L2);
-                                pick[c] = pick[m] = (sc <= sm) ? c : m;
+                                const double sm = steps(L3, L4, L1, L2), sc = steps(L1, L2, L3, L4);
+                                pick[c] = pick[m] = first_orientation(L1, L3, sc, sm, nunits) ? c : m;
                             }
                 orient = &(ocache[okey] = pick);
             }
