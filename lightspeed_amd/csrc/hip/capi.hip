@@ -864,14 +864,18 @@ const lsjk_pairlist::KGroupData& get_kgroups(lsjk_pairlist* pl, int L, int Lp, i
         while (v.size() % 64) v.push_back(make_int2(-1, 0));
         for (size_t c = 0; c < v.size(); c += 64) {
             G.chunk_b.push_back(pl->h_eb[v[c].x]);
-            // inside a chunk by the partner's K view column: neighbouring lanes then gather D from the
-            // same cache lines
-            auto col = [&](const int2& s) {
-                return s.x < 0 ? std::numeric_limits<int>::max()
-                               : pl->b2->h_kcart[pl->b2->h_cart[pl->h_eprim[s.x]]];
-            };
-            std::stable_sort(v.begin() + c, v.begin() + c + 64,
-                             [&](const int2& a, const int2& b) { return col(a) < col(b); });
+            // inside a chunk by the partner's K view column (padding last): neighbouring lanes then
+            // gather D from the same cache lines
+            unsigned long long key[64];
+            int2 in[64];
+            for (int t = 0; t < 64; t++) {
+                in[t] = v[c + t];
+                const unsigned int col = in[t].x < 0 ? 0xffffffffu
+                                                     : (unsigned int)pl->b2->h_kcart[pl->b2->h_cart[pl->h_eprim[in[t].x]]];
+                key[t] = ((unsigned long long)col << 6) | (unsigned long long)t;
+            }
+            std::sort(key, key + 64);
+            for (int t = 0; t < 64; t++) v[c + t] = in[key[t] & 63];
         }
         slot.insert(slot.end(), v.begin(), v.end());
         G.grp_slot[g + 1] = (int)slot.size();
@@ -880,11 +884,12 @@ const lsjk_pairlist::KGroupData& get_kgroups(lsjk_pairlist* pl, int L, int Lp, i
         const lsjk::Basis *b1 = pl->b1, *b2 = pl->b2;
         std::vector<int4> packed(slot.size());
         std::vector<double> ent(13 * slot.size(), 0.0);
+        int g = 0;  // the slot's group
         for (size_t q = 0; q < slot.size(); q++) {
+            while ((int)q >= G.grp_slot[g + 1]) g++;
             const int e = slot[q].x;
             packed[q] = make_int4(e, slot[q].y, 0, 0);
             if (e < 0) continue;
-            const int g = (int)(std::upper_bound(G.grp_slot.begin(), G.grp_slot.end(), (int)q) - G.grp_slot.begin()) - 1;
             const int s = pl->h_eprim[e];
             std::memcpy(&packed[q].z, &pl->h_eb[e], sizeof(float));
             packed[q].w = b2->h_kblk[b2->h_blk[s]];

@@ -10,8 +10,8 @@
 //     accumulators per pair, then the bra Hermite -> Cartesian transform shared with J.
 // A symmetric list adds the transposed block for pairs of distinct primitives.
 //
-// Kernels: one_e_st<LA,LB> (thread per pair, list order), one_e_v<LA,LB> (thread per pair,
-// writes the pair's Hermite accumulators); j_bra_scatter then transforms V.
+// Kernels: one_e_st<LA,LB> (thread per pair, list order), one_e_v<LA,LB> (thread per pair and part of
+// the charges, adds to the pair's Hermite accumulators); j_bra_scatter then transforms V.
 #include "coulomb_impl.hpp"
 
 namespace lsjk {
