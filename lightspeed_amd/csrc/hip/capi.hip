@@ -151,14 +151,27 @@ void block_put(void* p, bool busy)
 
 constexpr int kSide = 4;
 
+// Every copy goes over the library stream: it and the side streams are non-blocking streams, which the
+// null stream does not order.  An upload is complete when dev_upload returns (pageable memory; `v` may
+// go), and ordered before every kernel that is launched after it.
 template <typename T>
 T* dev_upload(const std::vector<T>& v)
 {
     T* p = nullptr;
     size_t bytes = std::max<size_t>(1, v.size()) * sizeof(T);
     HIPCHK(device_malloc((void**)&p, bytes));
-    if (!v.empty()) HIPCHK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+    if (!v.empty()) {
+        HIPCHK(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, S.stream));
+        HIPCHK(hipStreamSynchronize(S.stream));
+    }
     return p;
+}
+
+// To the host, behind what the library stream holds; complete on return.
+void dev_download(void* dst, const void* src, size_t bytes)
+{
+    if (bytes) HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, S.stream));
+    HIPCHK(hipStreamSynchronize(S.stream));
 }
 
 template <typename T>
@@ -1302,7 +1315,7 @@ void finish_call(bool count, const lsjk::CallScalars* sc)
     S.ms[1] = m1;
     if (count) {
         lsjk::CallScalars h;
-        HIPCHK(hipMemcpy(&h, sc, sizeof(h), hipMemcpyDeviceToHost));
+        dev_download(&h, sc, sizeof(h));
         std::memcpy(S.counts, h.counts, sizeof(S.counts));
         std::memcpy(S.counts32, h.counts32, sizeof(S.counts32));
         std::memcpy(S.wsteps, h.wsteps, sizeof(S.wsteps));
@@ -1482,7 +1495,7 @@ void unit_features(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34c, int L1
 std::vector<lsjk::KUnitG> download_units(const lsjk::KUnitG* d, int n)
 {
     std::vector<lsjk::KUnitG> h((size_t)std::max(n, 0));
-    if (n > 0) HIPCHK(hipMemcpy(h.data(), d, (size_t)n * sizeof(lsjk::KUnitG), hipMemcpyDeviceToHost));
+    dev_download(h.data(), d, h.size() * sizeof(lsjk::KUnitG));
     return h;
 }
 
@@ -1513,8 +1526,7 @@ const float* screen_tau(lsjk_screen* sc, const lsjk_pairlist* pl12, const lsjk_p
         HIPCHK(device_malloc((void**)&df, std::max(nunits, 1) * sizeof(float)));
         lsjk::launch_mlp_forward(sc->d_params, sc->ni, nunits, dx, df, S.stream);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(S.stream));
-        if (nunits) HIPCHK(hipMemcpy(f.data(), df, nunits * sizeof(float), hipMemcpyDeviceToHost));
+        dev_download(f.data(), df, f.size() * sizeof(float));
     } catch (...) {
         dev_free(dx);
         dev_free(df);
@@ -3039,8 +3051,7 @@ int lsjk_unit_magnitudes(const lsjk_pairlist* pl, int L1, int L2, int L3, int L4
         try {
             launch_k_unit_mag_sp(L1, L2, L3, L4, ka, kg, units.first, units.second, smin, d, S.stream);
             HIPCHK(hipGetLastError());
-            HIPCHK(hipStreamSynchronize(S.stream));
-            HIPCHK(hipMemcpy(mag, d, (size_t)units.second * sizeof(float), hipMemcpyDeviceToHost));
+            dev_download(mag, d, (size_t)units.second * sizeof(float));
         } catch (...) {
             dev_free(d);
             throw;

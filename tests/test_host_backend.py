@@ -1,0 +1,101 @@
+"""The host side of liblsjk (layouts, buffers, launch decisions) on a machine without a GPU: hip_stub.cpp
+stands in for the HIP runtime, "device" memory is host memory and kernels do not run.  Every case runs
+in a process of its own, so that one that dies names itself:
+
+    python tests/test_host_backend.py <built stub> <case>
+"""
+import ctypes
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+THRE = 1.0e-12
+CASES = {}
+
+
+def case(f):
+    CASES[f.__name__] = f
+    return f
+
+
+class Env:
+    """The package over the stub."""
+
+    def __init__(self, so):
+        self.stub = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)  # before liblsjk.so
+        for f in ("stub_uploaded", "stub_live_bytes", "stub_largest"):
+            getattr(self.stub, f).restype = ctypes.c_size_t
+        for f in ("stub_bad_frees", "stub_null_stream_copies", "stub_live_blocks", "stub_launches"):
+            getattr(self.stub, f).restype = ctypes.c_long
+        self.stub.stub_fail_from.argtypes = [ctypes.c_size_t]
+        self.stub.stub_fail_at.argtypes = [ctypes.c_long]
+        self.stub.stub_answer.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
+        sys.path[:0] = [ROOT, HERE]
+        import capi_ctypes
+        import lightspeed_amd as ls
+        self.ls, self.C = ls, capi_ctypes
+        self.res, self.ew = ls.ResourceList.build(), ls.Ewald([1.0], [-1.0])
+
+    def basis(self, n, basis="6-31gs"):
+        from lightspeed_amd import workloads as W
+        return self.ls.Basis.from_gbs_file(W.water_cluster(n, W.water_cluster_box(n), n), basis)
+
+    def pairs(self, b1, b2=None, thre=THRE):
+        return self.ls.PairList.build_schwarz(b1, b2 or b1, b2 is None, thre)
+
+    def tensor(self, *shape):
+        return self.ls.Tensor.array(np.zeros(shape))
+
+    def launches(self, part):
+        return self.stub.stub_launches(part.encode())
+
+
+@case
+def copies_are_ordered(E):
+    """No copy goes over the null stream, which does not order the library's streams, and none (nor a
+    wait) falls into a graph's recording: lists made before, lists made by the call, results, counters."""
+    I, t = E.ls.IntBox, THRE
+    b1, b2 = E.basis(2), E.basis(1, "cc-pvdz")
+    p1, p2 = E.pairs(b1), E.pairs(b2)
+    E.ls.set_counting(True)
+    for n, a, b in ((b1, p1, p1), (b2, p2, p2), (b2, p1, p2)):
+        for thredp in (t, 1.0e-6):
+            I.coulomb(E.res, E.ew, a, b, E.tensor(n.nao, n.nao), t, thredp)
+    for symm in (True, False):
+        I.exchange(E.res, E.ew, p1, p1, E.tensor(b1.nao, b1.nao), symm, t, 1.0e-6)
+    E.ls.last_counts()
+    E.ls.set_counting(False)
+    D = E.tensor(b2.nao, b2.nao)
+    I.coulombGrad(E.res, E.ew, p2, D, D, t, t)
+    I.exchangeGrad(E.res, E.ew, p2, D, D, True, True, True, t, t)
+    I.overlap(E.res, p2)
+    I.potential(E.res, E.ew, p2, E.tensor(9, 4))
+    d = E.ls.DeviceArray([b2.ncart, b2.ncart])
+    E.ls.count_quartets(p2, p2, d.ptr, d.ptr, True, t)
+    batch = E.ls.JKBatch.build(E.res, [p1, p2])
+    buf = [E.ls.DeviceArray([batch.nelem]) for _ in range(3)]
+    for thresp in (t, 1.0e-11, 1.0e-10, 1.0e-9, 1.0e-8, t):  # more thresholds than unit lists are kept for
+        batch.jk_device(E.ew, buf[0].ptr, thresp, thresp, buf[1].ptr, buf[2].ptr)
+    assert E.stub.stub_null_stream_copies() == 0
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.check_call(["g++", "-shared", "-fPIC", "-O1", "-std=c++17", os.path.join(HERE, "hip_stub.cpp"), "-o", so])
+    return so
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_host(stub, name):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), stub, name], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-4000:])
+
+
+if __name__ == "__main__":
+    CASES[sys.argv[2]](Env(sys.argv[1]))
