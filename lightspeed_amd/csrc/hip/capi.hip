@@ -3481,7 +3481,7 @@ int lsjk_potential(const lsjk_pairlist* pl, int nterm, const double* scales, con
             throw LsjkError(LSJK_E_INVALID, "lsjk_potential: null or invalid argument");
         Ewald ew;
         check_ewald(nterm, scales, omegas, ew);
-        if (ew.n == 0 || ncharge == 0) return;
+        if (ew.n == 0 || ncharge == 0 || pl->npair == 0) return;
         hipStream_t st = S.stream;
         const Basis *b1 = pl->b1, *b2 = pl->b2;
         double* vp = nullptr;

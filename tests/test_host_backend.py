@@ -84,6 +84,35 @@ def copies_are_ordered(E):
     assert E.stub.stub_null_stream_copies() == 0
 
 
+@case
+def empty_lists(E):
+    """Every entry point on a list without pairs adds nothing and returns."""
+    I, t = E.ls.IntBox, THRE
+    bas = E.basis(1)
+    n = bas.nao
+    none = E.pairs(bas, thre=1.0e10)
+    some = E.pairs(bas)
+    assert none.npair == 0 and some.npair > 0
+    D = E.tensor(n, n)
+    for a, b in ((none, none), (none, some), (some, none)):
+        I.coulomb(E.res, E.ew, a, b, D, t, t)
+        I.exchange(E.res, E.ew, a, b, D, True, t, t)
+        I.exchange(E.res, E.ew, a, b, D, False, t, 1.0e-6)
+    I.coulombGrad(E.res, E.ew, none, D, D, t, t)
+    I.exchangeGrad(E.res, E.ew, none, D, D, True, True, True, t, t)
+    I.overlap(E.res, none)
+    I.kinetic(E.res, none)
+    for charges in (0, 1, 300):
+        I.potential(E.res, E.ew, none, E.tensor(charges, 4))
+    d = E.ls.DeviceArray([n, n])
+    E.ls.count_quartets(none, none, d.ptr, d.ptr, True, t)
+    for lists in ([none], [none, some]):
+        batch = E.ls.JKBatch.build(E.res, lists)
+        buf = [E.ls.DeviceArray([batch.nelem]) for _ in range(3)]
+        for _ in range(2):
+            batch.jk_device(E.ew, buf[0].ptr, t, t, buf[1].ptr, buf[2].ptr)
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
