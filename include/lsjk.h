@@ -282,7 +282,7 @@ int lsjk_memset_zero(void* dst, size_t bytes);
 /* A device buffer for one call's operands or results, from the blocks that the session keeps (at most
  * 128 MiB of idle ones, freed by lsjk_finalize).  Release it with busy = 0 when nothing queued uses it
  * any more (after a call that waits: a copy to the host), else with busy = 1: it is then freed, which
- * waits.  Not for lsjk_free. */
+ * waits.  Once only: a block that is not on loan is refused, as any block of these is by lsjk_free. */
 int lsjk_buffer_acquire(void** ptr, size_t bytes);
 int lsjk_buffer_release(void* ptr, int busy);
 /* lsjk_memcpy_htod and lsjk_memset_zero without waiting: in order before the builds that follow.  src

@@ -128,10 +128,17 @@ void* block_get(size_t bytes)
     return p;
 }
 
+bool block_idle(const void* p)
+{
+    return std::any_of(S.idle.begin(), S.idle.end(), [p](const std::pair<void*, size_t>& b) { return b.first == p; });
+}
+
 // `busy`: work that uses the block may still be queued (hipFree waits for it; such a block is not kept).
 void block_put(void* p, bool busy)
 {
     if (!p) return;
+    // given back already: freed here, it would be handed out again
+    if (block_idle(p)) throw LsjkError(LSJK_E_INVALID, "lsjk_buffer_release: the block is not on loan");
     const auto it = S.lent.find(p);
     const size_t bytes = it == S.lent.end() ? 0 : it->second;  // 0: of a session that has ended
     if (it != S.lent.end()) S.lent.erase(it);
@@ -3653,6 +3660,8 @@ int lsjk_malloc(void** ptr, size_t bytes)
 int lsjk_free(void* ptr)
 {
     return guarded([&] {
+        if (ptr && (S.lent.count(ptr) || block_idle(ptr)))
+            throw LsjkError(LSJK_E_INVALID, "lsjk_free: a block of lsjk_buffer_acquire");
         if (ptr) HIPCHK(hipFree(ptr));
     });
 }

@@ -113,6 +113,52 @@ def empty_lists(E):
             batch.jk_device(E.ew, buf[0].ptr, t, t, buf[1].ptr, buf[2].ptr)
 
 
+@case
+def call_buffers(E):
+    """A block given back twice, or freed by lsjk_free, is refused and stays what it was; what is idle is
+    bounded by 128 MiB and 16 blocks; a block given back busy is freed."""
+    E.ls.hip_init(0)
+    L = E.C.load()
+    L.lsjk_buffer_acquire.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+    L.lsjk_buffer_release.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    release = L.lsjk_buffer_release
+    held_by_session = E.stub.stub_live_bytes(), E.stub.stub_live_blocks()
+
+    def get(nbytes):
+        p = ctypes.c_void_p()
+        assert L.lsjk_buffer_acquire(ctypes.byref(p), nbytes) == 0
+        return p.value
+
+    def idle():
+        """Bytes and blocks beyond the session's own (nothing is on loan)."""
+        return E.stub.stub_live_bytes() - held_by_session[0], E.stub.stub_live_blocks() - held_by_session[1]
+
+    mib = 1 << 20
+    a = get(mib)
+    assert L.lsjk_free(a) != 0  # on loan
+    assert release(a, 0) == 0
+    for busy in (0, 1):
+        assert release(a, busy) != 0  # idle
+    assert L.lsjk_free(a) != 0
+    b, c = get(mib), get(mib)
+    assert b == a and c != a  # not handed out twice
+    assert release(b, 1) == 0 and release(c, 0) == 0
+    assert idle() == (mib, 1)
+    for p in [get(40 * mib) for _ in range(5)]:
+        assert release(p, 0) == 0
+    assert idle()[0] <= 128 * mib
+    for p in [get(mib) for _ in range(40)]:
+        assert release(p, 0) == 0
+    nbytes, blocks = idle()
+    assert blocks <= 16 and nbytes <= 128 * mib
+    p = get(200 * mib)  # larger than all that may be idle
+    assert release(p, 0) == 0 and idle() == (nbytes, blocks)
+    p = get(3 * mib)
+    assert idle()[1] == blocks + 1 and release(p, 1) == 0 and idle() == (nbytes, blocks)
+    assert release(None, 0) == 0 and E.stub.stub_bad_frees() == 0
+    assert L.lsjk_finalize() == 0 and E.stub.stub_bad_frees() == 0
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
