@@ -87,7 +87,8 @@ struct Session {
 };
 Session S;
 
-// hipMalloc; out of memory, the idle blocks go first.
+// hipMalloc; out of memory, the idle blocks go first.  The error is the caller's: it does not stay
+// behind for the check after the next launches.
 hipError_t device_malloc(void** p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
@@ -98,6 +99,7 @@ hipError_t device_malloc(void** p, size_t bytes)
         S.idle_bytes = 0;
         e = hipMalloc(p, bytes);
     }
+    if (e != hipSuccess) (void)hipGetLastError();
     return e;
 }
 
@@ -288,6 +290,22 @@ struct Workspace {
     std::vector<std::pair<void**, size_t>> req;
     template <typename T>
     void add(T** p, size_t count) { req.push_back({(void**)p, std::max<size_t>(1, count) * sizeof(T)}); }
+    // A last piece that the call can do without: left out (null) where the rest fits and it does not.
+    template <typename T>
+    void add_optional(T** p, size_t count)
+    {
+        add(p, count);
+        optional = true;
+    }
+    bool optional = false;
+    bool drop_optional()
+    {
+        if (!optional) return false;
+        *req.back().first = nullptr;
+        req.pop_back();
+        optional = false;
+        return true;
+    }
     // ext: carve the pieces from this fixed buffer of ext_bytes (nothing is allocated; a request
     // that does not fit raises); nullptr: from the session workspace, grown as needed.
     void commit(void* ext = nullptr, size_t ext_bytes = 0, const char* who = nullptr)
@@ -295,6 +313,7 @@ struct Workspace {
         size_t total = 0;
         for (auto& r : req) total += (r.second + 255) & ~size_t(255);
         if (ext) {
+            if (total > ext_bytes && drop_optional()) return commit(ext, ext_bytes, who);
             if (total > ext_bytes)
                 throw LsjkError(LSJK_E_UNSUPPORTED, std::string(who ? who : "lsjk") + ": the call needs " +
                                                         std::to_string(total) + " bytes of scratch, more than the " +
@@ -310,7 +329,9 @@ struct Workspace {
             if (S.ws) HIPCHK(hipFree(S.ws));
             S.ws = nullptr;
             S.ws_bytes = 0;
-            HIPCHK(device_malloc(&S.ws, total));
+            const hipError_t e = device_malloc(&S.ws, total);
+            if (e == hipErrorOutOfMemory && drop_optional()) return commit();
+            HIPCHK(e);
             S.ws_bytes = total;
         }
         size_t off = 0;
@@ -1579,7 +1600,8 @@ struct CallOpts {
 };
 
 // Elements of KArgs::rw for a bra list and the ket partners' basis.  It is formed up to 4 GiB (about
-// 20,000 primitives with 18,000 shells); 0 above that: the kernel then sieves with the largest |D|.
+// 20,000 primitives with 18,000 shells); 0 above that, and not where the memory cannot be had: the
+// kernel then sieves with the largest |D|.
 size_t rowmax_elems(const lsjk_pairlist* pl12, const lsjk::Basis* b4)
 {
     const size_t n = (size_t)pl12->nrow * (pl12->kmaxL2 + 1) * (size_t)lsjk::blk_ld(b4);
@@ -1996,8 +2018,8 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
             wsp.add(&Dsh, blk_elems(b2, b4));
         }
         const size_t nrw = rowmax_elems(pl12, b4);
-        if (nrw) wsp.add(&rw, nrw);
         if (tune) wsp.add(&Ks, mat_elems(b1, b3));
+        if (nrw) wsp.add_optional(&rw, nrw);
         commit_ws(wsp, o, who);
         const bool timed = !o.graph;
 
@@ -2577,6 +2599,7 @@ struct lsjk_batch {
     size_t nelem = 0;
     void* ws = nullptr;  // fixed workspace of the captured graphs
     size_t ws_bytes = 0;
+    bool no_rowmax = false;  // its scratch could not be had with the rows' maxima (KArgs::rw)
     std::vector<BatchGraph> graphs;  // most recent last
 };
 
@@ -2703,7 +2726,8 @@ size_t batch_ws_bytes(const lsjk_batch* b, bool mixed, size_t* jbytes)
     size_t j = r(((size_t)pl->npair + 1) * sizeof(float)) + r((h + lsjk::kMaxHerm) * sizeof(double)) + r(h * sizeof(double));
     if (mixed) j += r(h * sizeof(float));
     *jbytes = j;
-    return j + r(blk_elems(b->basis, b->basis) * sizeof(double)) + r(rowmax_elems(pl, b->basis) * sizeof(unsigned int));
+    const size_t nrw = b->no_rowmax ? 0 : rowmax_elems(pl, b->basis);
+    return j + r(blk_elems(b->basis, b->basis) * sizeof(double)) + (nrw ? r(nrw * sizeof(unsigned int)) : 0);
 }
 
 void batch_jk(lsjk_batch* b, const double* D_dev, int nterm, const double* scales, const double* omegas, float thresp,
@@ -2749,14 +2773,20 @@ void batch_jk(lsjk_batch* b, const double* D_dev, int nterm, const double* scale
     }
     // then capture the same launches into a graph, for the next calls with these arguments
     size_t jbytes = 0;
-    const size_t need = batch_ws_bytes(b, thredp > thresp, &jbytes);
+    size_t need = batch_ws_bytes(b, thredp > thresp, &jbytes);
     if (need > b->ws_bytes) {
         for (auto& g : b->graphs) batch_drop_graph(g);  // they use the old workspace
         b->graphs.clear();
         if (b->ws) HIPCHK(hipFree(b->ws));
         b->ws = nullptr;
         b->ws_bytes = 0;
-        HIPCHK(device_malloc(&b->ws, need));
+        hipError_t e = device_malloc(&b->ws, need);
+        if (e == hipErrorOutOfMemory && !b->no_rowmax) {
+            b->no_rowmax = true;
+            need = batch_ws_bytes(b, thredp > thresp, &jbytes);
+            e = device_malloc(&b->ws, need);
+        }
+        HIPCHK(e);
         b->ws_bytes = need;
     }
     if (b->graphs.size() >= kBatchGraphsKept) {

@@ -19,11 +19,12 @@ constexpr int kHostToDevice = 1, kDeviceToHost = 2;
 std::map<void*, size_t> live;
 std::map<const void*, std::string> kernels;  // host stub of a kernel -> its name
 std::vector<std::string> launched;
-size_t fail_from = SIZE_MAX;  // allocations of at least this size fail
-long fail_at = -1;            // so does the one after this many more
+long fail_at = -1;  // the allocation after this many more fails, and its retries (same size)
+size_t failing = 0;
 long bad_frees = 0, null_stream_copies = 0;
 bool capturing = false;  // copies from pageable memory and waits are errors then
-size_t uploaded = 0, largest = 0;
+size_t uploaded = 0;
+long allocations = 0;
 int last_error = kSuccess;
 std::string answer;  // what the next copy to the host of this size gives
 struct Call {
@@ -101,11 +102,12 @@ int hipGetLastError(void)
 
 int hipMalloc(void** p, size_t n)
 {
-    if (n >= fail_from || fail_at == 0) return fail_at = -1, set(kOutOfMemory);
-    if (fail_at > 0) fail_at--;
+    if (fail_at >= 0 && fail_at-- == 0) failing = n;
+    if (n == failing) return set(kOutOfMemory);
+    failing = 0;
     *p = std::calloc(n ? n : 1, 1);
     live[*p] = n;
-    if (n > largest) largest = n;
+    allocations++;
     return kSuccess;
 }
 int hipFree(void* p)
@@ -141,7 +143,6 @@ int hipEventSynchronize(void*) { return kSuccess; }
 int hipEventElapsedTime(float* ms, void*, void*) { return *ms = 1.0f, kSuccess; }
 
 // ---- what the tests ask
-void stub_fail_from(size_t bytes) { fail_from = bytes; }
 void stub_fail_at(long n) { fail_at = n; }
 void stub_answer(const void* p, size_t n) { answer.assign(static_cast<const char*>(p), n); }
 long stub_bad_frees(void) { return bad_frees; }
@@ -154,8 +155,7 @@ size_t stub_live_bytes(void)
     return n;
 }
 long stub_live_blocks(void) { return static_cast<long>(live.size()); }
-size_t stub_largest(void) { return largest; }
-void stub_clear_largest(void) { largest = 0; }
+long stub_allocations(void) { return allocations; }
 // launches so far of kernels with `part` in their (mangled) names
 long stub_launches(const char* part)
 {

@@ -28,11 +28,10 @@ class Env:
 
     def __init__(self, so):
         self.stub = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)  # before liblsjk.so
-        for f in ("stub_uploaded", "stub_live_bytes", "stub_largest"):
+        for f in ("stub_uploaded", "stub_live_bytes"):
             getattr(self.stub, f).restype = ctypes.c_size_t
-        for f in ("stub_bad_frees", "stub_null_stream_copies", "stub_live_blocks", "stub_launches"):
+        for f in ("stub_bad_frees", "stub_null_stream_copies", "stub_live_blocks", "stub_launches", "stub_allocations"):
             getattr(self.stub, f).restype = ctypes.c_long
-        self.stub.stub_fail_from.argtypes = [ctypes.c_size_t]
         self.stub.stub_fail_at.argtypes = [ctypes.c_long]
         self.stub.stub_answer.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
         sys.path[:0] = [ROOT, HERE]
@@ -157,6 +156,47 @@ def call_buffers(E):
     assert idle()[1] == blocks + 1 and release(p, 1) == 0 and idle() == (nbytes, blocks)
     assert release(None, 0) == 0 and E.stub.stub_bad_frees() == 0
     assert L.lsjk_finalize() == 0 and E.stub.stub_bad_frees() == 0
+
+
+@case
+def exchange_without_row_maxima(E):
+    """Where the scratch with the sieve's row maxima cannot be had, the build goes without them; so does a
+    batch, whose graph is recorded all the same.  The next call is as ever."""
+    bas = E.basis(3)
+    n, t = bas.nao, THRE
+    pl = E.pairs(bas)
+    E.ls.IntBox.overlap(E.res, pl)  # the list's own arrays
+    D, K = E.ls.DeviceArray([n, n]), E.ls.DeviceArray([n, n])
+
+    def build(thredp):
+        before = E.launches("k_rowmax"), E.launches("k_ket")
+        E.ls.IntBox.exchange_device(E.ew, pl, pl, D.ptr, True, t, thredp, K.ptr)
+        return E.launches("k_rowmax") - before[0], E.launches("k_ket") - before[1]
+
+    E.stub.stub_fail_at(0)  # the call's scratch is what it allocates first
+    rowmax, ket = build(t)
+    assert rowmax == 0 and ket > 0
+    assert build(t) == (1, ket)
+    assert build(1.0e-6)[0] == 1
+
+    def batch():
+        b = E.ls.JKBatch.build(E.res, [pl, pl])
+        return b, [E.ls.DeviceArray([b.nelem]) for _ in range(3)]
+
+    def jk(b, buf, thredp=t):
+        first = E.stub.stub_allocations(), E.launches("k_rowmax")
+        b.jk_device(E.ew, buf[0].ptr, t, thredp, buf[1].ptr, buf[2].ptr)
+        return E.stub.stub_allocations() - first[0], E.launches("k_rowmax") - first[1]
+
+    jk(*batch())
+    nalloc, rowmax = jk(*batch())
+    assert rowmax == 2  # the call's own run and the recorded one
+    b, buf = batch()
+    E.stub.stub_fail_at(nalloc - 1)  # the graph's scratch is what it allocates last
+    assert jk(b, buf) == (nalloc, 1)
+    assert jk(b, buf) == (0, 0)  # replayed
+    assert jk(b, buf, 1.0e-6)[1] == 1  # another graph, more scratch: again without
+    E.ls.IntBox.coulomb_device(E.ew, pl, pl, D.ptr, t, t, K.ptr)
 
 
 @pytest.fixture(scope="module")
