@@ -732,8 +732,8 @@ long long j_chunk(long long nket, long long ntile, int L)
 const lsjk_pairlist::GradPairs& get_grad_pairs(lsjk_pairlist* pl)
 {
     using namespace lsjk;
-    auto& gd = pl->grad;
-    if (gd.built) return gd;
+    if (pl->grad.built) return pl->grad;
+    lsjk_pairlist::GradPairs gd;  // the list's own only once it is whole: an allocation may fail
     const Basis* b = pl->b1;
     std::vector<int> order(pl->npair);
     std::vector<int> cls(pl->npair);
@@ -782,11 +782,17 @@ const lsjk_pairlist::GradPairs& get_grad_pairs(lsjk_pairlist* pl)
         bound[q] = pl->h_bound[k];
         prim[q] = make_int2(i, j);
     }
-    gd.d_g = dev_upload(g);
-    gd.d_b = dev_upload(bound);
-    gd.d_prim = dev_upload(prim);
+    try {
+        gd.d_g = dev_upload(g);
+        gd.d_b = dev_upload(bound);
+        gd.d_prim = dev_upload(prim);
+    } catch (...) {
+        dev_free(gd.d_g);
+        dev_free(gd.d_b);
+        throw;
+    }
     gd.built = true;
-    return gd;
+    return pl->grad = gd;
 }
 
 // How one class pair of the exchange gradient is cut into waves.  chunk: pairs of class 2 one wave

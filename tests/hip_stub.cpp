@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <sstream>
 #include <string>
 #include <vector>
 
@@ -18,7 +19,7 @@ constexpr int kHostToDevice = 1, kDeviceToHost = 2;
 
 std::map<void*, size_t> live;
 std::map<const void*, std::string> kernels;  // host stub of a kernel -> its name
-std::vector<std::string> launched;
+std::vector<std::string> launched;  // name and shape of each launch
 long fail_at = -1;  // the allocation after this many more fails, and its retries (same size)
 size_t failing = 0;
 long bad_frees = 0, null_stream_copies = 0;
@@ -78,11 +79,12 @@ int __hipPopCallConfiguration(Dim3* grid, Dim3* block, size_t* lds, void** strea
     *stream = pushed.stream;
     return kSuccess;
 }
-int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void**, size_t, void*)
+int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void**, size_t lds, void*)
 {
     if (!grid.x || !grid.y || !grid.z || !block.x) return set(kInvalid);
-    const auto it = kernels.find(f);
-    launched.push_back(it == kernels.end() ? "?" : it->second);
+    std::ostringstream s;
+    s << kernels[f] << ' ' << grid.x << 'x' << grid.y << 'x' << grid.z << " of " << block.x << " lds " << lds;
+    launched.push_back(s.str());
     return kSuccess;
 }
 
@@ -156,6 +158,14 @@ size_t stub_live_bytes(void)
 }
 long stub_live_blocks(void) { return static_cast<long>(live.size()); }
 long stub_allocations(void) { return allocations; }
+// the launches from number `first` on, a line each
+const char* stub_launch_log(long first)
+{
+    static std::string all;
+    all.clear();
+    for (size_t i = first; i < launched.size(); i++) all += launched[i] + "\n";
+    return all.c_str();
+}
 // launches so far of kernels with `part` in their (mangled) names
 long stub_launches(const char* part)
 {

@@ -32,6 +32,8 @@ class Env:
             getattr(self.stub, f).restype = ctypes.c_size_t
         for f in ("stub_bad_frees", "stub_null_stream_copies", "stub_live_blocks", "stub_launches", "stub_allocations"):
             getattr(self.stub, f).restype = ctypes.c_long
+        self.stub.stub_launch_log.restype = ctypes.c_char_p
+        self.stub.stub_launch_log.argtypes = [ctypes.c_long]
         self.stub.stub_fail_at.argtypes = [ctypes.c_long]
         self.stub.stub_answer.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
         sys.path[:0] = [ROOT, HERE]
@@ -197,6 +199,46 @@ def exchange_without_row_maxima(E):
     assert jk(b, buf) == (0, 0)  # replayed
     assert jk(b, buf, 1.0e-6)[1] == 1  # another graph, more scratch: again without
     E.ls.IntBox.coulomb_device(E.ew, pl, pl, D.ptr, t, t, K.ptr)
+
+
+@case
+def failed_allocations(E):
+    """Whichever of its allocations a call fails at, the same call afterwards launches what it does on
+    fresh lists."""
+    I, t = E.ls.IntBox, THRE
+    bas = E.basis(1, "6-31gs")
+    D = E.tensor(bas.nao, bas.nao)
+    calls = {
+        "J": lambda p: I.coulomb(E.res, E.ew, p, p, D, t, t),
+        "K": lambda p: I.exchange(E.res, E.ew, p, p, D, True, t, t),
+        "K, general": lambda p: I.exchange(E.res, E.ew, p, p, D, False, t, t),
+        "J gradient": lambda p: I.coulombGrad(E.res, E.ew, p, D, D, t, t),
+        "K gradient": lambda p: I.exchangeGrad(E.res, E.ew, p, D, D, True, True, True, t, t),
+        "V": lambda p: I.potential(E.res, E.ew, p, E.tensor(50, 4)),
+    }
+
+    def launches(f, p):
+        first = E.launches("")
+        f(p)
+        return E.stub.stub_launch_log(first).decode()
+
+    for name, f in calls.items():
+        p = E.pairs(bas)
+        n = E.stub.stub_allocations()
+        fresh = launches(f, p)
+        n = E.stub.stub_allocations() - n
+        assert fresh and launches(f, p) == fresh
+        failed = 0
+        for k in range(n + 1):
+            p = E.pairs(bas)
+            E.stub.stub_fail_at(k)
+            try:
+                f(p)
+            except RuntimeError:
+                failed += 1
+            E.stub.stub_fail_at(-1)
+            assert launches(f, p) == fresh, (name, k)
+        assert failed >= n // 2, (name, failed, n)
 
 
 @pytest.fixture(scope="module")
