@@ -1667,9 +1667,10 @@ static void coulomb_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, c
         double* kd = nullptr;
         double* jp = nullptr;
         Workspace wsp;
-        // one ket more than the list's: the kernels read one past a range's end
-        wsp.add(&kb, (size_t)pl34->npair + 1);
-        wsp.add(&kd, pl34->hoff[2 * kMaxL + 1] + kMaxHerm);
+        // j_quartets loads one ket ahead: at a list's end one float past kb and at most four doubles past
+        // kd, unused, out of the piece that lies behind (kd, jp; pieces are at least 256 bytes)
+        wsp.add(&kb, (size_t)pl34->npair);
+        wsp.add(&kd, pl34->hoff[2 * kMaxL + 1]);
         wsp.add(&jp, pl12->hoff[2 * kMaxL + 1]);
         float* kd32 = nullptr;
         if (mixed) wsp.add(&kd32, pl34->hoff[2 * kMaxL + 1]);
@@ -2729,7 +2730,7 @@ size_t batch_ws_bytes(const lsjk_batch* b, bool mixed, size_t* jbytes)
     auto r = [](size_t n) { return (std::max<size_t>(1, n) + 255) & ~size_t(255); };
     const lsjk_pairlist* pl = b->list;
     const size_t h = pl->hoff[2 * lsjk::kMaxL + 1];
-    size_t j = r(((size_t)pl->npair + 1) * sizeof(float)) + r((h + lsjk::kMaxHerm) * sizeof(double)) + r(h * sizeof(double));
+    size_t j = r((size_t)pl->npair * sizeof(float)) + r(h * sizeof(double)) + r(h * sizeof(double));
     if (mixed) j += r(h * sizeof(float));
     *jbytes = j;
     const size_t nrw = b->no_rowmax ? 0 : rowmax_elems(pl, b->basis);
@@ -3309,8 +3310,9 @@ int lsjk_coulomb_grad(const lsjk_pairlist* pl, const double* Dbra_dev, const dou
         double* kd = nullptr;
         double* vp = nullptr;
         Workspace wsp;
-        wsp.add(&kb, (size_t)pl->npair + 1);
-        wsp.add(&kd, pl->hoff[2 * kMaxL + 1] + kMaxHerm);
+        // read one ket ahead, as in coulomb_call
+        wsp.add(&kb, (size_t)pl->npair);
+        wsp.add(&kd, pl->hoff[2 * kMaxL + 1]);
         wsp.add(&vp, hoff2[2 * kMaxL + 1]);
         wsp.commit();
         const JTaskList& seg = *get_jtasks(pl, pl);
@@ -3595,9 +3597,8 @@ int lsjk_count_quartets(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, co
         double* Dsh = nullptr;
         unsigned long long* out = nullptr;
         Workspace wsp;
-        // one ket more than the list's: the kernels read one past a range's end
-        wsp.add(&kb, (size_t)pl34->npair + 1);
-        wsp.add(&kd, pl34->hoff[2 * kMaxL + 1] + kMaxHerm);
+        wsp.add(&kb, (size_t)pl34->npair);
+        wsp.add(&kd, pl34->hoff[2 * kMaxL + 1]);
         wsp.add(&Dsh, (size_t)b2->nblk * b4->nblk);
         wsp.add(&out, 2 * 625);
         wsp.commit();

@@ -299,7 +299,7 @@ constexpr int j_waves(int L12, int L34, int route, bool bare)
 // Persistent kernel: each wave takes (64 bra pairs x ket range) tasks from a queue until it is
 // empty.  The workgroup's waves share an LDS copy of the tables (JLds).  Lanes own bra pairs; the
 // kets are read at wave-uniform addresses (scalar loads) one ket ahead of their use, in bound order
-// (the lists and per-call buffers are padded by one ket).  Quartets with est = B12 * B34' at or above
+// (the lists are padded by one ket; behind the per-call buffers lies more of the same scratch).  Quartets with est = B12 * B34' at or above
 // thresp are evaluated in FP64 (kRoutePlain), or on the mixed route (kRouteMixed) a ket step with any
 // quartet at or above thredp in FP64 and the others in FP32.
 template <int L12, int L34, int ROUTE, bool BARE>
@@ -309,7 +309,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(j_waves(L12
     using Lds = JLds<L12, L34, ROUTE>;
     constexpr int H12 = nherm(L12), H34 = nherm(L34), L = L12 + L34, HL = nherm(L);
     constexpr bool MIXED = ROUTE == kRouteMixed;
-    constexpr int DN = H34 <= 4 ? H34 : 1;  // ket densities loaded ahead
+    constexpr int DN = H34 <= 4 ? H34 : 1;  // ket densities loaded ahead (coulomb_call's scratch: at most 4)
     extern __shared__ double s_dyn[];
     double* s_tab64 = s_dyn;
     float* s_tab32 = reinterpret_cast<float*>(reinterpret_cast<char*>(s_dyn) + Lds::kBytes64);

@@ -241,6 +241,44 @@ def failed_allocations(E):
         assert failed >= n // 2, (name, failed, n)
 
 
+@case
+def noalloc_scratch_limit(E):
+    """lsjk_coulomb_noalloc takes what fits its 64 MiB (a float bound and H doubles per ket pair, H doubles
+    per bra pair, each of the three rounded up to 256 bytes), here to the byte."""
+    E.ls.hip_init(0)
+    L, ptr = E.C.load(), ctypes.c_void_p
+    n, m, H = 64000, 174760, 35  # pairs of two d functions
+    r = lambda b: (b + 255) // 256 * 256  # noqa: E731
+    assert r(4 * n) + r(8 * H * n) + r(8 * H * m) == 64 << 20
+
+    def pairs(npair):
+        nprim = int(np.ceil(np.sqrt(npair)))
+        f, i = np.ones(nprim), np.arange(nprim, dtype=np.int32)
+        xyz = np.linspace(0.0, 1.0, 3 * nprim)
+        p = np.arange(npair)
+        b, l = ptr(), ptr()
+        two, cart = np.full(nprim, 2, np.int32), np.ascontiguousarray(6 * i)
+        assert L.lsjk_basis_create(nprim, f.ctypes.data, f.ctypes.data, xyz.ctypes.data, two.ctypes.data, cart.ctypes.data,
+                                   6 * nprim, ctypes.byref(b)) == 0
+        p1, p2 = (np.ascontiguousarray(v, np.int32) for v in (p // nprim, p % nprim))
+        bound = np.ones(npair, np.float32)
+        assert L.lsjk_pairlist_create(b, b, 0, npair, p1.ctypes.data, p2.ctypes.data, bound.ctypes.data, ctypes.byref(l)) == 0
+        return l
+
+    bra, larger, ket = pairs(m), pairs(m + 1), pairs(n)
+    D = np.zeros((6 * 253) ** 2)
+    J = np.zeros((6 * 419) ** 2)
+    one, bare = np.array([1.0]), np.array([-1.0])
+
+    def call(f, bra, ket):
+        return f(bra, ket, D.ctypes.data, 1, one.ctypes.data, bare.ctypes.data, THRE, THRE, J.ctypes.data)
+
+    for b in (bra, larger):
+        assert call(L.lsjk_coulomb, b, ket) == 0  # the task lists
+    assert call(L.lsjk_coulomb_noalloc, bra, ket) == 0, L.lsjk_last_error()
+    assert call(L.lsjk_coulomb_noalloc, larger, ket) != 0
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
