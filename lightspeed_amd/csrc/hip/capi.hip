@@ -1,11 +1,13 @@
 // C-ABI of liblsjk: session, device-resident basis / pair-list layouts, and the orchestration of
 // the J and K kernels on the library stream.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <limits>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <tuple>
 #include <numeric>
@@ -13,6 +15,8 @@
 #include <type_traits>
 #include <stdexcept>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../../include/lsjk.h"
@@ -164,16 +168,21 @@ constexpr int kSide = 4;
 // null stream does not order.  An upload is complete when dev_upload returns (pageable memory; `v` may
 // go), and ordered before every kernel that is launched after it.
 template <typename T>
-T* dev_upload(const std::vector<T>& v)
+T* dev_upload(const T* v, size_t n)
 {
     T* p = nullptr;
-    size_t bytes = std::max<size_t>(1, v.size()) * sizeof(T);
-    HIPCHK(device_malloc((void**)&p, bytes));
-    if (!v.empty()) {
-        HIPCHK(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, S.stream));
+    HIPCHK(device_malloc((void**)&p, std::max<size_t>(1, n) * sizeof(T)));
+    if (n) {
+        HIPCHK(hipMemcpyAsync(p, v, n * sizeof(T), hipMemcpyHostToDevice, S.stream));
         HIPCHK(hipStreamSynchronize(S.stream));
     }
     return p;
+}
+
+template <typename T>
+T* dev_upload(const std::vector<T>& v)
+{
+    return dev_upload(v.data(), v.size());
 }
 
 // To the host, behind what the library stream holds; complete on return.
@@ -381,19 +390,26 @@ void check_ewald(int nterm, const double* scales, const double* omegas, lsjk::Ew
 
 // ------------------------------------------------------------------ pair-list layouts
 
-// The packed K entry of row primitive r of b1 and partner primitive s of b2 (kKEntDoubles, see KEnt).
-void kent_record(const lsjk::Basis* b1, int r, const lsjk::Basis* b2, int s, double* g)
+// The packed K entry of row primitive r of b1 and partner primitive s of b2 (kKEntDoubles, see KEnt),
+// K = c c' exp(-e e' / p R^2) given.
+double kent_overlap(const lsjk::Basis* b1, int r, const lsjk::Basis* b2, int s)
 {
-    const double er = b1->h_e[r], es = b2->h_e[s], p = er + es, ip = 1.0 / p;
+    const double er = b1->h_e[r], es = b2->h_e[s], ip = 1.0 / (er + es);
     double R2 = 0.0;
     for (int d = 0; d < 3; d++) {
         const double dd = b1->h_xyz[3 * r + d] - b2->h_xyz[3 * s + d];
         R2 += dd * dd;
     }
+    return b1->h_c[r] * b2->h_c[s] * std::exp(-er * es * ip * R2);
+}
+
+void kent_record(const lsjk::Basis* b1, int r, const lsjk::Basis* b2, int s, double K, double* g)
+{
+    const double er = b1->h_e[r], es = b2->h_e[s], p = er + es, ip = 1.0 / p;
     g[0] = p;
     // K_AB sqrt(2 pi^(5/2)) / p: the product of the two sides' values times (p + q)^(-1/2) is the
     // quartet prefactor 2 pi^(5/2) K_AB K_CD / (p q sqrt(p + q))
-    g[1] = b1->h_c[r] * b2->h_c[s] * std::exp(-er * es * ip * R2) * lsjk::kKPrefRoot * ip;
+    g[1] = K * lsjk::kKPrefRoot * ip;
     for (int d = 0; d < 3; d++) {
         const double A = b1->h_xyz[3 * r + d], B = b2->h_xyz[3 * s + d];
         const double P = (er * A + es * B) * ip;
@@ -520,6 +536,7 @@ void build_pairlist(lsjk_pairlist* pl)
     }
     const int ne = (int)ents.size();
     pl->nent = ne;
+    pl->h_eK.resize(ne);
     std::vector<float> eb(ne);
     std::vector<int> eprim(ne), ecart(ne), eblk(ne), keblk(ne);
     // packed entries (kKEntDoubles per entry, see KEnt): p, K, P, P - A, A - B, {cart, blk}, 1/(2p),
@@ -536,7 +553,8 @@ void build_pairlist(lsjk_pairlist* pl)
         keblk[q] = b2->h_kblk[eblk[q]];
         const int ids[2] = {ecart[q], eblk[q]}, kids[2] = {b2->h_kcart[ecart[q]], keblk[q]};
         double* g = eg.data() + (size_t)kKEntDoubles * q;
-        kent_record(b1, r, b2, s, g);
+        pl->h_eK[q] = kent_overlap(b1, r, b2, s);
+        kent_record(b1, r, b2, s, pl->h_eK[q], g);
         // FP32-route copy: P in FP64, the rest rounded to FP32
         double* h = eg32.data() + (size_t)kKEnt32Doubles * q;
         h[0] = g[2];
@@ -894,66 +912,113 @@ const lsjk_pairlist::KGroupData& get_kgroups(lsjk_pairlist* pl, int L, int Lp, i
         for (int q = 0; q < pl->nmol; q++) G.mol_grp[q + 1] += G.mol_grp[q];
     }
     const int m = pl->kmaxL2 + 1;
-    std::vector<int2> slot;
-    std::vector<int> grp_rows((size_t)G.ngroup * gsize, -1);
-    G.grp_rank.assign((size_t)G.ngroup * gsize, std::numeric_limits<int>::max());
+    const lsjk::Basis *b1 = pl->b1, *b2 = pl->b2;
+    // where each group's slots lie: its rows' entries, padded to whole chunks
     G.grp_slot.assign(G.ngroup + 1, 0);
+    int most = 0;
     for (int g = 0; g < G.ngroup; g++) {
+        long long n = 0;
+        for (int i = gstart[g]; i < gstart[g + 1]; i++) {
+            const size_t r = (size_t)rows[G.order[i]] * m + Lp;
+            n += pl->h_row_start[r + 1] - pl->h_row_start[r];
+        }
+        n = (n + 63) / 64 * 64;
+        if (G.grp_slot[g] + n > std::numeric_limits<int>::max())
+            throw LsjkError(LSJK_E_UNSUPPORTED, "lsjk: too many exchange ket slots");
+        G.grp_slot[g + 1] = G.grp_slot[g] + (int)n;
+        most = std::max(most, (int)n);
+    }
+    const size_t ns = (size_t)G.grp_slot[G.ngroup];
+    G.slot.resize(ns);
+    G.chunk_b.resize(ns / 64);
+    G.grp_rows.assign((size_t)G.ngroup * gsize, -1);
+    G.grp_rank.assign((size_t)G.ngroup * gsize, std::numeric_limits<int>::max());
+    std::vector<int4> packed(ns);
+    std::unique_ptr<double[]> ent(new double[13 * ns]);  // the 13 fields of all slots (KGroups::ent)
+    struct Scratch {
         std::vector<int2> v;
-        for (int t = 0; t < gsize && gstart[g] + t < gstart[g + 1]; t++) {
+        std::vector<unsigned long long> order;
+    };
+    // one group's slots; nothing is allocated
+    auto fill = [&](int g, Scratch& w) {
+        const size_t q0 = (size_t)G.grp_slot[g], nq = (size_t)G.grp_slot[g + 1] - q0;
+        size_t n = 0;
+        for (int t = 0; gstart[g] + t < gstart[g + 1]; t++) {
             const int r = rows[G.order[gstart[g] + t]];
-            grp_rows[(size_t)g * gsize + t] = r;
+            G.grp_rows[(size_t)g * gsize + t] = r;
             G.grp_rank[(size_t)g * gsize + t] = mrank[r];
             for (int e = pl->h_row_start[(size_t)r * m + Lp]; e < pl->h_row_start[(size_t)r * m + Lp + 1]; e++)
-                v.push_back(make_int2(e, t));
+                w.v[n++] = make_int2(e, t);
         }
-        std::stable_sort(v.begin(), v.end(), [&](const int2& a, const int2& b) { return pl->h_eb[a.x] > pl->h_eb[b.x]; });
-        while (v.size() % 64) v.push_back(make_int2(-1, 0));
-        for (size_t c = 0; c < v.size(); c += 64) {
-            G.chunk_b.push_back(pl->h_eb[v[c].x]);
+        // descending bounds, ties in entry order: one integer each, the inverted bound (bounds are
+        // not negative) over the place
+        for (size_t i = 0; i < n; i++) {
+            unsigned int b;
+            std::memcpy(&b, &pl->h_eb[w.v[i].x], sizeof(b));
+            w.order[i] = ((unsigned long long)~b << 32) | i;
+        }
+        std::sort(w.order.begin(), w.order.begin() + n);
+        for (size_t c = 0; c < nq; c += 64) {
             // inside a chunk by the partner's K view column (padding last): neighbouring lanes then
             // gather D from the same cache lines
             unsigned long long key[64];
             int2 in[64];
             for (int t = 0; t < 64; t++) {
-                in[t] = v[c + t];
-                const unsigned int col = in[t].x < 0 ? 0xffffffffu
-                                                     : (unsigned int)pl->b2->h_kcart[pl->b2->h_cart[pl->h_eprim[in[t].x]]];
+                in[t] = c + t < n ? w.v[w.order[c + t] & 0xffffffffu] : make_int2(-1, 0);
+                const unsigned int col = in[t].x < 0 ? 0xffffffffu : (unsigned int)b2->h_kcart[b2->h_cart[pl->h_eprim[in[t].x]]];
                 key[t] = ((unsigned long long)col << 6) | (unsigned long long)t;
             }
+            G.chunk_b[(q0 + c) / 64] = pl->h_eb[in[0].x];
             std::sort(key, key + 64);
-            for (int t = 0; t < 64; t++) v[c + t] = in[key[t] & 63];
+            double f[13][64];
+            for (int t = 0; t < 64; t++) {
+                const int2 sl = in[key[t] & 63];
+                G.slot[q0 + c + t] = sl;
+                int4& pk = packed[q0 + c + t];
+                pk = make_int4(sl.x, sl.y, 0, 0);
+                if (sl.x < 0) {
+                    for (int k = 0; k < 13; k++) f[k][t] = 0.0;
+                    continue;
+                }
+                const int s = pl->h_eprim[sl.x];
+                std::memcpy(&pk.z, &pl->h_eb[sl.x], sizeof(float));
+                pk.w = b2->h_kblk[b2->h_blk[s]];
+                double rec[lsjk::kKEntDoubles];
+                kent_record(b1, G.grp_rows[(size_t)g * gsize + sl.y], b2, s, pl->h_eK[sl.x], rec);
+                for (int k = 0; k < 11; k++) f[k][t] = rec[k];
+                f[11][t] = rec[12];
+                const long long cart = b2->h_kcart[b2->h_cart[s]];
+                std::memcpy(&f[12][t], &cart, sizeof(cart));
+            }
+            for (int k = 0; k < 13; k++) std::memcpy(ent.get() + k * ns + q0 + c, f[k], sizeof(f[k]));
         }
-        slot.insert(slot.end(), v.begin(), v.end());
-        G.grp_slot[g + 1] = (int)slot.size();
+    };
+    // The groups over host threads, 8192 slots (about 1 ms) and more to each: a batch of 60 clusters has
+    // 750,000 slots, which took 140 of a first pass's 530 ms on one thread.
+    const int nthread = (int)std::min<size_t>({ns / 8192 + 1, 8, std::max(1u, std::thread::hardware_concurrency())});
+    std::vector<Scratch> scratch(nthread);
+    for (auto& w : scratch) {
+        w.v.resize(most);
+        w.order.resize(most);
     }
+    std::atomic<int> next{0};
+    auto work = [&](Scratch& w) {
+        for (int g; (g = next++) < G.ngroup;) fill(g, w);
+    };
     {
-        const lsjk::Basis *b1 = pl->b1, *b2 = pl->b2;
-        std::vector<int4> packed(slot.size());
-        std::vector<double> ent(13 * slot.size(), 0.0);
-        int g = 0;  // the slot's group
-        for (size_t q = 0; q < slot.size(); q++) {
-            while ((int)q >= G.grp_slot[g + 1]) g++;
-            const int e = slot[q].x;
-            packed[q] = make_int4(e, slot[q].y, 0, 0);
-            if (e < 0) continue;
-            const int s = pl->h_eprim[e];
-            std::memcpy(&packed[q].z, &pl->h_eb[e], sizeof(float));
-            packed[q].w = b2->h_kblk[b2->h_blk[s]];
-            double rec[lsjk::kKEntDoubles];
-            kent_record(b1, grp_rows[(size_t)g * gsize + slot[q].y], b2, s, rec);
-            for (int f = 0; f < 11; f++) ent[f * slot.size() + q] = rec[f];
-            ent[11 * slot.size() + q] = rec[12];
-            const long long cart = b2->h_kcart[b2->h_cart[s]];
-            std::memcpy(&ent[12 * slot.size() + q], &cart, sizeof(cart));
+        std::vector<std::thread> helpers;
+        helpers.reserve(nthread);
+        try {
+            for (int i = 1; i < nthread; i++) helpers.emplace_back(work, std::ref(scratch[i]));
+        } catch (const std::system_error&) {  // fewer of them, then
         }
-        G.d_ent = dev_upload(ent);
-        G.d_slot = dev_upload(packed);
+        work(scratch[0]);
+        for (auto& h : helpers) h.join();
     }
+    G.d_ent = dev_upload(ent.get(), 13 * ns);
+    G.d_slot = dev_upload(packed);
     G.d_grp_slot = dev_upload(G.grp_slot);
-    G.d_grp_rows = dev_upload(grp_rows);
-    G.slot = slot;
-    G.grp_rows = grp_rows;
+    G.d_grp_rows = dev_upload(G.grp_rows);
     G.d_grp_rank = dev_upload(G.grp_rank);
     G.d_chunk_b = dev_upload(G.chunk_b);
     return pl->kgroups.emplace(key, std::move(G)).first->second;
@@ -979,33 +1044,30 @@ constexpr int kKThrespCached = 4;
 // round-robin workgroup-to-XCD dispatch each XCD (one L2) works through neighbouring bra rows, in
 // tiles of rows x groups (below).  The tiles pay off with the K view copy of D (neighbouring
 // shells in neighbouring columns); in the basis order they measured no faster.
-std::pair<const lsjk::KUnitG*, int> get_kunits_g(const lsjk_pairlist* pl12c, const lsjk_pairlist* pl34c, int L1,
-                                                 int L2, int L3, int L4, bool tri, float thresp, double* cost_out)
+//
+// The key of a class's unit list in its bra list: rows per ket group (bits 40..47), thresp bits
+// (8..39), class and triangle flag.
+std::pair<unsigned long long, long long> kunits_key(const lsjk_pairlist* pl34, int L1, int L2, int L3, int L4, bool tri,
+                                                    float thresp)
 {
-    using lsjk::KUnitG;
-    lsjk_pairlist* pl12 = const_cast<lsjk_pairlist*>(pl12c);
-    lsjk_pairlist* pl34 = const_cast<lsjk_pairlist*>(pl34c);
-    const int gsize = kgroup_for(pl34, L3, L4);
     unsigned int tb;
     std::memcpy(&tb, &thresp, sizeof(tb));
-    // key: rows per ket group (bits 40..47), thresp bits (8..39), class and triangle flag
-    const long long cls = ((long long)gsize << 40) | ((long long)tb << 8) |
-                          (((((L1 * 3 + L2) * 3 + L3) * 3 + L4) << 1) | (tri ? 1 : 0));
-    const auto key = std::make_pair(pl34->uid, cls);
-    auto it = pl12->kunits_g.find(key);
-    if (it == pl12->kunits_g.end()) {
-        // the unit lists depend on thresp: keep those of at most kKThrespCached values per ket list
-        {
-            std::set<long long> seen;
-            for (const auto& kv : pl12->kunits_g)
-                if (kv.first.first == pl34->uid) seen.insert((kv.first.second >> 8) & 0xffffffffLL);
-            if (!seen.count((cls >> 8) & 0xffffffffLL) && (int)seen.size() >= kKThrespCached) {
-                auto same = [&](const std::pair<unsigned long long, long long>& k) { return k.first == pl34->uid; };
-                erase_if_key(pl12->kunits_g, same, true);
-                erase_if_key(pl12->kcost_g, same, false);
-                pl12->kunits_gen++;
-            }
-        }
+    return {pl34->uid, ((long long)kgroup_for(pl34, L3, L4) << 40) | ((long long)tb << 8) |
+                           (((((L1 * 3 + L2) * 3 + L3) * 3 + L4) << 1) | (tri ? 1 : 0))};
+}
+
+// The units with their costs, in spatial row order: all that a choice between two classes needs.
+struct KUnitPlan {
+    std::vector<std::pair<long long, lsjk::KUnitG>> v;
+    double total = 0.0;
+};
+
+KUnitPlan plan_kunits(lsjk_pairlist* pl12, lsjk_pairlist* pl34, int L1, int L2, int L3, int L4, bool tri, float thresp)
+{
+    using lsjk::KUnitG;
+    const int gsize = kgroup_for(pl34, L3, L4);
+    KUnitPlan plan;
+    {
         const auto& rows1 = pl12->h_rows[L1][L2];
         const auto& G34 = get_kgroups(pl34, L3, L4, gsize);
         const auto& G12 = get_kgroups(pl12, L1, L2, kgroup_for(pl12, L1, L2));  // its row order only
@@ -1018,8 +1080,8 @@ std::pair<const lsjk::KUnitG*, int> get_kunits_g(const lsjk_pairlist* pl12c, con
         const auto& mrank = get_mrank(pl12);
         const int m12 = pl12->kmaxL2 + 1;
         // chunk bounds per group, and the smallest rank of each group (triangle mode)
-        std::vector<std::pair<long long, KUnitG>> v;
-        double total = 0.0;
+        auto& v = plan.v;
+        double& total = plan.total;
         for (int i1 : G12.order) {
             const int r1 = rows1[i1];
             const int a0 = pl12->h_row_start[(size_t)r1 * m12 + L2], a1 = pl12->h_row_start[(size_t)r1 * m12 + L2 + 1];
@@ -1123,6 +1185,41 @@ std::pair<const lsjk::KUnitG*, int> get_kunits_g(const lsjk_pairlist* pl12c, con
             }
             v.swap(w);
         }
+    }
+    return plan;
+}
+
+// `ready`: the class's plan, where the caller has it.
+std::pair<const lsjk::KUnitG*, int> get_kunits_g(const lsjk_pairlist* pl12c, const lsjk_pairlist* pl34c, int L1,
+                                                 int L2, int L3, int L4, bool tri, float thresp, double* cost_out,
+                                                 KUnitPlan* ready = nullptr)
+{
+    using lsjk::KUnitG;
+    lsjk_pairlist* pl12 = const_cast<lsjk_pairlist*>(pl12c);
+    lsjk_pairlist* pl34 = const_cast<lsjk_pairlist*>(pl34c);
+    const auto key = kunits_key(pl34, L1, L2, L3, L4, tri, thresp);
+    auto it = pl12->kunits_g.find(key);
+    if (it == pl12->kunits_g.end()) {
+        // the unit lists depend on thresp: keep those of at most kKThrespCached values per ket list
+        {
+            std::set<long long> seen;
+            for (const auto& kv : pl12->kunits_g)
+                if (kv.first.first == pl34->uid) seen.insert((kv.first.second >> 8) & 0xffffffffLL);
+            if (!seen.count((key.second >> 8) & 0xffffffffLL) && (int)seen.size() >= kKThrespCached) {
+                auto same = [&](const std::pair<unsigned long long, long long>& k) { return k.first == pl34->uid; };
+                erase_if_key(pl12->kunits_g, same, true);
+                erase_if_key(pl12->kcost_g, same, false);
+                pl12->kunits_gen++;
+            }
+        }
+        KUnitPlan plan;
+        if (ready)
+            plan = std::move(*ready);
+        else
+            plan = plan_kunits(pl12, pl34, L1, L2, L3, L4, tri, thresp);
+        auto& v = plan.v;
+        const auto& rows1 = pl12->h_rows[L1][L2];
+        const auto& G12 = get_kgroups(pl12, L1, L2, kgroup_for(pl12, L1, L2));  // its row order only
         auto bucket = [](long long c) { return c > 0 ? 64 - __builtin_clzll((unsigned long long)c) : 0; };
         std::stable_sort(v.begin(), v.end(), [&](const std::pair<long long, KUnitG>& a,
                                                  const std::pair<long long, KUnitG>& b) {
@@ -1172,9 +1269,9 @@ std::pair<const lsjk::KUnitG*, int> get_kunits_g(const lsjk_pairlist* pl12c, con
             throw LsjkError(LSJK_E_UNSUPPORTED, "lsjk: too many exchange work units");
         KUnitG* d = u.empty() ? nullptr : dev_upload(u);
         it = pl12->kunits_g.insert({key, {(void*)d, (int)u.size()}}).first;
-        pl12->kcost_g[key] = total;
+        pl12->kcost_g[key] = {plan.total, (int)u.size()};
     }
-    if (cost_out) *cost_out = pl12->kcost_g[key];
+    if (cost_out) *cost_out = pl12->kcost_g[key].first;
     return {static_cast<const KUnitG*>(it->second.first), it->second.second};
 }
 
@@ -2171,16 +2268,34 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
                             for (int L4 = 0; L4 <= b4->maxL; L4++) {
                                 const int c = kcount_index(L1, L2, L3, L4), m = kcount_index(L3, L4, L1, L2);
                                 if (c >= m) continue;
-                                int nunits = 0;  // of the class asked for last
-                                auto steps = [&](int A, int B, int C, int D_) {
-                                    nunits = 0;
-                                    if (pl12->h_rows[A][B].empty() || pl34->h_rows[C][D_].empty()) return 0.0;
-                                    double cost = 0.0;
-                                    nunits = (int)get_kunits_g(pl12, pl34, A, B, C, D_, false, thresp, &cost).second;
-                                    return cost;
-                                };
-                                const double sm = steps(L3, L4, L1, L2), sc = steps(L1, L2, L3, L4);
-                                pick[c] = pick[m] = first_orientation(L1, L3, sc, sm, nunits) ? c : m;
+                                if (pl12->h_rows[L1][L2].empty() || pl12->h_rows[L3][L4].empty()) {
+                                    pick[c] = pick[m] = c;
+                                    continue;
+                                }
+                                // both planned, the one that runs ordered and uploaded; of the other the
+                                // steps and the count stay
+                                auto* pl = const_cast<lsjk_pairlist*>(pl12);
+                                KUnitPlan plan[2];
+                                std::pair<double, int> cost[2];
+                                bool planned[2] = {false, false};
+                                for (int q = 0; q < 2; q++) {
+                                    const int A = q ? L3 : L1, B = q ? L4 : L2, C = q ? L1 : L3, E = q ? L2 : L4;
+                                    const auto key = kunits_key(pl, A, B, C, E, false, thresp);
+                                    const auto known = pl->kcost_g.find(key);
+                                    if (known != pl->kcost_g.end()) {
+                                        cost[q] = known->second;
+                                        continue;
+                                    }
+                                    plan[q] = plan_kunits(pl, pl, A, B, C, E, false, thresp);
+                                    planned[q] = true;
+                                    cost[q] = {plan[q].total, (int)plan[q].v.size()};
+                                }
+                                const int q = first_orientation(L1, L3, cost[0].first, cost[1].first, cost[0].second) ? 0 : 1;
+                                pick[c] = pick[m] = q ? m : c;
+                                get_kunits_g(pl, pl, q ? L3 : L1, q ? L4 : L2, q ? L1 : L3, q ? L2 : L4, false, thresp, nullptr,
+                                             planned[q] ? &plan[q] : nullptr);
+                                pl->kcost_g[kunits_key(pl, q ? L1 : L3, q ? L2 : L4, q ? L3 : L1, q ? L4 : L2, false, thresp)] =
+                                    cost[1 - q];
                             }
                 orient = &(ocache[okey] = pick);
             }

@@ -149,6 +149,7 @@ struct PairList {
     } grad;
     // host copies of the entry bounds and partner primitives (K view order)
     std::vector<float> h_eb;
+    std::vector<double> h_eK;  // c c' exp(-e e' / p R^2) of each
     std::vector<int> h_eprim;
     // spatial (Morton) rank of each basis-1 primitive: the order of the ket groups, and the total
     // order of the triangle mode; built on first use
@@ -178,7 +179,8 @@ struct PairList {
     // cached K build unit lists (device pointer, count) keyed by (ket list uid, class and
     // triangle flag, thresp bits), and their estimated cost
     std::map<std::pair<unsigned long long, long long>, std::pair<void*, int>> kunits_g;
-    std::map<std::pair<unsigned long long, long long>, double> kcost_g;
+    // cost and number of a class's units, same key; kept also where the list itself is not formed
+    std::map<std::pair<unsigned long long, long long>, std::pair<double, int>> kcost_g;
     // symmetric-mode K: for each pair of mirror classes (L1 L2 | L3 L4) / (L3 L4 | L1 L2), the one
     // that evaluates both (with the transposed block), chosen by timing both at first use; keyed by
     // (ket list uid, thresp bits << 1 | mixed route), class counter index -> chosen class counter

@@ -279,6 +279,22 @@ def noalloc_scratch_limit(E):
     assert call(L.lsjk_coulomb_noalloc, larger, ket) != 0
 
 
+@case
+def first_pass_lists(E):
+    """The first exchange over a list makes its scratch, six arrays per ket class and one unit list per
+    launch, none for the mirror classes that do not run; the other route's first call makes no more."""
+    bas = E.basis(2)
+    pl = E.pairs(bas)
+    E.ls.IntBox.overlap(E.res, pl)  # the list's own arrays
+    D, K = E.ls.DeviceArray([bas.nao, bas.nao]), E.ls.DeviceArray([bas.nao, bas.nao])
+    for thredp, expected in ((THRE, None), (1.0e-6, 0), (THRE, 0)):
+        before = E.stub.stub_allocations(), E.launches("k_ket")
+        E.ls.IntBox.exchange_device(E.ew, pl, pl, D.ptr, True, THRE, thredp, K.ptr)
+        made, launched = E.stub.stub_allocations() - before[0], E.launches("k_ket") - before[1]
+        assert launched == 45  # 81 classes of s, p and d rows and partners, 36 of them mirrors
+        assert made == (1 + 6 * 9 + launched if expected is None else expected)
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
