@@ -3538,7 +3538,7 @@ int lsjk_exchange_grad(const lsjk_pairlist* pl, const double* D13_dev, const dou
         pa.nblk = b->nblk;
         pa.blk_cart = b->d_blk_cart;
         pa.blk_L = b->d_blk_L;
-        pa.flags = S.d_sc->queue;
+        pa.maxima = reinterpret_cast<unsigned long long*>(S.d_sc->queue);
         pa.sc = S.d_sc;
         launch_k_grad_prep(pa, st);
         // all class pairs (the lane's class x the walked one), heaviest first over the side streams
@@ -3575,11 +3575,16 @@ int lsjk_exchange_grad(const lsjk_pairlist* pl, const double* D13_dev, const dou
         };
         if (ew.n > 0) {
             pass(pa.S13, pa.S24);
-            // the antisymmetric parts contribute only where both densities have one
-            unsigned int anti[2] = {0, 0};
-            HIPCHK(hipMemcpyAsync(anti, pa.flags, sizeof(anti), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
-            if (anti[0] && anti[1]) pass(pa.A13, pa.A24);
+            // The antisymmetric parts contribute only where both densities have one.  Densities that are
+            // symmetric but for rounding (the transform to Cartesian functions sums a d-d block and
+            // its transpose in different orders) have parts of some 2^-50 of their largest element:
+            // up to 2^-43 of it in both, the contribution is below 2^-86 of the symmetric parts'.
+            double m[4];
+            dev_download(m, pa.maxima, sizeof(m));
+            if (m[1] > 0.0 && m[3] > 0.0) {
+                const bool finite = std::isfinite(m[0]) && std::isfinite(m[2]);
+                if (!finite || (m[1] / m[0]) * (m[3] / m[2]) > std::ldexp(1.0, -86)) pass(pa.A13, pa.A24);
+            }
             launch_k_grad_atoms(gp, gd.d_prim, b->d_atom, pl->npair, b->natom, G_dev, st);
         }
         HIPCHK(hipGetLastError());

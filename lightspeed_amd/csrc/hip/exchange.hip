@@ -187,27 +187,39 @@ void launch_k_blockmax(const double* D, int ldD, const int* bc2, const int* bL2,
 __global__ __launch_bounds__(256) void k_grad_prep(KGradPrepArgs a)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)a.nblk * a.nblk) return;
-    const int bi = (int)(t / a.nblk), bj = (int)(t - (long long)bi * a.nblk);
-    const int oi = a.blk_cart[bi], oj = a.blk_cart[bj], ni = ncart(a.blk_L[bi]), nj = ncart(a.blk_L[bj]);
-    double m = 0.0;
-    bool anti13 = false, anti24 = false;
-    for (int i = oi; i < oi + ni; i++)
-        for (int j = oj; j < oj + nj; j++) {
-            const size_t ij = (size_t)i * a.n + j, ji = (size_t)j * a.n + i;
-            const double u = a.D13[ij], v = a.D13[ji], x = a.D24[ij], y = a.D24[ji];
-            a.S13[ij] = 0.5 * (u + v);
-            a.A13[ij] = 0.5 * (u - v);
-            a.S24[ij] = 0.5 * (x + y);
-            a.A24[ij] = 0.5 * (x - y);
-            anti13 = anti13 || u != v;
-            anti24 = anti24 || x != y;
-            m = fmax(m, fmax(fabs(x), fabs(y)));
-        }
-    a.Dsh[t] = m;
-    if (anti13) atomicOr(a.flags, 1u);
-    if (anti24) atomicOr(a.flags + 1, 1u);
-    atomicMax(&a.sc->dmax_bits, (unsigned long long)__double_as_longlong(m));
+    double m = 0.0, m13 = 0.0, a13 = 0.0, a24 = 0.0;
+    if (t < (long long)a.nblk * a.nblk) {
+        const int bi = (int)(t / a.nblk), bj = (int)(t - (long long)bi * a.nblk);
+        const int oi = a.blk_cart[bi], oj = a.blk_cart[bj], ni = ncart(a.blk_L[bi]), nj = ncart(a.blk_L[bj]);
+        for (int i = oi; i < oi + ni; i++)
+            for (int j = oj; j < oj + nj; j++) {
+                const size_t ij = (size_t)i * a.n + j, ji = (size_t)j * a.n + i;
+                const double u = a.D13[ij], v = a.D13[ji], x = a.D24[ij], y = a.D24[ji];
+                a.S13[ij] = 0.5 * (u + v);
+                a.A13[ij] = 0.5 * (u - v);
+                a.S24[ij] = 0.5 * (x + y);
+                a.A24[ij] = 0.5 * (x - y);
+                m13 = fmax(m13, fmax(fabs(u), fabs(v)));
+                a13 = fmax(a13, fabs(a.A13[ij]));
+                a24 = fmax(a24, fabs(a.A24[ij]));
+                m = fmax(m, fmax(fabs(x), fabs(y)));
+            }
+        a.Dsh[t] = m;
+    }
+    // one atomic per wave and maximum: all waves share the addresses
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        m = fmax(m, __shfl_xor(m, o));
+        m13 = fmax(m13, __shfl_xor(m13, o));
+        a13 = fmax(a13, __shfl_xor(a13, o));
+        a24 = fmax(a24, __shfl_xor(a24, o));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        const double top[4] = {m13, a13, m, a24};
+#pragma unroll
+        for (int k = 0; k < 4; k++) atomicMax(a.maxima + k, (unsigned long long)__double_as_longlong(top[k]));
+        atomicMax(&a.sc->dmax_bits, (unsigned long long)__double_as_longlong(m));
+    }
 }
 
 void launch_k_grad_prep(const KGradPrepArgs& a, hipStream_t s)

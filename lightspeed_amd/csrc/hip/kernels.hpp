@@ -160,14 +160,14 @@ constexpr int grad_ncomp(int L1, int L2, int L3, int L4) { return ncart(L1) * nc
 constexpr bool grad_expanded(int L1, int L2, int L3, int L4) { return grad_ncomp(L1, L2, L3, L4) <= 81; }
 constexpr bool grad_unrolled(int L1, int L2, int L3, int L4) { return grad_ncomp(L1, L2, L3, L4) <= 324; }
 // Per block pair: the symmetric and antisymmetric parts of D13 and D24, the block maxima of D24
-// (the larger of the two triangles'), max|D24|, and flags[0], flags[1] = whether D13, D24 have an
-// antisymmetric part.
+// (the larger of the two triangles'), max|D24|, and maxima[0 .. 3] = max|D13|, max|A13|, max|D24|,
+// max|A24| (bits of doubles).
 struct KGradPrepArgs {
     const double *D13, *D24;
     int n, nblk;
     const int *blk_cart, *blk_L;
     double *S13, *S24, *A13, *A24, *Dsh;
-    unsigned int* flags;
+    unsigned long long* maxima;
     CallScalars* sc;
 };
 void launch_k_grad_prep(const KGradPrepArgs& a, hipStream_t s);
