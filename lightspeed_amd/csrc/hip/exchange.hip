@@ -141,18 +141,20 @@ void launch_k_kview(const KViewArgs& a, hipStream_t s)
     hipLaunchKernelGGL(k_kview, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
 }
 
-__global__ void fill_zero(unsigned int* p, size_t n)
+// n words and the ntail (at most 3) bytes behind them.
+__global__ void fill_zero(unsigned int* p, size_t n, int ntail)
 {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        p[i] = 0u;
+    const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (size_t i = i0; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0u;
+    if (i0 < (size_t)ntail) reinterpret_cast<unsigned char*>(p + n)[i0] = 0;
 }
 
 void launch_fill(void* p, size_t bytes, hipStream_t s)
 {
-    size_t n = bytes / 4;
-    if (n == 0) return;
-    int blocks = (int)std::min<size_t>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(fill_zero, dim3(blocks), dim3(256), 0, s, (unsigned int*)p, n);
+    if (bytes == 0) return;
+    const size_t n = bytes / 4;
+    int blocks = (int)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 4096));
+    hipLaunchKernelGGL(fill_zero, dim3(blocks), dim3(256), 0, s, (unsigned int*)p, n, (int)(bytes % 4));
 }
 
 // Plain copy, 16 bytes per lane per step (grid-stride); the tail below 16 bytes byte-wise.
