@@ -866,9 +866,6 @@ const std::vector<int>& get_mrank(lsjk_pairlist* pl)
     return pl->h_mrank;
 }
 
-// Ket groups of the (row L, partner Lp) class of a list (see KGroups): the class's rows in spatial
-// order, gsize per group, each group's partner entries merged by bound (descending, ties by
-// entry index) and padded to a multiple of 64 slots.
 // Rows per ket group of (row L, partner L) of a list: the autotuned value or kgroup_size.
 int kgroup_for(const lsjk_pairlist* pl, int L, int Lp)
 {
@@ -876,6 +873,9 @@ int kgroup_for(const lsjk_pairlist* pl, int L, int Lp)
     return it != pl->kgsize.end() ? it->second : lsjk::kgroup_size(L, Lp);
 }
 
+// Ket groups of the (row L, partner Lp) class of a list (see KGroups): the class's rows in spatial
+// order, gsize per group, each group's partner entries merged by bound (descending, ties by
+// entry index) and padded to a multiple of 64 slots.
 const lsjk_pairlist::KGroupData& get_kgroups(lsjk_pairlist* pl, int L, int Lp, int gsize)
 {
     const int key = (L * 8 + Lp) * 256 + gsize;
@@ -2395,8 +2395,8 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
 // 4), per K class the work-unit split target (how finely few-unit classes are cut: 3072 .. 49152
 // units).  Class launches are serialised on one stream and timed with HIP events (lsjk's per-launch
 // profiling), each candidate twice (the faster counts); the fastest candidate is kept per group
-// pair / class.  Group size, waves per workgroup and register budgets are compile-time template
-// parameters of the kernels and are not searched here.
+// pair / class.  The rows per ket group are searched together with the mirror-class orientations;
+// waves per workgroup and register budgets are compile-time and are not.
 namespace {
 constexpr float kJScales[] = {0.25f, 0.5f, 1.0f, 2.0f, 4.0f};
 constexpr long long kKSplits[] = {3072, 12288, 49152};

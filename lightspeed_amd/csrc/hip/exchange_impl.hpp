@@ -348,8 +348,8 @@ __device__ __forceinline__ KEnt<float> load_ent32_uniform(const double* __restri
 
 // LDS of one k_ket workgroup: the staged table blocks first, FP64 (routes with FP64 quartets,
 // nrys <= 3) then FP32 (routes with FP32 quartets, nrys <= 5), then kKWaves group accumulators
-// (gsize x N1 x N3 doubles each, gsize = rows per ket group) and kKWaves slot queues.  The FP64 table at address 0 keeps a bin's coefficient offsets
-// (0..8 nrys * 24 bytes) inside the immediate offset field of the paired LDS reads, so the table
+// (gsize x N1 x N3 doubles each, gsize = rows per ket group) and kKWaves slot queues.  The FP64 table at
+// address 0 keeps a bin's coefficient offsets (0..8 nrys * 24 bytes) inside the immediate offset field of the paired LDS reads, so the table
 // lookup needs one address per bin.
 template <int L1, int L2, int L3, int L4, int ROUTE>
 struct KKetLds {
@@ -397,8 +397,8 @@ __device__ __forceinline__ KEnt<float> ent_to_f32(const KEnt<double>& e)
 // Waves per SIMD the compiler is asked to keep room for (register budget 512 / waves): FP64 classes
 // with an operator-term loop whose register count sits just above an occupancy step are held below it
 // where that costs at most a few spilled dwords and measured faster (classes that already spill, or
-// spill more, ran 15-55 % slower when held).  The bare 1/r kernels need no hold ((ss|ss) 44 registers,
-// (ss|sp) 77).  1 = no constraint.
+// spill more, ran 15-55 % slower when held).  The bare 1/r kernels need no hold ((ss|ss) 48 registers,
+// (ss|sp) 78; steps at 64 and 80).  1 = no constraint.
 constexpr int kket_class(int L1, int L2, int L3, int L4) { return ((L1 * 3 + L2) * 3 + L3) * 3 + L4; }
 constexpr int kket_waves(int L1, int L2, int L3, int L4, int route, bool bare)
 {

@@ -182,8 +182,9 @@ struct PairList {
     // cost and number of a class's units, same key; kept also where the list itself is not formed
     std::map<std::pair<unsigned long long, long long>, std::pair<double, int>> kcost_g;
     // symmetric-mode K: for each pair of mirror classes (L1 L2 | L3 L4) / (L3 L4 | L1 L2), the one
-    // that evaluates both (with the transposed block), chosen by timing both at first use; keyed by
-    // (ket list uid, thresp bits << 1 | mixed route), class counter index -> chosen class counter
+    // that evaluates both (with the transposed block), by estimated wave steps or the autotuner's
+    // timing; keyed by (ket list uid, thresp bits << 2 | learned route << 1 | mixed route), class
+    // counter index -> chosen class counter
     // index.  Every class pair with work has an entry once the map is stored.
     std::map<std::pair<unsigned long long, unsigned long long>, std::map<int, int>> korient;
 };

@@ -324,7 +324,6 @@ void launch_j_quartets_sym(int L12, int L34, int route, const JQuartetArgs& a, c
 void launch_j_quartets(int L12, int L34, int route, const JQuartetArgs& a, const JTask* tasks, int ntask,
                        unsigned int* qctr, hipStream_t s);
 
-
 // Work-queue counters of one call (CallScalars::queue, zeroed with the call's scalars): J classes
 // at jcount_index.
 
@@ -333,11 +332,9 @@ void launch_j_quartets(int L12, int L34, int route, const JQuartetArgs& a, const
 // the device's per-workgroup limit.
 int persistent_grid(const void* kernel, int block, size_t lds, long long nwork_groups);
 
-// blk_lo / blk_hi (nullptr: dense): per block 2, the range of blocks 4 of its molecule (batch
-// basis); band = the largest such range.
 // Dynamic LDS of one k_ket workgroup (as KKetLds lays it out): the staged Rys table blocks (FP64
-// for routes with FP64 quartets and nrys <= 3, FP32 for routes with FP32 quartets and nrys <= 5),
-// 8-byte aligned, then kKWaves accumulators of gsize x N1 x N3 doubles.
+// for nrys <= 3, FP32 on the mixed route for nrys <= 5), 8-byte aligned, then kKWaves accumulators
+// of gsize x N1 x N3 doubles and kKWaves slot queues.
 inline size_t kket_lds_bytes(const RysTable& tab, int L1, int L2, int L3, int L4, int route, int gsize)
 {
     const int NR = (L1 + L2 + L3 + L4) / 2 + 1;
@@ -366,6 +363,8 @@ struct KViewArgs {
     CallScalars* sc;
 };
 void launch_k_kview(const KViewArgs& a, hipStream_t s);
+// blk_lo / blk_hi (nullptr: dense): per block 2, the range of blocks 4 of its molecule (batch
+// basis); band = the largest such range.
 void launch_k_blockmax(const double* D, int ldD, const int* blk_cart2, const int* blk_L2, int nblk2,
                        const int* blk_cart4, const int* blk_L4, int nblk4, double* Dsh, int ldDsh, const int* blk_lo,
                        const int* blk_hi, int band, CallScalars* sc, hipStream_t s);
@@ -373,7 +372,7 @@ void launch_k_blockmax(const double* D, int ldD, const int* blk_cart2, const int
 // b12 b34 >= smin (classes with s and p functions only).
 void launch_k_unit_mag_sp(int L1, int L2, int L3, int L4, const KArgs& a, const KGroups& kg, const KUnitG* units,
                           int nunits, float smin, float* out, hipStream_t s);
-// K build classes (routes plain, FP64 part, FP32 part) over ket-group units.
+// K build classes (kRoutePlain or kRouteMixed) over ket-group units.
 void launch_k_ket(int L1, int L2, int L3, int L4, int route, const KArgs& a, const KGroups& g, const KUnitG* units,
                   int nunits, hipStream_t s);
 void launch_fill(void* p, size_t bytes, hipStream_t s);
