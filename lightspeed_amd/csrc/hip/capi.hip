@@ -3610,12 +3610,11 @@ static void one_e_st(const lsjk_pairlist* pl, double* Sout, double* Tout)
     a.S = Sout;
     a.T = Tout;
     a.ld = b2->ncart;
-    Fanout fo;
-    fo.begin();
+    // In a row: a class takes 5-15 us, the fork and join of the side streams 55 (overlap of H2O/STO-3G
+    // 125 us with them, 48 without; no faster with them up to (H2O)90/cc-pVDZ, 151,000 pairs).
     for (size_t c = 0; c + 1 < pl->cls_start.size(); c++)
         launch_one_e_st(pl->cls_L1[c], pl->cls_L2[c], a, pl->cls_start[c], pl->cls_start[c + 1] - pl->cls_start[c],
-                        fo.pick());
-    fo.end();
+                        S.stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(S.stream));
 }
@@ -3670,18 +3669,25 @@ int lsjk_potential(const lsjk_pairlist* pl, int nterm, const double* scales, con
         a.nA = ncharge;
         a.vp = vp;
         // the charges are cut so that the classes together give about 32 waves per compute unit, with at
-        // least 4 charges a wave; the classes run side by side
+        // least 4 charges a wave
         const long long waves = ((long long)pl->npair + 63) / 64 + (long long)pl->cls_L1.size();
         const int nsplit = (int)std::max<long long>(1, std::min<long long>((ncharge + 3) / 4, 32ll * S.num_cu / waves));
         if (nsplit > 1) launch_fill(vp, pl->hoff[2 * kMaxL + 1] * sizeof(double), st);
+        // The classes side by side where that gives more than the fork and join cost (55 us).  A class's
+        // time goes with its longest chain, the charges of a wave and then nsplit additions to one
+        // address: classes x chain is 27 ((H2O)1/6-31G**, its 3 charges, 152 us side by side and 82
+        // in a row), 117 ((H2O)12, 184 and 154; (H2O)12/cc-pVDZ, 436 both), 181 ((H2O)24/cc-pVDZ, 1554
+        // and 1602), 218 ((H2O)48/6-31G**, 1004 and 1085), 2300 ((H2O)1 with 1000 charges, 286 and 362).
+        const long long chain = (ncharge + nsplit - 1) / nsplit + (nsplit > 1 ? nsplit : 0);
+        const bool side = chain * (long long)pl->cls_L1.size() >= 150;
         Fanout fo;
-        fo.begin();
+        if (side) fo.begin();
         for (size_t c = 0; c + 1 < pl->cls_start.size(); c++) {
             const int L = pl->cls_L1[c] + pl->cls_L2[c];
             launch_one_e_v(pl->cls_L1[c], pl->cls_L2[c], a, pl->cls_start[c], pl->cls_start[c + 1] - pl->cls_start[c],
-                           nsplit, pl->hstart[L], pl->hoff[L], fo.pick());
+                           nsplit, pl->hstart[L], pl->hoff[L], side ? fo.pick() : st);
         }
-        fo.end();
+        if (side) fo.end();
         JScatterArgs sa{};
         sa.p1 = pl->d_p1;
         sa.p2 = pl->d_p2;

@@ -25,7 +25,7 @@ size_t failing = 0;
 long bad_frees = 0, null_stream_copies = 0;
 bool capturing = false;  // copies from pageable memory and waits are errors then
 size_t uploaded = 0;
-long allocations = 0;
+long allocations = 0, event_waits = 0;
 int last_error = kSuccess;
 std::string answer;  // what the next copy to the host of this size gives
 struct Call {
@@ -130,7 +130,7 @@ int hipMemcpyAsync(void* dst, const void* src, size_t n, int kind, void* stream)
 int hipStreamCreateWithFlags(void** s, unsigned) { return handle(s); }
 int hipStreamDestroy(void*) { return kSuccess; }
 int hipStreamSynchronize(void*) { return set(capturing ? kCapture : kSuccess); }
-int hipStreamWaitEvent(void*, void*, unsigned) { return kSuccess; }
+int hipStreamWaitEvent(void*, void*, unsigned) { return event_waits++, kSuccess; }
 int hipStreamBeginCapture(void*, int) { return capturing = true, kSuccess; }
 int hipStreamEndCapture(void*, void** g) { return capturing = false, handle(g); }
 int hipGraphInstantiate(void** e, void*, void*, char*, size_t) { return handle(e); }
@@ -158,6 +158,7 @@ size_t stub_live_bytes(void)
 }
 long stub_live_blocks(void) { return static_cast<long>(live.size()); }
 long stub_allocations(void) { return allocations; }
+long stub_event_waits(void) { return event_waits; }
 // the launches from number `first` on, a line each
 const char* stub_launch_log(long first)
 {

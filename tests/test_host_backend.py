@@ -30,7 +30,8 @@ class Env:
         self.stub = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)  # before liblsjk.so
         for f in ("stub_uploaded", "stub_live_bytes"):
             getattr(self.stub, f).restype = ctypes.c_size_t
-        for f in ("stub_bad_frees", "stub_null_stream_copies", "stub_live_blocks", "stub_launches", "stub_allocations"):
+        for f in ("stub_bad_frees", "stub_null_stream_copies", "stub_live_blocks", "stub_launches", "stub_allocations",
+                  "stub_event_waits"):
             getattr(self.stub, f).restype = ctypes.c_long
         self.stub.stub_launch_log.restype = ctypes.c_char_p
         self.stub.stub_launch_log.argtypes = [ctypes.c_long]
@@ -293,6 +294,25 @@ def first_pass_lists(E):
         made, launched = E.stub.stub_allocations() - before[0], E.launches("k_ket") - before[1]
         assert launched == 45  # 81 classes of s, p and d rows and partners, 36 of them mirrors
         assert made == (1 + 6 * 9 + launched if expected is None else expected)
+
+
+@case
+def one_electron_streams(E):
+    """Overlap, kinetic energy and the potential of few charges launch their classes in a row: fork and
+    join of the side streams cost more than small classes gain by running side by side."""
+    I = E.ls.IntBox
+    pl = E.pairs(E.basis(3))
+
+    def waits(f):
+        f()
+        before = E.stub.stub_event_waits()
+        f()
+        return E.stub.stub_event_waits() - before
+
+    V = lambda n: waits(lambda: I.potential(E.res, E.ew, pl, E.tensor(n, 4)))  # noqa: E731
+    assert waits(lambda: I.overlap(E.res, pl)) == waits(lambda: I.kinetic(E.res, pl)) == 0
+    assert V(1) == V(9) == 0
+    assert V(100000) > 0
 
 
 @pytest.fixture(scope="module")
