@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <limits>
 #include <map>
 #include <memory>
@@ -386,6 +387,44 @@ void check_ewald(int nterm, const double* scales, const double* omegas, lsjk::Ew
         ew.n++;
     }
     ew.plain = ew.n == 1 && ew.omega[0] == -1.0;
+}
+
+// ------------------------------------------------------------------ host threads
+
+// Host threads for `items` pieces of work, at least `each` of them to a thread.
+int host_threads(size_t items, size_t each)
+{
+    return (int)std::min<size_t>({items / each + 1, 8, std::max(1u, std::thread::hardware_concurrency())});
+}
+
+// f(i, t) for i = 0 .. n - 1 in any order, over nthread threads of which this is number t = 0 (fewer
+// where they cannot be had).  The first exception ends the rest and is thrown on.
+template <typename F>
+void host_parallel(int n, int nthread, F&& f)
+{
+    std::atomic<int> next{0};
+    std::exception_ptr failed;
+    std::mutex mu;
+    auto work = [&](int t) {
+        for (int i; (i = next++) < n;) {
+            try {
+                f(i, t);
+            } catch (...) {
+                std::lock_guard<std::mutex> lk(mu);
+                if (!failed) failed = std::current_exception();
+                next = n;
+            }
+        }
+    };
+    std::vector<std::thread> helpers;
+    helpers.reserve(nthread);
+    try {
+        for (int t = 1; t < std::min(n, nthread); t++) helpers.emplace_back(work, t);
+    } catch (const std::system_error&) {
+    }
+    work(0);
+    for (auto& h : helpers) h.join();
+    if (failed) std::rethrow_exception(failed);
 }
 
 // ------------------------------------------------------------------ pair-list layouts
@@ -995,26 +1034,13 @@ const lsjk_pairlist::KGroupData& get_kgroups(lsjk_pairlist* pl, int L, int Lp, i
     };
     // The groups over host threads, 8192 slots (about 1 ms) and more to each: a batch of 60 clusters has
     // 750,000 slots, which took 140 of a first pass's 530 ms on one thread.
-    const int nthread = (int)std::min<size_t>({ns / 8192 + 1, 8, std::max(1u, std::thread::hardware_concurrency())});
+    const int nthread = host_threads(ns, 8192);
     std::vector<Scratch> scratch(nthread);
     for (auto& w : scratch) {
         w.v.resize(most);
         w.order.resize(most);
     }
-    std::atomic<int> next{0};
-    auto work = [&](Scratch& w) {
-        for (int g; (g = next++) < G.ngroup;) fill(g, w);
-    };
-    {
-        std::vector<std::thread> helpers;
-        helpers.reserve(nthread);
-        try {
-            for (int i = 1; i < nthread; i++) helpers.emplace_back(work, std::ref(scratch[i]));
-        } catch (const std::system_error&) {  // fewer of them, then
-        }
-        work(scratch[0]);
-        for (auto& h : helpers) h.join();
-    }
+    host_parallel(G.ngroup, nthread, [&](int g, int t) { fill(g, scratch[t]); });
     G.d_ent = dev_upload(ent.get(), 13 * ns);
     G.d_slot = dev_upload(packed);
     G.d_grp_slot = dev_upload(G.grp_slot);
@@ -1045,26 +1071,34 @@ constexpr int kKThrespCached = 4;
 // tiles of rows x groups (below).  The tiles pay off with the K view copy of D (neighbouring
 // shells in neighbouring columns); in the basis order they measured no faster.
 //
+// A class's units are planned, ordered and uploaded in turn (plan_kunits, order_kunits, make_kunits).
+struct KClass {
+    int L1, L2, L3, L4;
+    bool tri;
+};
+
 // The key of a class's unit list in its bra list: rows per ket group (bits 40..47), thresp bits
 // (8..39), class and triangle flag.
-std::pair<unsigned long long, long long> kunits_key(const lsjk_pairlist* pl34, int L1, int L2, int L3, int L4, bool tri,
-                                                    float thresp)
+std::pair<unsigned long long, long long> kunits_key(const lsjk_pairlist* pl34, const KClass& k, float thresp)
 {
     unsigned int tb;
     std::memcpy(&tb, &thresp, sizeof(tb));
-    return {pl34->uid, ((long long)kgroup_for(pl34, L3, L4) << 40) | ((long long)tb << 8) |
-                           (((((L1 * 3 + L2) * 3 + L3) * 3 + L4) << 1) | (tri ? 1 : 0))};
+    return {pl34->uid, ((long long)kgroup_for(pl34, k.L3, k.L4) << 40) | ((long long)tb << 8) |
+                           (((((k.L1 * 3 + k.L2) * 3 + k.L3) * 3 + k.L4) << 1) | (k.tri ? 1 : 0))};
 }
 
 // The units with their costs, in spatial row order: all that a choice between two classes needs.
+// Reads the lists and their ket groups only (plans of several classes are made at once).
 struct KUnitPlan {
     std::vector<std::pair<long long, lsjk::KUnitG>> v;
     double total = 0.0;
 };
 
-KUnitPlan plan_kunits(lsjk_pairlist* pl12, lsjk_pairlist* pl34, int L1, int L2, int L3, int L4, bool tri, float thresp)
+KUnitPlan plan_kunits(lsjk_pairlist* pl12, lsjk_pairlist* pl34, const KClass& k, float thresp)
 {
     using lsjk::KUnitG;
+    const int L1 = k.L1, L2 = k.L2, L3 = k.L3, L4 = k.L4;
+    const bool tri = k.tri;
     const int gsize = kgroup_for(pl34, L3, L4);
     KUnitPlan plan;
     {
@@ -1189,37 +1223,15 @@ KUnitPlan plan_kunits(lsjk_pairlist* pl12, lsjk_pairlist* pl34, int L1, int L2, 
     return plan;
 }
 
-// `ready`: the class's plan, where the caller has it.
-std::pair<const lsjk::KUnitG*, int> get_kunits_g(const lsjk_pairlist* pl12c, const lsjk_pairlist* pl34c, int L1,
-                                                 int L2, int L3, int L4, bool tri, float thresp, double* cost_out,
-                                                 KUnitPlan* ready = nullptr)
+// The units of a plan in dispatch order.
+std::vector<lsjk::KUnitG> order_kunits(lsjk_pairlist* pl12, const KClass& k, KUnitPlan& plan)
 {
     using lsjk::KUnitG;
-    lsjk_pairlist* pl12 = const_cast<lsjk_pairlist*>(pl12c);
-    lsjk_pairlist* pl34 = const_cast<lsjk_pairlist*>(pl34c);
-    const auto key = kunits_key(pl34, L1, L2, L3, L4, tri, thresp);
-    auto it = pl12->kunits_g.find(key);
-    if (it == pl12->kunits_g.end()) {
-        // the unit lists depend on thresp: keep those of at most kKThrespCached values per ket list
-        {
-            std::set<long long> seen;
-            for (const auto& kv : pl12->kunits_g)
-                if (kv.first.first == pl34->uid) seen.insert((kv.first.second >> 8) & 0xffffffffLL);
-            if (!seen.count((key.second >> 8) & 0xffffffffLL) && (int)seen.size() >= kKThrespCached) {
-                auto same = [&](const std::pair<unsigned long long, long long>& k) { return k.first == pl34->uid; };
-                erase_if_key(pl12->kunits_g, same, true);
-                erase_if_key(pl12->kcost_g, same, false);
-                pl12->kunits_gen++;
-            }
-        }
-        KUnitPlan plan;
-        if (ready)
-            plan = std::move(*ready);
-        else
-            plan = plan_kunits(pl12, pl34, L1, L2, L3, L4, tri, thresp);
+    std::vector<KUnitG> u;
+    {
         auto& v = plan.v;
-        const auto& rows1 = pl12->h_rows[L1][L2];
-        const auto& G12 = get_kgroups(pl12, L1, L2, kgroup_for(pl12, L1, L2));  // its row order only
+        const auto& rows1 = pl12->h_rows[k.L1][k.L2];
+        const auto& G12 = get_kgroups(pl12, k.L1, k.L2, kgroup_for(pl12, k.L1, k.L2));  // its row order only
         auto bucket = [](long long c) { return c > 0 ? 64 - __builtin_clzll((unsigned long long)c) : 0; };
         std::stable_sort(v.begin(), v.end(), [&](const std::pair<long long, KUnitG>& a,
                                                  const std::pair<long long, KUnitG>& b) {
@@ -1236,7 +1248,6 @@ std::pair<const lsjk::KUnitG*, int> get_kunits_g(const lsjk_pairlist* pl12c, con
         constexpr size_t W = lsjk::kKWaves;
         std::vector<int> pos1(rows1.size(), 0);  // spatial position of each bra row
         for (size_t q = 0; q < G12.order.size(); q++) pos1[G12.order[q]] = (int)q;
-        std::vector<KUnitG> u;
         u.reserve(v.size());
         for (size_t s0 = 0; s0 < v.size();) {
             size_t s1 = s0;
@@ -1267,12 +1278,144 @@ std::pair<const lsjk::KUnitG*, int> get_kunits_g(const lsjk_pairlist* pl12c, con
         }
         if (u.size() > (size_t)std::numeric_limits<int>::max() / lsjk::kKWaves)
             throw LsjkError(LSJK_E_UNSUPPORTED, "lsjk: too many exchange work units");
-        KUnitG* d = u.empty() ? nullptr : dev_upload(u);
-        it = pl12->kunits_g.insert({key, {(void*)d, (int)u.size()}}).first;
-        pl12->kcost_g[key] = {plan.total, (int)u.size()};
+    }
+    return u;
+}
+
+// Which of two mirror classes runs, the first (L1 L2 | L3 L4) with L1 < L3, or L1 = L3 and L2 < L4
+// (steps_c wave steps over nunits units), or its mirror (steps_m)?  By the wave steps, weighed by what a
+// step costs in either orientation; all pairs timed in both at (H2O)64/6-31G**, (H2O)128/6-31G* and
+// (H2O)30/cc-pVDZ (decaying densities) and C19H40/cc-pVDZ:
+//  * L1 < L3: the mirror's ket has the lower row, whose transfer from C is shorter or absent (L3 = 0)
+//    and whose lists fill the lanes better.  At equal steps (ss|ds) 1.27, 1.64, 0.58, 0.68 ms against
+//    (ds|ss) 0.55, 0.81, 0.21, 0.64; (ss|ps) 1.69, 1.62, 1.39, 1.94 against 1.64, 1.43, 0.80, 1.58;
+//    (sd|pp) with 1.02-1.14 of its steps 0.54, 0.50, 0.16, 0.33 against 0.48, 0.38, 0.15, 0.32.  The
+//    mirror is kept up to 1.25 times the steps; beyond, (ps|ds) and (pd|ds) kinds are faster as they are.
+//  * L1 = L3 = 0: the first class's ket (s L4) recurs at D and comes in groups of 64 rows, worth about a
+//    quarter of the steps ((ss|sd) 0.61 and 0.97 ms with 1.22 of the steps of (sd|ss), 1.01 and 1.64) if
+//    its fewer, longer units still fill the device's 24 waves per CU three times; with fewer, the last
+//    ones run alone ((ss|sp) 1.47 against 0.82 ms at 16500 units of equal steps, 1.98 against 1.71 at
+//    13000, but 1.98 against 2.25 at 20700 and 1.84 against 2.27 at 83000).
+bool first_orientation(int L1, int L3, double steps_c, double steps_m, int nunits)
+{
+    if (L1 < L3) return 1.25 * steps_c < steps_m;
+    if (L1 == 0) return nunits >= 3 * 24 * S.num_cu ? steps_c <= 1.25 * steps_m : 1.05 * steps_c < steps_m;
+    return steps_c <= steps_m;
+}
+
+// The unit list of one class, or of the one of two mirror classes that first_orientation picks (cls[0]
+// the class of the lower index); `chosen` is filled.
+struct KUnitJob {
+    KClass cls[2];
+    int n = 1, chosen = 0;
+    std::pair<double, int> cost[2];
+    std::vector<lsjk::KUnitG> u;
+    bool made = false;
+};
+
+// Units of jobs worked on at a time (52 bytes each on the host).
+constexpr double kKUnitsAtOnce = 8.0e6;
+
+// Makes the unit lists that are missing, the jobs over host threads: planning and ordering them on one
+// thread was about 80 % of the host's time for a first pass over a list ((H2O)64/6-31G**: 360 ms of
+// host time, 100 over eight threads).  The upload and everything that changes the lists stays on
+// this thread.
+void make_kunits(lsjk_pairlist* pl12, lsjk_pairlist* pl34, std::vector<KUnitJob>& jobs, float thresp)
+{
+    if (jobs.empty()) return;
+    // the unit lists depend on thresp: keep those of at most kKThrespCached values per ket list
+    {
+        const long long cls = kunits_key(pl34, jobs[0].cls[0], thresp).second;
+        std::set<long long> seen;
+        for (const auto& kv : pl12->kunits_g)
+            if (kv.first.first == pl34->uid) seen.insert((kv.first.second >> 8) & 0xffffffffLL);
+        if (!seen.count((cls >> 8) & 0xffffffffLL) && (int)seen.size() >= kKThrespCached) {
+            auto same = [&](const std::pair<unsigned long long, long long>& k) { return k.first == pl34->uid; };
+            erase_if_key(pl12->kunits_g, same, true);
+            erase_if_key(pl12->kcost_g, same, false);
+            pl12->kunits_gen++;
+        }
+    }
+    // the groups of all classes, which the threads then only read; each job's size
+    get_mrank(pl12);
+    std::vector<std::pair<double, int>> order;  // (bra row, ket chunk) steps, job
+    std::vector<double> units(jobs.size(), 0.0);
+    double steps = 0.0;
+    for (size_t i = 0; i < jobs.size(); i++) {
+        double n = 0.0;
+        for (int q = 0; q < jobs[i].n; q++) {
+            const KClass& k = jobs[i].cls[q];
+            const auto& G34 = get_kgroups(pl34, k.L3, k.L4, kgroup_for(pl34, k.L3, k.L4));
+            get_kgroups(pl12, k.L1, k.L2, kgroup_for(pl12, k.L1, k.L2));
+            const double rows = (double)pl12->h_rows[k.L1][k.L2].size() / std::max(1, pl34->nmol);
+            n += rows * (double)(G34.slot.size() / 64);
+            units[i] += rows * (double)G34.ngroup + (double)kKUnitsTargetDefault;
+        }
+        order.push_back({n, (int)i});
+        steps += n;
+    }
+    std::sort(order.begin(), order.end(), [](const auto& a, const auto& b) {  // the longest first
+        return a.first != b.first ? a.first > b.first : a.second < b.second;
+    });
+    const int nthread = host_threads((size_t)steps, 20000);
+    for (size_t i0 = 0; i0 < order.size();) {
+        size_t i1 = i0;
+        for (double n = 0.0; i1 < order.size() && (i1 == i0 || n + units[order[i1].second] <= kKUnitsAtOnce); i1++)
+            n += units[order[i1].second];
+        host_parallel((int)(i1 - i0), nthread, [&](int i, int) {
+            KUnitJob& job = jobs[order[i0 + i].second];
+            KUnitPlan plan[2];
+            bool planned[2] = {false, false};
+            auto make_plan = [&](int q) {
+                plan[q] = plan_kunits(pl12, pl34, job.cls[q], thresp);
+                job.cost[q] = {plan[q].total, (int)plan[q].v.size()};
+                planned[q] = true;
+            };
+            for (int q = 0; q < job.n; q++) {
+                const auto known = pl12->kcost_g.find(kunits_key(pl34, job.cls[q], thresp));
+                if (known != pl12->kcost_g.end())
+                    job.cost[q] = known->second;
+                else
+                    make_plan(q);
+            }
+            if (job.n == 2)
+                job.chosen = first_orientation(job.cls[0].L1, job.cls[0].L3, job.cost[0].first, job.cost[1].first,
+                                               job.cost[0].second) ? 0 : 1;
+            const KClass& k = job.cls[job.chosen];
+            if (pl12->kunits_g.count(kunits_key(pl34, k, thresp))) return;
+            if (!planned[job.chosen]) make_plan(job.chosen);
+            job.u = order_kunits(pl12, k, plan[job.chosen]);
+            job.made = true;
+        });
+        for (size_t i = i0; i < i1; i++) {
+            KUnitJob& job = jobs[order[i].second];
+            if (job.made) {
+                const auto key = kunits_key(pl34, job.cls[job.chosen], thresp);
+                void* d = job.u.empty() ? nullptr : dev_upload(job.u);
+                pl12->kunits_g.insert({key, {d, (int)job.u.size()}});
+            }
+            for (int q = 0; q < job.n; q++) pl12->kcost_g[kunits_key(pl34, job.cls[q], thresp)] = job.cost[q];
+            job.u = {};
+        }
+        i0 = i1;
+    }
+}
+
+std::pair<const lsjk::KUnitG*, int> get_kunits_g(const lsjk_pairlist* pl12c, const lsjk_pairlist* pl34c, int L1,
+                                                 int L2, int L3, int L4, bool tri, float thresp, double* cost_out)
+{
+    lsjk_pairlist* pl12 = const_cast<lsjk_pairlist*>(pl12c);
+    lsjk_pairlist* pl34 = const_cast<lsjk_pairlist*>(pl34c);
+    const KClass k{L1, L2, L3, L4, tri};
+    const auto key = kunits_key(pl34, k, thresp);
+    if (!pl12->kunits_g.count(key)) {
+        std::vector<KUnitJob> one(1);
+        one[0].cls[0] = k;
+        make_kunits(pl12, pl34, one, thresp);
     }
     if (cost_out) *cost_out = pl12->kcost_g[key].first;
-    return {static_cast<const KUnitG*>(it->second.first), it->second.second};
+    const auto& u = pl12->kunits_g[key];
+    return {static_cast<const lsjk::KUnitG*>(u.first), u.second};
 }
 
 lsjk::KGroups kgroups_args(const lsjk_pairlist::KGroupData& G)
@@ -2050,27 +2193,6 @@ lsjk_basis* basis_new(int nprim, const double* c, const double* e, const double*
 
 }  // namespace
 
-// Which of two mirror classes runs, the first (L1 L2 | L3 L4) with L1 < L3, or L1 = L3 and L2 < L4
-// (steps_c wave steps over nunits units), or its mirror (steps_m)?  By the wave steps, weighed by what a
-// step costs in either orientation; all pairs timed in both at (H2O)64/6-31G**, (H2O)128/6-31G* and
-// (H2O)30/cc-pVDZ (decaying densities) and C19H40/cc-pVDZ:
-//  * L1 < L3: the mirror's ket has the lower row, whose transfer from C is shorter or absent (L3 = 0)
-//    and whose lists fill the lanes better.  At equal steps (ss|ds) 1.27, 1.64, 0.58, 0.68 ms against
-//    (ds|ss) 0.55, 0.81, 0.21, 0.64; (ss|ps) 1.69, 1.62, 1.39, 1.94 against 1.64, 1.43, 0.80, 1.58;
-//    (sd|pp) with 1.02-1.14 of its steps 0.54, 0.50, 0.16, 0.33 against 0.48, 0.38, 0.15, 0.32.  The
-//    mirror is kept up to 1.25 times the steps; beyond, (ps|ds) and (pd|ds) kinds are faster as they are.
-//  * L1 = L3 = 0: the first class's ket (s L4) recurs at D and comes in groups of 64 rows, worth about a
-//    quarter of the steps ((ss|sd) 0.61 and 0.97 ms with 1.22 of the steps of (sd|ss), 1.01 and 1.64) if
-//    its fewer, longer units still fill the device's 24 waves per CU three times; with fewer, the last
-//    ones run alone ((ss|sp) 1.47 against 0.82 ms at 16500 units of equal steps, 1.98 against 1.71 at
-//    13000, but 1.98 against 2.25 at 20700 and 1.84 against 2.27 at 83000).
-bool first_orientation(int L1, int L3, double steps_c, double steps_m, int nunits)
-{
-    if (L1 < L3) return 1.25 * steps_c < steps_m;
-    if (L1 == 0) return nunits >= 3 * 24 * S.num_cu ? steps_c <= 1.25 * steps_m : 1.05 * steps_c < steps_m;
-    return steps_c <= steps_m;
-}
-
 // lsjk_exchange: workspace, unit lists, mirror-class choices, the launches on the library stream.
 static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, const double* D24_dev, int D24symm,
                           int nterm, const double* scales, const double* omegas, float thresp, float thredp,
@@ -2260,43 +2382,43 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
             // choice; the autotuner times both (twice each, on the library stream,
             // into a scratch K) and keeps the faster.  A class that is its own mirror takes the row
             // triangle instead.
-            if (symmode && !tune && !orient && ew.n > 0 && !o.graph) {
-                std::map<int, int> pick;
+            auto* w12 = const_cast<lsjk_pairlist*>(pl12);
+            auto* w34 = const_cast<lsjk_pairlist*>(pl34);
+            // The classes with work, as (L1 L2 | L3 L4): f(class).  In the
+            // symmetric mode a mirror pair's class that `orient` stores (else the one of the lower
+            // index; both classes of a pair never run together), or of all pairs the lower (`both`).
+            auto for_classes = [&](bool both, auto&& f) {
                 for (int L1 = 0; L1 <= b1->maxL; L1++)
-                    for (int L2 = 0; L2 <= b2->maxL; L2++)
-                        for (int L3 = 0; L3 <= b3->maxL; L3++)
+                    for (int L3 = 0; L3 <= b3->maxL; L3++)
+                        for (int L2 = 0; L2 <= b2->maxL; L2++)
                             for (int L4 = 0; L4 <= b4->maxL; L4++) {
+                                if (pl12->h_rows[L1][L2].empty() || pl34->h_rows[L3][L4].empty()) continue;
                                 const int c = kcount_index(L1, L2, L3, L4), m = kcount_index(L3, L4, L1, L2);
-                                if (c >= m) continue;
-                                if (pl12->h_rows[L1][L2].empty() || pl12->h_rows[L3][L4].empty()) {
-                                    pick[c] = pick[m] = c;
-                                    continue;
+                                if (symmode && c != m) {
+                                    const auto it = orient && !both ? orient->find(c) : std::map<int, int>::const_iterator();
+                                    const int pick = (orient && !both && it != orient->end()) ? it->second : std::min(c, m);
+                                    if (pick != c) continue;
                                 }
-                                // both planned, the one that runs ordered and uploaded; of the other the
-                                // steps and the count stay
-                                auto* pl = const_cast<lsjk_pairlist*>(pl12);
-                                KUnitPlan plan[2];
-                                std::pair<double, int> cost[2];
-                                bool planned[2] = {false, false};
-                                for (int q = 0; q < 2; q++) {
-                                    const int A = q ? L3 : L1, B = q ? L4 : L2, C = q ? L1 : L3, E = q ? L2 : L4;
-                                    const auto key = kunits_key(pl, A, B, C, E, false, thresp);
-                                    const auto known = pl->kcost_g.find(key);
-                                    if (known != pl->kcost_g.end()) {
-                                        cost[q] = known->second;
-                                        continue;
-                                    }
-                                    plan[q] = plan_kunits(pl, pl, A, B, C, E, false, thresp);
-                                    planned[q] = true;
-                                    cost[q] = {plan[q].total, (int)plan[q].v.size()};
-                                }
-                                const int q = first_orientation(L1, L3, cost[0].first, cost[1].first, cost[0].second) ? 0 : 1;
-                                pick[c] = pick[m] = q ? m : c;
-                                get_kunits_g(pl, pl, q ? L3 : L1, q ? L4 : L2, q ? L1 : L3, q ? L2 : L4, false, thresp, nullptr,
-                                             planned[q] ? &plan[q] : nullptr);
-                                pl->kcost_g[kunits_key(pl, q ? L1 : L3, q ? L2 : L4, q ? L3 : L1, q ? L4 : L2, false, thresp)] =
-                                    cost[1 - q];
+                                f(KClass{L1, L2, L3, L4, symmode && c == m});
                             }
+            };
+            std::vector<KUnitJob> jobs;
+            if (symmode && !tune && !orient && !o.graph) {
+                for_classes(true, [&](const KClass& k) {
+                    KUnitJob job;
+                    job.cls[0] = k;
+                    job.cls[1] = KClass{k.L3, k.L4, k.L1, k.L2, false};
+                    job.n = k.tri ? 1 : 2;
+                    jobs.push_back(std::move(job));
+                });
+                make_kunits(w12, w34, jobs, thresp);
+                std::map<int, int> pick;
+                for (const auto& job : jobs) {
+                    if (job.n != 2) continue;
+                    const KClass& k = job.cls[0];
+                    const int c = kcount_index(k.L1, k.L2, k.L3, k.L4), m = kcount_index(k.L3, k.L4, k.L1, k.L2);
+                    pick[c] = pick[m] = job.chosen ? m : c;
+                }
                 orient = &(ocache[okey] = pick);
             }
             if (tune) {
@@ -2344,30 +2466,23 @@ static void exchange_call(const lsjk_pairlist* pl12, const lsjk_pairlist* pl34, 
                             }
                 orient = &(ocache[okey] = tuned);
             }
+            // the lists that are missing still, together
+            jobs.clear();
+            for_classes(false, [&](const KClass& k) {
+                if (w12->kunits_g.count(kunits_key(w34, k, thresp))) return;
+                KUnitJob job;
+                job.cls[0] = k;
+                jobs.push_back(std::move(job));
+            });
+            make_kunits(w12, w34, jobs, thresp);
             std::vector<KL> kls;
-            for (int L1 = 0; L1 <= b1->maxL; L1++)
-                for (int L3 = 0; L3 <= b3->maxL; L3++)
-                    for (int L2 = 0; L2 <= b2->maxL; L2++)
-                        for (int L4 = 0; L4 <= b4->maxL; L4++) {
-                            bool tri = false;
-                            if (symmode) {
-                                const int c = kcount_index(L1, L2, L3, L4), m = kcount_index(L3, L4, L1, L2);
-                                if (c == m) {
-                                    tri = true;
-                                } else {
-                                    // the stored choice, else the class of the lower index (both
-                                    // classes of a pair never run together)
-                                    const auto it = orient ? orient->find(c) : std::map<int, int>::const_iterator();
-                                    const int pick = (orient && it != orient->end()) ? it->second : std::min(c, m);
-                                    if (pick != c) continue;
-                                }
-                            }
-                            KL k;
-                            if (!make_kl(L1, L2, L3, L4, tri, K13_dev, k)) continue;
-                            // evaluated for the mirror class too: its diagonal blocks are the transposes
-                            k.ka.mirror_diag = (symmode && !tri) ? 1 : 0;
-                            kls.push_back(k);
-                        }
+            for_classes(false, [&](const KClass& c) {
+                KL k;
+                if (!make_kl(c.L1, c.L2, c.L3, c.L4, c.tri, K13_dev, k)) return;
+                // evaluated for the mirror class too: its diagonal blocks are the transposes
+                k.ka.mirror_diag = (symmode && !c.tri) ? 1 : 0;
+                kls.push_back(k);
+            });
             // heaviest classes first (estimated cost)
             std::stable_sort(kls.begin(), kls.end(), [](const KL& a, const KL& b) { return a.cost > b.cost; });
             fo.begin();
