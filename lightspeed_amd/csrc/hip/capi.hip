@@ -1101,124 +1101,122 @@ KUnitPlan plan_kunits(lsjk_pairlist* pl12, lsjk_pairlist* pl34, const KClass& k,
     const bool tri = k.tri;
     const int gsize = kgroup_for(pl34, L3, L4);
     KUnitPlan plan;
+    const auto& rows1 = pl12->h_rows[L1][L2];
+    const auto& G34 = get_kgroups(pl34, L3, L4, gsize);
+    const auto& G12 = get_kgroups(pl12, L1, L2, kgroup_for(pl12, L1, L2));  // its row order only
+    // the class's unit-split target: autotuned (this list on both sides) or the default
+    long long kKUnitsTarget = kKUnitsTargetDefault;
+    if (pl12 == pl34) {
+        auto ks = pl12->ksplit.find(kcount_index_host(L1, L2, L3, L4));
+        if (ks != pl12->ksplit.end()) kKUnitsTarget = ks->second;
+    }
+    const auto& mrank = get_mrank(pl12);
+    const int m12 = pl12->kmaxL2 + 1;
+    // chunk bounds per group, and the smallest rank of each group (triangle mode)
+    auto& v = plan.v;
+    double& total = plan.total;
+    for (int i1 : G12.order) {
+        const int r1 = rows1[i1];
+        const int a0 = pl12->h_row_start[(size_t)r1 * m12 + L2], a1 = pl12->h_row_start[(size_t)r1 * m12 + L2 + 1];
+        // bounds are sorted descending: the partners with b12 >= x are a prefix
+        auto npass = [&](double x) {
+            int lo = a0, hi = a1;
+            while (lo < hi) {
+                const int mid = (lo + hi) / 2;
+                if ((double)pl12->h_eb[mid] >= x) lo = mid + 1; else hi = mid;
+            }
+            return (long long)(lo - a0);
+        };
+        const int rank1 = tri ? mrank[r1] : -1;
+        // a batch list pairs a row only with the groups of its own molecule
+        const int g0 = pl34->nmol > 0 ? G34.mol_grp[pl12->h_mol[r1]] : 0;
+        const int g1 = pl34->nmol > 0 ? G34.mol_grp[pl12->h_mol[r1] + 1] : G34.ngroup;
+        for (int g = g0; g < g1; g++) {
+            if (tri) {
+                int rmax = -1;
+                for (int t = 0; t < gsize; t++) {
+                    const int rk = G34.grp_rank[(size_t)g * gsize + t];
+                    if (rk != std::numeric_limits<int>::max()) rmax = std::max(rmax, rk);
+                }
+                if (rmax < rank1) continue;
+            }
+            long long c = 0;
+            for (int s = G34.grp_slot[g]; s < G34.grp_slot[g + 1]; s += 64)
+                c += npass((double)thresp / (double)G34.chunk_b[s / 64]);
+            v.push_back({c, KUnitG{i1, g, rank1, 0}});
+            total += (double)c;
+        }
+    }
+    // classes with few (row, group) pairs: split the groups' chunk ranges so that the launch
+    // has enough waves to fill the device
+    long long nchunk = 0;
+    for (const auto& x : v) nchunk += (G34.grp_slot[x.second.g + 1] - G34.grp_slot[x.second.g]) / 64;
+    const int per = (int)std::max<long long>(1, std::min<long long>(
+        (long long)(v.size() >= kKUnitsTarget ? 1 << 15 : (nchunk + kKUnitsTarget - 1) / kKUnitsTarget), 1 << 15));
     {
-        const auto& rows1 = pl12->h_rows[L1][L2];
-        const auto& G34 = get_kgroups(pl34, L3, L4, gsize);
-        const auto& G12 = get_kgroups(pl12, L1, L2, kgroup_for(pl12, L1, L2));  // its row order only
-        // the class's unit-split target: autotuned (this list on both sides) or the default
-        long long kKUnitsTarget = kKUnitsTargetDefault;
-        if (pl12 == pl34) {
-            auto ks = pl12->ksplit.find(kcount_index_host(L1, L2, L3, L4));
-            if (ks != pl12->ksplit.end()) kKUnitsTarget = ks->second;
-        }
-        const auto& mrank = get_mrank(pl12);
-        const int m12 = pl12->kmaxL2 + 1;
-        // chunk bounds per group, and the smallest rank of each group (triangle mode)
-        auto& v = plan.v;
-        double& total = plan.total;
-        for (int i1 : G12.order) {
-            const int r1 = rows1[i1];
+        std::vector<std::pair<long long, KUnitG>> w;
+        w.reserve(v.size());
+        for (const auto& x : v) {
+            const int g = x.second.g;
+            const int nch = (G34.grp_slot[g + 1] - G34.grp_slot[g]) / 64;
+            if (nch >= (1 << 15)) throw LsjkError(LSJK_E_UNSUPPORTED, "lsjk: exchange ket group too large");
+            const int r1 = rows1[x.second.i1];
             const int a0 = pl12->h_row_start[(size_t)r1 * m12 + L2], a1 = pl12->h_row_start[(size_t)r1 * m12 + L2 + 1];
-            // bounds are sorted descending: the partners with b12 >= x are a prefix
-            auto npass = [&](double x) {
-                int lo = a0, hi = a1;
-                while (lo < hi) {
-                    const int mid = (lo + hi) / 2;
-                    if ((double)pl12->h_eb[mid] >= x) lo = mid + 1; else hi = mid;
-                }
-                return (long long)(lo - a0);
-            };
-            const int rank1 = tri ? mrank[r1] : -1;
-            // a batch list pairs a row only with the groups of its own molecule
-            const int g0 = pl34->nmol > 0 ? G34.mol_grp[pl12->h_mol[r1]] : 0;
-            const int g1 = pl34->nmol > 0 ? G34.mol_grp[pl12->h_mol[r1] + 1] : G34.ngroup;
-            for (int g = g0; g < g1; g++) {
-                if (tri) {
-                    int rmax = -1;
-                    for (int t = 0; t < gsize; t++) {
-                        const int rk = G34.grp_rank[(size_t)g * gsize + t];
-                        if (rk != std::numeric_limits<int>::max()) rmax = std::max(rmax, rk);
-                    }
-                    if (rmax < rank1) continue;
-                }
+            // equal pieces of at most `per` chunks
+            const int npiece = (nch + per - 1) / per, step = (nch + npiece - 1) / npiece;
+            for (int c0 = 0; c0 < nch; c0 += step) {
+                const int nc = std::min(step, nch - c0);
                 long long c = 0;
-                for (int s = G34.grp_slot[g]; s < G34.grp_slot[g + 1]; s += 64)
-                    c += npass((double)thresp / (double)G34.chunk_b[s / 64]);
-                v.push_back({c, KUnitG{i1, g, rank1, 0}});
-                total += (double)c;
+                if (step < nch)
+                    for (int k = 0; k < nc; k++) {
+                        const double x0 = (double)thresp / (double)G34.chunk_b[G34.grp_slot[g] / 64 + c0 + k];
+                        c += (long long)(std::partition_point(pl12->h_eb.begin() + a0, pl12->h_eb.begin() + a1,
+                                                              [&](float b) { return (double)b >= x0; }) -
+                                         (pl12->h_eb.begin() + a0));
+                    }
+                else
+                    c = x.first;
+                KUnitG uu = x.second;
+                uu.crange = c0 | (nc << 16);
+                w.push_back({c, uu});
             }
         }
-        // classes with few (row, group) pairs: split the groups' chunk ranges so that the launch
-        // has enough waves to fill the device
-        long long nchunk = 0;
-        for (const auto& x : v) nchunk += (G34.grp_slot[x.second.g + 1] - G34.grp_slot[x.second.g]) / 64;
-        const int per = (int)std::max<long long>(1, std::min<long long>(
-            (long long)(v.size() >= kKUnitsTarget ? 1 << 15 : (nchunk + kKUnitsTarget - 1) / kKUnitsTarget), 1 << 15));
-        {
-            std::vector<std::pair<long long, KUnitG>> w;
-            w.reserve(v.size());
-            for (const auto& x : v) {
-                const int g = x.second.g;
-                const int nch = (G34.grp_slot[g + 1] - G34.grp_slot[g]) / 64;
-                if (nch >= (1 << 15)) throw LsjkError(LSJK_E_UNSUPPORTED, "lsjk: exchange ket group too large");
-                const int r1 = rows1[x.second.i1];
-                const int a0 = pl12->h_row_start[(size_t)r1 * m12 + L2], a1 = pl12->h_row_start[(size_t)r1 * m12 + L2 + 1];
-                // equal pieces of at most `per` chunks
-                const int npiece = (nch + per - 1) / per, step = (nch + npiece - 1) / npiece;
-                for (int c0 = 0; c0 < nch; c0 += step) {
-                    const int nc = std::min(step, nch - c0);
-                    long long c = 0;
-                    if (step < nch)
-                        for (int k = 0; k < nc; k++) {
-                            const double x0 = (double)thresp / (double)G34.chunk_b[G34.grp_slot[g] / 64 + c0 + k];
-                            c += (long long)(std::partition_point(pl12->h_eb.begin() + a0, pl12->h_eb.begin() + a1,
-                                                                  [&](float b) { return (double)b >= x0; }) -
-                                             (pl12->h_eb.begin() + a0));
-                        }
-                    else
-                        c = x.first;
-                    KUnitG uu = x.second;
-                    uu.crange = c0 | (nc << 16);
-                    w.push_back({c, uu});
-                }
-            }
-            v.swap(w);
+        v.swap(w);
+    }
+    // still few units (heavy classes: few rows, costly quartets): split each unit's walk over
+    // its bra row's partners into pieces, so that the launch has enough waves; each piece adds
+    // its part of the same K block
+    if (v.size() < (size_t)kKUnitsTarget / 4) {
+        long long walk_total = 0;
+        std::vector<int> walk(v.size());
+        for (size_t q = 0; q < v.size(); q++) {
+            const KUnitG& x = v[q].second;
+            const int r1 = rows1[x.i1];
+            const int a0 = pl12->h_row_start[(size_t)r1 * m12 + L2], a1 = pl12->h_row_start[(size_t)r1 * m12 + L2 + 1];
+            // partners that can pass with the unit's first (largest-bound) chunk
+            const double x0 = (double)thresp / (double)G34.chunk_b[G34.grp_slot[x.g] / 64 + (x.crange & 0xffff)];
+            walk[q] = (a1 - a0 >= 0xffff) ? 0 : (int)(std::partition_point(pl12->h_eb.begin() + a0, pl12->h_eb.begin() + a1,
+                                                                            [&](float b) { return (double)b >= x0; }) -
+                                                       (pl12->h_eb.begin() + a0));
+            walk_total += walk[q];
         }
-        // still few units (heavy classes: few rows, costly quartets): split each unit's walk over
-        // its bra row's partners into pieces, so that the launch has enough waves; each piece adds
-        // its part of the same K block
-        if (v.size() < (size_t)kKUnitsTarget / 4) {
-            long long walk_total = 0;
-            std::vector<int> walk(v.size());
-            for (size_t q = 0; q < v.size(); q++) {
-                const KUnitG& x = v[q].second;
-                const int r1 = rows1[x.i1];
-                const int a0 = pl12->h_row_start[(size_t)r1 * m12 + L2], a1 = pl12->h_row_start[(size_t)r1 * m12 + L2 + 1];
-                // partners that can pass with the unit's first (largest-bound) chunk
-                const double x0 = (double)thresp / (double)G34.chunk_b[G34.grp_slot[x.g] / 64 + (x.crange & 0xffff)];
-                walk[q] = (a1 - a0 >= 0xffff) ? 0 : (int)(std::partition_point(pl12->h_eb.begin() + a0, pl12->h_eb.begin() + a1,
-                                                                                [&](float b) { return (double)b >= x0; }) -
-                                                           (pl12->h_eb.begin() + a0));
-                walk_total += walk[q];
+        const long long piece = std::max<long long>(1, (walk_total + kKUnitsTarget / 4 - 1) / (kKUnitsTarget / 4));
+        std::vector<std::pair<long long, KUnitG>> w;
+        for (size_t q = 0; q < v.size(); q++) {
+            const int n = walk[q];
+            if (n <= piece) {
+                w.push_back(v[q]);
+                continue;
             }
-            const long long piece = std::max<long long>(1, (walk_total + kKUnitsTarget / 4 - 1) / (kKUnitsTarget / 4));
-            std::vector<std::pair<long long, KUnitG>> w;
-            for (size_t q = 0; q < v.size(); q++) {
-                const int n = walk[q];
-                if (n <= piece) {
-                    w.push_back(v[q]);
-                    continue;
-                }
-                const int np = (int)((n + piece - 1) / piece), step = (n + np - 1) / np;
-                for (int p0 = 0; p0 < n; p0 += step) {
-                    KUnitG uu = v[q].second;
-                    // the last piece runs to the end of the row's partners (the stop test ends it)
-                    uu.prange = p0 | ((p0 + step < n ? step : 0) << 16);
-                    w.push_back({std::max<long long>(1, v[q].first / np), uu});
-                }
+            const int np = (int)((n + piece - 1) / piece), step = (n + np - 1) / np;
+            for (int p0 = 0; p0 < n; p0 += step) {
+                KUnitG uu = v[q].second;
+                // the last piece runs to the end of the row's partners (the stop test ends it)
+                uu.prange = p0 | ((p0 + step < n ? step : 0) << 16);
+                w.push_back({std::max<long long>(1, v[q].first / np), uu});
             }
-            v.swap(w);
         }
+        v.swap(w);
     }
     return plan;
 }
@@ -1228,57 +1226,55 @@ std::vector<lsjk::KUnitG> order_kunits(lsjk_pairlist* pl12, const KClass& k, KUn
 {
     using lsjk::KUnitG;
     std::vector<KUnitG> u;
-    {
-        auto& v = plan.v;
-        const auto& rows1 = pl12->h_rows[k.L1][k.L2];
-        const auto& G12 = get_kgroups(pl12, k.L1, k.L2, kgroup_for(pl12, k.L1, k.L2));  // its row order only
-        auto bucket = [](long long c) { return c > 0 ? 64 - __builtin_clzll((unsigned long long)c) : 0; };
-        std::stable_sort(v.begin(), v.end(), [&](const std::pair<long long, KUnitG>& a,
-                                                 const std::pair<long long, KUnitG>& b) {
-            return bucket(a.first) > bucket(b.first);
-        });
-        // Workgroup w (units kKWaves w .. kKWaves w + kKWaves - 1) runs on XCD w % 8.  Each bucket is
-        // cut into 8 contiguous ranges (bands of neighbouring bra rows); workgroups take kKWaves
-        // consecutive units of range w % 8.  Inside a range the units go in tiles of kKTileRows
-        // rows x kKTileGroups ket groups (spatial order both ways), so that an XCD's L2 holds the
-        // tile's block of the K view D: rows = the tile's bra partners, columns = the groups'
-        // partners.  Inside a tile the units are sorted by cost, so the waves of one workgroup
-        // (which holds its slots until its last wave ends) cost about the same.  Units that do not
-        // fill a whole workgroup of their range go at the bucket's end.
-        constexpr size_t W = lsjk::kKWaves;
-        std::vector<int> pos1(rows1.size(), 0);  // spatial position of each bra row
-        for (size_t q = 0; q < G12.order.size(); q++) pos1[G12.order[q]] = (int)q;
-        u.reserve(v.size());
-        for (size_t s0 = 0; s0 < v.size();) {
-            size_t s1 = s0;
-            while (s1 < v.size() && bucket(v[s1].first) == bucket(v[s0].first)) s1++;
-            const size_t n = s1 - s0, per = ((n + 7) / 8 + W - 1) / W * W;
-            for (size_t x = 0; x < 8; x++) {
-                const size_t b = std::min(n, x * per), e = std::min(n, (x + 1) * per);
-                std::stable_sort(v.begin() + s0 + b, v.begin() + s0 + e,
-                                 [&](const std::pair<long long, KUnitG>& a, const std::pair<long long, KUnitG>& c) {
-                                     const int ra = pos1[a.second.i1] / kKTileRows, rc = pos1[c.second.i1] / kKTileRows;
-                                     if (ra != rc) return ra < rc;
-                                     const int ga = a.second.g / kKTileGroups, gc = c.second.g / kKTileGroups;
-                                     if (ga != gc) return ga < gc;
-                                     if (a.first != c.first) return a.first > c.first;
-                                     if (pos1[a.second.i1] != pos1[c.second.i1]) return pos1[a.second.i1] < pos1[c.second.i1];
-                                     return a.second.g < c.second.g;
-                                 });
-            }
-            std::vector<KUnitG> rest;
-            for (size_t k = 0; k < per; k += W)
-                for (size_t x = 0; x < 8; x++) {
-                    const size_t b = x * per + k, e = std::min(std::min(n, (x + 1) * per), b + W);
-                    if (b >= e) continue;
-                    for (size_t q = b; q < e; q++) (e - b == W ? u : rest).push_back(v[s0 + q].second);
-                }
-            u.insert(u.end(), rest.begin(), rest.end());
-            s0 = s1;
+    auto& v = plan.v;
+    const auto& rows1 = pl12->h_rows[k.L1][k.L2];
+    const auto& G12 = get_kgroups(pl12, k.L1, k.L2, kgroup_for(pl12, k.L1, k.L2));  // its row order only
+    auto bucket = [](long long c) { return c > 0 ? 64 - __builtin_clzll((unsigned long long)c) : 0; };
+    std::stable_sort(v.begin(), v.end(), [&](const std::pair<long long, KUnitG>& a,
+                                             const std::pair<long long, KUnitG>& b) {
+        return bucket(a.first) > bucket(b.first);
+    });
+    // Workgroup w (units kKWaves w .. kKWaves w + kKWaves - 1) runs on XCD w % 8.  Each bucket is
+    // cut into 8 contiguous ranges (bands of neighbouring bra rows); workgroups take kKWaves
+    // consecutive units of range w % 8.  Inside a range the units go in tiles of kKTileRows
+    // rows x kKTileGroups ket groups (spatial order both ways), so that an XCD's L2 holds the
+    // tile's block of the K view D: rows = the tile's bra partners, columns = the groups'
+    // partners.  Inside a tile the units are sorted by cost, so the waves of one workgroup
+    // (which holds its slots until its last wave ends) cost about the same.  Units that do not
+    // fill a whole workgroup of their range go at the bucket's end.
+    constexpr size_t W = lsjk::kKWaves;
+    std::vector<int> pos1(rows1.size(), 0);  // spatial position of each bra row
+    for (size_t q = 0; q < G12.order.size(); q++) pos1[G12.order[q]] = (int)q;
+    u.reserve(v.size());
+    for (size_t s0 = 0; s0 < v.size();) {
+        size_t s1 = s0;
+        while (s1 < v.size() && bucket(v[s1].first) == bucket(v[s0].first)) s1++;
+        const size_t n = s1 - s0, per = ((n + 7) / 8 + W - 1) / W * W;
+        for (size_t x = 0; x < 8; x++) {
+            const size_t b = std::min(n, x * per), e = std::min(n, (x + 1) * per);
+            std::stable_sort(v.begin() + s0 + b, v.begin() + s0 + e,
+                             [&](const std::pair<long long, KUnitG>& a, const std::pair<long long, KUnitG>& c) {
+                                 const int ra = pos1[a.second.i1] / kKTileRows, rc = pos1[c.second.i1] / kKTileRows;
+                                 if (ra != rc) return ra < rc;
+                                 const int ga = a.second.g / kKTileGroups, gc = c.second.g / kKTileGroups;
+                                 if (ga != gc) return ga < gc;
+                                 if (a.first != c.first) return a.first > c.first;
+                                 if (pos1[a.second.i1] != pos1[c.second.i1]) return pos1[a.second.i1] < pos1[c.second.i1];
+                                 return a.second.g < c.second.g;
+                             });
         }
-        if (u.size() > (size_t)std::numeric_limits<int>::max() / lsjk::kKWaves)
-            throw LsjkError(LSJK_E_UNSUPPORTED, "lsjk: too many exchange work units");
+        std::vector<KUnitG> rest;
+        for (size_t k = 0; k < per; k += W)
+            for (size_t x = 0; x < 8; x++) {
+                const size_t b = x * per + k, e = std::min(std::min(n, (x + 1) * per), b + W);
+                if (b >= e) continue;
+                for (size_t q = b; q < e; q++) (e - b == W ? u : rest).push_back(v[s0 + q].second);
+            }
+        u.insert(u.end(), rest.begin(), rest.end());
+        s0 = s1;
     }
+    if (u.size() > (size_t)std::numeric_limits<int>::max() / lsjk::kKWaves)
+        throw LsjkError(LSJK_E_UNSUPPORTED, "lsjk: too many exchange work units");
     return u;
 }
 
