@@ -1,16 +1,18 @@
 // Exchange (K) build: small helper kernels (D block maxima, fills, copies) and the class
-// dispatcher; the quartet kernels are in exchange_impl.hpp (instantiated by exchange_k<L1><L2>.hip).
+// dispatcher; the quartet kernels are in exchange_impl.hpp (instantiated by exchange_k<L1><L2>.hip and exchange_kt<L1><L2>.hip).
 #include "internal.hpp"
 #include "kernels.hpp"
 
 namespace lsjk {
 
-template <int L1, int L2>
+template <int L1, int L2, bool BARE>
 void launch_k_ket_l12(int L3, int L4, int route, const KArgs& a, const KGroups& kg, const KUnitG* units, int nunits,
                       hipStream_t s);
 #define LSJK_KET_EXTERN(X, Y)                                                                                \
-    extern template void launch_k_ket_l12<X, Y>(int, int, int, const KArgs&, const KGroups&, const KUnitG*, int, \
-                                                hipStream_t);
+    extern template void launch_k_ket_l12<X, Y, true>(int, int, int, const KArgs&, const KGroups&, const KUnitG*, \
+                                                      int, hipStream_t);                                     \
+    extern template void launch_k_ket_l12<X, Y, false>(int, int, int, const KArgs&, const KGroups&, const KUnitG*, \
+                                                       int, hipStream_t);
 LSJK_KET_EXTERN(0, 0) LSJK_KET_EXTERN(0, 1) LSJK_KET_EXTERN(0, 2)
 LSJK_KET_EXTERN(1, 0) LSJK_KET_EXTERN(1, 1) LSJK_KET_EXTERN(1, 2)
 LSJK_KET_EXTERN(2, 0) LSJK_KET_EXTERN(2, 1) LSJK_KET_EXTERN(2, 2)
@@ -288,7 +290,10 @@ void launch_k_ket(int L1, int L2, int L3, int L4, int route, const KArgs& a, con
 {
     if (nunits <= 0) return;
 #define CASE(X, Y) \
-    if (L1 == X && L2 == Y) return launch_k_ket_l12<X, Y>(L3, L4, route, a, kg, units, nunits, s);
+    if (L1 == X && L2 == Y) {                                                                                \
+        if (a.ew.plain) return launch_k_ket_l12<X, Y, true>(L3, L4, route, a, kg, units, nunits, s);         \
+        return launch_k_ket_l12<X, Y, false>(L3, L4, route, a, kg, units, nunits, s);                        \
+    }
     CASE(0, 0) CASE(0, 1) CASE(0, 2) CASE(1, 0) CASE(1, 1) CASE(1, 2) CASE(2, 0) CASE(2, 1) CASE(2, 2)
 #undef CASE
 }

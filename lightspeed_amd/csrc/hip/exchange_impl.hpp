@@ -1,6 +1,9 @@
 // Exchange (K) quartet kernel templates, shared by the translation units that instantiate them
-// (exchange_k<L1><L2>.hip: one per bra row and partner angular momentum, so the 324 instantiations
-// compile in parallel).
+// (exchange_k<L1><L2>.hip for one bare 1/r term and exchange_kt<L1><L2>.hip for any terms: one per bra
+// row and partner angular momentum, so the 324 instantiations compile in parallel, and a process
+// loads the code of the operators it uses: a unit's code goes to the device at the first launch
+// from it, about 2.8 ms per MB.  The first exchange call of a process with one term, s to d
+// functions, took 24.5 ms with both in one unit).
 // Direct exchange (K) build on gfx950.
 //
 // K13 += sum_{2,4} (12|34) D24 over the quartets the reference evaluates
@@ -811,15 +814,15 @@ __global__ __launch_bounds__(64 * kKWaves) void k_unit_mag(KArgs a, KGroups kg, 
 }
 
 // Launch of one K build class with bra row and partner angular momenta L1, L2 (instantiated in
-// exchange_k<L1><L2>.hip).
-template <int L1, int L2>
+// exchange_k<L1><L2>.hip, exchange_kt<L1><L2>.hip).
+template <int L1, int L2, bool BARE>
 void launch_k_ket_l12(int L3, int L4, int route, const KArgs& a, const KGroups& kg, const KUnitG* units, int nunits,
                       hipStream_t s)
 {
     dim3 grid((unsigned)((nunits + kKWaves - 1) / kKWaves)), block(64 * kKWaves);
 #define ONE(C, D, R)                                                                                \
     {                                                                                               \
-        auto* kernel = a.ew.plain ? k_ket<L1, L2, C, D, R, true> : k_ket<L1, L2, C, D, R, false>;   \
+        auto* kernel = k_ket<L1, L2, C, D, R, BARE>;                                                \
         const size_t lds = KKetLds<L1, L2, C, D, R>::bytes(a.rys, kg.gsize);                        \
         if (lds > kMaxLdsPerGroup || lds != kket_lds_bytes(a.rys, L1, L2, C, D, R, kg.gsize))      \
             throw std::runtime_error("lsjk: k_ket LDS request too large or inconsistent");         \

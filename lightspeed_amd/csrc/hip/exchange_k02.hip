@@ -1,6 +1,6 @@
-// Instantiations of the K build kernels with bra row and partner angular momenta 0 and 2.
+// Instantiations of the K build kernels with bra row and partner angular momenta 0 and 2, one bare 1/r term.
 #include "exchange_impl.hpp"
 
 namespace lsjk {
-template void launch_k_ket_l12<0, 2>(int, int, int, const KArgs&, const KGroups&, const KUnitG*, int, hipStream_t);
+template void launch_k_ket_l12<0, 2, true>(int, int, int, const KArgs&, const KGroups&, const KUnitG*, int, hipStream_t);
 }  // namespace lsjk

@@ -1,6 +1,6 @@
-// Instantiations of the K build kernels with bra row and partner angular momenta 2 and 1.
+// Instantiations of the K build kernels with bra row and partner angular momenta 2 and 1, one bare 1/r term.
 #include "exchange_impl.hpp"
 
 namespace lsjk {
-template void launch_k_ket_l12<2, 1>(int, int, int, const KArgs&, const KGroups&, const KUnitG*, int, hipStream_t);
+template void launch_k_ket_l12<2, 1, true>(int, int, int, const KArgs&, const KGroups&, const KUnitG*, int, hipStream_t);
 }  // namespace lsjk

@@ -19,6 +19,7 @@ constexpr int kHostToDevice = 1, kDeviceToHost = 2;
 
 std::map<void*, size_t> live;
 std::map<const void*, std::string> kernels;  // host stub of a kernel -> its name
+std::map<const void*, std::string> units;    // code object -> the names of its kernels, a line each
 std::vector<std::string> launched;  // name and shape of each launch
 long fail_at = -1;  // the allocation after this many more fails, and its retries (same size)
 size_t failing = 0;
@@ -61,9 +62,10 @@ extern "C" {
 
 void** __hipRegisterFatBinary(const void*) { return new void*(nullptr); }
 void __hipUnregisterFatBinary(void**) {}
-void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*)
+void __hipRegisterFunction(void** unit, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*)
 {
     kernels[host] = name;
+    units[unit] += std::string(name) + "\n";
 }
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 int __hipPushCallConfiguration(Dim3 grid, Dim3 block, size_t lds, void* stream)
@@ -166,6 +168,13 @@ const char* stub_launch_log(long first)
     all.clear();
     for (size_t i = first; i < launched.size(); i++) all += launched[i] + "\n";
     return all.c_str();
+}
+// the kernels of code object i (what the first launch of one of them loads)
+const char* stub_unit(long i)
+{
+    for (const auto& u : units)
+        if (i-- == 0) return u.second.c_str();
+    return nullptr;
 }
 // launches so far of kernels with `part` in their (mangled) names
 long stub_launches(const char* part)

@@ -35,6 +35,8 @@ class Env:
             getattr(self.stub, f).restype = ctypes.c_long
         self.stub.stub_launch_log.restype = ctypes.c_char_p
         self.stub.stub_launch_log.argtypes = [ctypes.c_long]
+        self.stub.stub_unit.restype = ctypes.c_char_p
+        self.stub.stub_unit.argtypes = [ctypes.c_long]
         self.stub.stub_fail_at.argtypes = [ctypes.c_long]
         self.stub.stub_answer.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
         sys.path[:0] = [ROOT, HERE]
@@ -313,6 +315,18 @@ def one_electron_streams(E):
     assert waits(lambda: I.overlap(E.res, pl)) == waits(lambda: I.kinetic(E.res, pl)) == 0
     assert V(1) == V(9) == 0
     assert V(100000) > 0
+
+
+@case
+def exchange_code_by_operator(E):
+    """The exchange kernels of one 1/r term and those of any terms are in code objects of their own, so that
+    a process loads what it uses (k_ket's last template argument)."""
+    kinds = []
+    while E.stub.stub_unit(len(kinds)) is not None:
+        names = [k for k in E.stub.stub_unit(len(kinds)).decode().split() if "5k_ketI" in k]
+        kinds.append({k.split("5k_ketI")[1].split("EEEv")[0][-1] for k in names})
+    assert sum(1 for k in kinds if k == {"1"}) == sum(1 for k in kinds if k == {"0"}) == 9
+    assert all(len(k) <= 1 for k in kinds)
 
 
 @pytest.fixture(scope="module")
